@@ -225,7 +225,7 @@ def main():
     fold_ms, fold_launches = stages32["fold"]
     fold_avg_ms = fold_ms / max(1, fold_launches)
     achieved = fold_bytes / (fold_avg_ms * 1e-3) / 1e9
-    kname = "k_fold_chunks"
+    kname = "k_fold_sorted"
     traffic, traffic_src = measured_traffic(kname, S, n, k)
     result["roofline"] = {"kernel": kname, "bound": "hbm", "achieved": achieved,
                           "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,

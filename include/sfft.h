@@ -158,10 +158,11 @@ int sfft_plan_set_precision(sfft_plan *plan, sfft_precision precision);
 /* Fold schedule of a v1/v2 plan (no counterpart in the reference; it maps
  * src/computefourier-1.0-2.0.cc:222-275 onto the GPU).  fold_mode 0: one
  * workgroup per (signal, loop) folds into LDS and transforms there; 1: a
- * signal-major streamed fold with stream_blocks resident workgroups (0: twice
- * the CU count), then the bucket FFTs, which for v2 store the buckets by
+ * fold that walks the taps of all loops in address order, then the bucket
+ * FFTs, which for v2 store the buckets by
  * alias row so that estimation reads them contiguously; 2: as 1 with the
- * buckets in natural order.  Schedules never change results.
+ * buckets in natural order.  stream_blocks is accepted and reported back;
+ * the folds size their own grids.  Schedules never change results.
  * Returns 0 or -1. */
 int sfft_plan_set_schedule(sfft_plan *plan, int fold_mode, int stream_blocks);
 int sfft_plan_get_schedule(const sfft_plan *plan, int *fold_mode, int *stream_blocks);

@@ -236,7 +236,7 @@ int64_t Plan::output_capacity() const
 int64_t Plan::plan_bytes() const
 {
   return (int64_t)(taps_loc.bytes + taps_est.bytes + tapsT_loc32.bytes +
-                   tapsT_est32.bytes + win_loc.bytes + win_est.bytes +
+                   tapsT_est32.bytes + tapsT_loc.bytes + tapsT_est.bytes + win_loc.bytes + win_est.bytes +
                    tw64.bytes + tw32.bytes + v3_time1.bytes + v3_time2.bytes +
                    v3_freq1.bytes + v3_freq2.bytes);
 }
@@ -377,9 +377,8 @@ Plan *make_plan(int n, int k, sfft_version v)
     P->own_stream = true;
     return P;
   }
-  // tuning overrides for experiments: fold schedule and its resident blocks
+  // tuning override for experiments: the fold schedule
   if (const char *e = std::getenv("SFFT_FOLD_MODE")) P->fold_mode = std::min(2, std::max(0, std::atoi(e)));
-  if (const char *e = std::getenv("SFFT_FOLD_BLOCKS")) P->stream_blocks = std::atoi(e);
   P->v12 = derive_v12(n, k, v == SFFT_VERSION_2);
   std::string why = check_v12(P->v12);
   if (!why.empty()) {
@@ -404,6 +403,8 @@ Plan *make_plan(int n, int k, sfft_version v)
             upload(P->taps_est, to_d2(fe.time, fe.time.size())) &&
             upload(P->tapsT_loc32, taps_by_bucket<float2>(fl.time, p.B_loc, P->tR_loc)) &&
             upload(P->tapsT_est32, taps_by_bucket<float2>(fe.time, p.B_est, P->tR_est)) &&
+            upload(P->tapsT_loc, taps_by_bucket<double2>(fl.time, p.B_loc, P->tR_loc)) &&
+            upload(P->tapsT_est, taps_by_bucket<double2>(fe.time, p.B_est, P->tR_est)) &&
             upload(P->win_loc, est_window(fl.freq, p.n, p.B_loc)) &&
             upload(P->win_est, est_window(fe.freq, p.n, p.B_est)) &&
             upload(P->tw64, to_d2(tw, tw.size())) &&
@@ -471,6 +472,8 @@ Plan *clone_plan(const Plan *src, Workspace *ws, hipStream_t stream)
   P->taps_est = src->taps_est;
   P->tapsT_loc32 = src->tapsT_loc32;
   P->tapsT_est32 = src->tapsT_est32;
+  P->tapsT_loc = src->tapsT_loc;
+  P->tapsT_est = src->tapsT_est;
   P->tR_loc = src->tR_loc;
   P->tR_est = src->tR_est;
   P->seg_rows = src->seg_rows;
@@ -501,6 +504,7 @@ void free_plan(Plan *P)
   if (P->stream && (P->own_stream || P->owns_tables)) (void)hipStreamSynchronize(P->stream);
   if (P->owns_tables) {
     DevBuf *bufs[] = {&P->taps_loc, &P->taps_est, &P->tapsT_loc32, &P->tapsT_est32,
+                      &P->tapsT_loc, &P->tapsT_est,
                       &P->win_loc, &P->win_est, &P->tw64, &P->tw32,
                       &P->v3_time1, &P->v3_time2, &P->v3_freq1, &P->v3_freq2};
     for (DevBuf *b : bufs) b->release();
@@ -980,6 +984,8 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   a.taps_est = P->taps_est.as<const double2>();
   a.tapsT_loc32 = P->tapsT_loc32.as<const float2>();
   a.tapsT_est32 = P->tapsT_est32.as<const float2>();
+  a.tapsT_loc = P->tapsT_loc.as<const double2>();
+  a.tapsT_est = P->tapsT_est.as<const double2>();
   a.tR_loc = P->tR_loc;
   a.tR_est = P->tR_est;
   a.seg_rows = P->seg_rows;
@@ -1021,13 +1027,6 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
                   p.W_comb % (n / p.B_est) == 0 && n / p.W_comb >= 64 &&
                   std::max(p.B_loc, p.B_est) <= (fp32 ? 2 : 1) * kMaxLdsFft64;
   P->last_rows_layout = a.rows_layout;
-  a.stream_blocks = P->stream_blocks;
-  if (a.stream_blocks <= 0) {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-      (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    a.stream_blocks = 2 * cus;  // 8 resident wavefronts per CU
-  }
 
   // an arena workspace creates no runtime objects: no timing events, no
   // second stream, no graphs
@@ -1130,8 +1129,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
     // batch of this shape; the workspace and staging addresses are part of
     // the key (kernel arguments and copy nodes hold them)
     const uint64_t key = (uint64_t)S | (uint64_t)fp32 << 32 | (uint64_t)want_sparse << 33 |
-                         (uint64_t)want_dense << 34 | (uint64_t)a.fold_mode << 35 |
-                         (uint64_t)a.stream_blocks << 36;
+                         (uint64_t)want_dense << 34 | (uint64_t)a.fold_mode << 35;
     const uint64_t sig = workspace_signature(*P->ws) ^
                          ((uint64_t)io.cap * 0x9e3779b97f4a7c15ull + (uint64_t)a.ref_conj);
     hipGraphExec_t ex = nullptr;

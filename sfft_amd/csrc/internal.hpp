@@ -188,7 +188,7 @@ struct Plan {
   V3Params v3;
   sfft_precision precision = SFFT_PRECISION_FP64;
   int fold_mode = 1;       // see k::V12Launch::fold_mode
-  int stream_blocks = 0;   // 0: derived from the CU count
+  int stream_blocks = 0;   // kept for sfft_plan_get_schedule; the folds size their own grids
   bool last_fp32 = false;  // precision of the buckets in ws_xsamp
   bool last_rows_layout = false;  // the last batch stored buckets by alias row
   bool ref_conj = true;
@@ -204,6 +204,7 @@ struct Plan {
   // v1/v2 device tables
   DevBuf taps_loc, taps_est;      // double2[w]
   DevBuf tapsT_loc32, tapsT_est32;  // float2[B * ceil(w/B)]: FP32 taps by bucket
+  DevBuf tapsT_loc, tapsT_est;      // double2[B * ceil(w/B)]: FP64 taps by bucket
   int tR_loc = 0, tR_est = 0;       // ceil(w/B) of each filter
   int seg_rows = 256;               // rows per chunk of the FP32 fold (sum order)
   DevBuf win_loc, win_est;        // double2[m+1]: freq[(n-d) mod n], d = -m/2..m/2
@@ -326,6 +327,7 @@ struct V12Launch {
   const double2 *taps_loc, *taps_est;
   // FP32 taps by bucket: tapsT[b * tR + k] = tap[b + k*B] (k < tR = ceil(w/B))
   const float2 *tapsT_loc32, *tapsT_est32;
+  const double2 *tapsT_loc, *tapsT_est;  // the FP64 taps likewise
   int tR_loc, tR_est;
   int seg_rows;    // rows per chunk of the FP32 fold (fixes its summation order)
   const double2 *win_loc, *win_est;
@@ -352,10 +354,9 @@ struct V12Launch {
   int64_t o_cap;            // sparse capacity per signal
   int64_t est_cap;          // upper bound of the located count per signal
   int fold_mode;            // 0: fused fold+FFT per (signal, loop) block;
-                            // 1: signal-major streamed fold, then bucket FFTs
-                            //    (alias-row layout where it applies);
+                            // 1: sorted fold, then bucket FFTs (alias-row
+                            //    layout where it applies);
                             // 2: as 1, buckets always in natural order
-  int stream_blocks;        // resident blocks of the streamed fold
   // scratch for transforms and selections that do not fit in LDS (null
   // when unused)
   double2 *comb_buf, *comb_tmp;  // S x comb_loops x W sub-sampled comb signals

@@ -15,6 +15,7 @@
 // (signal, chunk).  All index arithmetic is exact: for n = 2^p the low 32
 // bits of i * a already give (i * a) mod n.
 #include <algorithm>
+#include <climits>
 #include <mutex>
 #include <string>
 
@@ -219,195 +220,286 @@ __global__ void __launch_bounds__(kBlock) k_fold_fft64(V12Launch a, int l0, int 
   for (int j = threadIdx.x; j < B; j += T) out[j] = smem64[j];
 }
 
-// ---------------------------------------------------------------- streamed fold
-// The FP64 bucket sums, scheduled for the Infinity Cache (MALL): work items
-// are (signal, loop, 64 buckets), one per wavefront, numbered signal-major,
-// and a fixed set of resident wavefronts walks them in order.  Only a few
-// signals are then in flight at once, so the second and later touches of a
-// signal's 128-byte lines (20 loops gather ~20% of its samples) find them in
-// the MALL instead of HBM.  Each lane sums its bucket in ascending tap order
-// (identical arithmetic to the fused kernel); the B-point FFT follows in
-// the bucket FFT batches.  Buckets are written pre-FFT into xs64.
-constexpr int kFoldWaves = 4;  // wavefronts per block
+// ---------------------------------------------------------------- sorted fold
+// Bucket sums with the gathers in address order.  Loop l adds x[p] * tap[i]
+// into bucket b = i mod B for the taps i = b + kB < w at p = i*ai mod n;
+// p mod B = b*ai mod B, so bucket b only ever reads residue class
+// r = b*ai mod B, and b = r*a mod B (a*ai = 1 mod n).  Viewing the signal as
+// n/B rows of B samples (p = r + t*B), a workgroup takes the buckets of
+// f.res consecutive residues in every loop of the part, one (residue, loop)
+// pair per thread, and is the only reader of those residues' lines.  It
+// sorts its pairs' taps by row (a counting sort in LDS) and walks the sorted
+// list: neighbouring lanes read the same or the next row, so a 128-byte line
+// is requested once, whichever loops' taps meet in it, and every load of the
+// walk is independent of the others.  The products replace the taps in LDS,
+// and each pair's thread adds its own in the form's fixed order:
+//   FP64  ascending tap order, as the reference does;
+//   FP32  chunk by chunk of 2^seg_log rows, in ascending tap order within a
+//         chunk, with compensated (2Sum) sums, the chunks' sums added in
+//         chunk order.
+//
+// Bound by HBM on batches: the 850,060 gathers of a signal (n = 2^22, k = 64)
+// touch 422,076 lines, 13.83 GB per 256 signals, read in 2.96 ms (4.7 TB/s,
+// the rate of a large copy).  Before, with the gathers of a 256-row chunk in
+// flight at a time in tap order, 3.72 ms; the FP64 form, one wave per 64
+// buckets in tap order, took 1.03 ms per 64 signals against 0.80 ms.  One
+// signal is bound by the phases' latency: 19 us against 36 us (FP32), 17 us
+// against 24 us (FP64, n = 2^22, k = 100).
+constexpr int kMaxTaps = 32;           // taps per pair: 5 bits of a list entry
+constexpr int kFoldThreads = 512;      // and pairs per workgroup at most
+constexpr int kWalkAhead = 8;          // gathers in flight per thread
+constexpr int kSortAhead = 8;          // sort steps and tap loads in flight per thread
+constexpr int kPackLog = 3, kPackChunks = 1 << kPackLog;  // tap counts in one 64-bit word
+constexpr size_t kFoldLds = 150 * 1024;  // dynamic LDS of a workgroup at most
 
-struct FoldItems {
-  int l0, nl;          // loop range
-  int c_loc, c_est;    // 64-bucket chunks per location / estimation loop
-  int n_loc;           // location loops in the range
-  int64_t per_signal;  // items per signal
-  int64_t total;
+// Loops [l0, l0 + nl) of one bucket count and precision.
+struct FoldPart {
+  int fp32;
+  int l0, nl;
+  int B, logB;
+  int res, log_res;      // residues per workgroup
+  int groups;            // B / res
+  int tR;                // LDS stride of a pair's taps (max ceil(w/B), odd)
+  unsigned inv_tR;       // idx / tR = idx * inv_tR >> 20 for idx below kFoldThreads * tR
+  int nbins, bin_shift;  // sort bins of 2^bin_shift rows
+  int seg_log;           // FP32: rows per chunk 2^seg_log
+  int order_at;          // FP32: the taps' summation order, in words of LDS
 };
 
-__host__ __device__ inline FoldItems fold_items(const V12Launch &a, int l0, int nl)
+struct FoldParts {
+  FoldPart p[2];
+  int groups;  // workgroups per signal, all parts
+};
+
+// sum + cmp gains v, compensated (2Sum)
+__device__ __forceinline__ void add2(float2 &sum, float2 &cmp, float2 v)
 {
-  FoldItems f;
-  f.l0 = l0;
-  f.nl = nl;
-  f.c_loc = (a.B_loc + 63) / 64;
-  f.c_est = (a.B_est + 63) / 64;
-  const int l1 = l0 + nl;
-  f.n_loc = max(0, min(l1, a.Lloc) - l0);
-  f.per_signal = (int64_t)f.n_loc * f.c_loc + (int64_t)(nl - f.n_loc) * f.c_est;
-  f.total = f.per_signal * a.S;
-  return f;
+  float t = sum.x + v.x, bp = t - sum.x;
+  cmp.x += (sum.x - (t - bp)) + (v.x - bp);
+  sum.x = t;
+  t = sum.y + v.y;
+  bp = t - sum.y;
+  cmp.y += (sum.y - (t - bp)) + (v.y - bp);
+  sum.y = t;
 }
 
-__global__ void __launch_bounds__(64 * kFoldWaves) k_fold_stream(V12Launch a, FoldItems f)
+// Group g of the part's residues in signal s.
+template <bool FP32>
+__device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f, int s, int g,
+                                           double2 *smem64, int *sh)
 {
-  const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * kFoldWaves + (threadIdx.x >> 6);
-  const int64_t nwaves = (int64_t)gridDim.x * kFoldWaves;
-  const unsigned mask = (unsigned)a.n - 1;
-  const int stride = 2 * a.L + max(a.comb_loops, 1);
-  for (int64_t item = wave; item < f.total; item += nwaves) {
-    const int s = (int)(item / f.per_signal);
-    const int64_t r0 = item % f.per_signal;
-    int l, ch;
-    if (r0 < (int64_t)f.n_loc * f.c_loc) {
-      l = f.l0 + (int)(r0 / f.c_loc);
-      ch = (int)(r0 % f.c_loc);
+  using T2 = typename std::conditional<FP32, float2, double2>::type;
+  constexpr int T = kFoldThreads;
+  const int tid = threadIdx.x;
+  const int npairs = f.res * f.nl;
+  T2 *slots = reinterpret_cast<T2 *>(smem64);
+  int *bins = reinterpret_cast<int *>(smem64);  // until the list is built
+  uint2 *pp = reinterpret_cast<uint2 *>(smem64 + (npairs * f.tR * sizeof(T2) + 15) / 16);
+  int *tap_at = reinterpret_cast<int *>(pp + npairs);
+  uint16_t *list = reinterpret_cast<uint16_t *>(tap_at + npairs);
+  // FP32: the pair's taps in summation order, a byte each (tR4 of them); a
+  // second list when they take several passes
+  const int tR4 = (f.tR + 3) & ~3;
+  uint8_t *order = reinterpret_cast<uint8_t *>(
+      reinterpret_cast<uint32_t *>(smem64) + f.order_at) + tid * tR4;
+  uint8_t *order2 = order + npairs * tR4;
+  const int B = f.B, logB = f.logB;
+  const unsigned mask = (unsigned)a.n - 1, rmask = ((unsigned)a.n >> logB) - 1;
+  const int *prm = a.params + (int64_t)s * (2 * a.L + max(a.comb_loops, 1));
+  const bool has = tid < npairs;
+  const int l = f.l0 + (has ? tid >> f.log_res : 0);
+  const unsigned av = (unsigned)prm[l], ai = (unsigned)prm[a.L + l];
+  const unsigned res = (unsigned)(g * f.res + (tid & (f.res - 1)));
+  const int b = (int)((res * av) & (unsigned)(B - 1));
+  const int w = l < a.Lloc ? a.w_loc : a.w_est;
+  const int R = (has && b < w) ? (w - b + B - 1) / B : 0;
+  const unsigned p0 = ((unsigned)b * ai) & mask, step = ((unsigned)B * ai) & mask;
+  const unsigned row0 = p0 >> logB, srow = step >> logB;  // row of tap k: row0 + k srow
+  if (has) {
+    // the pair's first sample and stride, and its run of taps (bit 31: of
+    // the location filter)
+    pp[tid] = make_uint2(p0, step);
+    tap_at[tid] = b * (l < a.Lloc ? a.tR_loc : a.tR_est) | (l < a.Lloc ? INT_MIN : 0);
+  }
+  for (int i = tid; i < f.nbins; i += T) bins[i] = 0;
+  __syncthreads();
+  // FP32: taps by the low bits of their chunk, eight bits a count
+  uint64_t per_chunk = 0;
+  for (int k = 0; k < R; k++) {
+    const unsigned row = (row0 + (unsigned)k * srow) & rmask;
+    atomicAdd(&bins[row >> f.bin_shift], 1);
+    if (FP32) per_chunk += 1ull << (8 * ((row >> f.seg_log) & (kPackChunks - 1)));
+  }
+  __syncthreads();
+  int total;
+  {
+    const int C = (f.nbins + T - 1) / T;
+    const int lo = min(f.nbins, tid * C), hi = min(f.nbins, lo + C);
+    int sum = 0;
+    for (int i = lo; i < hi; i++) sum += bins[i];
+    int run = block_exclusive_scan(sum, sh, total);
+    for (int i = lo; i < hi; i++) {
+      const int v = bins[i];
+      bins[i] = run;
+      run += v;
+    }
+  }
+  __syncthreads();
+  // the list; FP32: the pair's taps sorted, stably, by the low bits of their
+  // chunk (place: the exclusive byte-wise prefix sum of the counts)
+  uint64_t place = per_chunk * 0x0101010101010100ull;
+  for (int k0 = 0; k0 < R; k0 += kSortAhead) {
+    int at[kSortAhead];
+#pragma unroll
+    for (int u = 0; u < kSortAhead; u++)
+      if (k0 + u < R) {
+        const unsigned row = (row0 + (unsigned)(k0 + u) * srow) & rmask;
+        at[u] = atomicAdd(&bins[row >> f.bin_shift], 1);
+        if (FP32) {
+          const int c8 = 8 * (int)((row >> f.seg_log) & (kPackChunks - 1));
+          order[(place >> c8) & 255] = (uint8_t)(k0 + u);
+          place += 1ull << c8;
+        }
+      }
+#pragma unroll
+    for (int u = 0; u < kSortAhead; u++)
+      if (k0 + u < R) list[at[u]] = (uint16_t)(tid << 5 | (k0 + u));
+  }
+  if (FP32) {
+    // the chunk's further bits, kPackLog at a time
+    for (int sft = kPackLog; (rmask >> f.seg_log) >> sft; sft += kPackLog) {
+      uint64_t cnt = 0;
+      for (int k = 0; k < R; k++)
+        cnt += 1ull << (8 * ((((row0 + (unsigned)k * srow) & rmask) >> (f.seg_log + sft)) &
+                             (kPackChunks - 1)));
+      uint64_t at = cnt * 0x0101010101010100ull;
+      for (int i = 0; i < R; i++) {
+        const unsigned k = order[i];
+        const int c8 = 8 * (int)((((row0 + k * srow) & rmask) >> (f.seg_log + sft)) &
+                                 (kPackChunks - 1));
+        order2[(at >> c8) & 255] = (uint8_t)k;
+        at += 1ull << c8;
+      }
+      uint8_t *t = order;
+      order = order2;
+      order2 = t;
+    }
+  }
+  __syncthreads();
+  const double2 *__restrict__ x = a.x[s];
+  double2 xv[kWalkAhead];
+  int at[kWalkAhead];
+  auto gather = [&](int j0) {
+#pragma unroll
+    for (int u = 0; u < kWalkAhead; u++) {
+      const int j = j0 + u * T;
+      at[u] = -1;
+      if (j < total) {
+        const unsigned e = list[j];
+        const int pr = (int)(e >> 5), k = (int)(e & 31);
+        const uint2 q = pp[pr];
+        xv[u] = x[(q.x + (unsigned)k * q.y) & mask];
+        at[u] = pr * f.tR + k;
+      }
+    }
+  };
+  gather(tid);  // in flight while the taps are staged
+  // the taps, by bucket, in coalesced runs
+  {
+    const T2 *tl, *te;
+    if constexpr (FP32) {
+      tl = a.tapsT_loc32;
+      te = a.tapsT_est32;
     } else {
-      const int64_t r1 = r0 - (int64_t)f.n_loc * f.c_loc;
-      l = f.l0 + f.n_loc + (int)(r1 / f.c_est);
-      ch = (int)(r1 % f.c_est);
+      tl = a.tapsT_loc;
+      te = a.tapsT_est;
     }
-    const bool isloc = l < a.Lloc;
-    const int B = isloc ? a.B_loc : a.B_est;
-    const int w = isloc ? a.w_loc : a.w_est;
-    const int m = ch * 64 + lane;
-    if (m >= B) continue;
-    const unsigned ai = (unsigned)a.params[(int64_t)s * stride + a.L + l];
-    const double2 *__restrict__ x = a.x[s];
-    const int64_t out = (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est) + m;
-    const int R = (w - m + B - 1) / B;  // taps m, m+B, ... below w
-    const double2 *__restrict__ taps = isloc ? a.taps_loc : a.taps_est;
+    const int cnt = npairs * f.tR;
+    for (int i0 = tid; i0 < cnt; i0 += kSortAhead * T) {
+      T2 t[kSortAhead];
+#pragma unroll
+      for (int u = 0; u < kSortAhead; u++) {
+        const int idx = min(i0 + u * T, cnt - 1);
+        const int pr = (int)(((unsigned)idx * f.inv_tR) >> 20), k = idx - pr * f.tR;
+        const int ta = tap_at[pr];
+        const T2 *tp = ta < 0 ? tl : te;
+        t[u] = tp[(ta & INT_MAX) + min(k, (ta < 0 ? a.tR_loc : a.tR_est) - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < kSortAhead; u++) slots[min(i0 + u * T, cnt - 1)] = t[u];
+    }
+  }
+  __syncthreads();
+  for (int j0 = tid;;) {
+#pragma unroll
+    for (int u = 0; u < kWalkAhead; u++) {
+      if (at[u] < 0) continue;
+      const T2 t = slots[at[u]];
+      if constexpr (FP32) {
+        slots[at[u]] = cmul(make_float2((float)xv[u].x, (float)xv[u].y), t);
+      } else {
+        slots[at[u]] = make_double2(xv[u].x * t.x - xv[u].y * t.y, xv[u].x * t.y + xv[u].y * t.x);
+      }
+    }
+    j0 += kWalkAhead * T;
+    if (j0 >= total) break;
+    gather(j0);
+  }
+  __syncthreads();
+  if (!has) return;
+  const T2 *mine = slots + tid * f.tR;
+  const int64_t out = (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est) + b;
+  if constexpr (FP32) {
+    float2 tot = make_float2(0.f, 0.f), sum = tot, cmp = tot;
+    unsigned chunk = ~0u;
+    for (int i0 = 0; i0 < R; i0 += 4) {
+      // four taps' products and chunks at a time
+      const unsigned four = *reinterpret_cast<const unsigned *>(order + i0);
+      float2 v[4];
+      unsigned c[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const unsigned k = min((four >> (8 * u)) & 255u, (unsigned)(R - 1));  // past R: unused
+        v[u] = mine[k];
+        c[u] = ((row0 + k * srow) & rmask) >> f.seg_log;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        if (i0 + u >= R) break;
+        if (c[u] != chunk) {
+          tot = make_float2(tot.x + (sum.x + cmp.x), tot.y + (sum.y + cmp.y));
+          sum = cmp = make_float2(0.f, 0.f);
+          chunk = c[u];
+        }
+        add2(sum, cmp, v[u]);
+      }
+    }
+    tot = make_float2(tot.x + (sum.x + cmp.x), tot.y + (sum.y + cmp.y));
+    a.xs32[out] = tot;
+  } else {
     double2 acc = make_double2(0.0, 0.0);
-    int r = 0;
-    for (; r + 8 <= R; r += 8) {
-      double2 xv[8], tv[8];
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        const unsigned i = (unsigned)(m + (r + q) * B);
-        xv[q] = x[(i * ai) & mask];
-        tv[q] = taps[i];
-      }
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        acc.x = acc.x + (xv[q].x * tv[q].x - xv[q].y * tv[q].y);
-        acc.y = acc.y + (xv[q].x * tv[q].y + xv[q].y * tv[q].x);
-      }
-    }
-    for (; r < R; r++) {
-      const unsigned i = (unsigned)(m + r * B);
-      const double2 xv = x[(i * ai) & mask], tv = taps[i];
-      acc.x = acc.x + (xv.x * tv.x - xv.y * tv.y);
-      acc.y = acc.y + (xv.x * tv.y + xv.y * tv.x);
+    for (int k = 0; k < R; k++) {
+      acc.x = acc.x + mine[k].x;
+      acc.y = acc.y + mine[k].y;
     }
     a.xs64[out] = acc;
   }
 }
 
-// ---------------------------------------------------------------- chunked fold
-// The FP32 form's bucket sums, grouped so that an XCD's L2 serves repeated
-// touches of a 128-byte line.  Loop l adds x[p] * tap[i] into bucket
-// b = i mod B for the taps i = b + kB < w at p = i*ai mod n; p mod B =
-// b*ai mod B, so bucket b only ever reads residue class r = b*ai mod B, and
-// b = r*a mod B (a*ai = 1 mod n).  A workgroup takes the buckets of kResPer
-// consecutive residues in every loop of the launch, one (residue, loop) pair
-// per thread: it is the only reader of those residues' lines (viewing the
-// signal as n/B rows of B samples, p = r + t*B).  Rows are walked in chunks
-// of 2^seg_log rows; each thread adds, chunk after chunk, its taps whose
-// sample lies in the chunk, in ascending tap order, with compensated (2Sum)
-// FP32 sums, and adds the chunks' sums in chunk order.  The workgroup's
-// threads work on the same chunk at about the same time, so the touches of
-// one line (taps of different loops in one row) fall within one memory round
-// trip and the L2 serves all but the first.  The pairs' taps are staged in
-// LDS by coalesced loads of their by-bucket runs.  This fixes the FP32 form's
-// summation order; with one chunk it is plain ascending tap order.
-constexpr int kResPer = 16;                        // residues per workgroup
-constexpr int kFoldResBlock = kResPer * kMaxLoops;  // 512: one pair per thread
-constexpr int kChunkBatch = 16;                    // gathers in flight per thread and round
-
-struct FoldChunks {
-  int l0, nl;        // loops [l0, l0 + nl), all with B buckets
-  int B, logB;
-  int res, groups;   // residues per workgroup, B / res
-  int seg_log, nseg; // rows per chunk 2^seg_log, chunks
-  int tR;            // LDS stride of a pair's taps (max ceil(w/B) of the loops)
-};
-
-__global__ void __launch_bounds__(kFoldResBlock) k_fold_chunks(V12Launch a, FoldChunks f)
+// grid: S x f.groups
+__global__ void __launch_bounds__(kFoldThreads) k_fold_sorted(V12Launch a, FoldParts f)
 {
-  extern __shared__ float2 s_tap[];  // pair-major, f.tR taps each
-  __shared__ int s_b[kFoldResBlock];
-  const int g = (int)(blockIdx.x % (unsigned)f.groups);
+  extern __shared__ double2 smem64[];
+  __shared__ int sh[16];
   const int s = (int)(blockIdx.x / (unsigned)f.groups);
-  const int tid = threadIdx.x;
-  const int npairs = f.res * f.nl;
-  const bool has = tid < npairs;
-  const int e = tid % f.res, jl = has ? tid / f.res : 0;
-  const int l = f.l0 + jl;
-  const bool isloc = l < a.Lloc;
-  const int *prm = a.params + (int64_t)s * (2 * a.L + max(a.comb_loops, 1));
-  const unsigned av = (unsigned)prm[l], ai = (unsigned)prm[a.L + l];
-  const int B = f.B, logB = f.logB;
-  const unsigned mask = (unsigned)a.n - 1;
-  const int b = (int)(((unsigned)(g * f.res + e) * av) & (unsigned)(B - 1));
-  const int w = isloc ? a.w_loc : a.w_est;
-  const int R = (has && b < w) ? (w - b + B - 1) / B : 0;
-  const unsigned p0 = ((unsigned)b * ai) & mask;
-  const unsigned step = ((unsigned)B * ai) & mask;
-  s_b[tid] = b;
-  __syncthreads();
-  for (int idx = tid; idx < npairs * f.tR; idx += blockDim.x) {
-    const int pr = idx / f.tR, k = idx - pr * f.tR;
-    const bool lp = f.l0 + pr / f.res < a.Lloc;
-    const int tRp = lp ? a.tR_loc : a.tR_est;
-    const float2 *T = lp ? a.tapsT_loc32 : a.tapsT_est32;
-    s_tap[idx] = k < tRp ? T[(int64_t)s_b[pr] * tRp + k] : make_float2(0.f, 0.f);
+  int g = (int)(blockIdx.x % (unsigned)f.groups);
+  FoldPart p = f.p[0];
+  if (g >= p.groups) {
+    g -= p.groups;
+    p = f.p[1];
   }
-  __syncthreads();
-  if (!has) return;  // no barrier below
-  const float2 *mytap = s_tap + tid * f.tR;
-  const double2 *__restrict__ x = a.x[s];
-  const int cshift = logB + f.seg_log;
-  float2 tot = make_float2(0.f, 0.f);
-  for (int c = 0; c < f.nseg; c++) {
-    unsigned m = 0, pp = p0;
-    for (int k = 0; k < R; k++) {
-      if ((int)(pp >> cshift) == c) m |= 1u << k;
-      pp = (pp + step) & mask;
-    }
-    float2 sum = make_float2(0.f, 0.f), cmp = make_float2(0.f, 0.f);
-    while (m) {
-      double2 xv[kChunkBatch];
-      int kk[kChunkBatch];
-#pragma unroll
-      for (int q = 0; q < kChunkBatch; q++) {
-        kk[q] = m ? __ffs(m) - 1 : -1;
-        if (kk[q] >= 0) {
-          xv[q] = x[(p0 + (unsigned)kk[q] * step) & mask];
-          m &= m - 1;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < kChunkBatch; q++) {
-        if (kk[q] >= 0) {
-          const float2 pr = cmul(make_float2((float)xv[q].x, (float)xv[q].y), mytap[kk[q]]);
-          float t = sum.x + pr.x, bp = t - sum.x;
-          cmp.x += (sum.x - (t - bp)) + (pr.x - bp);
-          sum.x = t;
-          t = sum.y + pr.y;
-          bp = t - sum.y;
-          cmp.y += (sum.y - (t - bp)) + (pr.y - bp);
-          sum.y = t;
-        }
-      }
-    }
-    const float2 part = make_float2(sum.x + cmp.x, sum.y + cmp.y);
-    tot = c == 0 ? part : make_float2(tot.x + part.x, tot.y + part.y);
-  }
-  a.xs32[(int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est) + b] = tot;
+  if (p.fp32) fold_group<true>(a, p, s, g, smem64, sh);
+  else fold_group<false>(a, p, s, g, smem64, sh);
 }
 
 // ---------------------------------------------------------------- v1 votes
@@ -1279,70 +1371,100 @@ int comb(const V12Launch &a, hipStream_t st)
   return 0;
 }
 
-// Loops of one bucket count folded by k_fold_chunks.
-static int fold_chunks(const V12Launch &a, hipStream_t st, int l0, int nl, int B)
+// The part of loops [l0, l0 + nl) with `res` residues per workgroup and its
+// LDS; false when the loops do not fit the kernel's limits.
+static bool fold_part(const V12Launch &a, bool fp32, int l0, int nl, int B, int res, FoldPart &f,
+                      size_t &lds)
 {
-  FoldChunks f;
+  const size_t elt = fp32 ? sizeof(float2) : sizeof(double2);
+  f.fp32 = fp32;
   f.l0 = l0;
   f.nl = nl;
   f.B = B;
   f.logB = 31 - __builtin_clz((unsigned)B);
-  f.res = std::min(kResPer, B);
+  f.res = std::min(res, B);
+  f.log_res = 31 - __builtin_clz((unsigned)f.res);
   f.groups = B / f.res;
   const int rows = a.n / B;
   const int seg = std::min(rows, a.seg_rows);
   f.seg_log = 31 - __builtin_clz((unsigned)seg);
-  f.nseg = rows / seg;
   f.tR = 0;
   if (l0 < a.Lloc) f.tR = std::max(f.tR, a.tR_loc);
   if (l0 + nl > a.Lloc) f.tR = std::max(f.tR, a.tR_est);
-  if (f.tR > 32) {  // tap masks are 32 bits; tolerances >= 5e-9 give at most 27 taps
-    set_error("fold: more than 32 taps per bucket");
-    return -1;
+  if (f.tR > kMaxTaps) return false;
+  f.tR |= 1;
+  f.inv_tR = (1u << 20) / (unsigned)f.tR + 1;
+  const size_t npairs = (size_t)f.res * nl;
+  const size_t slots = (npairs * f.tR * elt + 15) / 16 * 16;
+  f.nbins = rows;
+  f.bin_shift = 0;
+  while (f.nbins > 2048 || f.nbins * sizeof(int) > slots) {  // the bins use the slots' LDS
+    f.nbins >>= 1;
+    f.bin_shift++;
   }
-  const int threads = (f.res * nl + 63) / 64 * 64;
-  const size_t lds = (size_t)f.res * nl * f.tR * sizeof(float2);
-  allow_lds(k_fold_chunks, lds);
-  const dim3 grid((unsigned)((int64_t)a.S * f.groups));
-  hipLaunchKernelGGL(k_fold_chunks, grid, dim3(threads), lds, st, a, f);
-  return launched("fold_chunks");
+  lds = slots + npairs * (sizeof(uint2) + sizeof(int)) +
+        (npairs * f.tR * sizeof(uint16_t) + 3) / 4 * 4;
+  f.order_at = (int)(lds / 4);
+  if (fp32) lds += npairs * ((f.tR + 3) & ~3) * ((rows >> f.seg_log) > kPackChunks ? 2 : 1);
+  return npairs <= kFoldThreads && lds <= kFoldLds;
+}
+
+// Loops [0, n64) in FP64 (from loop `from` on) and [n64, L) in FP32.
+static int fold_sorted(const V12Launch &a, hipStream_t st, int from, int n64)
+{
+  // 16 residues (256 contiguous bytes of a row) read HBM 5-10 % faster than
+  // 8 on batches (FP32 256 x n = 2^22, k = 64: 3.20 against 3.56 ms beside
+  // the estimation; FP64 64 signals: 0.81 against 0.86 ms); a launch of few
+  // workgroups is faster spread over twice as many (one signal: 19.0 against
+  // 20.8 us), and two resident workgroups' LDS does not hold 16 residues of
+  // many FP64 loops
+  FoldParts f{};
+  size_t lds = 0;
+  int np = 0;
+  auto add = [&](bool fp32, int l0, int l1) {
+    if (l1 <= l0) return 0;
+    const int B = l0 < a.Lloc ? a.B_loc : a.B_est;
+    size_t b16 = 0;
+    const bool wide = (int64_t)a.S * B >= 16 * 512 && fold_part(a, fp32, l0, l1 - l0, B, 16, f.p[np], b16);
+    if (!wide && !fold_part(a, fp32, l0, l1 - l0, B, 8, f.p[np], b16)) {
+      set_error("fold: more than 32 taps per bucket");
+      return -1;
+    }
+    lds = std::max(lds, b16);
+    f.groups += f.p[np].groups;
+    np++;
+    return 0;
+  };
+  const bool same = a.B_loc == a.B_est;
+  const int cut = same ? n64 : a.Lloc;  // where the bucket count or precision changes
+  // (with both, they change at the same loop: n64 is 0, Lloc or L)
+  if (add(n64 == 0, from, cut) != 0 || add(cut >= n64, std::max(cut, from), a.L) != 0) return -1;
+  if (np == 0) return 0;
+  allow_lds(k_fold_sorted, lds);
+  hipLaunchKernelGGL(k_fold_sorted, dim3((unsigned)((int64_t)a.S * f.groups)), dim3(kFoldThreads),
+                     lds, st, a, f);
+  return launched("fold_sorted") == 0 ? 1 : -1;
 }
 
 int fold_fft(const V12Launch &a, hipStream_t st, int part)
 {
-  // loops [0, n64) in FP64, [n64, L) in FP32 (folded by k_fold_chunks, with
-  // the FFTs in part 1 whatever the schedule)
+  // loops [0, n64) in FP64, [n64, L) in FP32 (with the FFTs in part 1
+  // whatever the schedule)
   const int n64 = !a.fp32 ? a.L : (a.loc64 ? a.Lloc : 0);
   const int B64 = n64 == 0 ? 0 : (n64 > a.Lloc ? max(a.B_loc, a.B_est) : a.B_loc);
   int launches = 0;
   if (part == 0) {
-    if (n64 > 0 && a.fold_mode >= 1) {
-      const FoldItems f = fold_items(a, 0, n64);
-      const int64_t g =
-          std::min<int64_t>(a.stream_blocks, (f.total + kFoldWaves - 1) / kFoldWaves);
-      hipLaunchKernelGGL(k_fold_stream, dim3((unsigned)g), dim3(64 * kFoldWaves), 0, st, a, f);
-      if (launched("fold_stream64") != 0) return -1;
-      launches++;
-    } else if (n64 > 0) {
+    int from = 0;  // first loop of the sorted fold
+    if (n64 > 0 && a.fold_mode == 0) {
       allow_lds(k_fold_fft64, (size_t)B64 * sizeof(double2));
       hipLaunchKernelGGL(k_fold_fft64, dim3(a.S * n64), dim3(kBlock),
                          (size_t)B64 * sizeof(double2), st, a, 0, n64);
       if (launched("fold_fft64") != 0) return -1;
       launches++;
+      from = n64;
     }
-    if (n64 < a.L) {
-      // the FP32 loops, in runs of one bucket count
-      auto run = [&](int l0, int nl, int B) { return fold_chunks(a, st, l0, nl, B); };
-      if (n64 < a.Lloc && a.B_loc != a.B_est) {
-        if (run(n64, a.Lloc - n64, a.B_loc) != 0 || run(a.Lloc, a.L - a.Lloc, a.B_est) != 0)
-          return -1;
-        launches += 2;
-      } else {
-        if (run(n64, a.L - n64, n64 < a.Lloc ? a.B_loc : a.B_est) != 0) return -1;
-        launches++;
-      }
-    }
-    return launches;
+    const int rc = fold_sorted(a, st, from, n64);
+    return rc < 0 ? -1 : launches + rc;
   }
   // part 1: the bucket FFTs of every loop not fused into its fold
   if (a.rows_layout) {

@@ -2,9 +2,8 @@
 //
 // The schedules differ only in how the fold is mapped onto the GPU: the
 // fused kernel (one workgroup per (signal, loop) folding into LDS and
-// transforming there) or the signal-major streamed fold with R resident
-// workgroups followed by the bucket-FFT batches.  Every lane sums its bucket
-// in the same tap order in all of them, so the choice never changes a bit of
+// transforming there) or the sorted fold followed by the bucket-FFT batches.
+// Every bucket is summed in the same tap order in all of them, so the choice never changes a bit of
 // the result; B, the loop counts and the filters are the reference's and are
 // not tuned.  Candidates are timed on synthetic noise signals with a private
 // RNG stream, so tuning does not advance the plan's own draws.
@@ -53,9 +52,6 @@ int autotune_plan(Plan *P, int batch)
 {
   if (P->version == SFFT_VERSION_3) return 0;  // one schedule only
   const V12Params &p = P->v12;
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   // synthetic batch: at most 8 GiB of input
   const int64_t per = (int64_t)p.n * 16;
   const int S = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(batch, 1), (8LL << 30) / per));
@@ -79,8 +75,8 @@ int autotune_plan(Plan *P, int batch)
 
   std::vector<std::pair<int, int>> cand;
   if (std::max(p.B_loc, p.B_est) <= kMaxLdsFft64) cand.push_back({0, 0});
-  for (int r : {1, 2, 4}) cand.push_back({1, r * cus});
-  if (P->precision == SFFT_PRECISION_FP32_REFINE && p.comb) cand.push_back({2, cus});
+  cand.push_back({1, 0});
+  if (P->precision == SFFT_PRECISION_FP32_REFINE && p.comb) cand.push_back({2, 0});
   const int mode0 = P->fold_mode, blocks0 = P->stream_blocks;
   double best = 1e30;
   std::pair<int, int> pick{mode0, blocks0};

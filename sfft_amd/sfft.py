@@ -139,8 +139,8 @@ class sfft:
         self.precision = precision
 
     def set_schedule(self, fold_mode, stream_blocks=0):
-        """Fold schedule (0 fused, 1 streamed with stream_blocks resident
-        workgroups); never changes results."""
+        """Fold schedule (0 fused, 1 sorted, 2 sorted with the buckets in
+        natural order); never changes results."""
         if self._L.sfft_plan_set_schedule(self.sfft_plan, fold_mode, stream_blocks) != 0:
             raise SfftError(_lib.last_error())
 

@@ -478,3 +478,50 @@ def test_parted_batch_equals_single(torch_cuda, graphs):
         assert torch.equal(va[i, :c], v1[0, :c])
     del x
     torch.cuda.empty_cache()
+
+
+# Edges of the sorted fold: few residues (B below a workgroup's), the widest
+# spectrum of rows (chunk lists of several passes), 8 and 16 residues per
+# workgroup, location and estimation loops of different bucket counts.
+SORTED = [
+    (2, 1 << 13, 50, 1),    # 23 loops, 32 rows of 256 buckets
+    (1, 1 << 14, 50, 3),
+    (2, 1 << 24, 10, 1),    # 16,384 and 32,768 rows: up to three list passes
+    (2, 1 << 23, 50, 1),    # B_loc != B_est
+    (1, 1 << 22, 30, 2),    # v1: FP64 and FP32 loops of one launch
+    (2, 1 << 20, 300, 9),   # 16 residues per workgroup
+]
+
+
+@pytest.mark.parametrize("version,n,k,signals", SORTED)
+def test_sorted_fold_buckets(torch_cuda, version, n, k, signals):
+    """The last signal's buckets of a batch equal the oracle's bit for bit
+    (FP64 form) and the model of the FP32 form's summation order."""
+    torch = torch_cuda
+    print(f"case sorted fold v{version} n={n} k={k} x{signals}", flush=True)
+    xs = [signal_np(n, k, seed=8800 + i, snr_db=30.0)[0] for i in range(signals)]
+    xd = [torch.from_numpy(x).cuda() for x in xs]
+    for precision in ("fp64", "fp32_refine"):
+        plan = _gpu_plan(version, n, k, precision)
+        fr, va = plan.make_sparse_outputs(signals)
+        plan.execute_many_sparse(xd, fr, va)
+        got = plan.debug_buckets(signals - 1)
+        lt, lf = plan.filter(0)
+        et, ef = plan.filter(1)
+        P = oracle.V12(n, k, version == 2)
+        P.set_filters(lt, lf, et, ef)
+        oracle.seed_glibc(17, 4242)
+        for _ in range(signals):
+            a, ai, off = P.draw()
+        ref = P.exec(xs[-1], a, ai, off, trace=True)["x_samp"]
+        p = P.p
+        nmax = max(p.B_loc, p.B_est, p.W_comb if version == 2 else 0)
+        at = 0
+        for l in range(P.loops):
+            loc = l < p.loc_loops
+            B = p.B_loc if loc else p.B_est
+            want = ref[at:at + B]
+            if precision == "fp32_refine" and not (version == 1 and loc):
+                want = oracle.fp32_buckets(xs[-1], n, B, lt if loc else et, ai[l], 256, nmax)
+            assert np.array_equal(got[at:at + B], want), (precision, l)
+            at += B

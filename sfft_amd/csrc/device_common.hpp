@@ -130,13 +130,20 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *tmp, int &total)
 // IEEE bit patterns order like the values.  Requires N >= num + 1.
 // The cutoff is found by byte-wise radix selection from the top byte; once
 // at most 128 keys share the selected prefix, their exact rank is computed
-// directly.  Uses 256+16 ints of LDS at sh.  Contains barriers.
+// directly.  The top byte (seven exponent bits) takes few values, so its
+// histogram is counted once per value and wave, not by 64 atomics on one
+// word; the picked indices are compacted by wave ballots over contiguous
+// shares (a contiguous run per thread put a wave's reads on one bank).
+// With both, the comb kernel of one signal (4096 points, 1024 threads) went
+// from 28 to 25 us.
+// Uses 256+32 ints of LDS at sh.  Contains barriers.
 __device__ void block_top_num(const double *mag, int N, int num, int *out,
                               int *sh)
 {
   int *hist = sh;          // 256
-  int *misc = sh + 256;    // 16
+  int *misc = sh + 256;    // 32
   const int T = blockDim.x, tid = threadIdx.x;
+  const int lane = tid & 63, wid = tid >> 6, nw = T >> 6;
   // rank of the cutoff in ascending order among the keys matching prefix
   int rank = N - num - 1;
   uint64_t prefix = 0, hi_mask = 0;
@@ -146,9 +153,23 @@ __device__ void block_top_num(const double *mag, int N, int num, int *out,
     const int shift = pass * 8;
     for (int d = tid; d < 256; d += T) hist[d] = 0;
     __syncthreads();
-    for (int i = tid; i < N; i += T) {
-      const uint64_t key = (uint64_t)__double_as_longlong(mag[i]);
-      if ((key & hi_mask) == prefix) atomicAdd(&hist[(key >> shift) & 255], 1);
+    if (pass == 7) {
+      for (int i0 = wid * 64; i0 < N; i0 += T) {
+        const int i = i0 + lane;
+        const int d = i < N ? (int)((uint64_t)__double_as_longlong(mag[i]) >> 56) : -1;
+        uint64_t left = __ballot(d >= 0);
+        while (left) {  // wave-uniform
+          const int d0 = __shfl(d, __ffsll((unsigned long long)left) - 1, 64);
+          const uint64_t same = __ballot(d == d0);
+          if (lane == 0) atomicAdd(&hist[d0], __popcll(same));
+          left &= ~same;
+        }
+      }
+    } else {
+      for (int i = tid; i < N; i += T) {
+        const uint64_t key = (uint64_t)__double_as_longlong(mag[i]);
+        if ((key & hi_mask) == prefix) atomicAdd(&hist[(key >> shift) & 255], 1);
+      }
     }
     __syncthreads();
     if (tid < 64) {
@@ -218,40 +239,42 @@ __device__ void block_top_num(const double *mag, int N, int num, int *out,
     }
   }
   if (!direct) cut = prefix;
-  // contiguous chunk per thread so that the compaction keeps index order
-  const int C = (N + T - 1) / T;
-  const int lo = tid * C, hi = min(N, lo + C);
+  // a contiguous share per wave, 64 keys a step, so that ballots rank the
+  // picked keys in index order
+  const int share = ((N + nw - 1) / nw + 63) & ~63;
+  const int lo = min(N, wid * share), hi = min(N, lo + share);
   int ngt = 0, neq = 0;
-  for (int i = lo; i < hi; i++) {
-    const uint64_t key = (uint64_t)__double_as_longlong(mag[i]);
-    ngt += key > cut;
-    neq += key == cut;
+  for (int i0 = lo; i0 < hi; i0 += 64) {
+    const bool in = i0 + lane < hi;
+    const uint64_t key = in ? (uint64_t)__double_as_longlong(mag[i0 + lane]) : 0;
+    ngt += __popcll(__ballot(in && key > cut));
+    neq += __popcll(__ballot(in && key == cut));
   }
-  int tot_gt, tot_eq;
-  (void)block_exclusive_scan(ngt, misc, tot_gt);
-  const int eq_before = block_exclusive_scan(neq, misc, tot_eq);
+  __syncthreads();  // misc is still being read above
+  if (lane == 0) {
+    misc[wid] = ngt;
+    misc[16 + wid] = neq;
+  }
+  __syncthreads();
+  int tot_gt = 0, gt_before = 0, eq_before = 0;
+  for (int q = 0; q < nw; q++) {
+    tot_gt += misc[q];
+    gt_before += q < wid ? misc[q] : 0;
+    eq_before += q < wid ? misc[16 + q] : 0;
+  }
   const int need = num - tot_gt;  // ties to take, lowest indices first
-  int nsel = 0, er = eq_before;
-  for (int i = lo; i < hi; i++) {
-    const uint64_t key = (uint64_t)__double_as_longlong(mag[i]);
-    if (key > cut) nsel++;
-    else if (key == cut) {
-      nsel += er < need;
-      er++;
-    }
-  }
-  int tot_sel;
-  int pos = block_exclusive_scan(nsel, misc, tot_sel);
-  er = eq_before;
-  for (int i = lo; i < hi; i++) {
-    const uint64_t key = (uint64_t)__double_as_longlong(mag[i]);
-    bool take = false;
-    if (key > cut) take = true;
-    else if (key == cut) {
-      take = er < need;
-      er++;
-    }
-    if (take && pos < num) out[pos++] = i;
+  int pos = gt_before + min(eq_before, need);
+  const uint64_t below = (1ull << lane) - 1;
+  for (int i0 = lo; i0 < hi; i0 += 64) {
+    const bool in = i0 + lane < hi;
+    const uint64_t key = in ? (uint64_t)__double_as_longlong(mag[i0 + lane]) : 0;
+    const uint64_t eq = __ballot(in && key == cut);
+    const bool take =
+        in && (key > cut || (key == cut && eq_before + __popcll(eq & below) < need));
+    const uint64_t tk = __ballot(take);
+    if (take) out[pos + __popcll(tk & below)] = i0 + lane;
+    pos += __popcll(tk);
+    eq_before += __popcll(eq);
   }
   __syncthreads();
 }

@@ -262,7 +262,7 @@ int64_t Plan::bytes_per_signal() const
   int64_t b = (need64 ? xs * 16 : 0) + (fp32 ? xs * 8 : 0);
   if (need64 && Bm > kMaxLdsFft64) b += xs * 16;
   if (fp32 && Bm > 2 * kMaxLdsFft64) b += xs * 8;
-  if (p.comb && p.W_comb > k::kMaxLdsComb) b += (int64_t)p.comb_loops * p.W_comb * 40;
+  if (p.comb && p.W_comb > k::kMaxLdsComb) b += (int64_t)p.comb_loops * p.W_comb * 24;
   if (!p.comb && p.B_loc > k::kMaxLdsSelect) b += (int64_t)p.loc_loops * p.B_loc * 8;
   if (!p.comb) b += 4LL * k::vote_chunks(n, p.B_loc, p.B_thresh, p.loc_loops, p.thr_loops);
   return b + (int64_t)p.comb_loops * p.B_thresh * 4 + (int64_t)p.loc_loops * p.B_thresh * 4 +
@@ -941,7 +941,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   const size_t comb_elems = big_comb ? (size_t)S * cl * p.W_comb : 0;
   const size_t mag_elems =
       std::max(comb_elems, big_sel ? (size_t)S * p.loc_loops * p.B_loc : (size_t)0);
-  if ((big_comb && !P->ws->comb.ensure(comb_elems * 2 * sizeof(double2))) ||
+  if ((big_comb && !P->ws->comb.ensure(comb_elems * sizeof(double2))) ||
       (mag_elems && !P->ws->mag.ensure(mag_elems * sizeof(double))) ||
       (big64 && !P->ws->tmp64.ensure((size_t)S * xs * 16)) ||
       (big32 && !P->ws->tmp32.ensure((size_t)S * xs * 8)))
@@ -1014,8 +1014,10 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   a.o_cap = io.cap;
   a.est_cap = cap;
   a.comb_buf = big_comb ? P->ws->comb.as<double2>() : nullptr;
-  a.comb_tmp = big_comb ? P->ws->comb.as<double2>() + comb_elems : nullptr;
   a.mag_buf = mag_elems ? P->ws->mag.as<double>() : nullptr;
+  // a v1 selection above the LDS size: its candidate lists (two of B_loc
+  // ints a loop) or, with more picks than they take, its powers
+  a.cand_buf = big_sel ? P->ws->mag.as<int>() : nullptr;
   a.tmp64 = big64 ? P->ws->tmp64.as<double2>() : nullptr;
   a.tmp32 = big32 ? P->ws->tmp32.as<float2>() : nullptr;
   // the fused fold + FFT keeps a whole bucket array in LDS

@@ -359,8 +359,9 @@ struct V12Launch {
                             // 2: as 1, buckets always in natural order
   // scratch for transforms and selections that do not fit in LDS (null
   // when unused)
-  double2 *comb_buf, *comb_tmp;  // S x comb_loops x W sub-sampled comb signals
-  double *mag_buf;               // |.|^2 of comb or v1 selection arrays
+  double2 *comb_buf;  // S x comb_loops x W: comb transforms, then candidate lists
+  double *mag_buf;    // |.|^2 of comb or v1 selection arrays
+  int *cand_buf;      // v1: candidate lists of the selections, S x Lloc x 2 B_loc
   double2 *tmp64;                // S x xs: radix-2 pass copy of xs64
   float2 *tmp32;                 // S x xs: radix-2 pass copy of xs32
   // v2 with W a multiple of n/B: buckets after the FFT stored by alias row
@@ -453,6 +454,10 @@ int radix2_fft64(double2 *data, double2 *tmp, int N, int64_t nb_outer, int nb_in
                  int64_t si, const double2 *tw, int tw_nmax, hipStream_t st);
 int radix2_fft32(float2 *data, float2 *tmp, int N, int64_t nb_outer, int nb_inner, int64_t so,
                  int64_t si, const float2 *tw, int tw_nmax, hipStream_t st);
+
+// Powers |.|^2 of the comb transforms above the LDS size, into a.mag_buf
+// (a.comb_buf: their scratch).
+int comb_power(const V12Launch &a, hipStream_t st);
 
 // The allocation-free exec's scratch region (kNoAllocScratch bytes of
 // device memory per GPU, a file-scope __device__ array): noalloc_setup()

@@ -2,7 +2,10 @@
 //
 //   * N <= kMaxLdsFft64 (FP64) / 2*kMaxLdsFft64 (FP32): one workgroup per
 //     transform, in LDS (radix-2 DIT with the plan's twiddle table);
-//   * larger N: Stockham autosort passes in global memory, radix 4 (and one
+//   * larger forward N with the plan's table: the same butterflies in two
+//     launches, runs of the bit-reversed sequence and then columns across
+//     the runs;
+//   * other larger N: Stockham autosort passes in global memory, radix 4 (and one
 //     radix-2 pass for odd log2 N), twiddles from sincos in FP64.
 //
 // Transforms are addressed as base + outer*stride_outer + inner*stride_inner
@@ -114,12 +117,27 @@ __global__ void k_copy(const T2 *in, T2 *out, int N, int64_t total, int nb_inner
 
 // Radix-2 DIT transforms larger than one workgroup's LDS, with the same
 // butterflies and twiddles as lds_fft (so FP64 results are bit-identical to
-// the in-LDS form): the first log2 C stages run in LDS on the C-point runs
-// of the bit-reversed sequence (data -> tmp), the remaining stages as
-// global butterfly passes (tmp in place; the last pass writes data).
+// the in-LDS form), in two launches: the first log2 C stages run in LDS on
+// the C-point runs of the bit-reversed sequence (k_r2_runs, source -> tmp),
+// the remaining log2 R stages, R = N/C, on the columns j of the R x C array
+// of runs (k_r2_cols: kCols columns a workgroup, R x kCols points in LDS).
+// A launch per remaining stage instead moved the array once a stage: the
+// four 131,072-point comb transforms of a batch took 16 + 50 + 4 x 5.7 us
+// (gather, runs of 8192, passes), and 64 runs left most CUs idle; runs of
+// 1024 read straight from the signals (28 us, bound by the reads' latency)
+// and one column launch (13 us) do the same beside the same fold.
 //
 // Run c of the bit-reversed sequence holds x[q*R + bitrev(c)] at LDS
-// position bitrev(q), q < C, R = N/C runs.
+// position bitrev(q), q < C.
+template <typename T2>
+__device__ __forceinline__ void r2_run(T2 *buf, T2 *out, int logC, const T2 *tw, int tw_nmax)
+{
+  const int C = 1 << logC;
+  __syncthreads();
+  lds_fft(buf, logC, tw, tw_nmax >> logC);
+  for (int q = threadIdx.x; q < C; q += blockDim.x) out[q] = buf[q];
+}
+
 template <typename T2>
 __global__ void __launch_bounds__(kBlock) k_r2_runs(const T2 *data, T2 *tmp, int logN, int logC,
                                                   int nb_inner, int64_t so, int64_t si,
@@ -134,32 +152,106 @@ __global__ void __launch_bounds__(kBlock) k_r2_runs(const T2 *data, T2 *tmp, int
   const int64_t base = fft_base(t, nb_inner, so, si);
   const T2 *in = data + base + bitrev(c, logR);
   for (int q = threadIdx.x; q < C; q += blockDim.x) buf[bitrev(q, logC)] = in[(int64_t)q << logR];
-  __syncthreads();
-  lds_fft(buf, logC, tw, tw_nmax >> logC);
-  T2 *out = tmp + base + ((int64_t)c << logC);
-  for (int q = threadIdx.x; q < C; q += blockDim.x) out[q] = buf[q];
+  r2_run(buf, tmp + base + ((int64_t)c << logC), logC, tw, tw_nmax);
 }
 
-// Stage s (span 2^s) of every transform: one butterfly per thread.
-template <typename T2>
-__global__ void __launch_bounds__(256) k_r2_pass(const T2 *src, T2 *dst, int logN, int s,
-                                                 int64_t total, int nb_inner, int64_t so,
-                                                 int64_t si, const T2 *tw, int tw_nmax)
+// The runs of the comb transforms: point i of transform t = (s, c) is
+// x[s][off + i * sigma], off the comb loop's draw (params row s, entry
+// at + c); transforms W apart in tmp.
+__global__ void __launch_bounds__(kBlock) k_comb_runs(const double2 *const *x, const int *params,
+                                                    int stride, int at, int cl, int sigma,
+                                                    double2 *tmp, int logN, int logC,
+                                                    const double2 *tw, int tw_nmax)
 {
-  const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= total) return;
-  const int64_t t = g >> (logN - 1);
-  const int b = (int)(g & ((1 << (logN - 1)) - 1));
+  extern __shared__ char smem_raw[];
+  double2 *buf = reinterpret_cast<double2 *>(smem_raw);
+  const int C = 1 << logC;
+  const int logR = logN - logC;
+  const int t = blockIdx.x >> logR;
+  const int c = blockIdx.x & ((1 << logR) - 1);
+  const int s = t / cl;
+  const double2 *in = x[s] + params[(int64_t)s * stride + at + t % cl];
+  const int64_t first = (int64_t)bitrev(c, logR) * sigma, step = (int64_t)sigma << logR;
+  for (int q = threadIdx.x; q < C; q += blockDim.x) buf[bitrev(q, logC)] = in[first + q * step];
+  r2_run(buf, tmp + ((int64_t)t << logN) + ((int64_t)c << logC), logC, tw, tw_nmax);
+}
+
+// Stages logC + sc .. logC + sc + P - 1 of kCols columns held in LDS as
+// buf[c * kCols + column], as lds_fft_pass.
+constexpr int kCols = 16;
+
+template <typename T2, int P>
+__device__ __forceinline__ void cols_pass(T2 *buf, int logR, int logC, int sc, int j0,
+                                          const T2 *__restrict__ tw, int tw_nmax)
+{
+  constexpr int M = 1 << P;
+  const int h = 1 << (sc - 1);
+  const int groups = (kCols << logR) >> P;
+  for (int g = threadIdx.x; g < groups; g += blockDim.x) {
+    const int jj = g & (kCols - 1), gc = g / kCols;
+    const int jc = gc & (h - 1);
+    const int c0 = ((gc >> (sc - 1)) << (sc - 1 + P)) + jc;
+    T2 v[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) v[m] = buf[(c0 + m * h) * kCols + jj];
+#pragma unroll
+    for (int r = 0; r < P; r++) {
+      const int tstride = tw_nmax >> (logC + sc + r);
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        if (m & (1 << r)) continue;
+        const int m1 = m + (1 << r);
+        const T2 w = tw[(((jc + (m & ((1 << r) - 1)) * h) << logC) + j0 + jj) * tstride];
+        const T2 u = v[m];
+        const T2 t = cmul(v[m1], w);
+        v[m] = cadd(u, t);
+        v[m1] = csub(u, t);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < M; m++) buf[(c0 + m * h) * kCols + jj] = v[m];
+  }
+  __syncthreads();
+}
+
+// Columns j0 .. j0 + kCols - 1 of every transform, src -> dst; with MAG the
+// powers |.|^2 go to mag (transform t at t N) instead.
+template <typename T2, bool MAG>
+__global__ void __launch_bounds__(kBlock) k_r2_cols(const T2 *src, T2 *dst, double *mag, int logN,
+                                                    int logC, int nb_inner, int64_t so,
+                                                    int64_t si, const T2 *tw, int tw_nmax)
+{
+  extern __shared__ char smem_raw[];
+  T2 *buf = reinterpret_cast<T2 *>(smem_raw);
+  const int logR = logN - logC;
+  const int per = (1 << logC) / kCols;
+  const int64_t t = blockIdx.x / (unsigned)per;
+  const int j0 = (int)(blockIdx.x % (unsigned)per) * kCols;
   const int64_t base = fft_base(t, nb_inner, so, si);
-  const int h = 1 << (s - 1);
-  const int j = b & (h - 1);
-  const int i0 = ((b >> (s - 1)) << s) + j;
-  const int i1 = i0 + h;
-  const T2 w = tw[j * (tw_nmax >> s)];
-  const T2 u = src[base + i0];
-  const T2 v = cmul(src[base + i1], w);
-  dst[base + i0] = cadd(u, v);
-  dst[base + i1] = csub(u, v);
+  const int pts = kCols << logR;
+  for (int e = threadIdx.x; e < pts; e += blockDim.x)
+    buf[e] = src[base + ((int64_t)(e / kCols) << logC) + j0 + (e & (kCols - 1))];
+  __syncthreads();
+  int sc = 1;
+  for (; logR - sc + 1 >= 3; sc += 3) cols_pass<T2, 3>(buf, logR, logC, sc, j0, tw, tw_nmax);
+  if (logR - sc + 1 == 2) cols_pass<T2, 2>(buf, logR, logC, sc, j0, tw, tw_nmax);
+  else if (logR - sc + 1 == 1) cols_pass<T2, 1>(buf, logR, logC, sc, j0, tw, tw_nmax);
+  for (int e = threadIdx.x; e < pts; e += blockDim.x) {
+    const int64_t i = ((int64_t)(e / kCols) << logC) + j0 + (e & (kCols - 1));
+    const T2 z = buf[e];
+    if constexpr (MAG) mag[(t << logN) + i] = z.x * z.x + z.y * z.y;
+    else dst[base + i] = z;
+  }
+}
+
+// log2 C of an N-point transform in two launches: the largest run up to
+// 2^most that still gives the chip 512 workgroups, at least 2^10 points and
+// no more than 512 rows of columns.
+inline int run_log(int logN, int most, int64_t nb)
+{
+  int c = std::min(most, logN - 1);
+  while (c > 10 && c > logN - 9 && (nb << (logN - c)) < 512) c--;
+  return c;
 }
 
 template <typename T2>
@@ -172,26 +264,23 @@ int radix2(T2 *data, T2 *tmp, int N, int C, int64_t nb_outer, int nb_inner, int6
   while ((1 << logN) < N) logN++;
   while ((1 << logC) < C) logC++;
   const int64_t nb = nb_outer * nb_inner;
-  const int L = std::min(logN, logC);
-  const size_t lds = ((size_t)1 << L) * sizeof(T2);
-  if (lds > 65536) {
-    raise_lds_limit(reinterpret_cast<const void *>(k_lds_fft_batch<T2>));
-    raise_lds_limit(reinterpret_cast<const void *>(k_r2_runs<T2>));
-  }
   if (logN <= logC) {
+    const size_t lds = ((size_t)1 << logN) * sizeof(T2);
+    if (lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_lds_fft_batch<T2>));
     if (nb >= (1LL << 31)) return -1;
     hipLaunchKernelGGL(k_lds_fft_batch<T2>, dim3((unsigned)nb), dim3(kBlock), lds, st, data,
                        logN, nb_inner, so, si, tw, tw_nmax / N);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
-  if (!tmp || (nb << (logN - logC)) >= (1LL << 31)) return -1;
-  hipLaunchKernelGGL(k_r2_runs<T2>, dim3((unsigned)(nb << (logN - logC))), dim3(kBlock), lds,
+  logC = run_log(logN, logC, nb);
+  const size_t run_lds = sizeof(T2) << logC, col_lds = (sizeof(T2) * kCols) << (logN - logC);
+  if (!tmp || (nb << std::max(logN - logC, logC - 4)) >= (1LL << 31)) return -1;
+  if (run_lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_r2_runs<T2>));
+  if (col_lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_r2_cols<T2, false>));
+  hipLaunchKernelGGL(k_r2_runs<T2>, dim3((unsigned)(nb << (logN - logC))), dim3(kBlock), run_lds,
                      st, data, tmp, logN, logC, nb_inner, so, si, tw, tw_nmax);
-  const int64_t total = nb << (logN - 1);
-  const dim3 grid((unsigned)((total + 255) / 256));
-  for (int s = logC + 1; s <= logN; s++)
-    hipLaunchKernelGGL(k_r2_pass<T2>, grid, dim3(256), 0, st, tmp, s == logN ? data : tmp, logN,
-                       s, total, nb_inner, so, si, tw, tw_nmax);
+  hipLaunchKernelGGL((k_r2_cols<T2, false>), dim3((unsigned)(nb << (logC - 4))), dim3(kBlock),
+                     col_lds, st, tmp, data, nullptr, logN, logC, nb_inner, so, si, tw, tw_nmax);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -266,6 +355,26 @@ int radix2_fft32(float2 *data, float2 *tmp, int N, int64_t nb_outer, int nb_inne
 {
   return radix2<float2>(data, tmp, N, 2 * kMaxLdsFft64, nb_outer, nb_inner, so, si, tw,
                         tw_nmax, st);
+}
+
+int comb_power(const V12Launch &a, hipStream_t st)
+{
+  int logN = 0;
+  while ((1 << logN) < a.W) logN++;
+  const int64_t nb = (int64_t)a.S * a.comb_loops;
+  const int logC = run_log(logN, 13, nb);
+  const size_t run_lds = sizeof(double2) << logC;
+  const size_t col_lds = (sizeof(double2) * kCols) << (logN - logC);
+  if (a.tw_nmax < a.W || (nb << std::max(logN - logC, logC - 4)) >= (1LL << 31)) return -1;
+  if (run_lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_comb_runs));
+  if (col_lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_r2_cols<double2, true>));
+  hipLaunchKernelGGL(k_comb_runs, dim3((unsigned)(nb << (logN - logC))), dim3(kBlock), run_lds, st,
+                     a.x, a.params, 2 * a.L + std::max(a.comb_loops, 1), 2 * a.L, a.comb_loops,
+                     a.n / a.W, a.comb_buf, logN, logC, a.tw64, a.tw_nmax);
+  hipLaunchKernelGGL((k_r2_cols<double2, true>), dim3((unsigned)(nb << (logC - 4))), dim3(kBlock),
+                     col_lds, st, a.comb_buf, nullptr, a.mag_buf, logN, logC, 1, (int64_t)a.W,
+                     (int64_t)a.W, a.tw64, a.tw_nmax);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int batch_fft64(double2 *data, double2 *tmp, int N, int64_t nb_outer, int nb_inner,

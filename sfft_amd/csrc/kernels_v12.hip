@@ -31,6 +31,13 @@ namespace {
 
 __device__ __forceinline__ int ilog2(int v) { return 31 - __clz(v); }
 
+inline int pow2_ceil_int(int v)
+{
+  int p = 1;
+  while (p < v) p <<= 1;
+  return p;
+}
+
 __device__ __forceinline__ int64_t loop_offset(int l, int Lloc, int Bl, int Be)
 {
   return (int64_t)min(l, Lloc) * Bl + (int64_t)max(0, l - Lloc) * Be;
@@ -41,6 +48,10 @@ inline int64_t loop_offset_host(int l, int Lloc, int Bl, int Be)
   return (int64_t)std::min(l, Lloc) * Bl + (int64_t)std::max(0, l - Lloc) * Be;
 }
 
+// Levels of a selection above the LDS size: threads, entries picked per
+// chunk at most, entries per chunk, and of the last level.
+constexpr int kTopThreads = 512, kTopMax = 4096, kTopChunk = 4096, kTopLast = 16384;
+
 // ---------------------------------------------------------------- comb
 // One block per (signal, comb loop).  LDS: W double2.  TB threads: kBlock
 // for batches; more for a few signals, whose comb is on the latency path.
@@ -48,7 +59,7 @@ template <int TB>
 __global__ void __launch_bounds__(TB) k_comb(V12Launch a)
 {
   extern __shared__ double2 smem64[];
-  __shared__ int sh[256 + 16];
+  __shared__ int sh[256 + 32];
   const int cl = a.comb_loops;
   const int s = blockIdx.x / cl, c = blockIdx.x % cl;
   const int stride = 2 * a.L + max(cl, 1);
@@ -88,35 +99,55 @@ __global__ void __launch_bounds__(TB) k_comb(V12Launch a)
   }
 }
 
-// W above the LDS limit: the strided sub-samples go to comb_buf, the W-point
-// FFTs run as LDS radix-2 runs plus global passes, then k_comb_select_global.
-__global__ void k_comb_gather(V12Launch a)
-{
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int cl = a.comb_loops, W = a.W;
-  if (t >= (int64_t)a.S * cl * W) return;
-  const int i = (int)(t % W);
-  const int64_t sc = t / W;
-  const int s = (int)(sc / cl), c = (int)(sc % cl);
-  const int stride = 2 * a.L + max(cl, 1);
-  const int off = a.params[(int64_t)s * stride + 2 * a.L + c];
-  a.comb_buf[t] = a.x[s][(int64_t)off + (int64_t)i * (a.n / W)];
-}
+// Selections above the LDS size, in levels: block (t, chunk) takes `chunk`
+// entries of row t's list (the first level: every index of the row) and
+// writes the num largest of them, by block_top_num's rule, in list order, to
+// its place of the next list.  An entry in the row's num largest is in its
+// chunk's, and the lists stay in index order, so the last level (one chunk)
+// picks what one selection over the whole row would, ties included.  One
+// 256-thread workgroup over a whole row took 660 us for 100 of 131,072; two
+// levels (chunks of 4096, then 3200 candidates) take 28 us.
+struct TopLevel {
+  const double *mag;    // rows of `row` powers; null: |xs64|^2 of the v1 loops
+  int64_t row;
+  const int *list;      // entries per row: list_len (null on the first level)
+  int list_len, chunk, chunks;
+  int num;
+  int *out;             // per row: out_stride entries, num per chunk
+  int64_t out_stride;
+  bool comb_last;       // last level of a single comb loop: counts too
+};
 
-__global__ void __launch_bounds__(kBlock) k_comb_select_global(V12Launch a)
+__global__ void __launch_bounds__(kTopThreads) k_top_level(V12Launch a, TopLevel v)
 {
-  __shared__ int sh[256 + 16];
-  const int cl = a.comb_loops, W = a.W;
-  const int s = blockIdx.x / cl, c = blockIdx.x % cl;
-  const double2 *z = a.comb_buf + (int64_t)blockIdx.x * W;
-  double *mag = a.mag_buf + (int64_t)blockIdx.x * W;
-  for (int i = threadIdx.x; i < W; i += blockDim.x) mag[i] = z[i].x * z[i].x + z[i].y * z[i].y;
-  __threadfence_block();
+  extern __shared__ double lds_mag[];
+  __shared__ int sh[256 + 32];
+  __shared__ int pick[kTopMax];
+  const int t = (int)(blockIdx.x / (unsigned)v.chunks), ch = (int)(blockIdx.x % (unsigned)v.chunks);
+  const int e0 = ch * v.chunk, len = min(v.chunk, v.list_len - e0);
+  const int *list = v.list ? v.list + (int64_t)t * v.list_len + e0 : nullptr;
+  const double *mag = v.mag ? v.mag + t * v.row : nullptr;
+  const double2 *z = a.xs64 + (int64_t)(t / a.Lloc) * a.xs + (int64_t)(t % a.Lloc) * a.B_loc;
+  for (int i = threadIdx.x; i < len; i += blockDim.x) {
+    const int e = list ? list[i] : e0 + i;
+    if (mag) {
+      lds_mag[i] = mag[e];
+    } else {
+      const double2 y = z[e];
+      lds_mag[i] = y.x * y.x + y.y * y.y;
+    }
+  }
   __syncthreads();
-  block_top_num(mag, W, a.num, a.approved + ((int64_t)s * cl + c) * a.num, sh);
-  if (cl == 1 && threadIdx.x == 0) {
-    a.num_comb[s] = a.num;
-    a.count[s] = (int64_t)a.num * (a.n / W);
+  int *out = v.out + (int64_t)t * v.out_stride + (int64_t)ch * v.num;
+  const int take = min(v.num, len);
+  if (len > v.num) block_top_num(lds_mag, len, v.num, pick, sh);
+  for (int i = threadIdx.x; i < take; i += blockDim.x) {
+    const int p = len > v.num ? pick[i] : i;
+    out[i] = list ? list[p] : e0 + p;
+  }
+  if (v.comb_last && threadIdx.x == 0) {
+    a.num_comb[t] = a.num;
+    a.count[t] = (int64_t)a.num * (a.n / a.W);
   }
 }
 
@@ -510,7 +541,7 @@ template <bool GLOBAL>
 __global__ void __launch_bounds__(kBlock) k_select(V12Launch a)
 {
   extern __shared__ double lds_mag[];
-  __shared__ int sh[256 + 16];
+  __shared__ int sh[256 + 32];
   // above the LDS size the magnitudes go to mag_buf
   double *mag = GLOBAL ? a.mag_buf + (int64_t)blockIdx.x * a.B_loc : lds_mag;
   const int s = blockIdx.x / a.Lloc, l = blockIdx.x % a.Lloc;
@@ -1334,6 +1365,44 @@ void *noalloc_scratch(int dev)
   return g_scratch[dev];
 }
 
+// The a.num largest of each of `rows` rows of `len` entries (powers at mag,
+// null: the v1 loops' |xs64|^2) into out, a.num per row; lists: 2 len ints of
+// scratch per row.
+static int top_levels(const V12Launch &a, hipStream_t st, const double *mag, int len, int rows,
+                      int *lists, int *out, bool comb_last)
+{
+  TopLevel v;
+  v.mag = mag;
+  v.row = len;
+  v.list = nullptr;
+  v.num = a.num;
+  int *next = lists, *other = lists + (int64_t)rows * len;
+  if (a.num > kTopMax) {
+    set_error("selection of more than 4096 entries above the LDS size");
+    return -1;
+  }
+  while (true) {
+    v.list_len = len;
+    const bool last = len <= kTopLast;
+    // every level at least halves the list: num is at most half a chunk
+    v.chunk = last ? len : std::max(kTopChunk, 2 * pow2_ceil_int(a.num));
+    v.chunks = (len + v.chunk - 1) / v.chunk;
+    v.out = last ? out : next;
+    const int left = (v.chunks - 1) * v.num + std::min(v.num, len - (v.chunks - 1) * v.chunk);
+    v.out_stride = last ? v.num : left;
+    v.comb_last = last && comb_last;
+    const size_t lds = (size_t)v.chunk * sizeof(double);
+    allow_lds(k_top_level, lds + kTopMax * sizeof(int));  // with its static picks
+    hipLaunchKernelGGL(k_top_level, dim3((unsigned)(rows * v.chunks)), dim3(kTopThreads), lds, st,
+                       a, v);
+    if (launched("top_level") != 0) return -1;
+    if (last) return 0;
+    v.list = next;
+    std::swap(next, other);
+    len = left;
+  }
+}
+
 // Below this many comb transforms per batch they run with kCombWide threads.
 constexpr int kFewCombs = 64, kCombWide = 1024;
 
@@ -1351,17 +1420,14 @@ int comb(const V12Launch &a, hipStream_t st)
     }
     if (launched("comb") != 0) return -1;
   } else {
-    const int64_t total = (int64_t)a.S * a.comb_loops * a.W;
-    hipLaunchKernelGGL(k_comb_gather, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       a);
-    if (launched("comb_gather") != 0) return -1;
-    if (radix2_fft64(a.comb_buf, a.comb_tmp, a.W, (int64_t)a.S * a.comb_loops, 1, a.W, a.W,
-                     a.tw64, a.tw_nmax, st) != 0) {
+    if (comb_power(a, st) != 0) {
       set_error("comb FFT launch failed");
       return -1;
     }
-    hipLaunchKernelGGL(k_comb_select_global, dim3(a.S * a.comb_loops), dim3(kBlock), 0, st, a);
-    if (launched("comb_select") != 0) return -1;
+    int *lists = reinterpret_cast<int *>(a.comb_buf);  // the transforms are done
+    if (top_levels(a, st, a.mag_buf, a.W, a.S * a.comb_loops, lists, a.approved,
+                   a.comb_loops == 1) != 0)
+      return -1;
   }
   if (a.comb_loops > 1) {
     const size_t lb = (size_t)((a.W + 31) / 32) * 4;
@@ -1520,16 +1586,25 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
   return launches;
 }
 
-int select_vote_v1(const V12Launch &a, hipStream_t st)
+// The top buckets of every location loop: in LDS up to its size, above it
+// in levels; more picks than a level takes, over the HBM array.
+static int select_loops(const V12Launch &a, hipStream_t st)
 {
   if (a.B_loc <= kMaxLdsSelect) {
     allow_lds(k_select<false>, (size_t)a.B_loc * sizeof(double));
     hipLaunchKernelGGL(k_select<false>, dim3(a.S * a.Lloc), dim3(kBlock),
                        (size_t)a.B_loc * sizeof(double), st, a);
+  } else if (a.num <= kTopMax) {
+    return top_levels(a, st, nullptr, a.B_loc, a.S * a.Lloc, a.cand_buf, a.J, false);
   } else {
     hipLaunchKernelGGL(k_select<true>, dim3(a.S * a.Lloc), dim3(kBlock), 0, st, a);
   }
-  if (launched("select") != 0) return -1;
+  return launched("select");
+}
+
+int select_vote_v1(const V12Launch &a, hipStream_t st)
+{
+  if (select_loops(a, st) != 0) return -1;
   const size_t lb = (size_t)a.Lloc * ((a.B_loc + 31) / 32) * 4;
   const int chunks = vote_chunks(a.n, a.B_loc, a.num, a.Lloc, a.thr);
   const dim3 grid((unsigned)((int64_t)a.S * chunks));
@@ -1543,14 +1618,7 @@ int select_vote_v1(const V12Launch &a, hipStream_t st)
 
 int comb_vote_keys(const V12Launch &a, int64_t *keys, int64_t stride, hipStream_t st)
 {
-  if (a.B_loc <= kMaxLdsSelect) {
-    allow_lds(k_select<false>, (size_t)a.B_loc * sizeof(double));
-    hipLaunchKernelGGL(k_select<false>, dim3(a.S * a.Lloc), dim3(kBlock),
-                       (size_t)a.B_loc * sizeof(double), st, a);
-  } else {
-    hipLaunchKernelGGL(k_select<true>, dim3(a.S * a.Lloc), dim3(kBlock), 0, st, a);
-  }
-  if (launched("select (v2 votes)") != 0) return -1;
+  if (select_loops(a, st) != 0) return -1;
   const int64_t chunks = (a.est_cap + kBlock - 1) / kBlock;
   const size_t lb = (size_t)a.Lloc * ((a.B_loc + 31) / 32) * 4;
   allow_lds(k_comb_vote_keys, lb);

@@ -525,3 +525,25 @@ def test_sorted_fold_buckets(torch_cuda, version, n, k, signals):
                 want = oracle.fp32_buckets(xs[-1], n, B, lt if loc else et, ai[l], 256, nmax)
             assert np.array_equal(got[at:at + B], want), (precision, l)
             at += B
+
+
+@pytest.mark.parametrize("version,n,k,tones", [
+    (2, 1 << 20, 50, 0),     # W = 16384, two comb loops: all powers tie at zero
+    (2, 1 << 20, 50, 3),     # fewer tones than picks, the rest leakage
+    (2, 1 << 24, 10, 0),     # W = 2^18
+    (1, 1 << 24, 2000, 0),   # v1: 4000 of 32768 buckets, ties
+    (1, 1 << 24, 2000, 5),
+])
+def test_selection_levels(torch_cuda, version, n, k, tones):
+    """Selections above the LDS size pick the oracle's indices, ties at the
+    cutoff in index order."""
+    print(f"case selection v{version} n={n} k={k} tones={tones}", flush=True)
+    x = np.zeros(n, np.complex128)
+    if tones:
+        x, f, v = signal_np(n, tones, seed=12)
+    plan = _gpu_plan(version, n, k)
+    ref = _oracle_run(version, n, k, x, _plan_filters(plan))
+    out = _run_gpu_dense(torch_cuda, plan, x)
+    fr, va = _gpu_plan(version, n, k).execute_sparse_host(x)
+    assert np.array_equal(np.unique(fr), _located(ref, version))
+    assert np.array_equal(out, ref["out"])

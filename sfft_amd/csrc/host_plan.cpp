@@ -264,6 +264,10 @@ int64_t Plan::bytes_per_signal() const
   if (fp32 && Bm > 2 * kMaxLdsFft64) b += xs * 8;
   if (p.comb && p.W_comb > k::kMaxLdsComb) b += (int64_t)p.comb_loops * p.W_comb * 24;
   if (!p.comb && p.B_loc > k::kMaxLdsSelect) b += (int64_t)p.loc_loops * p.B_loc * 8;
+  // estimation entries of the alias-row layout (whether or not it applies)
+  if (p.comb)
+    b += (int64_t)p.comb_loops * p.B_thresh * p.loops() * (int64_t)k::rows_entry_bytes(fp32) +
+         4LL * p.loops();
   if (!p.comb) b += 4LL * k::vote_chunks(n, p.B_loc, p.B_thresh, p.loc_loops, p.thr_loops);
   return b + (int64_t)p.comb_loops * p.B_thresh * 4 + (int64_t)p.loc_loops * p.B_thresh * 4 +
          output_capacity() * (4 + 16 + 4) + (2 * p.loops() + p.comb_loops + 8) * 4;
@@ -428,7 +432,7 @@ size_t Workspace::device_bytes() const
 {
   const DevBuf *bufs[] = {&params, &xsamp, &xsamp32, &approved, &numcomb, &J, &hits,
                           &ptrs, &out_freq, &out_val, &count, &stage, &v3, &v3_status,
-                          &comb, &mag, &tmp64, &tmp32, &multi, &votes};
+                          &comb, &mag, &tmp64, &tmp32, &multi, &rows, &votes};
   size_t b = 0;
   for (const DevBuf *d : bufs) b += d->bytes;
   return b;
@@ -438,7 +442,7 @@ void Workspace::use_arena(Arena *a)
 {
   DevBuf *bufs[] = {&params, &xsamp, &xsamp32, &approved, &numcomb, &J, &hits,
                     &ptrs, &out_freq, &out_val, &count, &stage, &v3, &v3_status,
-                    &comb, &mag, &tmp64, &tmp32, &multi, &votes};
+                    &comb, &mag, &tmp64, &tmp32, &multi, &rows, &votes};
   for (DevBuf *d : bufs) d->arena = a;
 }
 
@@ -446,7 +450,7 @@ void Workspace::release()
 {
   DevBuf *bufs[] = {&params, &xsamp, &xsamp32, &approved, &numcomb, &J, &hits,
                     &ptrs, &out_freq, &out_val, &count, &stage, &v3, &v3_status,
-                    &comb, &mag, &tmp64, &tmp32, &multi, &votes};
+                    &comb, &mag, &tmp64, &tmp32, &multi, &rows, &votes};
   for (DevBuf *d : bufs) d->release();
   if (pinned && !pinned_view) (void)hipHostFree(pinned);
   pinned = nullptr;
@@ -824,7 +828,7 @@ static uint64_t workspace_signature(const Workspace &w)
 {
   const void *ptrs[] = {w.params.p, w.xsamp.p, w.xsamp32.p, w.approved.p, w.numcomb.p, w.J.p,
                         w.hits.p, w.ptrs.p, w.count.p, w.comb.p, w.mag.p, w.tmp64.p,
-                        w.tmp32.p, w.pinned};
+                        w.tmp32.p, w.rows.p, w.pinned};
   uint64_t h = 1469598103934665603ull;
   for (const void *q : ptrs) {
     h ^= (uint64_t)(uintptr_t)q;
@@ -874,6 +878,11 @@ static k::V12Launch sub_launch(const k::V12Launch &a, int base, int cnt, int str
   if (a.J) b.J = a.J + s0 * a.Lloc * a.num;
   if (a.hits) b.hits = a.hits + s0 * a.hits_cap;
   if (a.vote_cnt) b.vote_cnt = a.vote_cnt + s0 * vchunks;
+  if (a.rows_layout) {
+    b.rows_tab = static_cast<char *>(a.rows_tab) +
+                 s0 * a.comb_loops * a.num * a.L * (int64_t)k::rows_entry_bytes(a.fp32);
+    b.rows_odd = a.rows_odd + s0 * a.L;
+  }
   b.count = a.count + s0;
   if (a.o_freq) b.o_freq = a.o_freq + s0;
   if (a.o_val) b.o_val = a.o_val + s0;
@@ -946,6 +955,17 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
       (big64 && !P->ws->tmp64.ensure((size_t)S * xs * 16)) ||
       (big32 && !P->ws->tmp32.ensure((size_t)S * xs * 8)))
     return -1;
+  // the fused fold + FFT keeps a whole bucket array in LDS
+  const int fold_mode = std::max(p.B_loc, p.B_est) > kMaxLdsFft64 ? std::max(1, P->fold_mode)
+                                                                 : P->fold_mode;
+  // alias-row bucket layout (schedule 1): v2, W a multiple of n/B for both
+  // loop kinds, at least one wavefront of alias rows, FFTs in LDS
+  const bool rows_layout = p.comb && fold_mode == 1 && !dbg_votes &&
+                           p.W_comb % (n / p.B_loc) == 0 && p.W_comb % (n / p.B_est) == 0 &&
+                           n / p.W_comb >= 64 &&
+                           std::max(p.B_loc, p.B_est) <= (fp32 ? 2 : 1) * kMaxLdsFft64;
+  const size_t tab_rows = rows_layout ? ((size_t)S * cl * num * L * k::rows_entry_bytes(fp32) + 15) / 16 * 16 : 0;
+  if (rows_layout && !P->ws->rows.ensure(tab_rows + (size_t)S * L * sizeof(int))) return -1;
   // RNG draws in signal order (src/computefourier-1.0-2.0.cc:465-474, 62),
   // made once every buffer is in place so that a call failing above
   // consumes none.
@@ -1020,14 +1040,10 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   a.cand_buf = big_sel ? P->ws->mag.as<int>() : nullptr;
   a.tmp64 = big64 ? P->ws->tmp64.as<double2>() : nullptr;
   a.tmp32 = big32 ? P->ws->tmp32.as<float2>() : nullptr;
-  // the fused fold + FFT keeps a whole bucket array in LDS
-  a.fold_mode = std::max(p.B_loc, p.B_est) > kMaxLdsFft64 ? std::max(1, P->fold_mode)
-                                                          : P->fold_mode;
-  // alias-row bucket layout (schedule 1): v2, W a multiple of n/B for both
-  // loop kinds, at least one wavefront of alias rows, FFTs in LDS
-  a.rows_layout = p.comb && a.fold_mode == 1 && !dbg_votes && p.W_comb % (n / p.B_loc) == 0 &&
-                  p.W_comb % (n / p.B_est) == 0 && n / p.W_comb >= 64 &&
-                  std::max(p.B_loc, p.B_est) <= (fp32 ? 2 : 1) * kMaxLdsFft64;
+  a.fold_mode = fold_mode;
+  a.rows_layout = rows_layout;
+  a.rows_tab = rows_layout ? P->ws->rows.p : nullptr;
+  a.rows_odd = rows_layout ? reinterpret_cast<int *>(P->ws->rows.as<char>() + tab_rows) : nullptr;
   P->last_rows_layout = a.rows_layout;
 
   // an arena workspace creates no runtime objects: no timing events, no

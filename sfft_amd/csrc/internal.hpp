@@ -168,6 +168,7 @@ struct Workspace {
   // bucket FFT passes)
   DevBuf comb, mag, tmp64, tmp32;
   DevBuf multi;  // descriptors of a multi-plan launch
+  DevBuf rows;   // alias-row estimation: table entries and bucket flags
   DevBuf votes;  // v2 comb-vote diagnostic: S x 2 x located int64
   void *pinned = nullptr;
   size_t pinned_bytes = 0;
@@ -367,7 +368,10 @@ struct V12Launch {
   // v2 with W a multiple of n/B: buckets after the FFT stored by alias row
   // (see k_bucket_fft_rows); estimation reads them contiguously
   bool rows_layout;
+  void *rows_tab;  // S x comb_loops*num x L estimation entries (rows_entry_bytes each)
+  int *rows_odd;   // FP64: S x L, buckets the estimate has to divide
 };
+size_t rows_entry_bytes(bool fp32);
 // Blocks per signal of the v1 vote: its candidates (the ranges of the
 // selected buckets of loops 0..Lloc-thr) in chunks of 8 * 256.
 inline int vote_chunks(int n, int B_loc, int num, int Lloc, int thr)

@@ -833,25 +833,28 @@ __device__ __forceinline__ double median20(double (&v)[LMAX])
   return m;
 }
 
+// Lower median (rank (L-1)/2) of v[0..L), slots past L holding +inf.
+template <int LMAX>
+__device__ __forceinline__ double lower_median1(double (&v)[LMAX], int L)
+{
+  if constexpr (LMAX == 20) {
+    if (L == 20) return median20<LMAX>(v);
+  }
+  sort_net<LMAX>(v);
+  const int rank = (L - 1) / 2;
+  double m = v[0];
+#pragma unroll
+  for (int l = 1; l < LMAX; l++)
+    if (l == rank) m = v[l];
+  return m;
+}
+
 template <int LMAX>
 __device__ __forceinline__ double2 lower_median(double (&vr)[LMAX], double (&vi)[LMAX],
                                                 int L)
 {
-  if constexpr (LMAX == 20) {
-    if (L == 20) return make_double2(median20<LMAX>(vr), median20<LMAX>(vi));
-  }
-  sort_net<LMAX>(vr);
-  sort_net<LMAX>(vi);
-  const int rank = (L - 1) / 2;
-  double mr = vr[0], mi = vi[0];
-#pragma unroll
-  for (int l = 1; l < LMAX; l++) {
-    if (l == rank) {
-      mr = vr[l];
-      mi = vi[l];
-    }
-  }
-  return make_double2(mr, mi);
+  const double re = lower_median1<LMAX>(vr, L);
+  return make_double2(re, lower_median1<LMAX>(vi, L));
 }
 
 __device__ __forceinline__ double2 load_bucket(const V12Launch &a, bool fp32, bool isloc,
@@ -1112,7 +1115,17 @@ __device__ __forceinline__ unsigned inv_odd(unsigned a)
   return x;
 }
 
+// Zero or of a magnitude whose quotients by a filter power near one neither
+// overflow nor lose bits to underflow on the way (false for infinities and
+// NaN): the FP64 estimate divides such buckets by a tabulated reciprocal.
+__device__ __forceinline__ bool plain_value(double v)
+{
+  const double m = fabs(v);
+  return m == 0.0 || (m >= 0x1p-700 && m <= 0x1p700);
+}
+
 // Bucket FFTs of loops [l0, l0 + nl), written in the alias-row layout.
+// FP64: rows_odd[s L + l] says whether any bucket is not a plain value.
 template <bool FP32>
 __global__ void __launch_bounds__(kBlock) k_bucket_fft_rows(V12Launch a, int l0, int nl)
 {
@@ -1133,43 +1146,121 @@ __global__ void __launch_bounds__(kBlock) k_bucket_fft_rows(V12Launch a, int l0,
   __syncthreads();
   if constexpr (FP32) lds_fft(rbuf, logB, a.tw32, a.tw_nmax / B);
   else lds_fft(rbuf, logB, a.tw64, a.tw_nmax / B);
+  int odd = 0;
   for (int b = threadIdx.x; b < B; b += blockDim.x) {
     const int r = b % d, q = b / d;
-    io[r * rows + (int)(((unsigned)q * uinv) & (unsigned)(rows - 1))] = rbuf[b];
+    const T2 z = rbuf[b];
+    if (!FP32) odd |= !plain_value(z.x) | !plain_value(z.y);
+    io[r * rows + (int)(((unsigned)q * uinv) & (unsigned)(rows - 1))] = z;
   }
+  if (!FP32) {
+    odd = __syncthreads_or(odd);
+    if (threadIdx.x == 0) a.rows_odd[(int64_t)s * a.L + l] = odd;
+  }
+}
+
+// Per (signal, residue, loop): where the residue's bucket row lies and what
+// its buckets are multiplied or divided by.  Written once per batch by
+// k_rows_table; the workgroups of k_estimate_rows copy their residues'
+// entries to LDS (computing them there cost every 64 rows' workgroup the
+// hashing and the quotients again).
+struct RowEntry32 {
+  double gx, gy;    // G / |G|^2
+  unsigned off, q;  // byte offsets: loop l's row r; the residue's place in it
+};
+struct RowEntry64 {
+  double gx, gy;    // G
+  double den, inv;  // |G|^2 and its reciprocal
+  unsigned off, q;  // as above; bit 31 of q: not to be divided by inv
+};
+
+// One thread per (signal, residue slot, loop).
+template <bool FP32>
+__global__ void __launch_bounds__(kBlock) k_rows_table(V12Launch a)
+{
+  using Entry = typename std::conditional<FP32, RowEntry32, RowEntry64>::type;
+  constexpr unsigned kElt = FP32 ? sizeof(float2) : sizeof(double2);
+  const int L = a.L, cap = a.comb_loops * a.num;
+  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (t >= (int64_t)a.S * cap * L) return;
+  const int l = (int)(t % L);
+  const int64_t si = t / L;
+  const int s = (int)(si / cap), i = (int)(si % cap);
+  if (i >= a.num_comb[s]) return;
+  const unsigned ai =
+      (unsigned)a.params[(int64_t)s * (2 * L + max(a.comb_loops, 1)) + L + l];
+  int hashed;
+  double2 G;
+  hash_direct(a, l, ai, (unsigned)a.approved[si], hashed, G);
+  const int rows = a.n / a.W;
+  const int B = l < a.Lloc ? a.B_loc : a.B_est;
+  const int d = B / rows;
+  const unsigned uinv = inv_odd(ai) & (unsigned)(rows - 1);
+  const double den = G.x * G.x + G.y * G.y;
+  Entry e;
+  e.off = (unsigned)(loop_offset(l, a.Lloc, a.B_loc, a.B_est) + (hashed % d) * rows) * kElt;
+  e.q = (((unsigned)(hashed / d) * uinv) & (unsigned)(rows - 1)) * kElt;
+  if constexpr (FP32) {
+    e.gx = G.x / den;
+    e.gy = G.y / den;
+  } else {
+    e.gx = G.x;
+    e.gy = G.y;
+    e.den = den;
+    e.inv = 1.0 / den;
+    const bool near1 = den >= 0x1p-100 && den <= 0x1p100 &&
+                       (G.x == 0.0 || fabs(G.x) >= 0x1p-100) &&
+                       (G.y == 0.0 || fabs(G.y) >= 0x1p-100);
+    if (!near1) e.q |= 0x80000000u;
+  }
+  reinterpret_cast<Entry *>(a.rows_tab)[t] = e;
 }
 
 // Residues per tile of k_estimate_rows (RI / 4 per wavefront): 16 for
 // batches, 4 when a batch gives too few tiles to fill the chip.
 constexpr int kRI = 16, kRIsmall = 4;
 
-// Median value of one residue (table column il) at alias row jm: the L
-// bucket reads of the lane, each at byte offset t_base + (t_q + jm mod
-// rows) * sizeof(bucket) of the signal's bucket array xs (the alias-row
-// layout needs the bucket FFTs in LDS, so a signal's buckets span a few MB
-// and 32-bit offsets hold them).
-template <int LMAX, bool FULL, bool FP32, int RI>
-__device__ __forceinline__ double2 rows_median(const char *xs, const unsigned *t_base,
-                                               const int *t_q, const double2 *t_g,
-                                               const double *t_den, int il, int jm, int rows,
-                                               int L, bool conj, double sign)
+// RN(a / den) from inv = RN(1 / den): q0 is within 1.5 ulp of the quotient,
+// its residual is exact to 2^-53 of itself, and where the quotient lies next
+// to a rounding midpoint q0 is half an ulp away, so the corrected sum lies
+// on the quotient's side of the midpoint (Markstein).  Holds while nothing
+// over- or underflows: see plain_value.
+__device__ __forceinline__ double div_by(double a, double den, double inv)
 {
-  constexpr unsigned kElt = FP32 ? sizeof(float2) : sizeof(double2);
+  const double q0 = a * inv;
+  return fma(fma(-den, q0, a), inv, q0);
+}
+
+// v, negated where flip is the sign bit (exact; an integer operation)
+__device__ __forceinline__ double flip_sign(double v, unsigned flip)
+{
+  return __hiloint2double(__double2hiint(v) ^ (int)flip, __double2loint(v));
+}
+
+// Bucket of entry e at byte jm of the alias rows: a row starts on a multiple
+// of its length, so the place within it is or-ed on.
+template <typename T2, typename Entry>
+__device__ __forceinline__ T2 row_bucket(const char *xs, const Entry &e, unsigned jm,
+                                         unsigned row_mask)
+{
+  return *reinterpret_cast<const T2 *>(xs + (((e.q + jm) & row_mask) | e.off));
+}
+
+// Median value of one residue at the byte offset jm of its alias row; tab:
+// the residue's L entries in LDS, xs: the signal's buckets.
+template <int LMAX, bool FULL>
+__device__ __forceinline__ double2 rows_median(const char *xs, const RowEntry32 *tab, unsigned jm,
+                                               unsigned row_mask, int L, unsigned flip, bool)
+{
   double vr[LMAX], vi[LMAX];
 #pragma unroll
   for (int l = 0; l < LMAX; l++) {
     if (FULL || l < L) {
-      const unsigned off =
-          t_base[l * RI + il] + ((unsigned)(t_q[l * RI + il] + jm) & (unsigned)(rows - 1)) * kElt;
-      const double2 g = t_g[l * RI + il];
-      if constexpr (FP32) {
-        const float2 u = *reinterpret_cast<const float2 *>(xs + off);
-        mul_by_inverse((double)u.x, (double)u.y, g, sign, vr[l], vi[l]);
-      } else {
-        // the reference's operation order (cf12 383-398), as k_estimate_comb
-        divide_by_filter(*reinterpret_cast<const double2 *>(xs + off), g, t_den[l * RI + il],
-                         conj, vr[l], vi[l]);
-      }
+      const RowEntry32 e = tab[l];
+      const float2 u = row_bucket<float2>(xs, e, jm, row_mask);
+      const double ux = (double)u.x, uy = (double)u.y;
+      vr[l] = fma(ux, e.gx, uy * e.gy);  // as mul_by_inverse
+      vi[l] = flip_sign(fma(ux, e.gy, -(uy * e.gx)), flip);
     } else {
       vr[l] = __longlong_as_double(0x7ff0000000000000ll);  // +inf pads
       vi[l] = vr[l];
@@ -1178,17 +1269,59 @@ __device__ __forceinline__ double2 rows_median(const char *xs, const unsigned *t
   return lower_median<LMAX>(vr, vi, FULL ? LMAX : L);
 }
 
+// FP64: the reference's operation order (cf12 383-398); odd: with divisions,
+// one part and one quotient at a time (rare, so with few registers).
+template <int LMAX, bool FULL>
+__device__ __forceinline__ double2 rows_median(const char *xs, const RowEntry64 *tab, unsigned jm,
+                                               unsigned row_mask, int L, unsigned flip, bool odd)
+{
+  if (!odd) {
+    double vr[LMAX], vi[LMAX];
+#pragma unroll
+    for (int l = 0; l < LMAX; l++) {
+      if (FULL || l < L) {
+        const RowEntry64 e = tab[l];
+        const double2 u = row_bucket<double2>(xs, e, jm, row_mask);
+        vr[l] = div_by(u.x * e.gx + u.y * e.gy, e.den, e.inv);
+        vi[l] = flip_sign(div_by(u.x * e.gy - u.y * e.gx, e.den, e.inv), flip);
+      } else {
+        vr[l] = __longlong_as_double(0x7ff0000000000000ll);
+        vi[l] = vr[l];
+      }
+    }
+    return lower_median<LMAX>(vr, vi, FULL ? LMAX : L);
+  }
+  double part[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    double v[LMAX];
+#pragma unroll
+    for (int l = 0; l < LMAX; l++) {
+      if (FULL || l < L) {
+        const RowEntry64 e = tab[l];
+        const double2 u = row_bucket<double2>(xs, e, jm, row_mask);
+        v[l] = c == 0 ? (u.x * e.gx + u.y * e.gy) / e.den
+                      : flip_sign((u.x * e.gy - u.y * e.gx) / e.den, flip);
+      } else {
+        v[l] = __longlong_as_double(0x7ff0000000000000ll);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    part[c] = lower_median1<LMAX>(v, FULL ? LMAX : L);
+  }
+  return make_double2(part[0], part[1]);
+}
+
 // FULL: L == LMAX, so the loop over loops has no branch and the compiler
 // issues all bucket loads of a frequency before the first wait.
 template <int LMAX, bool FULL, bool FP32, int RI>
 __global__ void __launch_bounds__(kBlock) k_estimate_rows(V12Launch a, int tiles_i, int tiles_j)
 {
   using T2 = typename std::conditional<FP32, float2, double2>::type;
-  __shared__ unsigned t_base[RI * LMAX];  // byte offset of loop l's row r: (off_l + r*rows) * elt
-  __shared__ int t_q[RI * LMAX];        // q0 * u^-1 mod rows
-  __shared__ double2 t_g[RI * LMAX];    // FP32 form: G / |G|^2; FP64: G
-  __shared__ double t_den[FP32 ? 1 : RI * LMAX];  // FP64: |G|^2
+  using Entry = typename std::conditional<FP32, RowEntry32, RowEntry64>::type;
   __shared__ double2 stage[64 * (RI + 1)];  // [row][residue], padded
+  __shared__ Entry tab[RI * LMAX];
+  __shared__ int s_odd;
   int s;
   int64_t c;
   if (!xcd_block(blockIdx.x, a.S, (int64_t)tiles_i * tiles_j, s, c)) return;
@@ -1197,48 +1330,44 @@ __global__ void __launch_bounds__(kBlock) k_estimate_rows(V12Launch a, int tiles
   const int rows = a.n / a.W;
   if (ti * RI >= nc) return;
   const int L = a.L;
-  const int stride = 2 * L + max(a.comb_loops, 1);
-  const int *approved = a.approved + (int64_t)s * a.comb_loops * a.num;
-  for (int e = threadIdx.x; e < RI * L; e += blockDim.x) {
-    const int l = e / RI, il = e % RI;
-    const int i = ti * RI + il;
-    if (i < nc) {
-      const unsigned ai = (unsigned)a.params[(int64_t)s * stride + L + l];
-      int hashed;
-      double2 G;
-      hash_direct(a, l, ai, (unsigned)approved[i], hashed, G);
-      const int B = l < a.Lloc ? a.B_loc : a.B_est;
-      const int d = B / rows;
-      const unsigned uinv = inv_odd(ai) & (unsigned)(rows - 1);
-      const double den = G.x * G.x + G.y * G.y;
-      t_base[l * RI + il] =
-          (unsigned)(loop_offset(l, a.Lloc, a.B_loc, a.B_est) + (hashed % d) * rows) *
-          (unsigned)sizeof(T2);
-      t_q[l * RI + il] = (int)(((unsigned)(hashed / d) * uinv) & (unsigned)(rows - 1));
-      if (FP32) {
-        t_g[l * RI + il] = make_double2(G.x / den, G.y / den);
-      } else {
-        t_g[l * RI + il] = G;
-        t_den[l * RI + il] = den;
-      }
+  const int cap = a.comb_loops * a.num;
+  const int *approved = a.approved + (int64_t)s * cap;
+  {
+    // the tile's entries, contiguous in the table, copied as 8-byte words
+    const int cnt = min(RI, nc - ti * RI) * L * (int)(sizeof(Entry) / 8);
+    const uint64_t *src = reinterpret_cast<const uint64_t *>(
+        reinterpret_cast<const Entry *>(a.rows_tab) + ((int64_t)s * cap + ti * RI) * L);
+    uint64_t *dst = reinterpret_cast<uint64_t *>(tab);
+    int odd = 0;
+    for (int e = threadIdx.x; e < cnt; e += blockDim.x) {
+      const uint64_t w = src[e];
+      dst[e] = w;
+      if (!FP32 && e % (int)(sizeof(Entry) / 8) == (int)(sizeof(Entry) / 8) - 1)
+        odd |= (int)(w >> 63);
     }
+    if (!FP32) {
+      if ((int)threadIdx.x < L) odd |= a.rows_odd[(int64_t)s * L + threadIdx.x];
+      if (threadIdx.x == 0) s_odd = 0;
+      __syncthreads();
+      if (odd) s_odd = 1;
+    }
+    __syncthreads();
   }
-  __syncthreads();
   const T2 *xsig;
   if constexpr (FP32) xsig = a.xs32 + (int64_t)s * a.xs;
   else xsig = a.xs64 + (int64_t)s * a.xs;
   const char *xs = reinterpret_cast<const char *>(xsig);
-  const bool conj = a.ref_conj;
+  const bool odd = !FP32 && s_odd;
+  const unsigned flip = a.ref_conj ? 0u : 0x80000000u;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int j = tj * 64 + lane;             // one alias row per lane
-  const int jm = j & (rows - 1);
+  const unsigned row_mask = (unsigned)(rows - 1) * (unsigned)sizeof(T2);
+  const unsigned jm = (unsigned)(tj * 64 + lane) * (unsigned)sizeof(T2);  // an alias row a lane
   for (int q = 0; q < RI / 4; q++) {
     asm volatile("" ::: "memory");
-    const int il = wid * (RI / 4) + q;     // one residue per wavefront
-    if (ti * RI + il >= nc) break;         // wave-uniform; no barrier inside
+    const int il = wid * (RI / 4) + q;  // one residue per wavefront
+    if (ti * RI + il >= nc) break;      // wave-uniform; no barrier inside
     stage[lane * (RI + 1) + il] =
-        rows_median<LMAX, FULL, FP32, RI>(xs, t_base, t_q, t_g, t_den, il, jm, rows, L, conj,
-                                          a.conj_sign);
+        rows_median<LMAX, FULL>(xs, tab + il * L, jm, row_mask, L, flip, odd);
   }
   __syncthreads();
   // row by row: RI consecutive output slots per row
@@ -1434,8 +1563,17 @@ int comb(const V12Launch &a, hipStream_t st)
     hipLaunchKernelGGL(k_comb_merge, dim3(a.S), dim3(kBlock), lb, st, a);
     if (launched("comb_merge") != 0) return -1;
   }
+  if (a.rows_layout) {
+    const int64_t entries = (int64_t)a.S * a.comb_loops * a.num * a.L;
+    const dim3 grid((unsigned)((entries + kBlock - 1) / kBlock));
+    if (a.fp32) hipLaunchKernelGGL(k_rows_table<true>, grid, dim3(kBlock), 0, st, a);
+    else hipLaunchKernelGGL(k_rows_table<false>, grid, dim3(kBlock), 0, st, a);
+    if (launched("rows_table") != 0) return -1;
+  }
   return 0;
 }
+
+size_t rows_entry_bytes(bool fp32) { return fp32 ? sizeof(RowEntry32) : sizeof(RowEntry64); }
 
 // The part of loops [l0, l0 + nl) with `res` residues per workgroup and its
 // LDS; false when the loops do not fit the kernel's limits.

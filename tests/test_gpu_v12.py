@@ -547,3 +547,42 @@ def test_selection_levels(torch_cuda, version, n, k, tones):
     fr, va = _gpu_plan(version, n, k).execute_sparse_host(x)
     assert np.array_equal(np.unique(fr), _located(ref, version))
     assert np.array_equal(out, ref["out"])
+
+
+@pytest.mark.parametrize("kind", ["plain", "tiny", "huge", "inf", "nan", "zero", "mixed"])
+def test_alias_row_quotients(torch_cuda, kind):
+    """The alias-row estimation of the FP64 form (quotients from tabulated
+    reciprocals, divisions for buckets outside their range) gives the bits of
+    the natural-order one, which divides throughout."""
+    torch = torch_cuda
+    n, k = 1 << 18, 64
+    print(f"case alias-row quotients {kind}", flush=True)
+    x, f, v = signal_np(n, k, seed=31, snr_db=30.0)
+    xs = [x, x.copy()]
+    if kind == "tiny":
+        xs[1] *= 1e-230
+    elif kind == "huge":
+        xs[1] *= 1e250
+    elif kind == "inf":
+        xs[1][12345] = np.inf
+    elif kind == "nan":
+        xs[1][777] = np.nan
+    elif kind == "zero":
+        xs[1][:] = 0
+    elif kind == "mixed":  # buckets of few taps on the large samples
+        xs[1] *= 1e-300
+        xs[1][5000:5003] = 1e200
+    res = []
+    for mode in (1, 2):
+        for conj in (True, False):
+            plan = _gpu_plan(2, n, k)
+            plan.set_schedule(mode, 0)
+            plan.set_reference_conjugate(conj)
+            xd = [torch.from_numpy(a).cuda() for a in xs]
+            fr, va = plan.make_sparse_outputs(2)
+            c = plan.execute_many_sparse(xd, fr, va)
+            res.append([(fr[i, :c[i]].cpu().numpy(), va[i, :c[i]].cpu().numpy()) for i in (0, 1)])
+    for a, b in ((res[0], res[2]), (res[1], res[3])):
+        for i in (0, 1):
+            assert np.array_equal(a[i][0], b[i][0])
+            assert np.array_equal(a[i][1].view(np.float64), b[i][1].view(np.float64), equal_nan=True)

@@ -98,6 +98,119 @@ __device__ void lds_fft(T2 *buf, int logN, const T2 *__restrict__ tw, int tws)
   else if (logN - s + 1 == 1) lds_fft_pass<T2, 1>(buf, N, s, tw, tws);
 }
 
+// Where point i of an N-point transform in LDS lies.  The passes below read
+// points 1, 8, 64, ... apart, and the bit-reversed input arrives 2^(logN-6)
+// apart; laid out by i, each of these puts the lanes of a read on a few
+// banks.  Xor-ing higher bits into the low ones (a linear map, so
+// fft_slot(i + j) = fft_slot(i) ^ fft_slot(j) for i, j without common bits)
+// spreads all of them over the banks.  The bucket FFTs of 20 loops of 4096
+// FP64 points went from 20 to 12 us (with one group of eight points a thread
+// instead of two), of 8 x 20 loops of 16,384 FP32 points from 81 to 60 us.
+// k_v3_run keeps lds_fft: built on this one it once ended a run with an
+// illegal access (n = 2^22, k = 500) whose cause was not found.
+template <typename T2>
+__device__ __forceinline__ unsigned fft_slot(unsigned i, int logN)
+{
+  constexpr int kLog = sizeof(T2) == 16 ? 4 : 5;  // log2 of the points in a row of banks
+  unsigned p = i ^ ((i >> 3) & 7u) ^ (((i >> 6) & 3u) << 3);
+  if (logN >= 10) {
+    const unsigned t = i >> (logN - kLog);  // rotated: clear of the bits above
+    p ^= (t << 1 | t >> (kLog - 1)) & ((1u << kLog) - 1);
+  }
+  return p;
+}
+
+// Stages s .. s+R-1 of an in-place radix-2 DIT FFT over N points in LDS, in
+// registers: with h = 2^(s-1), the 2^R points i0 + m*h (m < 2^R) of a group
+// only meet each other in those stages, so one thread loads them, applies the
+// stages' butterflies in order (the same cmul / add / sub on the same
+// twiddles as one stage per pass) and stores them.  cnt transforms, N points
+// apart.  Starts with a barrier, before which the first group's twiddles are
+// on their way.
+template <typename T2, int R>
+__device__ __forceinline__ void slot_fft_pass(T2 *buf, int logN, int s, const T2 *__restrict__ tw,
+                                             int tws, int cnt)
+{
+  constexpr int M = 1 << R;
+  const int N = 1 << logN, h = 1 << (s - 1);
+  const int groups = cnt << (logN - R);
+  // twiddles of a group: stage s + r needs 2^r, w[2^r - 1 + q], for the
+  // lower points at j + q h within their butterfly block
+  auto twiddles = [&](int g, T2 (&w)[M - 1]) {
+    const int j = g & (h - 1);
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int q = 0; q < (1 << r); q++)
+        w[(1 << r) - 1 + q] = tw[(j + q * h) * ((N >> (s + r)) * tws)];
+  };
+  T2 w[M - 1];
+  int g = threadIdx.x;
+  if (g < groups) twiddles(g, w);
+  __syncthreads();
+  for (; g < groups;) {
+    const int gi = g & ((N >> R) - 1);  // the group within its transform
+    const int j = gi & (h - 1);
+    const int i0 = ((gi >> (s - 1)) << (s - 1 + R)) + j;  // group block * (h << R) + j
+    T2 *const at = buf + ((g >> (logN - R)) << logN);
+    const unsigned p0 = fft_slot<T2>((unsigned)i0, logN);
+    T2 v[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) v[m] = at[p0 ^ fft_slot<T2>((unsigned)(m * h), logN)];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        if (m & (1 << r)) continue;
+        const int m1 = m + (1 << r);
+        const T2 u = v[m];
+        const T2 t = cmul(v[m1], w[(1 << r) - 1 + (m & ((1 << r) - 1))]);
+        v[m] = cadd(u, t);
+        v[m1] = csub(u, t);
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < M; m++) at[p0 ^ fft_slot<T2>((unsigned)(m * h), logN)] = v[m];
+    g += blockDim.x;
+    if (g < groups) twiddles(g, w);
+  }
+}
+
+// lds_fft of cnt runs of N = 2^logN points, with point i of the bit-reversed
+// input and of the natural-order output at fft_slot(i) of its run.  tw[j * tws] = e^{-2 pi i j/N} where tws =
+// Nmax / N for a table built for Nmax.  Three stages per LDS pass
+// (slot_fft_pass); every butterfly is the radix-2 one, so results are those of
+// one stage per pass, bit for bit.  Starts and ends with a barrier.
+template <typename T2>
+__device__ __forceinline__ void slot_fft(T2 *buf, int logN, const T2 *__restrict__ tw, int tws,
+                                         int cnt = 1)
+{
+  int s = 1;
+  for (; logN - s + 1 >= 3; s += 3) slot_fft_pass<T2, 3>(buf, logN, s, tw, tws, cnt);
+  if (logN - s + 1 == 2) slot_fft_pass<T2, 2>(buf, logN, s, tw, tws, cnt);
+  else if (logN - s + 1 == 1) slot_fft_pass<T2, 1>(buf, logN, s, tw, tws, cnt);
+  __syncthreads();
+}
+
+// The input of slot_fft: point i from src(i), kFillAhead loads in flight.
+constexpr int kFillAhead = 8;
+template <typename T2, typename F>
+__device__ __forceinline__ void slot_fft_fill(T2 *buf, int logN, F src)
+{
+  const int N = 1 << logN, T = blockDim.x;
+  for (int i0 = threadIdx.x; i0 < N; i0 += kFillAhead * T) {
+    T2 v[kFillAhead];
+#pragma unroll
+    for (int u = 0; u < kFillAhead; u++) v[u] = src(min(i0 + u * T, N - 1));
+#pragma unroll
+    for (int u = 0; u < kFillAhead; u++)  // past the end: point N - 1 again, same value
+      buf[fft_slot<T2>(bitrev((unsigned)min(i0 + u * T, N - 1), logN), logN)] = v[u];
+  }
+}
+
+// Threads for one N-point transform in LDS: one group of eight points each.
+__host__ __device__ inline int fft_threads(int N) { return N / 8 < 64 ? 64 : N / 8 > 1024 ? 1024 : N / 8; }
+
 // Exclusive prefix sum over the block (blockDim.x a multiple of 64);
 // tmp holds >= 16 ints of LDS.  Contains barriers.
 __device__ __forceinline__ int block_exclusive_scan(int v, int *tmp, int &total)

@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(256) k_stockham(const T2 *in, T2 *out, int N, 
 
 // One workgroup per transform, in LDS; forward only (the plan's table).
 template <typename T2>
-__global__ void __launch_bounds__(kBlock) k_lds_fft_batch(T2 *data, int logN, int nb_inner,
+__global__ void __launch_bounds__(1024) k_lds_fft_batch(T2 *data, int logN, int nb_inner,
                                                           int64_t so, int64_t si, const T2 *tw,
                                                           int tws)
 {
@@ -99,10 +99,9 @@ __global__ void __launch_bounds__(kBlock) k_lds_fft_batch(T2 *data, int logN, in
   T2 *buf = reinterpret_cast<T2 *>(smem_raw);
   const int N = 1 << logN;
   T2 *io = data + fft_base(blockIdx.x, nb_inner, so, si);
-  for (int m = threadIdx.x; m < N; m += blockDim.x) buf[bitrev(m, logN)] = io[m];
-  __syncthreads();
-  lds_fft(buf, logN, tw, tws);
-  for (int m = threadIdx.x; m < N; m += blockDim.x) io[m] = buf[m];
+  slot_fft_fill(buf, logN, [&](int m) { return io[m]; });
+  slot_fft(buf, logN, tw, tws);
+  for (int m = threadIdx.x; m < N; m += blockDim.x) io[m] = buf[fft_slot<T2>(m, logN)];
 }
 
 template <typename T2>
@@ -128,14 +127,13 @@ __global__ void k_copy(const T2 *in, T2 *out, int N, int64_t total, int nb_inner
 // and one column launch (13 us) do the same beside the same fold.
 //
 // Run c of the bit-reversed sequence holds x[q*R + bitrev(c)] at LDS
-// position bitrev(q), q < C.
+// point bitrev(q), q < C.
 template <typename T2>
 __device__ __forceinline__ void r2_run(T2 *buf, T2 *out, int logC, const T2 *tw, int tw_nmax)
 {
   const int C = 1 << logC;
-  __syncthreads();
-  lds_fft(buf, logC, tw, tw_nmax >> logC);
-  for (int q = threadIdx.x; q < C; q += blockDim.x) out[q] = buf[q];
+  slot_fft(buf, logC, tw, tw_nmax >> logC);
+  for (int q = threadIdx.x; q < C; q += blockDim.x) out[q] = buf[fft_slot<T2>(q, logC)];
 }
 
 template <typename T2>
@@ -145,13 +143,12 @@ __global__ void __launch_bounds__(kBlock) k_r2_runs(const T2 *data, T2 *tmp, int
 {
   extern __shared__ char smem_raw[];
   T2 *buf = reinterpret_cast<T2 *>(smem_raw);
-  const int C = 1 << logC;
   const int logR = logN - logC;
   const int64_t t = blockIdx.x >> logR;
   const int c = blockIdx.x & ((1 << logR) - 1);
   const int64_t base = fft_base(t, nb_inner, so, si);
   const T2 *in = data + base + bitrev(c, logR);
-  for (int q = threadIdx.x; q < C; q += blockDim.x) buf[bitrev(q, logC)] = in[(int64_t)q << logR];
+  slot_fft_fill(buf, logC, [&](int q) { return in[(int64_t)q << logR]; });
   r2_run(buf, tmp + base + ((int64_t)c << logC), logC, tw, tw_nmax);
 }
 
@@ -165,19 +162,18 @@ __global__ void __launch_bounds__(kBlock) k_comb_runs(const double2 *const *x, c
 {
   extern __shared__ char smem_raw[];
   double2 *buf = reinterpret_cast<double2 *>(smem_raw);
-  const int C = 1 << logC;
   const int logR = logN - logC;
   const int t = blockIdx.x >> logR;
   const int c = blockIdx.x & ((1 << logR) - 1);
   const int s = t / cl;
   const double2 *in = x[s] + params[(int64_t)s * stride + at + t % cl];
   const int64_t first = (int64_t)bitrev(c, logR) * sigma, step = (int64_t)sigma << logR;
-  for (int q = threadIdx.x; q < C; q += blockDim.x) buf[bitrev(q, logC)] = in[first + q * step];
+  slot_fft_fill(buf, logC, [&](int q) { return in[first + q * step]; });
   r2_run(buf, tmp + ((int64_t)t << logN) + ((int64_t)c << logC), logC, tw, tw_nmax);
 }
 
 // Stages logC + sc .. logC + sc + P - 1 of kCols columns held in LDS as
-// buf[c * kCols + column], as lds_fft_pass.
+// buf[c * kCols + column], as slot_fft_pass.
 constexpr int kCols = 16;
 
 template <typename T2, int P>
@@ -268,7 +264,7 @@ int radix2(T2 *data, T2 *tmp, int N, int C, int64_t nb_outer, int nb_inner, int6
     const size_t lds = ((size_t)1 << logN) * sizeof(T2);
     if (lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_lds_fft_batch<T2>));
     if (nb >= (1LL << 31)) return -1;
-    hipLaunchKernelGGL(k_lds_fft_batch<T2>, dim3((unsigned)nb), dim3(kBlock), lds, st, data,
+    hipLaunchKernelGGL(k_lds_fft_batch<T2>, dim3((unsigned)nb), dim3(fft_threads(N)), lds, st, data,
                        logN, nb_inner, so, si, tw, tw_nmax / N);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
@@ -388,7 +384,8 @@ int batch_fft64(double2 *data, double2 *tmp, int N, int64_t nb_outer, int nb_inn
     const size_t lds = (size_t)N * sizeof(double2);
     if (lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_lds_fft_batch<double2>));
     hipLaunchKernelGGL(k_lds_fft_batch<double2>, dim3((unsigned)(nb_outer * nb_inner)),
-                       dim3(kBlock), lds, st, data, logN, nb_inner, so, si, tw, tw_nmax / N);
+                       dim3(fft_threads(N)), lds, st, data, logN, nb_inner, so, si, tw,
+                       tw_nmax / N);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
   if (!tmp) return -1;
@@ -406,7 +403,8 @@ int batch_fft32(float2 *data, float2 *tmp, int N, int64_t nb_outer, int nb_inner
     const size_t lds = (size_t)N * sizeof(float2);
     if (lds > 65536) raise_lds_limit(reinterpret_cast<const void *>(k_lds_fft_batch<float2>));
     hipLaunchKernelGGL(k_lds_fft_batch<float2>, dim3((unsigned)(nb_outer * nb_inner)),
-                       dim3(kBlock), lds, st, data, logN, nb_inner, so, si, tw, tw_nmax / N);
+                       dim3(fft_threads(N)), lds, st, data, logN, nb_inner, so, si, tw,
+                       tw_nmax / N);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
   if (!tmp) return -1;

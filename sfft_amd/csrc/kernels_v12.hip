@@ -67,10 +67,8 @@ __global__ void __launch_bounds__(TB) k_comb(V12Launch a)
   const int W = a.W, logW = ilog2(W);
   const int sigma = a.n / W;
   const double2 *x = a.x[s];
-  for (int i = threadIdx.x; i < W; i += blockDim.x)
-    smem64[bitrev(i, logW)] = x[(int64_t)off + (int64_t)i * sigma];
-  __syncthreads();
-  lds_fft(smem64, logW, a.tw64, a.tw_nmax / W);
+  slot_fft_fill(smem64, logW, [&](int i) { return x[(int64_t)off + (int64_t)i * sigma]; });
+  slot_fft(smem64, logW, a.tw64, a.tw_nmax / W);
   // |.|^2 into the same LDS, as doubles (staged through registers: W is at
   // most kMaxLdsComb)
   constexpr int kPer = (kMaxLdsComb + TB - 1) / TB;
@@ -79,7 +77,7 @@ __global__ void __launch_bounds__(TB) k_comb(V12Launch a)
   for (int q = 0; q < kPer; q++) {
     const int i = threadIdx.x + q * TB;
     if (i < W) {
-      const double2 z = smem64[i];
+      const double2 z = smem64[fft_slot<double2>(i, logW)];
       v[q] = z.x * z.x + z.y * z.y;
     }
   }
@@ -241,14 +239,13 @@ __global__ void __launch_bounds__(kBlock) k_fold_fft64(V12Launch a, int l0, int 
 #pragma unroll
     for (int q = 0; q < kQ; q++) {
       const int m = mb + q * T;
-      if (m < B) smem64[bitrev(m, logB)] = acc[q];
+      if (m < B) smem64[fft_slot<double2>(bitrev(m, logB), logB)] = acc[q];
     }
   }
-  __syncthreads();
-  lds_fft(smem64, logB, a.tw64, a.tw_nmax / B);
+  slot_fft(smem64, logB, a.tw64, a.tw_nmax / B);
   double2 *out = a.xs64 + (int64_t)s * a.xs +
                  loop_offset(l, a.Lloc, a.B_loc, a.B_est);
-  for (int j = threadIdx.x; j < B; j += T) out[j] = smem64[j];
+  for (int j = threadIdx.x; j < B; j += T) out[j] = smem64[fft_slot<double2>(j, logB)];
 }
 
 // ---------------------------------------------------------------- sorted fold
@@ -1127,7 +1124,7 @@ __device__ __forceinline__ bool plain_value(double v)
 // Bucket FFTs of loops [l0, l0 + nl), written in the alias-row layout.
 // FP64: rows_odd[s L + l] says whether any bucket is not a plain value.
 template <bool FP32>
-__global__ void __launch_bounds__(kBlock) k_bucket_fft_rows(V12Launch a, int l0, int nl)
+__global__ void __launch_bounds__(1024) k_bucket_fft_rows(V12Launch a, int l0, int nl)
 {
   using T2 = typename std::conditional<FP32, float2, double2>::type;
   extern __shared__ char rraw[];
@@ -1142,14 +1139,13 @@ __global__ void __launch_bounds__(kBlock) k_bucket_fft_rows(V12Launch a, int l0,
   T2 *io;
   if constexpr (FP32) io = a.xs32; else io = a.xs64;
   io += (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est);
-  for (int m = threadIdx.x; m < B; m += blockDim.x) rbuf[bitrev(m, logB)] = io[m];
-  __syncthreads();
-  if constexpr (FP32) lds_fft(rbuf, logB, a.tw32, a.tw_nmax / B);
-  else lds_fft(rbuf, logB, a.tw64, a.tw_nmax / B);
+  slot_fft_fill(rbuf, logB, [&](int m) { return io[m]; });
+  if constexpr (FP32) slot_fft(rbuf, logB, a.tw32, a.tw_nmax / B);
+  else slot_fft(rbuf, logB, a.tw64, a.tw_nmax / B);
   int odd = 0;
   for (int b = threadIdx.x; b < B; b += blockDim.x) {
     const int r = b % d, q = b / d;
-    const T2 z = rbuf[b];
+    const T2 z = rbuf[fft_slot<T2>(b, logB)];
     if (!FP32) odd |= !plain_value(z.x) | !plain_value(z.y);
     io[r * rows + (int)(((unsigned)q * uinv) & (unsigned)(rows - 1))] = z;
   }
@@ -1676,11 +1672,11 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
     const int Bm = max(a.B_loc, a.B_est);
     if (a.fp32) {
       allow_lds(k_bucket_fft_rows<true>, (size_t)Bm * sizeof(float2));
-      hipLaunchKernelGGL(k_bucket_fft_rows<true>, dim3(a.S * a.L), dim3(kBlock),
+      hipLaunchKernelGGL(k_bucket_fft_rows<true>, dim3(a.S * a.L), dim3(fft_threads(Bm)),
                          (size_t)Bm * sizeof(float2), st, a, 0, a.L);
     } else {
       allow_lds(k_bucket_fft_rows<false>, (size_t)Bm * sizeof(double2));
-      hipLaunchKernelGGL(k_bucket_fft_rows<false>, dim3(a.S * a.L), dim3(kBlock),
+      hipLaunchKernelGGL(k_bucket_fft_rows<false>, dim3(a.S * a.L), dim3(fft_threads(Bm)),
                          (size_t)Bm * sizeof(double2), st, a, 0, a.L);
     }
     if (launched("bucket_fft_rows") != 0) return -1;

@@ -138,3 +138,39 @@ def test_top_num_cutoff_model(kind):
         keys = mag.astype(np.float64).view(np.uint64)
         cut = _cutoff_model(keys, num)
         assert cut == int(np.sort(keys)[N - num - 1])
+
+
+def _slot(i, logN, row_log):
+    """fft_slot of device_common.hpp: row_log 4 (FP64) or 5 (FP32)."""
+    p = i ^ ((i >> 3) & 7) ^ (((i >> 6) & 3) << 3)
+    if logN >= 10:
+        t = i >> (logN - row_log)
+        p ^= (t << 1 | t >> (row_log - 1)) & ((1 << row_log) - 1)
+    return p
+
+
+@pytest.mark.parametrize("row_log", [4, 5])
+@pytest.mark.parametrize("logN", [1, 3, 5, 8, 9, 10, 11, 12, 13, 14])
+def test_fft_slots(logN, row_log):
+    """Every point has a slot of its own within the transform, the map is
+    linear over disjoint bits (the passes xor the slots of i0 and m h), and
+    a half wave's points of a pass or of the bit-reversed fill meet in a row
+    of banks at most twice."""
+    N = 1 << logN
+    i = np.arange(N)
+    slots = np.array([_slot(int(q), logN, row_log) for q in i])
+    assert np.array_equal(np.sort(slots), i)
+    rng = np.random.default_rng(logN)
+    for a, b in rng.integers(0, N, (100, 2)):
+        b &= ~a
+        assert slots[a | b] == slots[a] ^ slots[b]
+    row = 1 << row_log
+    if logN < 10:
+        return
+    for s in range(1, logN - 1, 3):  # points 2^(s-1) apart in groups of 8
+        h = 1 << (s - 1)
+        g = np.arange(row)
+        i0 = ((g >> (s - 1)) << (s + 2)) + (g & (h - 1))
+        assert np.bincount(slots[i0] % row).max() <= 2, s
+    rev = np.array([int(format(q, "0%db" % logN)[::-1], 2) for q in range(row)])
+    assert np.bincount(slots[rev] % row).max() <= 2

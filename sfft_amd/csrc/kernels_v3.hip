@@ -1145,12 +1145,15 @@ constexpr int kClaimFree = 0, kClaimBusy = 1, kClaimDone = 2;
 // this is a guard against a defect, not a path of normal runs.
 constexpr int kClaimSpins = 1 << 20;
 
-// Marks a finished pre task done.  The workgroup barrier orders every
-// thread's stores before lane 0's device-scope release (the L2 written
-// back once), then the flag.  All threads; contains a barrier.
+// Marks a finished pre task done: every wave waits until its stores have
+// reached the L2 (a workgroup release alone does not: within a workgroup the
+// waves share an L1, so it leaves stores in flight across the barrier),
+// then lane 0's device-scope release writes the L2 back once, then the
+// flag.  All threads; contains a barrier.
 __device__ __forceinline__ void publish_task(int *cl)
 {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");

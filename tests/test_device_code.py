@@ -55,3 +55,18 @@ def test_called_functions_keep_their_return_address():
                 continue
             assert "s_getpc_b64 s[30:31]" not in body, (src, name)
     assert seen > 10
+
+
+def test_published_results_have_left_the_wave():
+    """A task's results are flagged done across XCDs by lane 0's L2
+    write-back; every wave waits for its own stores before the barrier that
+    precedes it."""
+    with tempfile.TemporaryDirectory() as d:
+        asm = _assembly("kernels_v3.hip", os.path.join(d, "v3.s"))
+    lines = [l.strip() for l in asm.splitlines()]
+    backs = [i for i, l in enumerate(lines) if l.startswith("buffer_wbl2")]
+    assert backs
+    for i in backs:
+        b = max(j for j in range(i) if lines[j].startswith("s_barrier"))
+        waits = [l for l in lines[b - 4:b] if l.startswith("s_waitcnt")]
+        assert any("vmcnt(0)" in l for l in waits), lines[b - 4:b + 1]

@@ -106,7 +106,8 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
         }
         if (kinds.is_device(o)) {
           de[s] = reinterpret_cast<double2 *>(o);
-          if (k::zero_dense(de[s], n, st) != 0) return fail(c0);
+          // v1/v2 batches clear their dense outputs themselves
+          if (P->version == SFFT_VERSION_3 && k::zero_dense(de[s], n, st) != 0) return fail(c0);
         } else {
           via_ws[s] = 1;
           nws++;
@@ -142,10 +143,18 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
     io.freq = any_sparse ? fr.data() : nullptr;
     io.val = any_sparse ? va.data() : nullptr;
     io.dense = dense ? de.data() : nullptr;
+    io.zero_dense = P->version != SFFT_VERSION_3;
     io.cap = cap;
     io.counts = counts.data();
     const int rc = exec_batch(P, io);
-    if (rc < 0) return fail(c0);
+    if (rc < 0) {
+      // (what follows is best effort; the call's error stays)
+      const std::string why = last_error();
+      for (int s = 0; s < S; s++)
+        if (de[s]) (void)k::zero_dense(de[s], n, st);
+      set_error(why);
+      return fail(c0);
+    }
     partial |= rc > 0;
     // results that went through the plan's buffers
     for (int s = 0; s < S; s++) {

@@ -249,12 +249,13 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int *tmp, int &total)
 // shares (a contiguous run per thread put a wave's reads on one bank).
 // With both, the comb kernel of one signal (4096 points, 1024 threads) went
 // from 28 to 25 us.
-// Uses 256+32 ints of LDS at sh.  Contains barriers.
+// Uses kTopScratch ints of LDS at sh.  Contains barriers, none after the
+// last writes of out.
+constexpr int kTopScratch = 2 * 256 + 32;
 __device__ void block_top_num(const double *mag, int N, int num, int *out,
                               int *sh)
 {
-  int *hist = sh;          // 256
-  int *misc = sh + 256;    // 32
+  int *misc = sh + 512;    // 32
   const int T = blockDim.x, tid = threadIdx.x;
   const int lane = tid & 63, wid = tid >> 6, nw = T >> 6;
   // rank of the cutoff in ascending order among the keys matching prefix
@@ -264,8 +265,12 @@ __device__ void block_top_num(const double *mag, int N, int num, int *out,
   bool direct = false;
   for (int pass = 7; pass >= 0; --pass) {
     const int shift = pass * 8;
-    for (int d = tid; d < 256; d += T) hist[d] = 0;
-    __syncthreads();
+    // two histograms in turn, cleared in pairs
+    int *hist = sh + 256 * (pass & 1);
+    if (pass & 1) {
+      for (int d = tid; d < 512; d += T) sh[d] = 0;
+      __syncthreads();
+    }
     if (pass == 7) {
       for (int i0 = wid * 64; i0 < N; i0 += T) {
         const int i = i0 + lane;
@@ -307,6 +312,7 @@ __device__ void block_top_num(const double *mag, int N, int num, int *out,
         misc[0] = 4 * tid + q;
         misc[1] = rank - cum;
         misc[2] = h[q];
+        misc[3] = 0;
       }
     }
     __syncthreads();
@@ -320,8 +326,6 @@ __device__ void block_top_num(const double *mag, int N, int num, int *out,
       // (#keys < it) <= rank < (#keys <= it)
       // the 128 keys as low words in hist[0..128), high words in hist[128..256)
       unsigned *klo = reinterpret_cast<unsigned *>(hist), *khi = klo + 128;
-      if (tid == 0) misc[3] = 0;
-      __syncthreads();
       for (int i = tid; i < N; i += T) {
         const uint64_t key = (uint64_t)__double_as_longlong(mag[i]);
         if ((key & hi_mask) == prefix) {
@@ -389,7 +393,6 @@ __device__ void block_top_num(const double *mag, int N, int num, int *out,
     pos += __popcll(tk);
     eq_before += __popcll(eq);
   }
-  __syncthreads();
 }
 
 }  // namespace dev

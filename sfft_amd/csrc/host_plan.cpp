@@ -1031,6 +1031,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   a.o_freq = want_sparse ? reinterpret_cast<int32_t *const *>(dtab + tab_bytes) : nullptr;
   a.o_val = want_sparse ? reinterpret_cast<double2 *const *>(dtab + 2 * tab_bytes) : nullptr;
   a.o_dense = want_dense ? reinterpret_cast<double2 *const *>(dtab + 3 * tab_bytes) : nullptr;
+  a.zero_dense = want_dense && io.zero_dense;
   a.o_cap = io.cap;
   a.est_cap = cap;
   a.comb_buf = big_comb ? P->ws->comb.as<double2>() : nullptr;
@@ -1128,7 +1129,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
     if ((launches[2] = k::fold_fft(a, st, 1)) < 0) return -1;
     mark(3);
     if (!p.comb && k::select_vote_v1(a, st) != 0) return -1;
-    launches[3] = p.comb ? 0 : 4;
+    launches[3] = p.comb ? 0 : 3;
     if (two_streams) HIP_OK(hipStreamWaitEvent(st, P->ev_join, 0));
     mark(4);
     if (k::estimate(a, st) != 0) return -1;
@@ -1147,7 +1148,8 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
     // batch of this shape; the workspace and staging addresses are part of
     // the key (kernel arguments and copy nodes hold them)
     const uint64_t key = (uint64_t)S | (uint64_t)fp32 << 32 | (uint64_t)want_sparse << 33 |
-                         (uint64_t)want_dense << 34 | (uint64_t)a.fold_mode << 35;
+                         (uint64_t)want_dense << 34 | (uint64_t)a.fold_mode << 35 |
+                         (uint64_t)a.zero_dense << 40;
     const uint64_t sig = workspace_signature(*P->ws) ^
                          ((uint64_t)io.cap * 0x9e3779b97f4a7c15ull + (uint64_t)a.ref_conj);
     hipGraphExec_t ex = nullptr;

@@ -286,7 +286,8 @@ struct BatchIO {
   const double2 *const *in = nullptr;
   int32_t *const *freq = nullptr;   // sparse frequencies, cap entries each
   double2 *const *val = nullptr;    // sparse values, cap entries each
-  double2 *const *dense = nullptr;  // n values each, already zero-filled
+  double2 *const *dense = nullptr;  // n values each (entries may be null)
+  bool zero_dense = false;          // v1/v2: the batch clears them (else they are clear)
   int64_t cap = 0;
   int64_t *counts = nullptr;        // host: S located counts (out)
   // the plan's workspace is an arena: no graph capture, no timing events,
@@ -352,6 +353,7 @@ struct V12Launch {
   int32_t *const *o_freq;   // S pointers or null
   double2 *const *o_val;    // S pointers or null
   double2 *const *o_dense;  // S pointers or null
+  bool zero_dense;          // the fold's launch clears the dense outputs
   int64_t o_cap;            // sparse capacity per signal
   int64_t est_cap;          // upper bound of the located count per signal
   int fold_mode;            // 0: fused fold+FFT per (signal, loop) block;

@@ -59,7 +59,7 @@ template <int TB>
 __global__ void __launch_bounds__(TB) k_comb(V12Launch a)
 {
   extern __shared__ double2 smem64[];
-  __shared__ int sh[256 + 32];
+  __shared__ int sh[kTopScratch];
   const int cl = a.comb_loops;
   const int s = blockIdx.x / cl, c = blockIdx.x % cl;
   const int stride = 2 * a.L + max(cl, 1);
@@ -119,7 +119,7 @@ struct TopLevel {
 __global__ void __launch_bounds__(kTopThreads) k_top_level(V12Launch a, TopLevel v)
 {
   extern __shared__ double lds_mag[];
-  __shared__ int sh[256 + 32];
+  __shared__ int sh[kTopScratch];
   __shared__ int pick[kTopMax];
   const int t = (int)(blockIdx.x / (unsigned)v.chunks), ch = (int)(blockIdx.x % (unsigned)v.chunks);
   const int e0 = ch * v.chunk, len = min(v.chunk, v.list_len - e0);
@@ -139,6 +139,7 @@ __global__ void __launch_bounds__(kTopThreads) k_top_level(V12Launch a, TopLevel
   int *out = v.out + (int64_t)t * v.out_stride + (int64_t)ch * v.num;
   const int take = min(v.num, len);
   if (len > v.num) block_top_num(lds_mag, len, v.num, pick, sh);
+  __syncthreads();
   for (int i = threadIdx.x; i < take; i += blockDim.x) {
     const int p = len > v.num ? pick[i] : i;
     out[i] = list ? list[p] : e0 + p;
@@ -297,6 +298,10 @@ struct FoldPart {
 struct FoldParts {
   FoldPart p[2];
   int groups;  // workgroups per signal, all parts
+  // the workgroups past S * groups clear the dense outputs, zero_blocks per
+  // signal (the estimates are written later on the stream): a launch less,
+  // and the stores run beside the gathers
+  int zero_blocks;
 };
 
 // sum + cmp gains v, compensated (2Sum)
@@ -514,11 +519,21 @@ __device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f
   }
 }
 
-// grid: S x f.groups
+// grid: S x f.groups, then S x f.zero_blocks
 __global__ void __launch_bounds__(kFoldThreads) k_fold_sorted(V12Launch a, FoldParts f)
 {
   extern __shared__ double2 smem64[];
   __shared__ int sh[16];
+  if (blockIdx.x >= (unsigned)(a.S * f.groups)) {
+    const unsigned z = blockIdx.x - (unsigned)(a.S * f.groups);
+    double2 *out = a.o_dense[z / (unsigned)f.zero_blocks];
+    if (!out) return;  // not wanted on the device
+    const int64_t step = (int64_t)f.zero_blocks * kFoldThreads;
+    for (int64_t i = (int64_t)(z % (unsigned)f.zero_blocks) * kFoldThreads + threadIdx.x; i < a.n;
+         i += step)
+      out[i] = make_double2(0.0, 0.0);
+    return;
+  }
   const int s = (int)(blockIdx.x / (unsigned)f.groups);
   int g = (int)(blockIdx.x % (unsigned)f.groups);
   FoldPart p = f.p[0];
@@ -531,6 +546,8 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_sorted(V12Launch a, FoldP
 }
 
 // ---------------------------------------------------------------- v1 votes
+constexpr int kFftPer = 8;  // points per thread of k_bucket_fft_v1 at most
+
 // One block per (signal, location loop): top-num buckets by |.|^2.
 // LDS: B doubles.  v1 location loops are always FP64 (xs64): their top-2k
 // choice is made among leakage-level bucket powers FP32 cannot resolve.
@@ -538,7 +555,7 @@ template <bool GLOBAL>
 __global__ void __launch_bounds__(kBlock) k_select(V12Launch a)
 {
   extern __shared__ double lds_mag[];
-  __shared__ int sh[256 + 32];
+  __shared__ int sh[kTopScratch];
   // above the LDS size the magnitudes go to mag_buf
   double *mag = GLOBAL ? a.mag_buf + (int64_t)blockIdx.x * a.B_loc : lds_mag;
   const int s = blockIdx.x / a.Lloc, l = blockIdx.x % a.Lloc;
@@ -554,6 +571,52 @@ __global__ void __launch_bounds__(kBlock) k_select(V12Launch a)
   block_top_num(mag, B, a.num, a.J + ((int64_t)s * a.Lloc + l) * a.num, sh);
 }
 
+// v1: the bucket FFTs of every loop in one launch, a location loop's block
+// going on to select its top-num buckets from LDS (as k_select, whose launch
+// and reads this saves; the location and estimation loops were two
+// launches).  One signal, n = 2^20, k = 50: 17 us against 6 + 6 + 13.
+// LDS: the largest loop's points.
+__global__ void __launch_bounds__(1024) k_bucket_fft_v1(V12Launch a)
+{
+  extern __shared__ double2 smem64[];
+  __shared__ int sh[kTopScratch];
+  const int s = blockIdx.x / a.L, l = blockIdx.x % a.L;
+  const bool isloc = l < a.Lloc;
+  const int B = isloc ? a.B_loc : a.B_est, logB = ilog2(B), T = blockDim.x;
+  const int64_t at = (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est);
+  if (!isloc && a.fp32) {
+    float2 *buf = reinterpret_cast<float2 *>(smem64), *io = a.xs32 + at;
+    slot_fft_fill(buf, logB, [&](int m) { return io[m]; });
+    slot_fft(buf, logB, a.tw32, a.tw_nmax / B);
+    for (int m = threadIdx.x; m < B; m += T) io[m] = buf[fft_slot<float2>(m, logB)];
+    return;
+  }
+  double2 *io = a.xs64 + at;
+  slot_fft_fill(smem64, logB, [&](int m) { return io[m]; });
+  slot_fft(smem64, logB, a.tw64, a.tw_nmax / B);
+  if (!isloc) {
+    for (int m = threadIdx.x; m < B; m += T) io[m] = smem64[fft_slot<double2>(m, logB)];
+    return;
+  }
+  double v[kFftPer];
+#pragma unroll
+  for (int q = 0; q < kFftPer; q++) {
+    const int i = threadIdx.x + q * T;
+    if (i < B) {
+      const double2 z = smem64[fft_slot<double2>(i, logB)];
+      io[i] = z;
+      v[q] = z.x * z.x + z.y * z.y;
+    }
+  }
+  __syncthreads();
+  double *mag = reinterpret_cast<double *>(smem64);
+#pragma unroll
+  for (int q = 0; q < kFftPer; q++)
+    if (threadIdx.x + q * T < B) mag[threadIdx.x + q * T] = v[q];
+  __syncthreads();
+  block_top_num(mag, B, a.num, a.J + ((int64_t)s * a.Lloc + l) * a.num, sh);
+}
+
 // A frequency f is a hit when, in at least thr of the location loops, its
 // permuted position p = f*ai mod n lies in the range
 // [ceil((J-1/2) n/B), ceil((J+1/2) n/B)) of a selected bucket J
@@ -562,12 +625,13 @@ __global__ void __launch_bounds__(kBlock) k_select(V12Launch a)
 // bucket, then offset in the range); a candidate is counted only from the
 // first such loop that selects it, so every hit appears once.  The candidate
 // list of a signal is cut into chunks of kVoteChunk, one block each:
-// k_vote_count counts each chunk's hits, k_vote_scan turns the counts into
-// offsets, k_vote_write writes the hits in candidate order.  LDS: Lloc * B
-// bits of selected-bucket flags.
+// k_vote_count counts each chunk's hits, k_vote_write writes the hits in
+// candidate order.  LDS: Lloc * B bits of selected-bucket flags
 constexpr int kVoteChunk = 8 * kBlock;
 static_assert(kVoteChunk == 2048, "vote_chunks() assumes chunks of 2048 candidates");
 
+// (the kernels evaluate a thread's eight candidates together, so that their
+// dependent reads overlap).
 struct VoteCtx {
   const int *prm, *J;
   const unsigned *selbits;
@@ -583,43 +647,66 @@ __device__ VoteCtx vote_setup(const V12Launch &a, int s, unsigned *selbits)
   v.words = (B + 31) / 32;
   v.prm = a.params + (int64_t)s * (2 * a.L + max(a.comb_loops, 1));
   v.mask = (unsigned)n - 1;
-  const int m = n / B;
-  v.half = m / 2;
-  v.logm = ilog2(m);
-  v.per_loop = (int64_t)num * m;
+  v.logm = ilog2(n) - ilog2(B);
+  v.half = (1 << v.logm) / 2;
+  v.per_loop = (int64_t)num << v.logm;
   v.total = (int64_t)max(Lloc - a.thr + 1, 0) * v.per_loop;
   v.J = a.J + (int64_t)s * Lloc * num;
   v.selbits = selbits;
   for (int i = threadIdx.x; i < Lloc * v.words; i += blockDim.x) selbits[i] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < Lloc * num; i += blockDim.x) {
-    const int l = i / num, b = v.J[i];
-    atomicOr(&selbits[l * v.words + (b >> 5)], 1u << (b & 31));
-  }
+  for (int l = 0; l < Lloc; l++)
+    for (int i = threadIdx.x; i < num; i += blockDim.x) {
+      const int b = v.J[l * num + i];
+      atomicOr(&selbits[l * v.words + (b >> 5)], 1u << (b & 31));
+    }
   __syncthreads();
   return v;
 }
 
-__device__ __forceinline__ int vote_keep(const V12Launch &a, const VoteCtx &v, int64_t c,
-                                         unsigned &loc)
+// Candidates ch kVoteChunk + i kBlock + threadIdx.x, i < 8: bit i of the
+// result says whether it is a hit, loc[i] its frequency.
+constexpr int kVotePer = kVoteChunk / kBlock;
+
+__device__ __forceinline__ unsigned vote_keep(const V12Launch &a, const VoteCtx &v, int ch,
+                                              unsigned (&loc)[kVotePer])
 {
-  if (c >= v.total) return 0;
-  const int l0 = (int)(c / v.per_loop);
-  const int64_t r = c % v.per_loop;
-  const int jb = v.J[(int64_t)l0 * a.num + (int)(r >> v.logm)];
-  const int q = (int)(r & ((1 << v.logm) - 1));
-  const unsigned m = 1u << v.logm;
-  const unsigned p = ((unsigned)jb * m - (unsigned)v.half + (unsigned)q + (unsigned)a.n) & v.mask;
-  loc = (p * (unsigned)v.prm[l0]) & v.mask;  // original frequency
-  int score = 0, earlier = 0;
-  for (int l = 0; l < a.Lloc; l++) {
-    const unsigned pl = (loc * (unsigned)v.prm[a.L + l]) & v.mask;
-    const unsigned bk = ((pl + (unsigned)v.half) & v.mask) >> v.logm;
-    const int sel = (v.selbits[l * v.words + (bk >> 5)] >> (bk & 31)) & 1;
-    score += sel;
-    earlier |= (l < l0) & sel;
+  int l0[kVotePer], score[kVotePer];
+  unsigned at[kVotePer], keep = 0, earlier = 0;
+#pragma unroll
+  for (int i = 0; i < kVotePer; i++) {
+    const int64_t c = (int64_t)ch * kVoteChunk + i * kBlock + threadIdx.x;
+    keep |= (c < v.total ? 1u : 0u) << i;
+    int64_t r = c < v.total ? c : 0;
+    int l = 0;
+    while (r >= v.per_loop) {  // few loops to start from
+      r -= v.per_loop;
+      l++;
+    }
+    l0[i] = l;
+    const int jb = v.J[(int64_t)l * a.num + (int)(r >> v.logm)];
+    at[i] = (((unsigned)jb << v.logm) - (unsigned)v.half +
+             ((unsigned)r & ((1u << v.logm) - 1)) + (unsigned)a.n) & v.mask;
   }
-  return (score >= a.thr) && !earlier;
+#pragma unroll
+  for (int i = 0; i < kVotePer; i++) {
+    loc[i] = (at[i] * (unsigned)v.prm[l0[i]]) & v.mask;  // original frequency
+    score[i] = 0;
+  }
+  for (int l = 0; l < a.Lloc; l++) {
+    const unsigned ai = (unsigned)v.prm[a.L + l];
+#pragma unroll
+    for (int i = 0; i < kVotePer; i++) {
+      const unsigned bk = ((((loc[i] * ai) & v.mask) + (unsigned)v.half) & v.mask) >> v.logm;
+      const int sel = (v.selbits[l * v.words + (bk >> 5)] >> (bk & 31)) & 1;
+      score[i] += sel;
+      earlier |= (unsigned)((l < l0[i]) & sel) << i;
+    }
+  }
+  unsigned hit = 0;
+#pragma unroll
+  for (int i = 0; i < kVotePer; i++) hit |= (score[i] >= a.thr ? 1u : 0u) << i;
+  return hit & keep & ~earlier;
 }
 
 // grid: S x chunks
@@ -629,51 +716,55 @@ __global__ void __launch_bounds__(kBlock) k_vote_count(V12Launch a, int chunks)
   __shared__ int sh[16];
   const int s = blockIdx.x / chunks, ch = blockIdx.x % chunks;
   const VoteCtx v = vote_setup(a, s, selbits);
-  int mine = 0;
-  for (int i = 0; i < kVoteChunk; i += blockDim.x) {
-    unsigned loc;
-    mine += vote_keep(a, v, (int64_t)ch * kVoteChunk + i + threadIdx.x, loc);
-  }
+  unsigned loc[kVotePer];
   int tot;
-  (void)block_exclusive_scan(mine, sh, tot);
+  (void)block_exclusive_scan(__popc(vote_keep(a, v, ch, loc)), sh, tot);
   if (threadIdx.x == 0) a.vote_cnt[blockIdx.x] = tot;
 }
 
-// grid: S; exclusive scan of a signal's chunk counts in place, and its
-// located count (at most hits_cap)
-__global__ void __launch_bounds__(kBlock) k_vote_scan(V12Launch a, int chunks)
-{
-  __shared__ int sh[16];
-  int *cnt = a.vote_cnt + (int64_t)blockIdx.x * chunks;
-  int64_t base = 0;
-  for (int c0 = 0; c0 < chunks; c0 += blockDim.x) {
-    const int c = c0 + threadIdx.x;
-    const int v = c < chunks ? cnt[c] : 0;
-    int tot;
-    const int pos = block_exclusive_scan(v, sh, tot);
-    if (c < chunks) cnt[c] = (int)min(base + pos, (int64_t)INT_MAX);
-    base += tot;
-  }
-  if (threadIdx.x == 0) a.count[blockIdx.x] = min(base, a.hits_cap);
-}
-
-// grid: S x chunks
+// grid: S x chunks.  A chunk's hits follow those of the signal's chunks
+// before it, whose counts the block sums itself (a scan kernel between the
+// two cost a launch); the last chunk writes the located count (at most
+// hits_cap).
 __global__ void __launch_bounds__(kBlock) k_vote_write(V12Launch a, int chunks)
 {
   extern __shared__ unsigned selbits[];
-  __shared__ int sh[16];
+  constexpr int NW = kBlock / 64;
+  __shared__ int64_t s_base[NW];
+  __shared__ int s_cnt[kVotePer * NW];
   const int s = blockIdx.x / chunks, ch = blockIdx.x % chunks;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int64_t before = 0;
+  for (int c = threadIdx.x; c < ch; c += kBlock) before += a.vote_cnt[(int64_t)s * chunks + c];
   const VoteCtx v = vote_setup(a, s, selbits);
-  int *hits = a.hits + (int64_t)s * a.hits_cap;
-  int64_t base = a.vote_cnt[blockIdx.x];
-  for (int i = 0; i < kVoteChunk; i += blockDim.x) {
-    unsigned loc = 0;
-    const int keep = vote_keep(a, v, (int64_t)ch * kVoteChunk + i + threadIdx.x, loc);
-    int tot;
-    const int pos = block_exclusive_scan(keep, sh, tot);
-    if (keep && base + pos < a.hits_cap) hits[base + pos] = (int)loc;
-    base += tot;
+  unsigned loc[kVotePer];
+  const unsigned keep = vote_keep(a, v, ch, loc);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+  if (lane == 0) s_base[wid] = before;
+#pragma unroll
+  for (int i = 0; i < kVotePer; i++) {
+    const uint64_t b = __ballot((keep >> i) & 1);
+    if (lane == 0) s_cnt[i * NW + wid] = __popcll(b);
   }
+  __syncthreads();
+  int64_t base = 0;
+#pragma unroll
+  for (int w = 0; w < NW; w++) base += s_base[w];
+  int *hits = a.hits + (int64_t)s * a.hits_cap;
+#pragma unroll
+  for (int i = 0; i < kVotePer; i++) {
+    const uint64_t b = __ballot((keep >> i) & 1);
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      if (w == wid && ((keep >> i) & 1)) {
+        const int64_t pos = base + __popcll(b & ((1ull << lane) - 1));
+        if (pos < a.hits_cap) hits[pos] = (int)loc[i];
+      }
+      base += s_cnt[i * NW + w];
+    }
+  }
+  if (ch == chunks - 1 && threadIdx.x == 0) a.count[s] = min(base, a.hits_cap);
 }
 
 // ---------------------------------------------------------------- v2 votes (diagnostic)
@@ -864,6 +955,23 @@ __device__ __forceinline__ double2 load_bucket(const V12Launch &a, bool fp32, bo
   return a.xs64[idx];
 }
 
+// load_bucket without a branch between the precisions (two 8-byte words
+// wherever they lie), so that several can be in flight.
+template <bool FP32>
+__device__ __forceinline__ double2 raw_bucket(const V12Launch &a, bool isloc, int64_t idx)
+{
+  if constexpr (!FP32) {
+    return a.xs64[idx];
+  } else {
+    const bool wide = a.loc64 && isloc;
+    const double *p = wide ? reinterpret_cast<const double *>(a.xs64 + idx)
+                           : reinterpret_cast<const double *>(a.xs32 + idx);
+    const double w0 = p[0], w1 = p[wide ? 1 : 0];
+    const float fx = __int_as_float(__double2loint(w0)), fy = __int_as_float(__double2hiint(w0));
+    return wide ? make_double2(w0, w1) : make_double2((double)fx, (double)fy);
+  }
+}
+
 // bucket / G with the reference's operation order (division by |G|^2)
 __device__ __forceinline__ void divide_by_filter(double2 U, double2 G, double den,
                                                  bool conj, double &vr, double &vi)
@@ -892,10 +1000,10 @@ __device__ __forceinline__ void hash_direct(const V12Launch &a, int l, unsigned 
 {
   const bool isloc = l < a.Lloc;
   const int B = isloc ? a.B_loc : a.B_est;
-  const int m = a.n / B;
+  const int logm = ilog2(a.n) - ilog2(B), m = 1 << logm;
   const unsigned p = (ai * h) & ((unsigned)a.n - 1);
-  hashed = (int)(p / (unsigned)m);
-  int dist = (int)(p % (unsigned)m);
+  hashed = (int)(p >> logm);
+  int dist = (int)(p & (unsigned)(m - 1));
   if (dist > m / 2) {
     hashed = (hashed + 1) & (B - 1);
     dist -= m;
@@ -1376,7 +1484,9 @@ __global__ void __launch_bounds__(kBlock) k_estimate_rows(V12Launch a, int tiles
   }
 }
 
-// v1: one thread per hit of the vote list.
+// v1: one thread per hit of the vote list.  Few hits, so bound by the reads'
+// latency: kHitAhead loops' reads are issued together.
+constexpr int kHitAhead = 4;  // divides every median network's size
 template <int LMAX, bool FP32>
 __global__ void __launch_bounds__(kBlock) k_estimate_hits(V12Launch a, int64_t chunks)
 {
@@ -1395,18 +1505,28 @@ __global__ void __launch_bounds__(kBlock) k_estimate_hits(V12Launch a, int64_t c
   const int64_t sbase = (int64_t)s * a.xs;
   double vr[LMAX], vi[LMAX];
 #pragma unroll
-  for (int l = 0; l < LMAX; l++) {
-    if (l < L) {
+  for (int l0 = 0; l0 < LMAX; l0 += kHitAhead) {
+    // buckets and filter values of kHitAhead loops in flight (past L: the
+    // last loop's again, unused)
+    double2 U[kHitAhead], G[kHitAhead];
+#pragma unroll
+    for (int u = 0; u < kHitAhead; u++) {
+      const int l = min(l0 + u, L - 1);
       const bool isloc = l < a.Lloc;
       int hashed;
-      double2 G;
-      hash_direct(a, l, s_ai[l], h, hashed, G);
-      const double2 U = load_bucket(a, FP32, isloc,
-                                    sbase + loop_offset(l, a.Lloc, a.B_loc, a.B_est) + hashed);
-      divide_by_filter(U, G, G.x * G.x + G.y * G.y, a.ref_conj, vr[l], vi[l]);
-    } else {
-      vr[l] = __longlong_as_double(0x7ff0000000000000ll);
-      vi[l] = vr[l];
+      hash_direct(a, l, s_ai[l], h, hashed, G[u]);
+      U[u] = raw_bucket<FP32>(a, isloc,
+                              sbase + loop_offset(l, a.Lloc, a.B_loc, a.B_est) + hashed);
+    }
+#pragma unroll
+    for (int u = 0; u < kHitAhead; u++) {
+      const int l = l0 + u;
+      if (l < L) {
+        divide_by_filter(U[u], G[u], G[u].x * G[u].x + G[u].y * G[u].y, a.ref_conj, vr[l], vi[l]);
+      } else {
+        vr[l] = __longlong_as_double(0x7ff0000000000000ll);
+        vi[l] = vr[l];
+      }
     }
   }
   write_result(a, s, t, h, lower_median<LMAX>(vr, vi, L));
@@ -1639,11 +1759,20 @@ static int fold_sorted(const V12Launch &a, hipStream_t st, int from, int n64)
   const int cut = same ? n64 : a.Lloc;  // where the bucket count or precision changes
   // (with both, they change at the same loop: n64 is 0, Lloc or L)
   if (add(n64 == 0, from, cut) != 0 || add(cut >= n64, std::max(cut, from), a.L) != 0) return -1;
-  if (np == 0) return 0;
+  f.zero_blocks = a.zero_dense ? (int)std::min<int64_t>(512, (a.n + 4095) / 4096) : 0;
+  if (np == 0 && f.zero_blocks == 0) return 0;
   allow_lds(k_fold_sorted, lds);
-  hipLaunchKernelGGL(k_fold_sorted, dim3((unsigned)((int64_t)a.S * f.groups)), dim3(kFoldThreads),
-                     lds, st, a, f);
+  hipLaunchKernelGGL(k_fold_sorted,
+                     dim3((unsigned)((int64_t)a.S * (f.groups + f.zero_blocks))),
+                     dim3(kFoldThreads), lds, st, a, f);
   return launched("fold_sorted") == 0 ? 1 : -1;
+}
+
+// Whether the bucket FFTs of a v1 batch select the top buckets too.
+static bool v1_fft_select(const V12Launch &a)
+{
+  return a.comb_loops == 0 && a.fold_mode >= 1 && a.B_loc <= kMaxLdsFft64 &&
+         a.B_est <= kMaxLdsFft64;
 }
 
 int fold_fft(const V12Launch &a, hipStream_t st, int part)
@@ -1681,6 +1810,15 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
     }
     if (launched("bucket_fft_rows") != 0) return -1;
     return 1;
+  }
+  if (v1_fft_select(a)) {
+    const size_t lds = std::max((size_t)a.B_loc * sizeof(double2),
+                                (size_t)a.B_est * (a.fp32 ? sizeof(float2) : sizeof(double2)));
+    // few signals: every thread the selection can use
+    const int T = a.S * a.Lloc < 256 ? 1024 : std::max(256, fft_threads(max(a.B_loc, a.B_est)));
+    allow_lds(k_bucket_fft_v1, lds);
+    hipLaunchKernelGGL(k_bucket_fft_v1, dim3(a.S * a.L), dim3(T), lds, st, a);
+    return launched("bucket_fft_v1") == 0 ? 1 : -1;
   }
   // the location and estimation loops as batches of one bucket count and
   // precision: in LDS up to the LDS size, else radix-2 runs plus global
@@ -1738,14 +1876,12 @@ static int select_loops(const V12Launch &a, hipStream_t st)
 
 int select_vote_v1(const V12Launch &a, hipStream_t st)
 {
-  if (select_loops(a, st) != 0) return -1;
+  if (!v1_fft_select(a) && select_loops(a, st) != 0) return -1;
   const size_t lb = (size_t)a.Lloc * ((a.B_loc + 31) / 32) * 4;
   const int chunks = vote_chunks(a.n, a.B_loc, a.num, a.Lloc, a.thr);
   const dim3 grid((unsigned)((int64_t)a.S * chunks));
   hipLaunchKernelGGL(k_vote_count, grid, dim3(kBlock), lb, st, a, chunks);
   if (launched("vote_count") != 0) return -1;
-  hipLaunchKernelGGL(k_vote_scan, dim3(a.S), dim3(kBlock), 0, st, a, chunks);
-  if (launched("vote_scan") != 0) return -1;
   hipLaunchKernelGGL(k_vote_write, grid, dim3(kBlock), lb, st, a, chunks);
   return launched("vote_write");
 }

@@ -586,3 +586,30 @@ def test_alias_row_quotients(torch_cuda, kind):
         for i in (0, 1):
             assert np.array_equal(a[i][0], b[i][0])
             assert np.array_equal(a[i][1].view(np.float64), b[i][1].view(np.float64), equal_nan=True)
+
+
+@pytest.mark.parametrize("version,precision,mode", [
+    (1, "fp64", 0), (1, "fp64", 1), (1, "fp32_refine", 0), (2, "fp64", 2), (2, "fp32_refine", 1)])
+def test_dense_outputs_are_cleared(torch_cuda, version, precision, mode):
+    """Dense device outputs that held other values read zero outside the
+    located set, for one signal and for several, whatever the schedule."""
+    torch = torch_cuda
+    n, k = 1 << 16, 50
+    print(f"case dense clear v{version} {precision} mode={mode}", flush=True)
+    xs = [signal_np(n, k, seed=70 + i)[0] for i in range(3)]
+    xd = [torch.from_numpy(x).cuda() for x in xs]
+    plan = _gpu_plan(version, n, k, precision)
+    plan.set_schedule(mode, 0)
+    fr, va = plan.make_sparse_outputs(3)
+    counts = plan.execute_many_sparse(xd, fr, va)
+    want = torch.zeros((3, n), dtype=torch.complex128, device="cuda")
+    for i in range(3):
+        want[i, fr[i, :int(counts[i])].long()] = va[i, :int(counts[i])]
+    plan.seed(17, 4242)
+    outs = [torch.full((n,), 7 + 7j, dtype=torch.complex128, device="cuda") for _ in range(3)]
+    plan.execute_many_device(xd, outs)
+    for i in range(3):
+        assert torch.equal(outs[i], want[i])
+    plan.seed(17, 4242)
+    plan.execute_device(xd[0], outs[1])
+    assert torch.equal(outs[1], want[0])

@@ -547,7 +547,7 @@ static int ensure_pinned(Plan *P, size_t bytes)
   if (P->ws->pinned) (void)hipHostFree(P->ws->pinned);
   P->ws->pinned = nullptr;
   P->ws->pinned_bytes = 0;
-  HIP_OK(hipHostMalloc(&P->ws->pinned, bytes, hipHostMallocDefault));
+  HIP_OK(hipHostMalloc(&P->ws->pinned, bytes, hipHostMallocMapped | hipHostMallocCoherent));
   P->ws->pinned_bytes = bytes;
   return 0;
 }
@@ -757,7 +757,7 @@ static int ensure_pinned_ws(Workspace *ws, size_t bytes)
   if (ws->pinned) (void)hipHostFree(ws->pinned);
   ws->pinned = nullptr;
   ws->pinned_bytes = 0;
-  HIP_OK(hipHostMalloc(&ws->pinned, bytes, hipHostMallocDefault));
+  HIP_OK(hipHostMalloc(&ws->pinned, bytes, hipHostMallocMapped | hipHostMallocCoherent));
   ws->pinned_bytes = bytes;
   return 0;
 }
@@ -884,6 +884,7 @@ static k::V12Launch sub_launch(const k::V12Launch &a, int base, int cnt, int str
     b.rows_odd = a.rows_odd + s0 * a.L;
   }
   b.count = a.count + s0;
+  if (a.count_host) b.count_host = a.count_host + s0;
   if (a.o_freq) b.o_freq = a.o_freq + s0;
   if (a.o_val) b.o_val = a.o_val + s0;
   if (a.o_dense) b.o_dense = a.o_dense + s0;
@@ -1050,7 +1051,23 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   // an arena workspace creates no runtime objects: no timing events, no
   // second stream, no graphs
   const bool timing = P->timing && !io.fixed_ws;
-  const bool two_streams = p.comb && !io.fixed_ws;
+  // the comb in the fold's launch, or (stage timing, combs above its LDS)
+  // on a second stream beside it
+  a.comb_fused = p.comb && !timing && k::fuse_comb(a);
+  const bool two_streams = p.comb && !io.fixed_ws && !a.comb_fused;
+  // the located counts: one comb loop's is known, others are written to the
+  // pinned staging by the kernel that finds them (a copy back cost every
+  // call a launch), or copied back to the staging of the allocation-free
+  // exec, which is not pinned
+  const bool known_count = p.comb && cl == 1;
+  a.count_host = known_count || io.fixed_ws ? nullptr : h_counts;
+  auto deliver_counts = [&]() -> int {
+    if (!known_count && io.fixed_ws)
+      HIP_OK(hipMemcpyAsync(h_counts, a.count, cnt_bytes, hipMemcpyDeviceToHost, st));
+    return 0;
+  };
+  if (known_count)
+    for (int s = 0; s < S; s++) h_counts[s] = (int64_t)num * (n / p.W_comb);
   if (timing && !P->ev_made) {
     for (hipEvent_t &e : P->ev) HIP_OK(hipEventCreate(&e));
     for (hipEvent_t &e : P->ev_comb) HIP_OK(hipEventCreate(&e));
@@ -1070,7 +1087,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
   // Not with stage timing, whose stages are whole-batch launches.
   // SFFT_PARTS overrides the part count (tuning experiments; 1: unparted).
   int parts = 1;
-  if (two_streams && fp32 && a.rows_layout && !timing && !dbg_votes && S >= 64) {
+  if (p.comb && !io.fixed_ws && fp32 && a.rows_layout && !timing && !dbg_votes && S >= 64) {
     parts = 2;
     if (const char *e = std::getenv("SFFT_PARTS")) parts = std::atoi(e);
     parts = std::max(1, std::min({parts, Plan::kMaxParts, S / 32}));
@@ -1090,11 +1107,13 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
                           hipMemcpyHostToDevice, st));
     if (parts > 1) {
       hipStream_t st2 = P->stream2, st3 = P->stream3;
-      HIP_OK(hipEventRecord(P->ev_fork, st));
-      HIP_OK(hipStreamWaitEvent(st2, P->ev_fork, 0));
-      if (k::comb(a, st2) != 0) return -1;
-      HIP_OK(hipEventRecord(P->ev_join, st2));
-      HIP_OK(hipStreamWaitEvent(st3, P->ev_join, 0));
+      if (two_streams) {
+        HIP_OK(hipEventRecord(P->ev_fork, st));
+        HIP_OK(hipStreamWaitEvent(st2, P->ev_fork, 0));
+        if (k::comb(a, st2) != 0 || k::rows_table(a, st2) != 0) return -1;
+        HIP_OK(hipEventRecord(P->ev_join, st2));
+        HIP_OK(hipStreamWaitEvent(st3, P->ev_join, 0));
+      }
       for (int q = 0; q < parts; q++) {
         const int b0 = (int)((int64_t)S * q / parts), b1 = (int)((int64_t)S * (q + 1) / parts);
         const k::V12Launch sa = sub_launch(a, b0, b1 - b0, stride, vchunks);
@@ -1105,23 +1124,23 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
       }
       HIP_OK(hipEventRecord(P->ev_est, st3));
       HIP_OK(hipStreamWaitEvent(st, P->ev_est, 0));
-      HIP_OK(hipMemcpyAsync(h_counts, a.count, cnt_bytes, hipMemcpyDeviceToHost, st));
-      return 0;
+      return deliver_counts();
     }
     if (two_streams) HIP_OK(hipEventRecord(P->ev_fork, st));
     mark(1);
     // the fold is enqueued before the comb: for a single signal the host's
     // launch calls are on the latency path, and the fold branch is longer
     if ((launches[1] = k::fold_fft(a, st, 0)) < 0) return -1;
-    if (p.comb && !two_streams) {
-      if (k::comb(a, st) != 0) return -1;
+    if (p.comb && !two_streams && !a.comb_fused) {
+      if (k::comb(a, st) != 0 || k::rows_table(a, st) != 0) return -1;
       launches[0] = cl > 1 ? 2 : 1;
-    } else if (p.comb) {
+    } else if (two_streams) {
       hipStream_t st2 = P->stream2;
       HIP_OK(hipStreamWaitEvent(st2, P->ev_fork, 0));
       if (timed) (void)hipEventRecord(P->ev_comb[0], st2);
       if (k::comb(a, st2) != 0) return -1;
       if (timed) (void)hipEventRecord(P->ev_comb[1], st2);
+      if (k::rows_table(a, st2) != 0) return -1;
       HIP_OK(hipEventRecord(P->ev_join, st2));
       launches[0] = cl > 1 ? 2 : 1;
     }
@@ -1137,8 +1156,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
     if (dbg_votes && k::comb_vote_keys(a, P->ws->votes.as<int64_t>(), 2 * cap, st) != 0)
       return -1;
     mark(5);
-    HIP_OK(hipMemcpyAsync(h_counts, a.count, cnt_bytes, hipMemcpyDeviceToHost, st));
-    return 0;
+    return deliver_counts();
   };
   P->last_fp32 = fp32;
   P->last_S = S;

@@ -350,6 +350,7 @@ struct V12Launch {
   int *vote_cnt;   // v1: S x vote_chunks hit counts, then offsets
   int64_t hits_cap;
   int64_t *count;  // S located counts
+  int64_t *count_host;      // the same in pinned host memory, or null
   int32_t *const *o_freq;   // S pointers or null
   double2 *const *o_val;    // S pointers or null
   double2 *const *o_dense;  // S pointers or null
@@ -370,6 +371,7 @@ struct V12Launch {
   // v2 with W a multiple of n/B: buckets after the FFT stored by alias row
   // (see k_bucket_fft_rows); estimation reads them contiguously
   bool rows_layout;
+  bool comb_fused;  // v2: the fold's launch runs the combs
   void *rows_tab;  // S x comb_loops*num x L estimation entries (rows_entry_bytes each)
   int *rows_odd;   // FP64: S x L, buckets the estimate has to divide
 };
@@ -474,6 +476,11 @@ int noalloc_setup();
 void *noalloc_scratch(int dev);
 
 int comb(const V12Launch &a, hipStream_t st);
+// Whether the fold's launch can run the combs too (V12Launch::comb_fused).
+bool fuse_comb(const V12Launch &a);
+// The alias-row estimation entries after comb() (with comb_fused the bucket
+// FFTs' launch writes them).
+int rows_table(const V12Launch &a, hipStream_t st);
 // part 0: the fold (fused with the bucket FFTs when fold_mode == 0);
 // part 1: the bucket FFTs (nothing when fused).  Returns launches or -1.
 int fold_fft(const V12Launch &a, hipStream_t st, int part);

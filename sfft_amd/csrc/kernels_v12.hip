@@ -53,15 +53,13 @@ inline int64_t loop_offset_host(int l, int Lloc, int Bl, int Be)
 constexpr int kTopThreads = 512, kTopMax = 4096, kTopChunk = 4096, kTopLast = 16384;
 
 // ---------------------------------------------------------------- comb
-// One block per (signal, comb loop).  LDS: W double2.  TB threads: kBlock
-// for batches; more for a few signals, whose comb is on the latency path.
+// Comb loop c of signal s by one workgroup of TB threads.  LDS: W double2 at
+// smem64, kTopScratch ints at sh.
 template <int TB>
-__global__ void __launch_bounds__(TB) k_comb(V12Launch a)
+__device__ __forceinline__ void comb_block(const V12Launch &a, int s, int c, double2 *smem64,
+                                           int *sh)
 {
-  extern __shared__ double2 smem64[];
-  __shared__ int sh[kTopScratch];
   const int cl = a.comb_loops;
-  const int s = blockIdx.x / cl, c = blockIdx.x % cl;
   const int stride = 2 * a.L + max(cl, 1);
   const int off = a.params[(int64_t)s * stride + 2 * a.L + c];
   const int W = a.W, logW = ilog2(W);
@@ -95,6 +93,17 @@ __global__ void __launch_bounds__(TB) k_comb(V12Launch a)
     a.num_comb[s] = a.num;
     a.count[s] = (int64_t)a.num * (a.n / W);
   }
+}
+
+// Combs in a launch of their own (beside the fold on a second stream):
+// kBlock threads for batches; more for a few signals, whose comb is on the
+// latency path.
+template <int TB>
+__global__ void __launch_bounds__(TB) k_comb(V12Launch a)
+{
+  extern __shared__ double2 smem64[];
+  __shared__ int sh[kTopScratch];
+  comb_block<TB>(a, blockIdx.x / a.comb_loops, blockIdx.x % a.comb_loops, smem64, sh);
 }
 
 // Selections above the LDS size, in levels: block (t, chunk) takes `chunk`
@@ -185,6 +194,7 @@ __global__ void __launch_bounds__(kBlock) k_comb_merge(V12Launch a)
   if (threadIdx.x == 0) {
     a.num_comb[s] = total;
     a.count[s] = (int64_t)total * (a.n / W);
+    if (a.count_host) a.count_host[s] = a.count[s];
   }
 }
 
@@ -292,7 +302,7 @@ struct FoldPart {
   unsigned inv_tR;       // idx / tR = idx * inv_tR >> 20 for idx below kFoldThreads * tR
   int nbins, bin_shift;  // sort bins of 2^bin_shift rows
   int seg_log;           // FP32: rows per chunk 2^seg_log
-  int order_at;          // FP32: the taps' summation order, in words of LDS
+  int order_at;          // the sorted list, then FP32 the taps' order: in words of LDS
 };
 
 struct FoldParts {
@@ -302,6 +312,9 @@ struct FoldParts {
   // signal (the estimates are written later on the stream): a launch less,
   // and the stores run beside the gathers
   int zero_blocks;
+  // the first workgroups run the combs of the batch's signals (S x comb
+  // loops, 0 when they have a launch of their own)
+  int combs;
 };
 
 // sum + cmp gains v, compensated (2Sum)
@@ -330,12 +343,6 @@ __device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f
   uint2 *pp = reinterpret_cast<uint2 *>(smem64 + (npairs * f.tR * sizeof(T2) + 15) / 16);
   int *tap_at = reinterpret_cast<int *>(pp + npairs);
   uint16_t *list = reinterpret_cast<uint16_t *>(tap_at + npairs);
-  // FP32: the pair's taps in summation order, a byte each (tR4 of them); a
-  // second list when they take several passes
-  const int tR4 = (f.tR + 3) & ~3;
-  uint8_t *order = reinterpret_cast<uint8_t *>(
-      reinterpret_cast<uint32_t *>(smem64) + f.order_at) + tid * tR4;
-  uint8_t *order2 = order + npairs * tR4;
   const int B = f.B, logB = f.logB;
   const unsigned mask = (unsigned)a.n - 1, rmask = ((unsigned)a.n >> logB) - 1;
   const int *prm = a.params + (int64_t)s * (2 * a.L + max(a.comb_loops, 1));
@@ -356,13 +363,8 @@ __device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f
   }
   for (int i = tid; i < f.nbins; i += T) bins[i] = 0;
   __syncthreads();
-  // FP32: taps by the low bits of their chunk, eight bits a count
-  uint64_t per_chunk = 0;
-  for (int k = 0; k < R; k++) {
-    const unsigned row = (row0 + (unsigned)k * srow) & rmask;
-    atomicAdd(&bins[row >> f.bin_shift], 1);
-    if (FP32) per_chunk += 1ull << (8 * ((row >> f.seg_log) & (kPackChunks - 1)));
-  }
+  for (int k = 0; k < R; k++)
+    atomicAdd(&bins[((row0 + (unsigned)k * srow) & rmask) >> f.bin_shift], 1);
   __syncthreads();
   int total;
   {
@@ -378,45 +380,15 @@ __device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f
     }
   }
   __syncthreads();
-  // the list; FP32: the pair's taps sorted, stably, by the low bits of their
-  // chunk (place: the exclusive byte-wise prefix sum of the counts)
-  uint64_t place = per_chunk * 0x0101010101010100ull;
   for (int k0 = 0; k0 < R; k0 += kSortAhead) {
     int at[kSortAhead];
 #pragma unroll
     for (int u = 0; u < kSortAhead; u++)
-      if (k0 + u < R) {
-        const unsigned row = (row0 + (unsigned)(k0 + u) * srow) & rmask;
-        at[u] = atomicAdd(&bins[row >> f.bin_shift], 1);
-        if (FP32) {
-          const int c8 = 8 * (int)((row >> f.seg_log) & (kPackChunks - 1));
-          order[(place >> c8) & 255] = (uint8_t)(k0 + u);
-          place += 1ull << c8;
-        }
-      }
+      if (k0 + u < R)
+        at[u] = atomicAdd(&bins[((row0 + (unsigned)(k0 + u) * srow) & rmask) >> f.bin_shift], 1);
 #pragma unroll
     for (int u = 0; u < kSortAhead; u++)
       if (k0 + u < R) list[at[u]] = (uint16_t)(tid << 5 | (k0 + u));
-  }
-  if (FP32) {
-    // the chunk's further bits, kPackLog at a time
-    for (int sft = kPackLog; (rmask >> f.seg_log) >> sft; sft += kPackLog) {
-      uint64_t cnt = 0;
-      for (int k = 0; k < R; k++)
-        cnt += 1ull << (8 * ((((row0 + (unsigned)k * srow) & rmask) >> (f.seg_log + sft)) &
-                             (kPackChunks - 1)));
-      uint64_t at = cnt * 0x0101010101010100ull;
-      for (int i = 0; i < R; i++) {
-        const unsigned k = order[i];
-        const int c8 = 8 * (int)((((row0 + k * srow) & rmask) >> (f.seg_log + sft)) &
-                                 (kPackChunks - 1));
-        order2[(at >> c8) & 255] = (uint8_t)k;
-        at += 1ull << c8;
-      }
-      uint8_t *t = order;
-      order = order2;
-      order2 = t;
-    }
   }
   __syncthreads();
   const double2 *__restrict__ x = a.x[s];
@@ -483,6 +455,32 @@ __device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f
   const T2 *mine = slots + tid * f.tR;
   const int64_t out = (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est) + b;
   if constexpr (FP32) {
+    // the taps in summation order, a byte each, where the list was: stable
+    // counting sorts by the chunk, kPackLog bits at a time, the counts and
+    // the places (their exclusive byte-wise prefix sum) in 64-bit words
+    const int tR4 = (f.tR + 3) & ~3;
+    uint8_t *order = reinterpret_cast<uint8_t *>(
+        reinterpret_cast<uint32_t *>(smem64) + f.order_at) + tid * tR4;
+    uint8_t *from = order + npairs * tR4;  // second list, for several passes
+    for (int sft = 0; sft == 0 || (rmask >> f.seg_log) >> sft; sft += kPackLog) {
+      auto bits = [&](unsigned k) {
+        return 8 * (int)((((row0 + k * srow) & rmask) >> (f.seg_log + sft)) & (kPackChunks - 1));
+      };
+      uint64_t place = 0;
+      for (int k = 0; k < R; k++) place += 1ull << bits(k);
+      place *= 0x0101010101010100ull;
+      if (sft) {
+        uint8_t *t = order;
+        order = from;
+        from = t;
+      }
+      for (int i = 0; i < R; i++) {
+        const unsigned k = sft ? from[i] : (unsigned)i;
+        const int c8 = bits(k);
+        order[(place >> c8) & 255] = (uint8_t)k;
+        place += 1ull << c8;
+      }
+    }
     float2 tot = make_float2(0.f, 0.f), sum = tot, cmp = tot;
     unsigned chunk = ~0u;
     for (int i0 = 0; i0 < R; i0 += 4) {
@@ -519,13 +517,20 @@ __device__ __forceinline__ void fold_group(const V12Launch &a, const FoldPart &f
   }
 }
 
-// grid: S x f.groups, then S x f.zero_blocks
+// grid: f.combs, S x f.groups, S x f.zero_blocks
 __global__ void __launch_bounds__(kFoldThreads) k_fold_sorted(V12Launch a, FoldParts f)
 {
   extern __shared__ double2 smem64[];
   __shared__ int sh[16];
-  if (blockIdx.x >= (unsigned)(a.S * f.groups)) {
-    const unsigned z = blockIdx.x - (unsigned)(a.S * f.groups);
+  unsigned blk = blockIdx.x;
+  if (blk < (unsigned)f.combs) {
+    comb_block<kFoldThreads>(a, (int)blk / a.comb_loops, (int)blk % a.comb_loops, smem64,
+                             reinterpret_cast<int *>(smem64 + a.W));
+    return;
+  }
+  blk -= (unsigned)f.combs;
+  if (blk >= (unsigned)(a.S * f.groups)) {
+    const unsigned z = blk - (unsigned)(a.S * f.groups);
     double2 *out = a.o_dense[z / (unsigned)f.zero_blocks];
     if (!out) return;  // not wanted on the device
     const int64_t step = (int64_t)f.zero_blocks * kFoldThreads;
@@ -534,8 +539,8 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_sorted(V12Launch a, FoldP
       out[i] = make_double2(0.0, 0.0);
     return;
   }
-  const int s = (int)(blockIdx.x / (unsigned)f.groups);
-  int g = (int)(blockIdx.x % (unsigned)f.groups);
+  const int s = (int)(blk / (unsigned)f.groups);
+  int g = (int)(blk % (unsigned)f.groups);
   FoldPart p = f.p[0];
   if (g >= p.groups) {
     g -= p.groups;
@@ -764,7 +769,10 @@ __global__ void __launch_bounds__(kBlock) k_vote_write(V12Launch a, int chunks)
       base += s_cnt[i * NW + w];
     }
   }
-  if (ch == chunks - 1 && threadIdx.x == 0) a.count[s] = min(base, a.hits_cap);
+  if (ch == chunks - 1 && threadIdx.x == 0) {
+    a.count[s] = min(base, a.hits_cap);
+    if (a.count_host) a.count_host[s] = min(base, a.hits_cap);
+  }
 }
 
 // ---------------------------------------------------------------- v2 votes (diagnostic)
@@ -1220,52 +1228,9 @@ __device__ __forceinline__ unsigned inv_odd(unsigned a)
   return x;
 }
 
-// Zero or of a magnitude whose quotients by a filter power near one neither
-// overflow nor lose bits to underflow on the way (false for infinities and
-// NaN): the FP64 estimate divides such buckets by a tabulated reciprocal.
-__device__ __forceinline__ bool plain_value(double v)
-{
-  const double m = fabs(v);
-  return m == 0.0 || (m >= 0x1p-700 && m <= 0x1p700);
-}
-
-// Bucket FFTs of loops [l0, l0 + nl), written in the alias-row layout.
-// FP64: rows_odd[s L + l] says whether any bucket is not a plain value.
-template <bool FP32>
-__global__ void __launch_bounds__(1024) k_bucket_fft_rows(V12Launch a, int l0, int nl)
-{
-  using T2 = typename std::conditional<FP32, float2, double2>::type;
-  extern __shared__ char rraw[];
-  T2 *rbuf = reinterpret_cast<T2 *>(rraw);
-  const int s = blockIdx.x / nl, l = l0 + blockIdx.x % nl;
-  const int B = l < a.Lloc ? a.B_loc : a.B_est;
-  const int logB = ilog2(B);
-  const int rows = a.n / a.W, d = B / rows;
-  const int stride = 2 * a.L + max(a.comb_loops, 1);
-  const unsigned ai = (unsigned)a.params[(int64_t)s * stride + a.L + l];
-  const unsigned uinv = inv_odd(ai) & (unsigned)(rows - 1);
-  T2 *io;
-  if constexpr (FP32) io = a.xs32; else io = a.xs64;
-  io += (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est);
-  slot_fft_fill(rbuf, logB, [&](int m) { return io[m]; });
-  if constexpr (FP32) slot_fft(rbuf, logB, a.tw32, a.tw_nmax / B);
-  else slot_fft(rbuf, logB, a.tw64, a.tw_nmax / B);
-  int odd = 0;
-  for (int b = threadIdx.x; b < B; b += blockDim.x) {
-    const int r = b % d, q = b / d;
-    const T2 z = rbuf[fft_slot<T2>(b, logB)];
-    if (!FP32) odd |= !plain_value(z.x) | !plain_value(z.y);
-    io[r * rows + (int)(((unsigned)q * uinv) & (unsigned)(rows - 1))] = z;
-  }
-  if (!FP32) {
-    odd = __syncthreads_or(odd);
-    if (threadIdx.x == 0) a.rows_odd[(int64_t)s * a.L + l] = odd;
-  }
-}
-
 // Per (signal, residue, loop): where the residue's bucket row lies and what
-// its buckets are multiplied or divided by.  Written once per batch by
-// k_rows_table; the workgroups of k_estimate_rows copy their residues'
+// its buckets are multiplied or divided by.  Written once per batch; the
+// workgroups of k_estimate_rows copy their residues'
 // entries to LDS (computing them there cost every 64 rows' workgroup the
 // hashing and the quotients again).
 struct RowEntry32 {
@@ -1278,14 +1243,13 @@ struct RowEntry64 {
   unsigned off, q;  // as above; bit 31 of q: not to be divided by inv
 };
 
-// One thread per (signal, residue slot, loop).
+// Entry t = (signal, residue slot, loop).
 template <bool FP32>
-__global__ void __launch_bounds__(kBlock) k_rows_table(V12Launch a)
+__device__ __forceinline__ void rows_entry(const V12Launch &a, int64_t t)
 {
   using Entry = typename std::conditional<FP32, RowEntry32, RowEntry64>::type;
   constexpr unsigned kElt = FP32 ? sizeof(float2) : sizeof(double2);
   const int L = a.L, cap = a.comb_loops * a.num;
-  const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (t >= (int64_t)a.S * cap * L) return;
   const int l = (int)(t % L);
   const int64_t si = t / L;
@@ -1318,6 +1282,63 @@ __global__ void __launch_bounds__(kBlock) k_rows_table(V12Launch a)
     if (!near1) e.q |= 0x80000000u;
   }
   reinterpret_cast<Entry *>(a.rows_tab)[t] = e;
+}
+
+// The entries in a launch of their own, after a comb on the second stream.
+template <bool FP32>
+__global__ void __launch_bounds__(kBlock) k_rows_table(V12Launch a)
+{
+  rows_entry<FP32>(a, (int64_t)blockIdx.x * kBlock + threadIdx.x);
+}
+
+// Zero or of a magnitude whose quotients by a filter power near one neither
+// overflow nor lose bits to underflow on the way (false for infinities and
+// NaN): the FP64 estimate divides such buckets by a tabulated reciprocal.
+__device__ __forceinline__ bool plain_value(double v)
+{
+  const double m = fabs(v);
+  return m == 0.0 || (m >= 0x1p-700 && m <= 0x1p700);
+}
+
+// Bucket FFTs of loops [l0, l0 + nl), written in the alias-row layout.
+// FP64: rows_odd[s L + l] says whether any bucket is not a plain value.
+// The workgroups past the transforms write the estimation entries, one a
+// thread, when the comb is done by now (a launch of their own cost a single
+// signal 4 us).
+template <bool FP32>
+__global__ void __launch_bounds__(1024) k_bucket_fft_rows(V12Launch a, int l0, int nl)
+{
+  using T2 = typename std::conditional<FP32, float2, double2>::type;
+  extern __shared__ char rraw[];
+  T2 *rbuf = reinterpret_cast<T2 *>(rraw);
+  if (blockIdx.x >= (unsigned)(a.S * nl)) {
+    rows_entry<FP32>(a, (int64_t)(blockIdx.x - (unsigned)(a.S * nl)) * blockDim.x + threadIdx.x);
+    return;
+  }
+  const int s = blockIdx.x / nl, l = l0 + blockIdx.x % nl;
+  const int B = l < a.Lloc ? a.B_loc : a.B_est;
+  const int logB = ilog2(B);
+  const int rows = a.n / a.W, d = B / rows;
+  const int stride = 2 * a.L + max(a.comb_loops, 1);
+  const unsigned ai = (unsigned)a.params[(int64_t)s * stride + a.L + l];
+  const unsigned uinv = inv_odd(ai) & (unsigned)(rows - 1);
+  T2 *io;
+  if constexpr (FP32) io = a.xs32; else io = a.xs64;
+  io += (int64_t)s * a.xs + loop_offset(l, a.Lloc, a.B_loc, a.B_est);
+  slot_fft_fill(rbuf, logB, [&](int m) { return io[m]; });
+  if constexpr (FP32) slot_fft(rbuf, logB, a.tw32, a.tw_nmax / B);
+  else slot_fft(rbuf, logB, a.tw64, a.tw_nmax / B);
+  int odd = 0;
+  for (int b = threadIdx.x; b < B; b += blockDim.x) {
+    const int r = b % d, q = b / d;
+    const T2 z = rbuf[fft_slot<T2>(b, logB)];
+    if (!FP32) odd |= !plain_value(z.x) | !plain_value(z.y);
+    io[r * rows + (int)(((unsigned)q * uinv) & (unsigned)(rows - 1))] = z;
+  }
+  if (!FP32) {
+    odd = __syncthreads_or(odd);
+    if (threadIdx.x == 0) a.rows_odd[(int64_t)s * a.L + l] = odd;
+  }
 }
 
 // Residues per tile of k_estimate_rows (RI / 4 per wavefront): 16 for
@@ -1651,6 +1672,8 @@ static int top_levels(const V12Launch &a, hipStream_t st, const double *mag, int
 // Below this many comb transforms per batch they run with kCombWide threads.
 constexpr int kFewCombs = 64, kCombWide = 1024;
 
+static int comb_merge(const V12Launch &a, hipStream_t st);
+
 int comb(const V12Launch &a, hipStream_t st)
 {
   if (a.W <= kMaxLdsComb) {
@@ -1674,22 +1697,24 @@ int comb(const V12Launch &a, hipStream_t st)
                    a.comb_loops == 1) != 0)
       return -1;
   }
-  if (a.comb_loops > 1) {
-    const size_t lb = (size_t)((a.W + 31) / 32) * 4;
-    hipLaunchKernelGGL(k_comb_merge, dim3(a.S), dim3(kBlock), lb, st, a);
-    if (launched("comb_merge") != 0) return -1;
-  }
-  if (a.rows_layout) {
-    const int64_t entries = (int64_t)a.S * a.comb_loops * a.num * a.L;
-    const dim3 grid((unsigned)((entries + kBlock - 1) / kBlock));
-    if (a.fp32) hipLaunchKernelGGL(k_rows_table<true>, grid, dim3(kBlock), 0, st, a);
-    else hipLaunchKernelGGL(k_rows_table<false>, grid, dim3(kBlock), 0, st, a);
-    if (launched("rows_table") != 0) return -1;
-  }
-  return 0;
+  return a.comb_loops > 1 ? comb_merge(a, st) : 0;
 }
 
 size_t rows_entry_bytes(bool fp32) { return fp32 ? sizeof(RowEntry32) : sizeof(RowEntry64); }
+
+static int64_t rows_entries(const V12Launch &a)
+{
+  return (int64_t)a.S * a.comb_loops * a.num * a.L;
+}
+
+int rows_table(const V12Launch &a, hipStream_t st)
+{
+  if (!a.rows_layout) return 0;
+  const dim3 grid((unsigned)((rows_entries(a) + kBlock - 1) / kBlock));
+  if (a.fp32) hipLaunchKernelGGL(k_rows_table<true>, grid, dim3(kBlock), 0, st, a);
+  else hipLaunchKernelGGL(k_rows_table<false>, grid, dim3(kBlock), 0, st, a);
+  return launched("rows_table");
+}
 
 // The part of loops [l0, l0 + nl) with `res` residues per workgroup and its
 // LDS; false when the loops do not fit the kernel's limits.
@@ -1722,50 +1747,95 @@ static bool fold_part(const V12Launch &a, bool fp32, int l0, int nl, int B, int 
     f.nbins >>= 1;
     f.bin_shift++;
   }
-  lds = slots + npairs * (sizeof(uint2) + sizeof(int)) +
-        (npairs * f.tR * sizeof(uint16_t) + 3) / 4 * 4;
+  lds = slots + npairs * (sizeof(uint2) + sizeof(int));
   f.order_at = (int)(lds / 4);
-  if (fp32) lds += npairs * ((f.tR + 3) & ~3) * ((rows >> f.seg_log) > kPackChunks ? 2 : 1);
+  const size_t list = (npairs * f.tR * sizeof(uint16_t) + 3) / 4 * 4;
+  const size_t order = npairs * ((f.tR + 3) & ~3) * ((rows >> f.seg_log) > kPackChunks ? 2 : 1);
+  lds += fp32 ? std::max(list, order) : list;
   return npairs <= kFoldThreads && lds <= kFoldLds;
 }
 
-// Loops [0, n64) in FP64 (from loop `from` on) and [n64, L) in FP32.
-static int fold_sorted(const V12Launch &a, hipStream_t st, int from, int n64)
+// The sorted fold of loops [0, n64) in FP64 (from loop `from` on) and
+// [n64, L) in FP32, and its LDS.  False when the loops do not fit.
+static bool fold_parts(const V12Launch &a, int from, int n64, FoldParts &f, size_t &lds)
 {
   // 16 residues (256 contiguous bytes of a row) read HBM 5-10 % faster than
   // 8 on batches (FP32 256 x n = 2^22, k = 64: 3.20 against 3.56 ms beside
   // the estimation; FP64 64 signals: 0.81 against 0.86 ms); a launch of few
   // workgroups is faster spread over twice as many (one signal: 19.0 against
-  // 20.8 us), and two resident workgroups' LDS does not hold 16 residues of
-  // many FP64 loops
-  FoldParts f{};
-  size_t lds = 0;
+  // 20.8 us), and a workgroup's LDS does not hold 16 residues of many FP64
+  // loops
+  f = FoldParts{};
+  lds = 0;
   int np = 0;
   auto add = [&](bool fp32, int l0, int l1) {
-    if (l1 <= l0) return 0;
+    if (l1 <= l0) return true;
     const int B = l0 < a.Lloc ? a.B_loc : a.B_est;
-    size_t b16 = 0;
-    const bool wide = (int64_t)a.S * B >= 16 * 512 && fold_part(a, fp32, l0, l1 - l0, B, 16, f.p[np], b16);
-    if (!wide && !fold_part(a, fp32, l0, l1 - l0, B, 8, f.p[np], b16)) {
-      set_error("fold: more than 32 taps per bucket");
-      return -1;
-    }
-    lds = std::max(lds, b16);
+    size_t need = 0;
+    const bool wide = (int64_t)a.S * B >= 16 * 512 &&
+                      fold_part(a, fp32, l0, l1 - l0, B, 16, f.p[np], need);
+    if (!wide && !fold_part(a, fp32, l0, l1 - l0, B, 8, f.p[np], need)) return false;
+    lds = std::max(lds, need);
     f.groups += f.p[np].groups;
     np++;
-    return 0;
+    return true;
   };
-  const bool same = a.B_loc == a.B_est;
-  const int cut = same ? n64 : a.Lloc;  // where the bucket count or precision changes
-  // (with both, they change at the same loop: n64 is 0, Lloc or L)
-  if (add(n64 == 0, from, cut) != 0 || add(cut >= n64, std::max(cut, from), a.L) != 0) return -1;
+  // where the bucket count or precision changes (with both, they change at
+  // the same loop: n64 is 0, Lloc or L)
+  const int cut = a.B_loc == a.B_est ? n64 : a.Lloc;
+  return add(n64 == 0, from, cut) && add(cut >= n64, std::max(cut, from), a.L);
+}
+
+// Loops in FP64 of a batch: the first ones.
+static int fp64_loops(const V12Launch &a)
+{
+  return !a.fp32 ? a.L : (a.loc64 ? a.Lloc : 0);
+}
+
+static size_t comb_lds(const V12Launch &a)
+{
+  return (size_t)a.W * sizeof(double2) + kTopScratch * sizeof(int);
+}
+
+bool fuse_comb(const V12Launch &a)
+{
+  // in the fold's launch the comb costs no second stream and no events; its
+  // LDS is every workgroup's of the launch, so it has to leave room for two
+  // on a CU, or the launch has to be small
+  if (a.comb_loops == 0 || a.W > kMaxLdsComb || a.fold_mode == 0) return false;
+  FoldParts f;
+  size_t lds;
+  if (!fold_parts(a, 0, fp64_loops(a), f, lds)) return false;
+  const size_t need = comb_lds(a);
+  return need <= std::max(lds, (size_t)79 * 1024) ||
+         (need <= kFoldLds && (int64_t)a.S * (f.groups + a.comb_loops) <= 256);
+}
+
+static int comb_merge(const V12Launch &a, hipStream_t st)
+{
+  const size_t lb = (size_t)((a.W + 31) / 32) * 4;
+  hipLaunchKernelGGL(k_comb_merge, dim3(a.S), dim3(kBlock), lb, st, a);
+  return launched("comb_merge");
+}
+
+static int fold_sorted(const V12Launch &a, hipStream_t st, int from, int n64)
+{
+  FoldParts f;
+  size_t lds = 0;
+  if (!fold_parts(a, from, n64, f, lds)) {
+    set_error("fold: more than 32 taps per bucket");
+    return -1;
+  }
   f.zero_blocks = a.zero_dense ? (int)std::min<int64_t>(512, (a.n + 4095) / 4096) : 0;
-  if (np == 0 && f.zero_blocks == 0) return 0;
+  f.combs = a.comb_fused ? a.S * a.comb_loops : 0;
+  if (f.combs) lds = std::max(lds, comb_lds(a));
+  const int64_t blocks = f.combs + (int64_t)a.S * (f.groups + f.zero_blocks);
+  if (blocks == 0) return 0;
   allow_lds(k_fold_sorted, lds);
-  hipLaunchKernelGGL(k_fold_sorted,
-                     dim3((unsigned)((int64_t)a.S * (f.groups + f.zero_blocks))),
-                     dim3(kFoldThreads), lds, st, a, f);
-  return launched("fold_sorted") == 0 ? 1 : -1;
+  hipLaunchKernelGGL(k_fold_sorted, dim3((unsigned)blocks), dim3(kFoldThreads), lds, st, a, f);
+  if (launched("fold_sorted") != 0) return -1;
+  if (f.combs && a.comb_loops > 1 && comb_merge(a, st) != 0) return -1;
+  return 1;
 }
 
 // Whether the bucket FFTs of a v1 batch select the top buckets too.
@@ -1779,7 +1849,7 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
 {
   // loops [0, n64) in FP64, [n64, L) in FP32 (with the FFTs in part 1
   // whatever the schedule)
-  const int n64 = !a.fp32 ? a.L : (a.loc64 ? a.Lloc : 0);
+  const int n64 = fp64_loops(a);
   const int B64 = n64 == 0 ? 0 : (n64 > a.Lloc ? max(a.B_loc, a.B_est) : a.B_loc);
   int launches = 0;
   if (part == 0) {
@@ -1798,15 +1868,17 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
   // part 1: the bucket FFTs of every loop not fused into its fold
   if (a.rows_layout) {
     // v2: every loop in one precision, written in the alias-row layout
-    const int Bm = max(a.B_loc, a.B_est);
+    const int Bm = max(a.B_loc, a.B_est), T = fft_threads(Bm);
+    const int64_t entries = a.comb_fused ? rows_entries(a) : 0;
+    const dim3 grid((unsigned)((int64_t)a.S * a.L + (entries + T - 1) / T));
     if (a.fp32) {
       allow_lds(k_bucket_fft_rows<true>, (size_t)Bm * sizeof(float2));
-      hipLaunchKernelGGL(k_bucket_fft_rows<true>, dim3(a.S * a.L), dim3(fft_threads(Bm)),
-                         (size_t)Bm * sizeof(float2), st, a, 0, a.L);
+      hipLaunchKernelGGL(k_bucket_fft_rows<true>, grid, dim3(T), (size_t)Bm * sizeof(float2), st,
+                         a, 0, a.L);
     } else {
       allow_lds(k_bucket_fft_rows<false>, (size_t)Bm * sizeof(double2));
-      hipLaunchKernelGGL(k_bucket_fft_rows<false>, dim3(a.S * a.L), dim3(fft_threads(Bm)),
-                         (size_t)Bm * sizeof(double2), st, a, 0, a.L);
+      hipLaunchKernelGGL(k_bucket_fft_rows<false>, grid, dim3(T), (size_t)Bm * sizeof(double2), st,
+                         a, 0, a.L);
     }
     if (launched("bucket_fft_rows") != 0) return -1;
     return 1;

@@ -546,6 +546,14 @@ __global__ void __launch_bounds__(kFoldThreads) k_fold_sorted(V12Launch a, FoldP
     g -= p.groups;
     p = f.p[1];
   }
+  // workgroups dispatched one after another take residues four groups apart
+  // (a rotation of g by two bits): with neighbours side by side in a row
+  // the same reads took longer (256 x n = 2^22 FP32 step 3.72 against 3.48
+  // ms, 64 signals FP64 1.10 against 1.02 ms, 8 x 2^24 2.92 against 2.87;
+  // one to six bits, bit reversal and a signal per XCD gave 3.42-3.73,
+  // 1.03-1.19 and 2.86-3.01, none better on all three)
+  const int lg = p.logB - p.log_res;
+  if (lg > 2) g = ((g << 2) | (g >> (lg - 2))) & (p.groups - 1);
   if (p.fp32) fold_group<true>(a, p, s, g, smem64, sh);
   else fold_group<false>(a, p, s, g, smem64, sh);
 }

@@ -38,6 +38,13 @@ constexpr int kPreAhead = 8;
 // Pairs per LDS chunk of the Gauss subtractions (fewer fitting than
 // kMinStageChunk: indices and values read from memory instead).
 constexpr int kStageChunk = 1024, kMinStageChunk = 32;
+// Entries a thread ranks per chunk, and values read ahead of a bucket's
+// subtractions.
+constexpr int kStageRanks = (3 * kStageChunk + kV3Block - 1) / kV3Block, kStageAhead = 4;
+// Hash slots and pairs per chunk of the Mansour subtractions, and the LDS
+// they take.
+constexpr int kMansourSlots = 256, kMansourChunk = 512;
+constexpr size_t kMansourBytes = (kMansourSlots + 2 * kMansourChunk) * sizeof(int);
 
 __device__ __forceinline__ int ilog2v(int v) { return 31 - __clz(v); }
 
@@ -99,19 +106,26 @@ __device__ __forceinline__ int ms_counted(double2 z, double invW)
   return re * re + im * im > 1e-6;
 }
 
-// MS bucket h less (r0, r1), its dirty bit set and the count updated.
-__device__ __forceinline__ void ms_sub(const Ctx &c, int h, double2 r0, double2 r1)
+// MS bucket h becomes (now, now1), loop 0's value having been old: its
+// dirty bit set and the count updated.
+__device__ __forceinline__ void ms_put(const Ctx &c, int h, double2 old, double2 now,
+                                       double2 now1)
 {
-  const double2 old = c.MS[2 * h];
-  const double2 now = csub(old, r0);
   c.MS[2 * h] = now;
-  c.MS[2 * h + 1] = csub(c.MS[2 * h + 1], r1);
+  c.MS[2 * h + 1] = now1;
   if (c.dirty) {
     const double invW = 1.0 / c.W;
     atomicOr(&c.dirty[h >> 5], 1u << (h & 31));
     const int d = ms_counted(now, invW) - ms_counted(old, invW);
     if (d) atomicAdd(c.cm, d);
   }
+}
+
+// MS bucket h less (r0, r1).
+__device__ __forceinline__ void ms_sub(const Ctx &c, int h, double2 r0, double2 r1)
+{
+  const double2 old = c.MS[2 * h];
+  ms_put(c, h, old, csub(old, r0), csub(c.MS[2 * h + 1], r1));
 }
 
 // ---------------------------------------------------------------- map
@@ -318,10 +332,13 @@ constexpr size_t kStagePairBytes = 6 * sizeof(double2) + sizeof(int) + 3 * sizeo
 // copies the chunk's bucket indices and removal values next to the bucket
 // arrays (one memory latency per chunk) and sorts the chunk's 3m entries
 // e = 3 u + q (pair u, q = 0, 1, 2 for its buckets h, h+1, h-1) by bucket:
-// counts, an exclusive scan, atomic placement, then each bucket's short
-// list re-sorted by e.  The owner of a bucket applies its entries in e
-// order, which is pair order and h, h+1, h-1 within a pair (cf3 465-482):
-// the subtractions a bucket sees and their order are unchanged.  stage
+// counts, an exclusive scan, atomic placement, then every entry moved to its
+// rank among the e of its bucket's list (one thread an entry: the buckets'
+// own threads sorting by insertion waited for LDS about L^2 / 4 times, 14 us
+// more for the 48 pairs of an 8-bucket filter).  The owner of a bucket applies
+// its entries in e order, which is pair order and h, h+1, h-1 within a pair
+// (cf3 465-482): the subtractions a bucket sees and their order are
+// unchanged.  stage
 // holds chunk * kStagePairBytes + (B + 16) * 4 bytes of LDS.  Called by
 // every thread of the block (barriers inside).
 __device__ void gauss_apply_staged(double2 *__restrict__ S0, double2 *__restrict__ S1, int B,
@@ -375,26 +392,47 @@ __device__ void gauss_apply_staged(double2 *__restrict__ S0, double2 *__restrict
       list[atomicAdd(&pos[b], 1)] = e;  // pos[b] ends at the end of bucket b
     }
     __syncthreads();
-    for (int tb = t; tb < B; tb += T) {
-      const int lo = tb ? pos[tb - 1] : 0, hi = pos[tb];
-      for (int i = lo + 1; i < hi; i++) {  // insertion sort by e (short lists)
-        const int v = list[i];
-        int j = i - 1;
-        while (j >= lo && list[j] > v) {
-          list[j + 1] = list[j];
-          j--;
+    // every entry's rank in its bucket's list, all entries at once
+    int slot_of[kStageRanks];
+#pragma unroll
+    for (int x = 0; x < kStageRanks; x++) {
+      const int e = t + x * T;
+      if (e >= 3 * m) break;
+      const int u = e / 3, q = e - 3 * u;
+      const int h = sh_idx[u];
+      const int b = q == 0 ? h : (q == 1 ? (h + 1) & bm : (h + bm) & bm);
+      const int lo = b ? pos[b - 1] : 0, hi = pos[b];
+      int before = lo;
+      for (int i = lo; i < hi; i++) before += list[i] < e;
+      slot_of[x] = before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < kStageRanks; x++) {
+      const int e = t + x * T;
+      if (e >= 3 * m) break;
+      list[slot_of[x]] = e;
+    }
+    __syncthreads();
+    // two threads per bucket, one for each offset's array
+    for (int tb = t; tb < 2 * B; tb += T) {
+      const int bk = tb & bm, off = tb < B ? 0 : 3;
+      double2 *__restrict__ S = tb < B ? S0 : S1;
+      const int lo = bk ? pos[bk - 1] : 0, hi = pos[bk];
+      double2 acc = S[bk];
+      for (int i0 = lo; i0 < hi; i0 += kStageAhead) {
+        double2 v[kStageAhead];
+#pragma unroll
+        for (int x = 0; x < kStageAhead; x++) {  // past the end: the last entry again, unused
+          const int e = list[min(i0 + x, hi - 1)];
+          const int u = e / 3;
+          v[x] = sv[6 * u + (e - 3 * u) + off];
         }
-        list[j + 1] = v;
+#pragma unroll
+        for (int x = 0; x < kStageAhead; x++)
+          if (i0 + x < hi) acc = csub(acc, v[x]);
       }
-      double2 a0 = S0[tb], a1 = S1[tb];
-      for (int i = lo; i < hi; i++) {
-        const int e = list[i];
-        const int u = e / 3, q = e - 3 * u;
-        a0 = csub(a0, sv[6 * u + q]);
-        a1 = csub(a1, sv[6 * u + 3 + q]);
-      }
-      S0[tb] = a0;
-      S1[tb] = a1;
+      S[bk] = acc;
     }
   }
   __syncthreads();
@@ -412,6 +450,54 @@ __device__ void mansour_removal(const Ctx &c, int key, double2 value, int &h, do
   sincos(PI2_OVER_N * key * (c.g0 + 1), &s1, &c1);
   r[0] = make_double2(W * (vr * c0 - vi * s0), W * (vr * s0 + vi * c0));
   r[1] = make_double2(W * (vr * c1 - vi * s1), W * (vr * s1 + vi * c1));
+}
+
+// The Mansour subtractions of cnt pairs, a chunk at a time: the pairs of a
+// chunk that fall on the same of kMansourSlots LDS hash slots are chained,
+// and the first pair of every bucket (the one whose chain holds no earlier
+// pair of that bucket) takes all of the bucket's pairs in pair order -- the
+// subtractions of a bucket and their order are those of one thread applying
+// every pair.  All first pairs read their buckets at once: with a thread per
+// residue of h a wave met its pairs one after another, a memory latency
+// each (a pass of 111 pairs took 26 us with it, 10 us now).  iw: kMansourBytes of LDS.  All
+// threads; contains barriers.
+__device__ __forceinline__ void mansour_apply_chained(const Ctx &c, const int *remi,
+                                                      const double2 *rem, int cnt, int *iw)
+{
+  constexpr int T = kV3Block;
+  static_assert(kMansourChunk <= T, "one pair a thread");
+  int *head = iw, *next = iw + kMansourSlots, *hs = next + kMansourChunk;
+  const int t = threadIdx.x;
+  for (int base = 0; base < cnt; base += kMansourChunk) {
+    const int m = min(kMansourChunk, cnt - base);
+    __threadfence_block();
+    __syncthreads();  // the previous chunk (and any other use of iw) is over
+    for (int j = t; j < kMansourSlots; j += T) head[j] = -1;
+    const int h = t < m ? remi[(int64_t)(base + t) * 3 + 2] : 0;
+    if (t < m) hs[t] = h;
+    __syncthreads();
+    if (t < m) next[t] = atomicExch(&head[h & (kMansourSlots - 1)], t);
+    __syncthreads();
+    if (t >= m) continue;  // (the loop's barriers are reached by every thread)
+    bool first = true, more = false;
+    for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q]) {
+      const bool same = hs[q] == h;
+      first &= !(same && q < t);
+      more |= same && q > t;
+    }
+    if (!first) continue;
+    const double2 *r = rem + (int64_t)(base + t) * 14 + 12;
+    ms_sub(c, h, r[0], r[1]);
+    for (int cur = t; more;) {  // later pairs of this bucket, ascending
+      int nxt = kMansourChunk;
+      for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q])
+        if (hs[q] == h && q > cur) nxt = min(nxt, q);
+      if (nxt == kMansourChunk) break;
+      r = rem + (int64_t)(base + nxt) * 14 + 12;
+      ms_sub(c, h, r[0], r[1]);
+      cur = nxt;
+    }
+  }
 }
 
 // Subtraction values of cnt (key, value) pairs, then their application in
@@ -449,28 +535,50 @@ __device__ __forceinline__ void removals(const Ctx &c, const int *keys, const do
 __device__ __forceinline__ void subtract(const Ctx &c, const int *keys, const double2 *vals,
                                          int cnt, int which)
 {
+  if (cnt == 0) return;
   const V3Launch &a = *c.a;
   // LDS staging for the applications
   const size_t room = c.room;
   double2 *const sv = c.stage;
   if (cnt <= kSerialApply && !a.serial_all &&
       room >= (size_t)kSerialApply * (14 * sizeof(double2) + 3 * sizeof(int))) {
-    // Few pairs: the removal values stay in LDS; one thread per Gauss
-    // bucket array applies them in pair order, and each Mansour bucket
-    // (in HBM) is updated by its owner thread h mod kV3Block in pair order
-    // -- every bucket sees the same subtractions in the same order.
+    // Few pairs: the removal values stay in LDS; the owner of a Gauss
+    // bucket applies them in pair order, and each Mansour bucket (in HBM)
+    // is updated by the lane of its first pair, in pair order -- every
+    // bucket sees the same subtractions in the same order.
     int *si = reinterpret_cast<int *>(sv + 14 * kSerialApply);
-    removals(c, keys, vals, cnt, which, sv, si);
-    __syncthreads();
-    if (which & 1) gauss_apply_few(c.GS0, c.GS1, c.B1, si, 0, sv, 0, cnt);
-    if (which & 2) gauss_apply_few(c.GP0, c.GP1, c.B2, si, 1, sv, 6, cnt);
-    if (which & 4) {
-      for (int i = 0; i < cnt; i++) {
-        const int h = si[i * 3 + 2];
-        if ((h & (kV3Block - 1)) != (int)threadIdx.x) continue;
-        ms_sub(c, h, sv[i * 14 + 12], sv[i * 14 + 13]);
+    // the last wave (no removal is computed there) loads the Mansour
+    // buckets meanwhile; pair j's lane j takes them when no earlier pair
+    // has the same bucket
+    const int mj = (int)threadIdx.x - (kV3Block - 64);
+    const bool mansour = (which & 4) && mj >= 0;
+    int mh = -1;
+    bool first = false, more = false;
+    double2 z0 = make_double2(0, 0), z1 = make_double2(0, 0);
+    if (mansour) {
+      if (mj < cnt) {
+        mh = keys[mj] & (c.W - 1);
+        z0 = c.MS[2 * mh];
+        z1 = c.MS[2 * mh + 1];
+      }
+      first = mj < cnt;
+#pragma unroll
+      for (int q = 0; q < kSerialApply; q++) {
+        const int hq = __shfl(mh, q, 64);
+        first &= !(q < mj && hq == mh);
+        more |= q > mj && hq == mh;
       }
     }
+    removals(c, keys, vals, cnt, which, sv, si);
+    __syncthreads();
+    if (mansour) {
+      if (first) ms_put(c, mh, z0, csub(z0, sv[mj * 14 + 12]), csub(z1, sv[mj * 14 + 13]));
+      if (first && more)
+        for (int i = mj + 1; i < cnt; i++)
+          if (si[i * 3 + 2] == mh) ms_sub(c, mh, sv[i * 14 + 12], sv[i * 14 + 13]);
+    }
+    if (which & 1) gauss_apply_few(c.GS0, c.GS1, c.B1, si, 0, sv, 0, cnt);
+    if (which & 2) gauss_apply_few(c.GP0, c.GP1, c.B2, si, 1, sv, 6, cnt);
     __threadfence_block();
     __syncthreads();
     return;
@@ -513,21 +621,15 @@ __device__ __forceinline__ void subtract(const Ctx &c, const int *keys, const do
     }
   }
   if (which & 4) {
-    constexpr int T = kV3Block;
-    const int t = threadIdx.x;
-    const int *__restrict__ remi = c.remi;
-    const double2 *__restrict__ rem = c.rem;
-    for (int i0 = 0; i0 < cnt; i0 += kApplyAhead) {
-      int hh[kApplyAhead];
-#pragma unroll
-      for (int u = 0; u < kApplyAhead; u++)
-        hh[u] = i0 + u < cnt ? remi[(i0 + u) * 3 + 2] : -1;
-#pragma unroll
-      for (int u = 0; u < kApplyAhead; u++) {
-        const int h = hh[u];
-        if (h < 0) break;
+    if (room >= kMansourBytes) {
+      mansour_apply_chained(c, c.remi, c.rem, cnt, reinterpret_cast<int *>(sv));
+    } else {
+      constexpr int T = kV3Block;
+      const int t = threadIdx.x;
+      for (int i = 0; i < cnt; i++) {
+        const int h = c.remi[i * 3 + 2];
         if ((h & (T - 1)) != t) continue;  // h = key mod W >= 0
-        const double2 *r = rem + (int64_t)(i0 + u) * 14 + 12;
+        const double2 *r = c.rem + (int64_t)i * 14 + 12;
         ms_sub(c, h, r[0], r[1]);
       }
     }
@@ -667,11 +769,12 @@ __device__ __forceinline__ bool mansour_bucket(const Ctx &c, const MansourConst 
 // evaluates only the acceptance test, on kSweepAhead steps' buckets loaded
 // together (one memory latency for them): each thread keeps its accepted
 // steps as bits, each wave writes the count of a step to rank[step NW +
-// wave]; a
-// block scan over rank (which is bucket order) gives every (step, wave) its
-// first slot; the second sweep estimates the accepted buckets and writes
-// each at that slot plus its accepted lanes below.  rank holds kV3Block
-// ints of LDS.
+// wave]; a block scan over rank (which is bucket order) gives every
+// (step, wave) its first slot, and the accepted buckets are listed in ef at
+// that slot plus the accepted lanes below.  Then one thread estimates each
+// listed bucket.  (Estimated where they lie, a few accepted buckets in every
+// step made every step pay two arctangents and a sine: 871 of 8192 buckets
+// took 33 us, 12 now.)  rank holds kV3Block ints of LDS.
 __device__ __forceinline__ int est_mansour(const Ctx &c, int *rank, int *sh)
 {
   constexpr int T = kV3Block, NW = T / 64, SEG = 64;
@@ -720,18 +823,22 @@ __device__ __forceinline__ int est_mansour(const Ctx &c, int *rank, int *sh)
     for (int st = 0; st < steps; st++) {
       const bool ok = (mine >> st) & 1;
       const uint64_t bal = __ballot(ok);
-      if (ok) {
-        const int bk = s0 + st * T + threadIdx.x;
-        int o = -1;
-        double2 v = make_double2(0, 0);
-        (void)mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
-        const int pos = rank[st * NW + wid] + __popcll(bal & ((1ull << lane) - 1));
-        c.ef[pos] = o;
-        c.ev[pos] = v;
-      }
+      if (ok)
+        c.ef[rank[st * NW + wid] + __popcll(bal & ((1ull << lane) - 1))] =
+            s0 + st * T + (int)threadIdx.x;
     }
     found += total;
     __syncthreads();  // rank is rewritten by the next segment
+  }
+  __threadfence_block();
+  __syncthreads();
+  for (int i = threadIdx.x; i < found; i += T) {
+    const int bk = c.ef[i];
+    int o = -1;
+    double2 v = make_double2(0, 0);
+    (void)mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
+    c.ef[i] = o;
+    c.ev[i] = v;
   }
   __threadfence_block();
   __syncthreads();
@@ -794,6 +901,7 @@ __device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *sh)
 // Returns false when the map would overflow.
 __device__ __forceinline__ bool map_add_found(const Ctx &c, int F, int *sh, int *s_size)
 {
+  if (F == 0) return true;
   const int T = blockDim.x;
   const int C = (F + T - 1) / T;
   const int lo = threadIdx.x * C, hi = min(F, lo + C);
@@ -809,14 +917,17 @@ __device__ __forceinline__ bool map_add_found(const Ctx &c, int F, int *sh, int 
   if (base + total > c.a->map_limit) return false;
   for (int i = lo; i < hi; i++) {
     int e = c.remi[i * 3];
+    // ans[f] = ans[f] + v (distinct keys within one pass; a new key's ans[f]
+    // is 0, added all the same: 0 + -0 is 0)
+    double2 v = make_double2(0.0, 0.0);
     if (e < 0) {
       e = base + pos++;
       c.keys[e] = c.ef[i];
-      c.vals[e] = make_double2(0.0, 0.0);
       map_insert_slot(c, c.ef[i], e);
+    } else {
+      v = c.vals[e];
     }
-    // ans[f] = ans[f] + v (distinct keys within one pass)
-    c.vals[e] = cadd(c.vals[e], c.ev[i]);
+    c.vals[e] = cadd(v, c.ev[i]);
   }
   __threadfence_block();
   __syncthreads();
@@ -1445,12 +1556,83 @@ __device__ void block_bitonic_u64(uint64_t *v, int P)
   __syncthreads();
 }
 
+// Entry e of the map as output t of signal s.
+__device__ __forceinline__ void put_result(const V3Launch &a, int s, const double2 *vals, int t,
+                                           int key, int e)
+{
+  const double2 v = vals[e];
+  if (a.o_freq && t < a.o_cap) {
+    int32_t *of = a.o_freq[s];
+    double2 *ov = a.o_val[s];
+    if (of) of[t] = key;
+    if (ov) ov[t] = v;
+  }
+  if (a.o_dense && a.o_dense[s]) a.o_dense[s][key] = v;
+}
+
 // The result of signal s: the map (M entries in insertion order) sorted by
 // frequency into the sparse outputs and scattered into the dense one; count
-// and status flags.  All threads; contains barriers.
+// and status flags.  The entries are counted into kResultBins equal bands of
+// frequency, placed band by band, and each ranked among its band's: a few
+// barriers, where a bitonic sort has one or two for each of its log^2 stages
+// (about 900 entries: 17 us, 4 us now; 52: 7.9 us, 2.6 us now).  Where the
+// frequencies crowd (a band of more than kResultBand) ranking would take as
+// many reads as the band has entries, and the bitonic sort is taken.  All
+// threads; contains barriers.
+constexpr int kResultBins = 1024, kResultBand = 64;
 __device__ void write_result(const V3Launch &a, int s, const int *keys, const double2 *vals,
                              int M, int flags, double2 *lds)
 {
+  constexpr int T = kV3Block, C = kResultBins / T;
+  __shared__ int s_scan[T / 64], s_most;
+  if (threadIdx.x == 0) {
+    a.count[s] = M;
+    a.status[s] = flags;
+  }
+  int *bin = reinterpret_cast<int *>(lds);  // counts, then starts, then ends
+  int2 *list = reinterpret_cast<int2 *>(bin + kResultBins);
+  if ((size_t)kResultBins * sizeof(int) + (size_t)M * sizeof(int2) <= a.lds_bytes) {
+    const int shift = max(0, ilog2v(a.n) - ilog2v(kResultBins));
+    const int t = threadIdx.x;
+    for (int i = t; i < kResultBins; i += T) bin[i] = 0;
+    if (t == 0) s_most = 0;
+    __syncthreads();
+    for (int i = t; i < M; i += T) atomicAdd(&bin[keys[i] >> shift], 1);
+    __syncthreads();
+    int v[C], sum = 0, most = 0;
+#pragma unroll
+    for (int u = 0; u < C; u++) {
+      v[u] = bin[t * C + u];
+      sum += v[u];
+      most = max(most, v[u]);
+    }
+    if (most > kResultBand) atomicMax(&s_most, most);
+    int total;
+    int run = block_exclusive_scan(sum, s_scan, total);  // (orders s_most)
+    if (s_most <= kResultBand) {
+#pragma unroll
+      for (int u = 0; u < C; u++) {
+        bin[t * C + u] = run;
+        run += v[u];
+      }
+      __syncthreads();
+      for (int i = t; i < M; i += T) {
+        const int key = keys[i];
+        list[atomicAdd(&bin[key >> shift], 1)] = make_int2(key, i);
+      }
+      __syncthreads();  // bin[b] is the end of band b
+      for (int i = t; i < M; i += T) {
+        const int2 x = list[i];
+        const int b = x.x >> shift;
+        const int lo = b ? bin[b - 1] : 0, hi = bin[b];
+        int pos = lo;
+        for (int q = lo; q < hi; q++) pos += list[q].x < x.x;
+        put_result(a, s, vals, pos, x.x, x.y);
+      }
+      return;
+    }
+    __syncthreads();  // bin is overwritten
+  }
   int P = 1;
   while (P < M) P <<= 1;
   uint64_t *srt = reinterpret_cast<uint64_t *>(lds);
@@ -1462,19 +1644,7 @@ __device__ void write_result(const V3Launch &a, int s, const int *keys, const do
   }
   for (int t = threadIdx.x; t < M; t += blockDim.x) {
     const int e = sortable ? (int)(srt[t] & 0xffffffffu) : t;
-    const int key = keys[e];
-    const double2 v = vals[e];
-    if (a.o_freq && t < a.o_cap) {
-      int32_t *of = a.o_freq[s];
-      double2 *ov = a.o_val[s];
-      if (of) of[t] = key;
-      if (ov) ov[t] = v;
-    }
-    if (a.o_dense && a.o_dense[s]) a.o_dense[s][key] = v;
-  }
-  if (threadIdx.x == 0) {
-    a.count[s] = M;
-    a.status[s] = flags;
+    put_result(a, s, vals, t, keys[e], e);
   }
 }
 

@@ -355,3 +355,23 @@ def test_v3_map_overflow_writes_every_result(torch_cuda):
                         dense.ctypes.data_as(C.c_void_p))
     assert "overflow" in _lib.last_error()
     assert not np.isnan(dense).any() and np.count_nonzero(dense) <= 12
+
+
+@pytest.mark.parametrize("k,width", [(200, 1536), (400, 40000), (60, 1 << 20)])
+def test_v3_result_order(torch_cuda, k, width):
+    """The result is sorted by counting into 1024 bands of frequency and
+    ranking within a band, or, where a band holds more than 64 entries, by a
+    bitonic sort: 200 tones in the lowest 1536 frequencies of 2^20 (130 in
+    one band), 400 in the lowest 40,000 (18) and 60 over the whole range, as
+    the oracle gives them (values within the 1e-9 of the parity test)."""
+    n = 1 << 20
+    print(f"case v3 result order k={k} width={width}", flush=True)
+    rng = np.random.default_rng(5)
+    X = np.zeros(n, np.complex128)
+    X[rng.choice(width, k, replace=False)] = np.exp(2j * np.pi * rng.random(k))
+    x = np.fft.ifft(X) * n
+    plan = sfft_amd.sfft(n, k, 3, seed=(17, 4242))
+    ref = _oracle_v3(n, k, x, _plan_filters(plan))
+    fr, va = plan.execute_sparse_host(x)
+    assert not ref["early"] and np.array_equal(fr, ref["freqs"])
+    assert np.abs(va - ref["vals"]).max() <= 1e-9 * np.abs(ref["vals"]).max()

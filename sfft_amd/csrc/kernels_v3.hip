@@ -6,9 +6,8 @@
 // Parallel within a signal: the filters (gathers, folds, FFTs in LDS), the
 // per-bucket estimation (atan2 / sincos), the result-map updates and the
 // subtraction values.  The subtractions themselves reach every bucket in the
-// reference's order (found-list order: short passes by one thread per bucket
-// array, longer ones by the thread owning the bucket), so every bucket sees
-// the same sequence of roundings as in the oracle.  The
+// reference's order (found-list order, by the thread that owns the bucket),
+// so every bucket sees the same sequence of roundings as in the oracle.  The
 // result map is iterated in insertion order (the reference's
 // tr1::unordered_map order is unreproducible; see the oracle).
 #include <algorithm>
@@ -26,25 +25,21 @@ namespace {
 
 constexpr int kV3Block = 512;
 static_assert((kV3Block & (kV3Block - 1)) == 0, "owner tests take residues by masking");
-// Subtraction passes of up to this many pairs run on one thread per bucket
-// array; longer ones on bucket-owner threads.
-constexpr int kSerialApply = 16;
-// Bucket indices an owner thread loads ahead in the subtraction scans.
-constexpr int kApplyAhead = 32;
+// Passes that found up to this many pairs keep them and their subtraction
+// values in LDS.
+constexpr int kFewPairs = 16;
 // Steps of a sweep over the Mansour buckets whose loads are issued together.
 constexpr int kSweepAhead = 4;
 // Loads the pre-kernel's gathers and folds issue together per thread.
 constexpr int kPreAhead = 8;
-// Pairs per LDS chunk of the Gauss subtractions (fewer fitting than
-// kMinStageChunk: indices and values read from memory instead).
-constexpr int kStageChunk = 1024, kMinStageChunk = 32;
-// Entries a thread ranks per chunk, and values read ahead of a bucket's
-// subtractions.
+// Pairs per LDS chunk of the subtractions (fewer fitting than
+// kMinStageChunk: one thread per bucket array).
+constexpr int kStageChunk = 1024, kMinStageChunk = 16;
+// Entries of one Gauss filter a thread ranks per chunk, values read ahead of
+// a bucket's subtractions, and hash slots of a chunk's Mansour buckets.
 constexpr int kStageRanks = (3 * kStageChunk + kV3Block - 1) / kV3Block, kStageAhead = 4;
-// Hash slots and pairs per chunk of the Mansour subtractions, and the LDS
-// they take.
-constexpr int kMansourSlots = 256, kMansourChunk = 512;
-constexpr size_t kMansourBytes = (kMansourSlots + 2 * kMansourChunk) * sizeof(int);
+constexpr int kMansourSlots = 256;
+static_assert(6 * kStageChunk <= 65536, "list entries are 16 bits");
 
 __device__ __forceinline__ int ilog2v(int v) { return 31 - __clz(v); }
 
@@ -59,9 +54,17 @@ __device__ __forceinline__ int wave_sum(int v)
 // int products in the reference wrap modulo 2^32 (cf3 381-382, 475, 743)
 __device__ __forceinline__ int wmul(int x, int y) { return (int)((unsigned)x * (unsigned)y); }
 
+// x a mod n for x, a >= 0 and n a power of two
 __device__ __forceinline__ int timesmod(int x, int a, int n)
 {
-  return (int)(((long long)x * a) % n);
+  return (int)((unsigned long long)x * (unsigned long long)a & (unsigned long long)(n - 1));
+}
+
+// x % n (the sign of x) for n a power of two
+__device__ __forceinline__ int smod(int x, int n)
+{
+  const int m = x & (n - 1);
+  return x < 0 && m ? m - n : m;
 }
 
 // Filter response at signed offset d from a window stored as
@@ -95,6 +98,8 @@ struct Ctx {
   int *cm;
   double2 *stage;  // LDS for the subtractions, room bytes
   size_t room;
+  int *lf;  // LDS: the first kFewPairs of ef and ev, of the last estimate
+  double2 *lv;
 };
 
 // The round-robin loop's test on a Mansour bucket (loop-0 value z): power
@@ -196,9 +201,9 @@ __device__ __forceinline__ GaussIdx gauss_index(const Ctx &c, int key, int B)
 {
   const int n = c.n;
   const unsigned n1 = (unsigned)n - 1;
-  const unsigned nb = (unsigned)n / (unsigned)B;
+  const unsigned nb = (unsigned)n >> ilog2v(B);
   GaussIdx x;
-  x.h = (int)(key * 1. / nb + 0.5) % B;
+  x.h = (int)(key * 1. / nb + 0.5) & (B - 1);
   const unsigned dist1 = ((unsigned)x.h * nb - (unsigned)key + (unsigned)n) & n1;
   x.dd[0] = dist1;
   x.dd[1] = (dist1 + (unsigned)n + nb) & n1;
@@ -212,8 +217,8 @@ __device__ __forceinline__ void gauss_values(const Ctx &c, int key, double2 valu
   const int n = c.n;
   const double PI2_DIV_N = 2 * M_PI / n;
   const double a1 = value.x, b1 = value.y;
-  const int ko = wmul(key, g) % n;
-  const int ko2 = wmul(key, (int)((unsigned)g + (unsigned)step)) % n;
+  const int ko = smod(wmul(key, g), n);
+  const int ko2 = smod(wmul(key, (int)((unsigned)g + (unsigned)step)), n);
   double b2, a2, b22, a22;
   sincos(PI2_DIV_N * ko, &b2, &a2);
   sincos(PI2_DIV_N * ko2, &b22, &a22);
@@ -245,27 +250,27 @@ __device__ void gauss_apply_pair(double2 *S0, double2 *S1, int B, int h, const d
   for (int q = 0; q < 3; q++) S1[bk[q]] = csub(S1[bk[q]], r[3 + q]);
 }
 
-// A few pairs (removal values in LDS: 14 per pair, this filter's at roff;
-// bucket index at 3 i + slot) applied by bucket owners: thread t takes its
+// A few pairs (removal values in LDS, nv per pair, bucket indices nf per
+// pair, both from this filter's first on) applied by bucket owners: thread t takes its
 // buckets t, t + blockDim, ... and walks the pairs in order, applying the
 // parts that land on the bucket (h, h+1, h-1 within a pair) -- the order
 // in which gauss_apply_pair applies them pair after pair.
 __device__ __forceinline__ void gauss_apply_few(double2 *S0, double2 *S1, int B, const int *si,
-                                                int slot, const double2 *sv, int roff, int cnt)
+                                                int nf, const double2 *sv, int nv, int cnt)
 {
   const int bm = B - 1;  // B a power of two
   for (int tb = threadIdx.x; tb < B; tb += blockDim.x) {
     double2 a0 = make_double2(0, 0), a1 = make_double2(0, 0);
     bool any = false;
     for (int i = 0; i < cnt; i++) {
-      const int h = si[i * 3 + slot];
+      const int h = si[i * nf];
       if ((unsigned)((tb - h + 1) & bm) > 2u) continue;
       if (!any) {
         a0 = S0[tb];
         a1 = S1[tb];
         any = true;
       }
-      const double2 *r = sv + i * 14 + roff;
+      const double2 *r = sv + i * nv;
       if (h == tb) {
         a0 = csub(a0, r[0]);
         a1 = csub(a1, r[3]);
@@ -286,158 +291,6 @@ __device__ __forceinline__ void gauss_apply_few(double2 *S0, double2 *S1, int B,
   }
 }
 
-// Pair i subtracts r[0..2] from buckets h, h+1, h-1 of S0 and r[3..5] from
-// those of S1 (in that order; with B <= 2 a bucket can be several of them).
-// Thread t owns the buckets b = t mod blockDim and takes the pairs in pair
-// order, kApplyAhead bucket indices loaded ahead (each batch costs one
-// memory latency).
-__device__ void gauss_apply_owned(double2 *__restrict__ S0, double2 *__restrict__ S1, int B,
-                                  const int *__restrict__ remi, int slot,
-                                  const double2 *__restrict__ rem, int roff, int cnt)
-{
-  constexpr int T = kV3Block;
-  const int t = threadIdx.x;
-  if (t >= B) return;
-  // B and T are powers of two: the buckets h-1, h, h+1 of a pair can only
-  // include one of this thread's (b mod T == t) when (h - t + 1) mod
-  // min(B, T) <= 2; only those pairs take the exact test below
-  const int M = min(B, T);
-  for (int i0 = 0; i0 < cnt; i0 += kApplyAhead) {
-    int hh[kApplyAhead];
-#pragma unroll
-    for (int u = 0; u < kApplyAhead; u++)
-      hh[u] = i0 + u < cnt ? remi[(i0 + u) * 3 + slot] : -1;
-#pragma unroll
-    for (int u = 0; u < kApplyAhead; u++) {
-      const int h = hh[u];
-      if (h < 0) break;
-      if ((unsigned)((h - t + 1) & (M - 1)) > 2u) continue;
-      const int bk[3] = {h, (h + 1) % B, (h + B - 1) % B};
-#pragma unroll
-      for (int q = 0; q < 3; q++) {
-        if (bk[q] % T != t) continue;
-        const double2 *r = rem + (int64_t)(i0 + u) * 14 + roff;
-        S0[bk[q]] = csub(S0[bk[q]], r[q]);
-        S1[bk[q]] = csub(S1[bk[q]], r[3 + q]);
-      }
-    }
-  }
-}
-
-// LDS bytes the staged application needs per pair of a chunk: 6 removal
-// values, the bucket index, three sort entries.
-constexpr size_t kStagePairBytes = 6 * sizeof(double2) + sizeof(int) + 3 * sizeof(int);
-
-// As gauss_apply_owned, a chunk of pairs at a time through LDS: the block
-// copies the chunk's bucket indices and removal values next to the bucket
-// arrays (one memory latency per chunk) and sorts the chunk's 3m entries
-// e = 3 u + q (pair u, q = 0, 1, 2 for its buckets h, h+1, h-1) by bucket:
-// counts, an exclusive scan, atomic placement, then every entry moved to its
-// rank among the e of its bucket's list (one thread an entry: the buckets'
-// own threads sorting by insertion waited for LDS about L^2 / 4 times, 14 us
-// more for the 48 pairs of an 8-bucket filter).  The owner of a bucket applies
-// its entries in e order, which is pair order and h, h+1, h-1 within a pair
-// (cf3 465-482): the subtractions a bucket sees and their order are
-// unchanged.  stage
-// holds chunk * kStagePairBytes + (B + 16) * 4 bytes of LDS.  Called by
-// every thread of the block (barriers inside).
-__device__ void gauss_apply_staged(double2 *__restrict__ S0, double2 *__restrict__ S1, int B,
-                                   const int *__restrict__ remi, int slot,
-                                   const double2 *__restrict__ rem, int roff, int cnt,
-                                   double2 *__restrict__ stage, int chunk)
-{
-  constexpr int T = kV3Block;
-  const int t = threadIdx.x;
-  const int bm = B - 1;  // B a power of two
-  double2 *__restrict__ sv = stage;
-  int *__restrict__ sh_idx = reinterpret_cast<int *>(sv + 6 * (size_t)chunk);
-  int *__restrict__ list = sh_idx + chunk;
-  int *__restrict__ pos = list + 3 * chunk;  // B bucket counts, then ends
-  int *__restrict__ sh = pos + B;            // scan scratch
-  const int C = (B + T - 1) / T;             // buckets per thread in the scan
-  for (int base = 0; base < cnt; base += chunk) {
-    const int m = min(chunk, cnt - base);
-    __syncthreads();  // the previous chunk is applied
-    for (int j = t; j < m; j += T) sh_idx[j] = remi[(int64_t)(base + j) * 3 + slot];
-    for (int j = t; j < 6 * m; j += T) {
-      const int u = j / 6, q = j - 6 * u;
-      sv[j] = rem[(int64_t)(base + u) * 14 + roff + q];
-    }
-    for (int b = t; b < B; b += T) pos[b] = 0;
-    __syncthreads();
-    for (int e = t; e < 3 * m; e += T) {
-      const int u = e / 3, q = e - 3 * u;
-      const int h = sh_idx[u];
-      const int b = q == 0 ? h : (q == 1 ? (h + 1) & bm : (h + bm) & bm);
-      atomicAdd(&pos[b], 1);
-    }
-    __syncthreads();
-    {
-      const int lo = t * C, hi = min(B, lo + C);
-      int sum = 0;
-      for (int b = lo; b < hi; b++) sum += pos[b];
-      int total;
-      int run = block_exclusive_scan(sum, sh, total);
-      for (int b = lo; b < hi; b++) {
-        const int v = pos[b];
-        pos[b] = run;  // start of bucket b's entries
-        run += v;
-      }
-    }
-    __syncthreads();
-    for (int e = t; e < 3 * m; e += T) {
-      const int u = e / 3, q = e - 3 * u;
-      const int h = sh_idx[u];
-      const int b = q == 0 ? h : (q == 1 ? (h + 1) & bm : (h + bm) & bm);
-      list[atomicAdd(&pos[b], 1)] = e;  // pos[b] ends at the end of bucket b
-    }
-    __syncthreads();
-    // every entry's rank in its bucket's list, all entries at once
-    int slot_of[kStageRanks];
-#pragma unroll
-    for (int x = 0; x < kStageRanks; x++) {
-      const int e = t + x * T;
-      if (e >= 3 * m) break;
-      const int u = e / 3, q = e - 3 * u;
-      const int h = sh_idx[u];
-      const int b = q == 0 ? h : (q == 1 ? (h + 1) & bm : (h + bm) & bm);
-      const int lo = b ? pos[b - 1] : 0, hi = pos[b];
-      int before = lo;
-      for (int i = lo; i < hi; i++) before += list[i] < e;
-      slot_of[x] = before;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int x = 0; x < kStageRanks; x++) {
-      const int e = t + x * T;
-      if (e >= 3 * m) break;
-      list[slot_of[x]] = e;
-    }
-    __syncthreads();
-    // two threads per bucket, one for each offset's array
-    for (int tb = t; tb < 2 * B; tb += T) {
-      const int bk = tb & bm, off = tb < B ? 0 : 3;
-      double2 *__restrict__ S = tb < B ? S0 : S1;
-      const int lo = bk ? pos[bk - 1] : 0, hi = pos[bk];
-      double2 acc = S[bk];
-      for (int i0 = lo; i0 < hi; i0 += kStageAhead) {
-        double2 v[kStageAhead];
-#pragma unroll
-        for (int x = 0; x < kStageAhead; x++) {  // past the end: the last entry again, unused
-          const int e = list[min(i0 + x, hi - 1)];
-          const int u = e / 3;
-          v[x] = sv[6 * u + (e - 3 * u) + off];
-        }
-#pragma unroll
-        for (int x = 0; x < kStageAhead; x++)
-          if (i0 + x < hi) acc = csub(acc, v[x]);
-      }
-      S[bk] = acc;
-    }
-  }
-  __syncthreads();
-}
-
 // update_mansour_loops2 (cf3 300-351)
 __device__ void mansour_removal(const Ctx &c, int key, double2 value, int &h, double2 *r)
 {
@@ -452,186 +305,313 @@ __device__ void mansour_removal(const Ctx &c, int key, double2 value, int &h, do
   r[1] = make_double2(W * (vr * c1 - vi * s1), W * (vr * s1 + vi * c1));
 }
 
-// The Mansour subtractions of cnt pairs, a chunk at a time: the pairs of a
-// chunk that fall on the same of kMansourSlots LDS hash slots are chained,
-// and the first pair of every bucket (the one whose chain holds no earlier
-// pair of that bucket) takes all of the bucket's pairs in pair order -- the
-// subtractions of a bucket and their order are those of one thread applying
-// every pair.  All first pairs read their buckets at once: with a thread per
-// residue of h a wave met its pairs one after another, a memory latency
-// each (a pass of 111 pairs took 26 us with it, 10 us now).  iw: kMansourBytes of LDS.  All
-// threads; contains barriers.
-__device__ __forceinline__ void mansour_apply_chained(const Ctx &c, const int *remi,
-                                                      const double2 *rem, int cnt, int *iw)
-{
-  constexpr int T = kV3Block;
-  static_assert(kMansourChunk <= T, "one pair a thread");
-  int *head = iw, *next = iw + kMansourSlots, *hs = next + kMansourChunk;
-  const int t = threadIdx.x;
-  for (int base = 0; base < cnt; base += kMansourChunk) {
-    const int m = min(kMansourChunk, cnt - base);
-    __threadfence_block();
-    __syncthreads();  // the previous chunk (and any other use of iw) is over
-    for (int j = t; j < kMansourSlots; j += T) head[j] = -1;
-    const int h = t < m ? remi[(int64_t)(base + t) * 3 + 2] : 0;
-    if (t < m) hs[t] = h;
-    __syncthreads();
-    if (t < m) next[t] = atomicExch(&head[h & (kMansourSlots - 1)], t);
-    __syncthreads();
-    if (t >= m) continue;  // (the loop's barriers are reached by every thread)
-    bool first = true, more = false;
-    for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q]) {
-      const bool same = hs[q] == h;
-      first &= !(same && q < t);
-      more |= same && q > t;
-    }
-    if (!first) continue;
-    const double2 *r = rem + (int64_t)(base + t) * 14 + 12;
-    ms_sub(c, h, r[0], r[1]);
-    for (int cur = t; more;) {  // later pairs of this bucket, ascending
-      int nxt = kMansourChunk;
-      for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q])
-        if (hs[q] == h && q > cur) nxt = min(nxt, q);
-      if (nxt == kMansourChunk) break;
-      r = rem + (int64_t)(base + nxt) * 14 + 12;
-      ms_sub(c, h, r[0], r[1]);
-      cur = nxt;
-    }
-  }
-}
-
-// Subtraction values of cnt (key, value) pairs, then their application in
-// pair order.  which: bit 0 Gauss-1, bit 1 Gauss-2, bit 2 Mansour.
-// Slots per pair in rem: [0..5] G1, [6..11] G2, [12..13] Mansour.
 // The removal values of cnt (key, value) pairs for the filters in which
-// (bit 0 Gauss-1, 1 Gauss-2, 2 Mansour) into r (14 per pair) and ri (3
-// bucket indices per pair).  One work item per (filter, pair); each
-// filter's pairs start on a wave boundary, so a wave runs one filter's
-// code and the filters' sincos and window loads proceed in parallel.
+// (bit 0 Gauss-1, 1 Gauss-2, 2 Mansour): nv values a pair in r0 (Gauss-1's
+// six, Gauss-2's six, Mansour's two, those of which alone) and nf bucket
+// indices a pair in ri0, in the same order.  One work item per (filter,
+// pair); each filter's pairs start on a wave boundary, so a wave runs one
+// filter's code and the filters' sincos and window loads proceed in
+// parallel.
+__device__ __forceinline__ int removal_values(int which)
+{
+  return 6 * (which & 1) + 6 * ((which >> 1) & 1) + 2 * ((which >> 2) & 1);
+}
+__device__ __forceinline__ int removal_indices(int which)
+{
+  return (which & 1) + ((which >> 1) & 1) + ((which >> 2) & 1);
+}
 __device__ __forceinline__ void removals(const Ctx &c, const int *keys, const double2 *vals,
                                          int cnt, int which, double2 *r0, int *ri0)
 {
   const V3Launch &a = *c.a;
-  int fs[3], nf = 0;
+  const int nv = removal_values(which), nf = removal_indices(which);
+  const int g1 = which & 1, g2 = (which >> 1) & 1;
+  int fs[3], k = 0;
   for (int f = 0; f < 3; f++)
-    if ((which >> f) & 1) fs[nf++] = f;
+    if ((which >> f) & 1) fs[k++] = f;
   const int stride = (cnt + 63) & ~63;
   for (int t = threadIdx.x; t < nf * stride; t += blockDim.x) {
-    const int q = t / stride, i = t - q * stride;
+    const int q = t < stride ? 0 : (t < 2 * stride ? 1 : 2), i = t - q * stride;
     if (i >= cnt) continue;
     const int f = fs[q];
     const int key = keys[i];
     const double2 v = vals[i];
-    double2 *r = r0 + (int64_t)i * 14;
-    int *ri = ri0 + (int64_t)i * 3;
+    double2 *r = r0 + i * nv;
+    int *ri = ri0 + i * nf;
     if (f == 0) gauss_removal(c, key, v, c.B1, a.win1, a.win1_half, c.gG, 1, ri[0], r);
     else if (f == 1)
-      gauss_removal(c, (timesmod(key, c.ai, c.n) + c.shift) % c.n, v, c.B2, a.win2,
-                    a.win2_half, wmul(c.aa, c.gG), 1, ri[1], r + 6);
-    else mansour_removal(c, key, v, ri[2], r + 12);
+      gauss_removal(c, smod(timesmod(key, c.ai, c.n) + c.shift, c.n), v, c.B2, a.win2,
+                    a.win2_half, wmul(c.aa, c.gG), 1, ri[g1], r + 6 * g1);
+    else mansour_removal(c, key, v, ri[g1 + g2], r + 6 * (g1 + g2));
   }
 }
 
+// LDS bytes apply_staged needs per pair and besides (NB Gauss buckets).
+__device__ __forceinline__ size_t staged_pair_bytes(int which)
+{
+  const int ng = (which & 1) + ((which >> 1) & 1);
+  return removal_values(which) * sizeof(double2) + removal_indices(which) * sizeof(int) +
+         sizeof(int) + 3 * ng * sizeof(unsigned short);
+}
+__device__ __forceinline__ size_t staged_fixed_bytes(int NB)
+{
+  return (NB + 16 + kMansourSlots) * sizeof(int);
+}
+
+// The application of m <= kStageChunk pairs whose removals (sv, si, laid out
+// by removals) are in LDS; iw: LDS for the lists below.  All filters at
+// once, a barrier serving each:
+// - Gauss: the entries e = 3 u + q (pair u; q = 0, 1, 2 for its buckets h,
+//   h+1, h-1; Gauss-2's after Gauss-1's) are sorted by bucket -- counts, an
+//   exclusive scan, atomic placement, then every entry moved to its rank
+//   among the e of its bucket's list, one thread an entry.  (Sorted by
+//   insertion, a thread a bucket, the 48 pairs of an 8-bucket filter took
+//   14 us more.)  A thread for each bucket of each offset's array applies
+//   its entries in e order, which is pair order and h, h+1, h-1 within a
+//   pair (cf3 465-482).
+// - Mansour: the pairs that fall on the same of kMansourSlots hash slots
+//   are chained, and the first pair of every bucket (the one whose chain
+//   holds no earlier pair of that bucket) takes all of the bucket's pairs
+//   in pair order, the buckets loaded before the sort.  (With a thread per
+//   residue of h a wave met its pairs one after another, a memory latency
+//   each: a pass of 111 pairs took 16 us more.)
+// So the subtractions a bucket sees and their order are those of one thread
+// applying pair after pair.  Called by every thread of the block; contains
+// barriers, none at its end.
+__device__ __forceinline__ void apply_staged(const Ctx &c, int which, const double2 *sv,
+                                             const int *si, int m, int *iw)
+{
+  constexpr int T = kV3Block, MP = (kStageChunk + T - 1) / T, MR = 2 * kStageRanks;
+  const int t = threadIdx.x;
+  const int nv = removal_values(which), nf = removal_indices(which);
+  const int ng = (which & 1) + ((which >> 1) & 1);
+  const int Ba = (which & 1) ? c.B1 : c.B2;  // buckets of the first Gauss filter here
+  const int Bb = ng == 2 ? c.B2 : 0;         // and of the second
+  const int NB = Ba + Bb, E = 3 * m * ng;
+  int *pos = iw, *sh = pos + NB, *head = sh + 16, *next = head + kMansourSlots;
+  unsigned short *list = reinterpret_cast<unsigned short *>(next + m);
+  // bin and value index of entry e
+  auto entry = [&](int e, int &vi) {
+    const bool second = e >= 3 * m;
+    const int e1 = second ? e - 3 * m : e;
+    const int u = e1 / 3, q = e1 - 3 * u;
+    const int h = si[u * nf + second], bm = (second ? Bb : Ba) - 1;  // powers of two
+    vi = u * nv + 6 * second + q;
+    return (second ? Ba : 0) + (q == 0 ? h : (q == 1 ? (h + 1) & bm : (h + bm) & bm));
+  };
+  int vi;
+  double2 z0[MP], z1[MP];
+  int hh[MP];
+#pragma unroll
+  for (int x = 0; x < MP; x++) {
+    hh[x] = 0;
+    z0[x] = z1[x] = make_double2(0, 0);
+    if ((which & 4) && t + x * T < m) {
+      hh[x] = si[(t + x * T) * nf + ng];
+      z0[x] = c.MS[2 * hh[x]];
+      z1[x] = c.MS[2 * hh[x] + 1];
+    }
+  }
+  for (int b = t; b < NB; b += T) pos[b] = 0;
+  if (which & 4)
+    for (int j = t; j < kMansourSlots; j += T) head[j] = -1;
+  __syncthreads();
+  for (int e = t; e < E; e += T) atomicAdd(&pos[entry(e, vi)], 1);
+  if (which & 4)
+#pragma unroll
+    for (int x = 0; x < MP; x++)
+      if (t + x * T < m) next[t + x * T] = atomicExch(&head[hh[x] & (kMansourSlots - 1)], t + x * T);
+  __syncthreads();
+  {
+    const int C = (NB + T - 1) / T;  // bins per thread in the scan
+    const int lo = min(NB, t * C), hi = min(NB, lo + C);
+    int sum = 0;
+    for (int b = lo; b < hi; b++) sum += pos[b];
+    int total;
+    int run = block_exclusive_scan(sum, sh, total);
+    for (int b = lo; b < hi; b++) {
+      const int v = pos[b];
+      pos[b] = run;  // start of bin b's entries
+      run += v;
+    }
+  }
+  __syncthreads();
+  for (int e = t; e < E; e += T) list[atomicAdd(&pos[entry(e, vi)], 1)] = (unsigned short)e;
+  __syncthreads();  // pos[b] is the end of bin b
+  int slot[MR];
+#pragma unroll
+  for (int x = 0; x < MR; x++) {
+    const int e = t + x * T;
+    if (e >= E) break;
+    const int b = entry(e, vi);
+    const int lo = b ? pos[b - 1] : 0, hi = pos[b];
+    int before = lo;
+    for (int i = lo; i < hi; i++) before += (int)list[i] < e;
+    slot[x] = before;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < MR; x++) {
+    const int e = t + x * T;
+    if (e >= E) break;
+    list[slot[x]] = (unsigned short)e;
+  }
+  if (which & 4) {
+#pragma unroll
+    for (int x = 0; x < MP; x++) {
+      const int j = t + x * T, h = hh[x];
+      if (j >= m) break;
+      bool first = true, more = false;
+      for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q]) {
+        const bool same = si[q * nf + ng] == h;
+        first &= !(same && q < j);
+        more |= same && q > j;
+      }
+      if (!first) continue;
+      const double2 *r = sv + j * nv + 6 * ng;
+      ms_put(c, h, z0[x], csub(z0[x], r[0]), csub(z1[x], r[1]));
+      for (int cur = j; more;) {  // later pairs of this bucket, ascending
+        int nxt = m;
+        for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q])
+          if (si[q * nf + ng] == h && q > cur) nxt = min(nxt, q);
+        if (nxt == m) break;
+        ms_sub(c, h, sv[nxt * nv + 6 * ng], sv[nxt * nv + 6 * ng + 1]);
+        cur = nxt;
+      }
+    }
+  }
+  __syncthreads();
+  for (int tb = t; tb < 2 * NB; tb += T) {
+    const int off = tb < NB ? 0 : 1, b = tb - off * NB;
+    // GS0, GS1, GP0, GP1 lie one after the other
+    const bool gp = b >= Ba || !(which & 1);
+    double2 *S = c.GS0 + (gp ? 2 * c.B1 + off * c.B2 + ((which & 1) ? b - Ba : b) : off * c.B1 + b);
+    const int lo = b ? pos[b - 1] : 0, hi = pos[b];
+    if (lo == hi) continue;
+    double2 acc = *S;
+    for (int i0 = lo; i0 < hi; i0 += kStageAhead) {
+      double2 v[kStageAhead];
+#pragma unroll
+      for (int x = 0; x < kStageAhead; x++) {  // past the end: the last entry again, unused
+        (void)entry(list[min(i0 + x, hi - 1)], vi);
+        v[x] = sv[vi + 3 * off];
+      }
+#pragma unroll
+      for (int x = 0; x < kStageAhead; x++)
+        if (i0 + x < hi) acc = csub(acc, v[x]);
+    }
+    *S = acc;
+  }
+}
+
+// Few pairs: kept, like their removal values, in LDS.
+__device__ __forceinline__ bool few_pairs(const Ctx &c, int cnt)
+{
+  return cnt <= kFewPairs && !c.a->serial_all &&
+         c.room >= (size_t)kFewPairs * (14 * sizeof(double2) + 3 * sizeof(int));
+}
+
+// The subtraction of the cnt <= kFewPairs pairs in lf, lv: the owner of a
+// Gauss bucket applies them in pair order, and each Mansour bucket (in HBM)
+// is updated by the lane of its first pair, in pair order -- every bucket
+// sees the same subtractions in the same order.  The last wave (no removal
+// is computed there) loads the Mansour buckets meanwhile.  Contains
+// barriers, none after the last update.
+__device__ __forceinline__ void subtract_few(const Ctx &c, int cnt, int which)
+{
+  double2 *const sv = c.stage;
+  int *const si = reinterpret_cast<int *>(sv + 14 * kFewPairs);
+  const int mj = (int)threadIdx.x - (kV3Block - 64);
+  const bool mansour = (which & 4) && mj >= 0;
+  int mh = -1;
+  bool first = false, more = false;
+  double2 z0 = make_double2(0, 0), z1 = make_double2(0, 0);
+  if (mansour) {
+    if (mj < cnt) {
+      mh = c.lf[mj] & (c.W - 1);
+      z0 = c.MS[2 * mh];
+      z1 = c.MS[2 * mh + 1];
+    }
+    first = mj < cnt;
+#pragma unroll
+    for (int q = 0; q < kFewPairs; q++) {
+      const int hq = __shfl(mh, q, 64);
+      first &= !(q < mj && hq == mh);
+      more |= q > mj && hq == mh;
+    }
+  }
+  removals(c, c.lf, c.lv, cnt, which, sv, si);
+  __syncthreads();
+  const int nv = removal_values(which), nf = removal_indices(which);
+  const int g1 = which & 1, g2 = (which >> 1) & 1;
+  if (mansour && first) {
+    const double2 *r = sv + 6 * (g1 + g2);
+    ms_put(c, mh, z0, csub(z0, r[mj * nv]), csub(z1, r[mj * nv + 1]));
+    if (more)
+      for (int i = mj + 1; i < cnt; i++)
+        if (si[i * nf + g1 + g2] == mh) ms_sub(c, mh, r[i * nv], r[i * nv + 1]);
+  }
+  if (g1) gauss_apply_few(c.GS0, c.GS1, c.B1, si, nf, sv, nv, cnt);
+  if (g2) gauss_apply_few(c.GP0, c.GP1, c.B2, si + g1, nf, sv + 6 * g1, nv, cnt);
+}
+
+// Subtraction of cnt (key, value) pairs from the buckets of the filters in
+// which, in pair order.  All threads; contains barriers, the last one at its
+// end.
 __device__ __forceinline__ void subtract(const Ctx &c, const int *keys, const double2 *vals,
                                          int cnt, int which)
 {
   if (cnt == 0) return;
-  const V3Launch &a = *c.a;
-  // LDS staging for the applications
-  const size_t room = c.room;
-  double2 *const sv = c.stage;
-  if (cnt <= kSerialApply && !a.serial_all &&
-      room >= (size_t)kSerialApply * (14 * sizeof(double2) + 3 * sizeof(int))) {
-    // Few pairs: the removal values stay in LDS; the owner of a Gauss
-    // bucket applies them in pair order, and each Mansour bucket (in HBM)
-    // is updated by the lane of its first pair, in pair order -- every
-    // bucket sees the same subtractions in the same order.
-    int *si = reinterpret_cast<int *>(sv + 14 * kSerialApply);
-    // the last wave (no removal is computed there) loads the Mansour
-    // buckets meanwhile; pair j's lane j takes them when no earlier pair
-    // has the same bucket
-    const int mj = (int)threadIdx.x - (kV3Block - 64);
-    const bool mansour = (which & 4) && mj >= 0;
-    int mh = -1;
-    bool first = false, more = false;
-    double2 z0 = make_double2(0, 0), z1 = make_double2(0, 0);
-    if (mansour) {
-      if (mj < cnt) {
-        mh = keys[mj] & (c.W - 1);
-        z0 = c.MS[2 * mh];
-        z1 = c.MS[2 * mh + 1];
-      }
-      first = mj < cnt;
-#pragma unroll
-      for (int q = 0; q < kSerialApply; q++) {
-        const int hq = __shfl(mh, q, 64);
-        first &= !(q < mj && hq == mh);
-        more |= q > mj && hq == mh;
-      }
+  if (few_pairs(c, cnt)) {
+    if ((int)threadIdx.x < cnt) {
+      c.lf[threadIdx.x] = keys[threadIdx.x];
+      c.lv[threadIdx.x] = vals[threadIdx.x];
     }
-    removals(c, keys, vals, cnt, which, sv, si);
     __syncthreads();
-    if (mansour) {
-      if (first) ms_put(c, mh, z0, csub(z0, sv[mj * 14 + 12]), csub(z1, sv[mj * 14 + 13]));
-      if (first && more)
-        for (int i = mj + 1; i < cnt; i++)
-          if (si[i * 3 + 2] == mh) ms_sub(c, mh, sv[i * 14 + 12], sv[i * 14 + 13]);
-    }
-    if (which & 1) gauss_apply_few(c.GS0, c.GS1, c.B1, si, 0, sv, 0, cnt);
-    if (which & 2) gauss_apply_few(c.GP0, c.GP1, c.B2, si, 1, sv, 6, cnt);
+    subtract_few(c, cnt, which);
     __threadfence_block();
     __syncthreads();
     return;
   }
+  const int nv = removal_values(which), nf = removal_indices(which);
+  const size_t fixed = staged_fixed_bytes(c.B1 + c.B2);
+  const int chunk =
+      c.room > fixed
+          ? (int)min((size_t)kStageChunk, (c.room - fixed) / staged_pair_bytes(which))
+          : 0;
+  if (chunk >= kMinStageChunk && !c.a->serial_all) {
+    // a chunk at a time through LDS: the removals, then their application
+    for (int base = 0; base < cnt; base += chunk) {
+      const int m = min(chunk, cnt - base);
+      double2 *const sv = c.stage;
+      int *const si = reinterpret_cast<int *>(sv + m * nv);
+      if (base) __syncthreads();  // the previous chunk is applied
+      removals(c, keys + base, vals + base, m, which, sv, si);
+      __syncthreads();
+      apply_staged(c, which, sv, si, m, si + m * nf);
+      __threadfence_block();
+    }
+    __syncthreads();
+    return;
+  }
+  // no room (tiny plans), or the diagnostic: one thread per bucket array
+  // applies every pair in turn
   removals(c, keys, vals, cnt, which, c.rem, c.remi);
   __threadfence_block();
   __syncthreads();
-  // One thread per bucket, each taking the pairs in pair order: a bucket
-  // sees the same subtractions in the same order as when one thread applies
-  // every pair in turn (cf3 465-482), so the results are the same.
-  if (cnt <= kSerialApply || c.a->serial_all) {
-    // few pairs: one thread per bucket array applies them all
-    if (threadIdx.x == 0 && (which & 1)) {
-      for (int i = 0; i < cnt; i++) gauss_apply_pair(c.GS0, c.GS1, c.B1, c.remi[i * 3], c.rem + (int64_t)i * 14);
-    } else if (threadIdx.x == 64 && (which & 2)) {
-      for (int i = 0; i < cnt; i++)
-        gauss_apply_pair(c.GP0, c.GP1, c.B2, c.remi[i * 3 + 1], c.rem + (int64_t)i * 14 + 6);
-    } else if (threadIdx.x == 128 && (which & 4)) {
-      for (int i = 0; i < cnt; i++) {
-        const int h = c.remi[i * 3 + 2];
-        const double2 *r = c.rem + (int64_t)i * 14 + 12;
-        ms_sub(c, h, r[0], r[1]);
-      }
-    }
-    __threadfence_block();
-    __syncthreads();
-    return;
-  }
-  {
-    // staged in LDS (kStagePairBytes per pair plus the bucket counts)
-    const size_t fixed = (size_t)(max(c.B1, c.B2) + 16) * sizeof(int);
-    const int chunk =
-        room > fixed ? (int)min((size_t)kStageChunk, (room - fixed) / kStagePairBytes) : 0;
-    if (chunk >= kMinStageChunk) {
-      if (which & 1) gauss_apply_staged(c.GS0, c.GS1, c.B1, c.remi, 0, c.rem, 0, cnt, sv, chunk);
-      if (which & 2) gauss_apply_staged(c.GP0, c.GP1, c.B2, c.remi, 1, c.rem, 6, cnt, sv, chunk);
-    } else {
-      if (which & 1) gauss_apply_owned(c.GS0, c.GS1, c.B1, c.remi, 0, c.rem, 0, cnt);
-      if (which & 2) gauss_apply_owned(c.GP0, c.GP1, c.B2, c.remi, 1, c.rem, 6, cnt);
-    }
-  }
-  if (which & 4) {
-    if (room >= kMansourBytes) {
-      mansour_apply_chained(c, c.remi, c.rem, cnt, reinterpret_cast<int *>(sv));
-    } else {
-      constexpr int T = kV3Block;
-      const int t = threadIdx.x;
-      for (int i = 0; i < cnt; i++) {
-        const int h = c.remi[i * 3 + 2];
-        if ((h & (T - 1)) != t) continue;  // h = key mod W >= 0
-        const double2 *r = c.rem + (int64_t)i * 14 + 12;
-        ms_sub(c, h, r[0], r[1]);
-      }
+  const int g1 = which & 1, g2 = (which >> 1) & 1;
+  const int *ri = c.remi;
+  const double2 *r = c.rem;
+  if (threadIdx.x == 0 && g1) {
+    for (int i = 0; i < cnt; i++)
+      gauss_apply_pair(c.GS0, c.GS1, c.B1, ri[(int64_t)i * nf], r + (int64_t)i * nv);
+  } else if (threadIdx.x == 64 && g2) {
+    for (int i = 0; i < cnt; i++)
+      gauss_apply_pair(c.GP0, c.GP1, c.B2, ri[(int64_t)i * nf + g1], r + (int64_t)i * nv + 6 * g1);
+  } else if (threadIdx.x == 128 && (which & 4)) {
+    for (int i = 0; i < cnt; i++) {
+      const double2 *q = r + (int64_t)i * nv + 6 * (g1 + g2);
+      ms_sub(c, ri[(int64_t)i * nf + g1 + g2], q[0], q[1]);
     }
   }
   __threadfence_block();
@@ -642,6 +622,17 @@ __device__ __forceinline__ void subtract(const Ctx &c, const int *keys, const do
 // An estimate's accepted buckets go to ef/ev in ascending bucket order (the
 // order the reference appends them in, hence the map's insertion order),
 // without a staging slot per bucket.
+
+// Entry pos of what an estimate found.
+__device__ __forceinline__ void found_at(const Ctx &c, int pos, int key, double2 val)
+{
+  c.ef[pos] = key;
+  c.ev[pos] = val;
+  if (pos < kFewPairs) {
+    c.lf[pos] = key;
+    c.lv[pos] = val;
+  }
+}
 
 // One step of kV3Block buckets (bucket = step start + threadIdx.x) whose
 // results are in registers: the accepted ones are written at base + their
@@ -665,8 +656,7 @@ __device__ __forceinline__ int emit_step(const Ctx &c, int base, bool ok, int ou
   __syncthreads();
   if (ok) {
     const int pos = off + __popcll(bal & ((1ull << lane) - 1));
-    c.ef[pos] = out;
-    c.ev[pos] = val;
+    found_at(c, pos, out, val);
   }
   return tot;
 }
@@ -837,8 +827,7 @@ __device__ __forceinline__ int est_mansour(const Ctx &c, int *rank, int *sh)
     int o = -1;
     double2 v = make_double2(0, 0);
     (void)mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
-    c.ef[i] = o;
-    c.ev[i] = v;
+    found_at(c, i, o, v);
   }
   __threadfence_block();
   __syncthreads();
@@ -849,10 +838,11 @@ __device__ __forceinline__ int est_mansour(const Ctx &c, int *rank, int *sh)
 // only: a bucket left unwritten holds the values that estimate rejected (an
 // accepted bucket is always written next, by the subtraction of what it
 // found), so it is rejected again and the result is the full sweep's.
-// Thread t takes bit word w = t (+ kV3Block ...): buckets 32 w .. 32 w + 31
-// in ascending order, so a block scan over the threads' accepted counts
-// ranks the accepted buckets in bucket order.  Clears the bits it reads.
-__device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *sh)
+// Thread t takes bit word w = t (+ kV3Block ...), buckets 32 w .. 32 w + 31,
+// and clears it; a block scan over the threads' bit counts lists the set
+// bits in bucket order (list: kV3Block ints of LDS), and one thread tests and
+// estimates each listed bucket, one load latency and one estimate for all.
+__device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *list, int *sh)
 {
   const int n = c.n, W = c.W;
   const double PI2 = 2 * M_PI;
@@ -865,32 +855,27 @@ __device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *sh)
   m.err_max = n * 1e-10;
   const int words = (W + 31) >> 5;
   int found = 0;
-  for (int w0 = 0; w0 < words; w0 += blockDim.x) {
+  for (int w0 = 0; w0 < words; w0 += kV3Block) {
     const int wd = w0 + threadIdx.x;
-    unsigned bits = 0, acc = 0;
+    unsigned bits = 0;
     if (wd < words) {
       bits = c.dirty[wd];
       c.dirty[wd] = 0u;
     }
-    for (unsigned b = bits; b; b &= b - 1) {
-      const int bk = wd * 32 + __ffs(b) - 1;
-      int o;
-      double2 v;
-      if (mansour_bucket<false>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v))
-        acc |= b & (~b + 1u);
-    }
     int total;
-    int pos = found + block_exclusive_scan(__popc(acc), sh, total);
-    for (; acc; acc &= acc - 1) {
-      const int bk = wd * 32 + __ffs(acc) - 1;
+    int pos = block_exclusive_scan(__popc(bits), sh, total);
+    for (int d0 = 0; d0 < total; d0 += kV3Block) {
+      for (; bits && pos < d0 + kV3Block; bits &= bits - 1) list[pos++ - d0] = wd * 32 + __ffs(bits) - 1;
+      __syncthreads();
       int o = -1;
       double2 v = make_double2(0, 0);
-      (void)mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
-      c.ef[pos] = o;
-      c.ev[pos] = v;
-      pos++;
+      bool ok = false;
+      if (d0 + (int)threadIdx.x < total) {
+        const int bk = list[threadIdx.x];
+        ok = mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
+      }
+      found += emit_step(c, found, ok, o, v, sh);  // (its barriers free list)
     }
-    found += total;
   }
   __threadfence_block();
   __syncthreads();
@@ -934,6 +919,56 @@ __device__ __forceinline__ bool map_add_found(const Ctx &c, int F, int *sh, int 
   if (threadIdx.x == 0) *s_size = base + total;
   __syncthreads();
   return true;
+}
+
+// map_add_found by one wave, for F <= kFewPairs pairs in lf, lv; *ok is what
+// map_add_found returns.  No barriers.
+__device__ __forceinline__ void map_add_wave(const Ctx &c, int F, int *s_size, int *ok)
+{
+  const int lane = threadIdx.x & 63;
+  const bool act = lane < F;
+  const int key = act ? c.lf[lane] : 0;
+  int e = act ? map_find(c, key) : 0;
+  const uint64_t fresh = __ballot(act && e < 0);
+  const int base = *s_size, total = __popcll(fresh);
+  const bool fits = base + total <= c.a->map_limit;
+  if (fits && act) {
+    double2 v = make_double2(0.0, 0.0);
+    if (e < 0) {
+      e = base + __popcll(fresh & ((1ull << lane) - 1));
+      c.keys[e] = key;
+      map_insert_slot(c, key, e);
+    } else {
+      v = c.vals[e];
+    }
+    c.vals[e] = cadd(v, c.lv[lane]);
+  }
+  if (lane == 0) {
+    *ok = fits;
+    if (fits) *s_size = base + total;
+  }
+}
+
+// The F found pairs (ef, ev) added to the map and subtracted from the
+// buckets of the filters in which; false when the map would overflow.  Of
+// few pairs, one wave adds to the map while others compute the removals: a
+// pass of the loop that finds a handful took 9.3 us, 6.9 us so.  All threads;
+// contains barriers, the last one at its end.
+__device__ __forceinline__ bool add_subtract(const Ctx &c, int F, int which, int *sh,
+                                             int *s_size, int *s_ok)
+{
+  if (F == 0) return true;
+  if (!few_pairs(c, F)) {
+    const bool ok = map_add_found(c, F, sh, s_size);
+    __syncthreads();
+    subtract(c, c.ef, c.ev, F, which);
+    return ok;
+  }
+  if ((threadIdx.x >> 6) == kV3Block / 64 - 2) map_add_wave(c, F, s_size, s_ok);
+  subtract_few(c, F, which);
+  __threadfence_block();
+  __syncthreads();
+  return *s_ok;
 }
 
 }  // namespace
@@ -1325,7 +1360,9 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   extern __shared__ double2 lds[];
   __shared__ int sh[16];
   __shared__ int s_rank[kV3Block];
-  __shared__ int s_size, s_flag, s_cnt[3], s_cm, s_claim;
+  __shared__ int s_size, s_flag, s_cnt[3], s_cm, s_claim, s_ok;
+  __shared__ int s_lf[kFewPairs];
+  __shared__ double2 s_lv[kFewPairs];
   // the Mansour buckets (pre tasks 0, 1) first: a task run here uses the
   // LDS from its start
   // (and Gauss-1, task 2, which is done by then too: one wait for all three)
@@ -1348,6 +1385,8 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   c.GS1 = lds + a.B1;
   c.GP0 = lds + 2 * a.B1;
   c.GP1 = lds + 2 * a.B1 + a.B2;
+  c.lf = s_lf;
+  c.lv = s_lv;
   c.MS = a.ms + (int64_t)s * 2 * a.W;
   c.keys = a.map_keys + (int64_t)s * a.Mcap;
   c.vals = a.map_vals + (int64_t)s * a.Mcap;
@@ -1365,7 +1404,8 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
     const size_t gauss = (2 * (size_t)a.B1 + 2 * (size_t)a.B2) * sizeof(double2);
     const size_t bits = (((size_t)W + 31) / 32 * sizeof(unsigned) + 15) / 16 * 16;
     const size_t rest = a.lds_bytes > gauss ? a.lds_bytes - gauss : 0;
-    const bool track = rest >= bits + (size_t)kMinStageChunk * 112 + 4 * ((size_t)max(a.B1, a.B2) + 16);
+    const bool track =
+        rest >= bits + kMinStageChunk * staged_pair_bytes(7) + staged_fixed_bytes(a.B1 + a.B2);
     c.dirty = track ? reinterpret_cast<unsigned *>(lds + 2 * a.B1 + 2 * a.B2) : nullptr;
     c.cm = &s_cm;
     c.stage = lds + 2 * a.B1 + 2 * a.B2 + (track ? bits / sizeof(double2) : 0);
@@ -1417,9 +1457,7 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   }
   subtract(c, c.keys, c.vals, s_size, 1);  // the map so far, insertion order
   F = est_gauss(c, c.GS0, c.GS1, a.B1, 1, 0, a.win1, a.win1_half, sh);
-  if (!map_add_found(c, F, sh, &s_size) && threadIdx.x == 0) s_flag |= 2;
-  __syncthreads();
-  subtract(c, c.ef, c.ev, F, 1 | 4);
+  if (!add_subtract(c, F, 1 | 4, sh, &s_size, &s_ok) && threadIdx.x == 0) s_flag |= 2;
 
   // ---- Gauss filter 2 (cf3 215-297): buckets from pre task 3 (run here:
   // in its own bucket arrays' LDS, phases and samples in the staging LDS)
@@ -1435,9 +1473,7 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   }
   subtract(c, c.keys, c.vals, s_size, 2);
   F = est_gauss(c, c.GP0, c.GP1, a.B2, c.aa, c.b, a.win2, a.win2_half, sh);
-  if (!map_add_found(c, F, sh, &s_size) && threadIdx.x == 0) s_flag |= 2;
-  __syncthreads();
-  subtract(c, c.ef, c.ev, F, 7);
+  if (!add_subtract(c, F, 7, sh, &s_size, &s_ok) && threadIdx.x == 0) s_flag |= 2;
 
   // ---- round robin until the three bucket counts repeat (cf3 997-1076)
   int prev[3] = {0, 0, 0};
@@ -1445,15 +1481,15 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   bool cm_valid = false;  // s_cm holds the Mansour count (uniform)
   for (; pass < a.max_passes; pass++) {
     const int sel = pass % 3;
-    if (sel == 0) F = c.dirty ? est_mansour_dirty(c, sh) : est_mansour(c, s_rank, sh);
+    if (sel == 0) F = c.dirty ? est_mansour_dirty(c, s_rank, sh) : est_mansour(c, s_rank, sh);
     else if (sel == 1) F = est_gauss(c, c.GS0, c.GS1, a.B1, 1, 0, a.win1, a.win1_half, sh);
     else F = est_gauss(c, c.GP0, c.GP1, a.B2, c.aa, c.b, a.win2, a.win2_half, sh);
-    if (!map_add_found(c, F, sh, &s_size)) {
+    if (!add_subtract(c, F, 7, sh, &s_size, &s_ok)) {
+      // (what was subtracted all the same is not read again)
       if (threadIdx.x == 0) s_flag |= 2;
       __syncthreads();
       break;
     }
-    subtract(c, c.ef, c.ev, F, 7);
     if (sel == 2) {
       if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
       __syncthreads();
@@ -1461,11 +1497,11 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
       for (int j = threadIdx.x; j < a.B1; j += blockDim.x) {
         // the reference counts elements 0..B1-1 of its interleaved array
         const double2 z = (j & 1) ? c.GS1[j >> 1] : c.GS0[j >> 1];
-        c1 += z.x * z.x + z.y * z.y > 1e-6;
+        c1 += __popcll(__ballot(z.x * z.x + z.y * z.y > 1e-6));  // (lane 0 is active)
       }
       for (int j = threadIdx.x; j < a.B2; j += blockDim.x) {
         const double2 z = (j & 1) ? c.GP1[j >> 1] : c.GP0[j >> 1];
-        c2 += z.x * z.x + z.y * z.y > 1e-6;
+        c2 += __popcll(__ballot(z.x * z.x + z.y * z.y > 1e-6));
       }
       // the Mansour count is kept up to date by every bucket write once it
       // has been counted in full (the first test)
@@ -1479,8 +1515,6 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
           for (int u = 0; u < kSweepAhead; u++) cm += j0 + u * kV3Block < W && ms_counted(z[u], invW);
         }
       }
-      c1 = wave_sum(c1);
-      c2 = wave_sum(c2);
       if (!cm_valid) cm = wave_sum(cm);
       if ((threadIdx.x & 63) == 0) {
         if (!cm_valid) atomicAdd(&s_cnt[0], cm);

@@ -25,9 +25,10 @@ namespace {
 
 constexpr int kV3Block = 512;
 static_assert((kV3Block & (kV3Block - 1)) == 0, "owner tests take residues by masking");
-// Passes that found up to this many pairs keep them and their subtraction
-// values in LDS.
-constexpr int kFewPairs = 16;
+// Passes that found up to this many pairs (a lane each) keep them and their
+// subtraction values in LDS.
+constexpr int kFewPairs = 64;
+static_assert(kV3Block / 64 == 8, "subtract_few gives each of eight waves a part");
 // Steps of a sweep over the Mansour buckets whose loads are issued together.
 constexpr int kSweepAhead = 4;
 // Loads the pre-kernel's gathers and folds issue together per thread.
@@ -188,9 +189,9 @@ __device__ void fft_pair(double2 *x0, double2 *x1, int B, const V3Launch &a)
 // update_gaussian_loops2 (cf3 354-463): what to subtract from buckets
 // h, h+1, h-1 of both loops for (key, value); r[0..5] = loop0 x3, loop1 x3.
 // update_gauss_loops2 (cf3 353-463) for one located (key, value) in a
-// Gauss filter of B buckets at offsets g, g + step: the centre bucket h, the
-// three window distances, then (gauss_values) the removal values r[0..2]
-// (offset g) and r[3..5] (g + step) for buckets h, h+1, h-1.  Split so the
+// Gauss filter of B buckets at offsets g, g + 1: the centre bucket h, the
+// three window distances, then (gauss_values) an offset's three removal
+// values, for buckets h, h+1, h-1.  Split so the
 // window loads of several removals can be issued together.
 struct GaussIdx {
   int h;
@@ -212,35 +213,30 @@ __device__ __forceinline__ GaussIdx gauss_index(const Ctx &c, int key, int B)
 }
 
 __device__ __forceinline__ void gauss_values(const Ctx &c, int key, double2 value, int g,
-                                             int step, const double2 F[3], double2 *r)
+                                             const double2 F[3], double2 *r)
 {
   const int n = c.n;
   const double PI2_DIV_N = 2 * M_PI / n;
   const double a1 = value.x, b1 = value.y;
   const int ko = smod(wmul(key, g), n);
-  const int ko2 = smod(wmul(key, (int)((unsigned)g + (unsigned)step)), n);
-  double b2, a2, b22, a22;
+  double b2, a2;
   sincos(PI2_DIV_N * ko, &b2, &a2);
-  sincos(PI2_DIV_N * ko2, &b22, &a22);
-  const double v1r = a1 * a2 - b1 * b2, v1i = a1 * b2 + b1 * a2;
-  const double v2r = a1 * a22 - b1 * b22, v2i = a1 * b22 + b1 * a22;
+  const double vr = a1 * a2 - b1 * b2, vi = a1 * b2 + b1 * a2;
 #pragma unroll
-  for (int q = 0; q < 3; q++) {
-    r[q] = make_double2(v1r * F[q].x - v1i * F[q].y, v1r * F[q].y + v1i * F[q].x);
-    r[3 + q] = make_double2(v2r * F[q].x - v2i * F[q].y, v2r * F[q].y + v2i * F[q].x);
-  }
+  for (int q = 0; q < 3; q++)
+    r[q] = make_double2(vr * F[q].x - vi * F[q].y, vr * F[q].y + vi * F[q].x);
 }
 
 __device__ void gauss_removal(const Ctx &c, int key, double2 value, int B,
-                              const double2 *win, int half, int g, int step,
-                              int &h, double2 *r)
+                              const double2 *win, int half, int g, int &h, double2 *r)
 {
   const GaussIdx x = gauss_index(c, key, B);
   h = x.h;
   double2 F[3];
 #pragma unroll
   for (int q = 0; q < 3; q++) F[q] = win_at(win, half, x.dd[q], c.n);
-  gauss_values(c, key, value, g, step, F, r);
+  gauss_values(c, key, value, g, F, r);
+  gauss_values(c, key, value, (int)((unsigned)g + 1u), F, r + 3);
 }
 
 __device__ void gauss_apply_pair(double2 *S0, double2 *S1, int B, int h, const double2 *r)
@@ -251,37 +247,65 @@ __device__ void gauss_apply_pair(double2 *S0, double2 *S1, int B, int h, const d
 }
 
 // A few pairs (removal values in LDS, nv per pair, bucket indices nf per
-// pair, both from this filter's first on) applied by bucket owners: thread t takes its
-// buckets t, t + blockDim, ... and walks the pairs in order, applying the
-// parts that land on the bucket (h, h+1, h-1 within a pair) -- the order
-// in which gauss_apply_pair applies them pair after pair.
+// pair, both from this filter's first on; cnt <= 64) applied by bucket
+// owners: thread t takes its buckets t, t + blockDim, ... and walks the
+// pairs in order, applying the parts that land on the bucket (h, h+1, h-1
+// within a pair) -- the order in which gauss_apply_pair applies them pair
+// after pair.  The bucket indices come from lanes (no LDS latency a pair),
+// kStageAhead pairs' values are read together, and a wave skips those of
+// which none lands on its buckets.
 __device__ __forceinline__ void gauss_apply_few(double2 *S0, double2 *S1, int B, const int *si,
                                                 int nf, const double2 *sv, int nv, int cnt)
 {
   const int bm = B - 1;  // B a power of two
-  for (int tb = threadIdx.x; tb < B; tb += blockDim.x) {
-    double2 a0 = make_double2(0, 0), a1 = make_double2(0, 0);
+  const int lane = threadIdx.x & 63;
+  const int hl = si[(lane < cnt ? lane : 0) * nf];
+  // whole waves throughout (lanes past the last bucket idle, not inactive):
+  // a lane holds a pair's index whether or not it has a bucket
+  const int w0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);
+  for (int t0 = w0; t0 < B; t0 += kV3Block) {
+    const int tb = t0 + lane;
+    const bool own = tb < B;
+    double2 a0 = S0[own ? tb : 0], a1 = S1[own ? tb : 0];
     bool any = false;
-    for (int i = 0; i < cnt; i++) {
-      const int h = si[i * nf];
-      if ((unsigned)((tb - h + 1) & bm) > 2u) continue;
-      if (!any) {
-        a0 = S0[tb];
-        a1 = S1[tb];
+    if (B < 4) {  // a bucket can be several of a pair's three
+      for (int i = 0; i < cnt; i++) {
+        const int h = __builtin_amdgcn_readlane(hl, i);
+        const double2 *r = sv + i * nv;
+        const int bk[3] = {h, (h + 1) & bm, (h + bm) & bm};
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+          if (own && bk[q] == tb) {
+            a0 = csub(a0, r[q]);
+            a1 = csub(a1, r[3 + q]);
+            any = true;
+          }
+      }
+    } else {
+      for (int i0 = 0; i0 < cnt; i0 += kStageAhead) {
+        int d[kStageAhead];  // 0, 1, 2: this bucket is h - 1, h, h + 1
+        bool hit = false;
+#pragma unroll
+        for (int u = 0; u < kStageAhead; u++) {
+          const int h = __builtin_amdgcn_readlane(hl, min(i0 + u, cnt - 1));
+          d[u] = own && i0 + u < cnt ? (tb - h + 1) & bm : 3;
+          hit |= d[u] < 3;
+        }
+        if (!hit) continue;
         any = true;
-      }
-      const double2 *r = sv + i * nv;
-      if (h == tb) {
-        a0 = csub(a0, r[0]);
-        a1 = csub(a1, r[3]);
-      }
-      if (((h + 1) & bm) == tb) {
-        a0 = csub(a0, r[1]);
-        a1 = csub(a1, r[4]);
-      }
-      if (((h + bm) & bm) == tb) {
-        a0 = csub(a0, r[2]);
-        a1 = csub(a1, r[5]);
+        double2 v0[kStageAhead], v1[kStageAhead];
+#pragma unroll
+        for (int u = 0; u < kStageAhead; u++) {  // (of no pair: pair cnt - 1, unused)
+          const double2 *r = sv + min(i0 + u, cnt - 1) * nv + (d[u] == 1 ? 0 : (d[u] == 2 ? 1 : 2));
+          v0[u] = r[0];
+          v1[u] = r[3];
+        }
+#pragma unroll
+        for (int u = 0; u < kStageAhead; u++)
+          if (d[u] < 3) {
+            a0 = csub(a0, v0[u]);
+            a1 = csub(a1, v1[u]);
+          }
       }
     }
     if (any) {
@@ -291,18 +315,15 @@ __device__ __forceinline__ void gauss_apply_few(double2 *S0, double2 *S1, int B,
   }
 }
 
-// update_mansour_loops2 (cf3 300-351)
-__device__ void mansour_removal(const Ctx &c, int key, double2 value, int &h, double2 *r)
+// update_mansour_loops2 (cf3 300-351), the removal at offset g
+__device__ __forceinline__ double2 mansour_value(const Ctx &c, int key, double2 value, int g)
 {
   const double PI2_OVER_N = 2 * M_PI / c.n;
   const int W = c.W;
-  h = key & (W - 1);
   const double vr = value.x, vi = value.y;
-  double s0, c0, s1, c1;
-  sincos(PI2_OVER_N * key * c.g0, &s0, &c0);
-  sincos(PI2_OVER_N * key * (c.g0 + 1), &s1, &c1);
-  r[0] = make_double2(W * (vr * c0 - vi * s0), W * (vr * s0 + vi * c0));
-  r[1] = make_double2(W * (vr * c1 - vi * s1), W * (vr * s1 + vi * c1));
+  double s0, c0;
+  sincos(PI2_OVER_N * key * g, &s0, &c0);
+  return make_double2(W * (vr * c0 - vi * s0), W * (vr * s0 + vi * c0));
 }
 
 // The removal values of cnt (key, value) pairs for the filters in which
@@ -338,11 +359,16 @@ __device__ __forceinline__ void removals(const Ctx &c, const int *keys, const do
     const double2 v = vals[i];
     double2 *r = r0 + i * nv;
     int *ri = ri0 + i * nf;
-    if (f == 0) gauss_removal(c, key, v, c.B1, a.win1, a.win1_half, c.gG, 1, ri[0], r);
+    if (f == 0) gauss_removal(c, key, v, c.B1, a.win1, a.win1_half, c.gG, ri[0], r);
     else if (f == 1)
       gauss_removal(c, smod(timesmod(key, c.ai, c.n) + c.shift, c.n), v, c.B2, a.win2,
-                    a.win2_half, wmul(c.aa, c.gG), 1, ri[g1], r + 6 * g1);
-    else mansour_removal(c, key, v, ri[g1 + g2], r + 6 * (g1 + g2));
+                    a.win2_half, wmul(c.aa, c.gG), ri[g1], r + 6 * g1);
+    else {
+      double2 *rm = r + 6 * (g1 + g2);
+      ri[g1 + g2] = key & (c.W - 1);
+      rm[0] = mansour_value(c, key, v, c.g0);
+      rm[1] = mansour_value(c, key, v, c.g0 + 1);
+    }
   }
 }
 
@@ -508,47 +534,71 @@ __device__ __forceinline__ void apply_staged(const Ctx &c, int which, const doub
 __device__ __forceinline__ bool few_pairs(const Ctx &c, int cnt)
 {
   return cnt <= kFewPairs && !c.a->serial_all &&
-         c.room >= (size_t)kFewPairs * (14 * sizeof(double2) + 3 * sizeof(int));
+         c.room >= (size_t)cnt * (14 * sizeof(double2) + 3 * sizeof(int));
 }
 
-// The subtraction of the cnt <= kFewPairs pairs in lf, lv: the owner of a
-// Gauss bucket applies them in pair order, and each Mansour bucket (in HBM)
-// is updated by the lane of its first pair, in pair order -- every bucket
-// sees the same subtractions in the same order.  The last wave (no removal
-// is computed there) loads the Mansour buckets meanwhile.  Contains
-// barriers, none after the last update.
+// The subtraction of the 0 < cnt <= kFewPairs pairs in lf, lv: a wave for
+// each filter and offset computes its removals, a lane a pair (both offsets
+// on one lane took their sines in turn); the owner of a Gauss bucket applies
+// them in pair order, and each Mansour bucket (in HBM) is updated by the
+// lane of its first pair, in pair order -- every bucket sees the same
+// subtractions in the same order.  The last wave (no removal is computed
+// there) loads the Mansour buckets meanwhile.  Contains barriers, none after
+// the last update.
 __device__ __forceinline__ void subtract_few(const Ctx &c, int cnt, int which)
 {
+  const V3Launch &a = *c.a;
   double2 *const sv = c.stage;
-  int *const si = reinterpret_cast<int *>(sv + 14 * kFewPairs);
-  const int mj = (int)threadIdx.x - (kV3Block - 64);
-  const bool mansour = (which & 4) && mj >= 0;
+  const int nv = removal_values(which), nf = removal_indices(which);
+  int *const si = reinterpret_cast<int *>(sv + cnt * nv);
+  const int g1 = which & 1, g2 = (which >> 1) & 1;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const bool mansour = (which & 4) && wave == kV3Block / 64 - 1;
   int mh = -1;
   bool first = false, more = false;
   double2 z0 = make_double2(0, 0), z1 = make_double2(0, 0);
   if (mansour) {
-    if (mj < cnt) {
-      mh = c.lf[mj] & (c.W - 1);
+    if (lane < cnt) {
+      mh = c.lf[lane] & (c.W - 1);
       z0 = c.MS[2 * mh];
       z1 = c.MS[2 * mh + 1];
     }
-    first = mj < cnt;
-#pragma unroll
-    for (int q = 0; q < kFewPairs; q++) {
-      const int hq = __shfl(mh, q, 64);
-      first &= !(q < mj && hq == mh);
-      more |= q > mj && hq == mh;
+    first = lane < cnt;
+    for (int q = 0; q < cnt; q++) {
+      const int hq = __builtin_amdgcn_readlane(mh, q);
+      first &= !(q < lane && hq == mh);
+      more |= q > lane && hq == mh;
     }
   }
-  removals(c, c.lf, c.lv, cnt, which, sv, si);
+  if (wave < 2 * nf && lane < cnt) {
+    const int f = wave >> 1, off = wave & 1;  // f-th filter here
+    const int key = c.lf[lane];
+    const double2 v = c.lv[lane];
+    double2 *r = sv + lane * nv;
+    if ((which & 4) && f == nf - 1) {
+      if (off == 0) si[lane * nf + f] = key & (c.W - 1);
+      r[6 * f + off] = mansour_value(c, key, v, c.g0 + off);
+    } else {
+      const bool second = f == 1 || !g1;  // Gauss-2
+      const int kf = second ? smod(timesmod(key, c.ai, c.n) + c.shift, c.n) : key;
+      const int g = second ? wmul(c.aa, c.gG) : c.gG;
+      const double2 *win = second ? a.win2 : a.win1;
+      const int half = second ? a.win2_half : a.win1_half;
+      const GaussIdx x = gauss_index(c, kf, second ? c.B2 : c.B1);
+      double2 F[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++) F[q] = win_at(win, half, x.dd[q], c.n);
+      if (off == 0) si[lane * nf + f] = x.h;
+      gauss_values(c, kf, v, (int)((unsigned)g + (unsigned)off), F, r + 6 * f + 3 * off);
+    }
+  }
   __syncthreads();
-  const int nv = removal_values(which), nf = removal_indices(which);
-  const int g1 = which & 1, g2 = (which >> 1) & 1;
   if (mansour && first) {
     const double2 *r = sv + 6 * (g1 + g2);
-    ms_put(c, mh, z0, csub(z0, r[mj * nv]), csub(z1, r[mj * nv + 1]));
+    ms_put(c, mh, z0, csub(z0, r[lane * nv]), csub(z1, r[lane * nv + 1]));
     if (more)
-      for (int i = mj + 1; i < cnt; i++)
+      for (int i = lane + 1; i < cnt; i++)
         if (si[i * nf + g1 + g2] == mh) ms_sub(c, mh, r[i * nv], r[i * nv + 1]);
   }
   if (g1) gauss_apply_few(c.GS0, c.GS1, c.B1, si, nf, sv, nv, cnt);
@@ -891,8 +941,9 @@ __device__ __forceinline__ bool map_add_found(const Ctx &c, int F, int *sh, int 
   const int C = (F + T - 1) / T;
   const int lo = threadIdx.x * C, hi = min(F, lo + C);
   int nnew = 0;
+  const bool empty = *s_size == 0;  // the keys of one pass are distinct
   for (int i = lo; i < hi; i++) {
-    const int e = map_find(c, c.ef[i]);
+    const int e = empty ? -1 : map_find(c, c.ef[i]);
     c.remi[i * 3] = e;  // remember (reused as scratch before removals)
     nnew += e < 0;
   }
@@ -952,7 +1003,7 @@ __device__ __forceinline__ void map_add_wave(const Ctx &c, int F, int *s_size, i
 // The F found pairs (ef, ev) added to the map and subtracted from the
 // buckets of the filters in which; false when the map would overflow.  Of
 // few pairs, one wave adds to the map while others compute the removals: a
-// pass of the loop that finds a handful took 9.3 us, 6.9 us so.  All threads;
+// pass of the loop that finds a handful took 9.3 us, 5.9 us so.  All threads;
 // contains barriers, the last one at its end.
 __device__ __forceinline__ bool add_subtract(const Ctx &c, int F, int which, int *sh,
                                              int *s_size, int *s_ok)
@@ -1363,6 +1414,18 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   __shared__ int s_size, s_flag, s_cnt[3], s_cm, s_claim, s_ok;
   __shared__ int s_lf[kFewPairs];
   __shared__ double2 s_lv[kFewPairs];
+  // the empty map, written while the pre tasks run (Hcap: a power of two,
+  // 128 or more)
+  {
+    int *const hidx = a.map_hidx + (int64_t)s * a.Hcap;
+    for (int i = threadIdx.x; i < a.Hcap / 4; i += blockDim.x)
+      reinterpret_cast<int4 *>(hidx)[i] = make_int4(-1, -1, -1, -1);
+    if (threadIdx.x == 0) {
+      s_size = 0;
+      s_flag = 0;
+    }
+    __threadfence_block();  // (need_tasks has barriers)
+  }
   // the Mansour buckets (pre tasks 0, 1) first: a task run here uses the
   // LDS from its start
   // (and Gauss-1, task 2, which is done by then too: one wait for all three)
@@ -1413,12 +1476,6 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
     if (track)
       for (int i = threadIdx.x; i < (W + 31) / 32; i += blockDim.x) c.dirty[i] = 0u;
   }
-  for (int i = threadIdx.x; i < a.Hcap; i += blockDim.x) c.hidx[i] = -1;
-  if (threadIdx.x == 0) {
-    s_size = 0;
-    s_flag = 0;
-  }
-  __threadfence_block();
   __syncthreads();
 
   // ---- Mansour filter (cf3 96-127): buckets from pre tasks 0, 1

@@ -375,3 +375,29 @@ def test_v3_result_order(torch_cuda, k, width):
     fr, va = plan.execute_sparse_host(x)
     assert not ref["early"] and np.array_equal(fr, ref["freqs"])
     assert np.abs(va - ref["vals"]).max() <= 1e-9 * np.abs(ref["vals"]).max()
+
+
+@pytest.mark.parametrize("n,k", [(1 << 14, 16), (1 << 16, 12), (1 << 18, 24), (1 << 20, 60),
+                                 (1 << 20, 110)])
+def test_v3_few_pairs_equal_serial(torch_cuda, n, k):
+    """A pass of up to 64 pairs keeps a pair on a lane and hands the bucket
+    indices to the owners of the buckets, which may be fewer than the pairs
+    (8 to 128 Gauss buckets here): the same bits as one thread applying every
+    pair in turn."""
+    torch = torch_cuda
+    print(f"case v3 few pairs n={n} k={k}", flush=True)
+    S = 6
+    xd = [torch.from_numpy(signal_np(n, k, seed=9500 + 3 * i + k)[0]).cuda() for i in range(S)]
+    a = sfft_amd.sfft(n, k, 3, seed=(41, 43))
+    b = sfft_amd.sfft(n, k, 3, seed=(41, 43))
+    b.debug_v3(serial_subtractions=True)
+    fa, va = a.make_sparse_outputs(S)
+    fb, vb = b.make_sparse_outputs(S)
+    ca = a.execute_many_sparse(xd, fa, va)
+    cb = b.execute_many_sparse(xd, fb, vb)
+    torch.cuda.synchronize()
+    assert np.array_equal(ca, cb) and int(ca.max()) > 0
+    for i in range(S):
+        c = int(ca[i])
+        assert torch.equal(fa[i, :c], fb[i, :c])
+        assert torch.equal(va[i, :c], vb[i, :c])

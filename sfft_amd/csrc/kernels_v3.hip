@@ -1049,6 +1049,9 @@ __device__ __forceinline__ bool add_subtract(const Ctx &c, int F, int which, int
 // the bucket keeps the reference's values (status bit 8).
 constexpr int kRefOff = kV3RefineOffsets;  // Mansour offsets: equations per bucket
 constexpr int kRefMax = 7;  // unknowns per bucket (located + unlocated)
+// Threads of a solve workgroup, and workgroups a launch aims at (a few per
+// CU; the classes are taken in turn).
+constexpr int kRefBlock = 128, kRefGrid = 2048;
 
 __device__ __forceinline__ double2 cis_mod(long long r, int n)
 {
@@ -1138,23 +1141,24 @@ __device__ __forceinline__ double2 gshfl2(double2 v, int src)
   return make_double2(__shfl(v.x, src, kRefOff), __shfl(v.y, src, kRefOff));
 }
 
-// Least squares over the kRefOff equations: y_l ~ sum_m X[m] e[m]_l, pc <=
-// kRefMax unknowns, by modified Gram-Schmidt QR of the columns (samples of
+// Least squares over the kRefOff equations: y_l ~ sum_m X[m] e[m]_l, pc <= P
+// unknowns, by modified Gram-Schmidt QR of the columns (samples of
 // unit exponentials: QR keeps their conditioning instead of squaring it).
 // e[m] is this lane's entry of column m, y its bucket value.  Returns the
 // squared residual (1e300 when the columns are dependent); X on every lane.
-__device__ __forceinline__ double ref_solve_lanes(const double2 (&e)[kRefMax], double2 y,
-                                                  int pc, double2 (&X)[kRefMax], int lane)
+template <int P>
+__device__ __forceinline__ double ref_solve_lanes(const double2 (&e)[P], double2 y,
+                                                  int pc, double2 (&X)[P], int lane)
 {
-  double2 Q[kRefMax], Rrow[kRefMax], z[kRefMax];  // Rrow: row `lane` of R
+  double2 Q[P], Rrow[P], z[P];  // Rrow: row `lane` of R
 #pragma unroll
-  for (int m = 0; m < kRefMax; m++) {
+  for (int m = 0; m < P; m++) {
     Rrow[m] = make_double2(0, 0);
     Q[m] = make_double2(0, 0);
     z[m] = make_double2(0, 0);
   }
 #pragma unroll
-  for (int m = 0; m < kRefMax; m++) {
+  for (int m = 0; m < P; m++) {
     if (m >= pc) break;
     Q[m] = e[m];
 #pragma unroll
@@ -1170,24 +1174,45 @@ __device__ __forceinline__ double ref_solve_lanes(const double2 (&e)[kRefMax], d
     Q[m] = make_double2(Q[m].x * inv, Q[m].y * inv);
   }
 #pragma unroll
-  for (int m = 0; m < kRefMax; m++)
+  for (int m = 0; m < P; m++)
     if (m < pc) z[m] = gsum2(cconjmul(Q[m], y));
   // back substitution: row m lives on lane m, X[m] is then broadcast
 #pragma unroll
-  for (int m = kRefMax - 1; m >= 0; m--) {
+  for (int m = P - 1; m >= 0; m--) {
     if (m >= pc) continue;
     double2 acc = z[m];
 #pragma unroll
-    for (int q = m + 1; q < kRefMax; q++)
+    for (int q = m + 1; q < P; q++)
       if (q < pc) acc = csub(acc, cmul(Rrow[q], X[q]));
     const double2 xm = make_double2(acc.x / Rrow[m].x, acc.y / Rrow[m].x);
     X[m] = gshfl2(xm, m);
   }
   double2 r = y;
 #pragma unroll
-  for (int m = 0; m < kRefMax; m++)
+  for (int m = 0; m < P; m++)
     if (m < pc) r = csub(r, cmul(X[m], e[m]));
   return gsum(r.x * r.x + r.y * r.y);
+}
+
+// refine_class for a class whose one located member is entry e0 of the map
+// and which holds no unlocated tone: the same operations with one column in
+// registers instead of kRefMax.  False (nothing written) when the residual
+// stays large.
+__device__ __forceinline__ bool refine_single(const V3Launch &a, int s, int g0, int j, int e0,
+                                              const int *keys, double2 *vals, int lane)
+{
+  const int n = a.n, W = a.W;
+  const unsigned mask = (unsigned)n - 1;
+  const long long fk = keys[e0];
+  const double2 mv = ref_row(a, s, lane)[j];
+  const double2 y = make_double2(mv.x / W, mv.y / W);
+  const double scale = gsum(y.x * y.x + y.y * y.y);
+  double2 X[1];
+  const double2 e[1] = {cis_mod((fk * ((long long)g0 + (long long)lane * a.ref_t)) & mask, n)};
+  const double tol = 1e-20 * (scale > 1e-8 ? scale : 1e-8);
+  if (ref_solve_lanes(e, y, 1, X, lane) > tol) return false;
+  if (lane == 0) vals[e0] = X[0];
+  return true;
 }
 
 // The refine solve of class j of signal s by a lane group (lane = this
@@ -1236,15 +1261,13 @@ __device__ __forceinline__ int refine_class(const V3Launch &a, int s, int g0, in
   const double2 mv = ref_row(a, s, lane)[j];
   const double2 y = make_double2(mv.x / W, mv.y / W);
   const double scale = gsum(y.x * y.x + y.y * y.y);
-  double2 e[kRefMax], w[kRefMax], X[kRefMax];
+  double2 e[kRefMax], X[kRefMax];
 #pragma unroll
   for (int m = 0; m < kRefMax; m++) {
     e[m] = make_double2(0, 0);
-    w[m] = make_double2(0, 0);
     X[m] = make_double2(0, 0);
     if (m < p) {
       e[m] = cis_mod((fk[m] * ((long long)g0 + (long long)lane * t)) & mask, n);
-      w[m] = cis_mod((fk[m] * t) & mask, n);
     }
   }
   const double tol = 1e-20 * (scale > 1e-8 ? scale : 1e-8);
@@ -1257,7 +1280,8 @@ __device__ __forceinline__ int refine_class(const V3Launch &a, int s, int g0, in
     for (int m = 0; m < kRefMax; m++) {
       if (m >= p) break;
       const double2 dn = gshfl2(d, lane + 1 < kRefOff ? lane + 1 : lane);
-      if (lane + 1 < len) d = csub(dn, cmul(w[m], d));
+      const double2 w = cis_mod((fk[m] * t) & mask, n);
+      if (lane + 1 < len) d = csub(dn, cmul(w, d));
       len--;
     }
     double2 X2[kRefMax];
@@ -1983,14 +2007,28 @@ __global__ void __launch_bounds__(kV3Block) k_v3_run(const V3Launch *__restrict_
   pre_task(groups[bb.x], bb.y, 4 + w % nref, lds, groups[bb.x].lds_bytes, nullptr, 0);
 }
 
-// The refine form after k_v3_run, in three kernels over the same
+// The refine form after k_v3_run, in four kernels over the same
 // (group, signal) blocks: k_v3_refine lists the located entries of every
 // residue class (linked lists through head, W entries in cf, and next, M
-// entries in remi) and the non-empty classes; k_v3_refine_solve solves
-// those, kRefOff lanes each (nsub workgroups per signal, the later ones
-// mostly idle); k_v3_refine_write sorts and writes the
-// result.  Groups without refine, and signals with the reference's early
-// return, wrote their result in k_v3_run and are skipped.
+// entries in remi) and the non-empty classes, those of one entry apart;
+// k_v3_refine_single solves the classes of one entry, kRefOff lanes each,
+// and hands on those with an unlocated tone; k_v3_refine_solve solves the
+// rest; k_v3_refine_write sorts and writes the result.  Nearly all classes
+// (94 of 100 with 1000 tones in 8192 classes) hold one entry.  With all of
+// them in the general solve (256 VGPRs, two waves a SIMD) two waves in five
+// ran the longer solve for one of their eight classes: 79 us for
+// 64 signals of up to 1000 tones; now 12 + 47.  Groups without refine,
+// and signals with the reference's early return, wrote their result in
+// k_v3_run and are skipped.
+//
+// The class lists (in cv, free after the loop): nz[0] and nz[1] the counts
+// of the classes of one entry and of the rest, the classes from nz[2] and
+// nz[2 + W] on, in no particular order.
+__device__ __forceinline__ int *refine_lists(const V3Launch &a, int s)
+{
+  return reinterpret_cast<int *>(a.cv + (int64_t)s * a.Fcap);
+}
+
 __global__ void __launch_bounds__(kV3Block) k_v3_refine(const V3Launch *__restrict__ groups,
                                                         const int2 *__restrict__ blocks)
 {
@@ -2001,44 +2039,65 @@ __global__ void __launch_bounds__(kV3Block) k_v3_refine(const V3Launch *__restri
   const int M = (int)a.count[s], W = a.W;
   const int *keys = a.map_keys + (int64_t)s * a.Mcap;
   int *head = a.cf + (int64_t)s * a.Fcap, *next = a.remi + (int64_t)s * a.Rcap * 3;
-  // the non-empty classes, for the solve (in cv, free after the loop):
-  // nz[0] their count, nz[1..] the classes in no particular order
-  int *nz = reinterpret_cast<int *>(a.cv + (int64_t)s * a.Fcap);
-  __shared__ int s_nz;
+  int *nz = refine_lists(a, s);
+  __shared__ int s_nz[2];
   for (int j = threadIdx.x; j < W; j += blockDim.x) head[j] = -1;
-  if (threadIdx.x == 0) s_nz = 0;
+  if (threadIdx.x < 2) s_nz[threadIdx.x] = 0;
+  __threadfence_block();
+  __syncthreads();
+  for (int e = threadIdx.x; e < M; e += blockDim.x)
+    next[e] = atomicExch(&head[keys[e] & (W - 1)], e);
   __threadfence_block();
   __syncthreads();
   for (int e = threadIdx.x; e < M; e += blockDim.x) {
     const int j = keys[e] & (W - 1);
-    const int old = atomicExch(&head[j], e);
-    next[e] = old;
-    if (old < 0) nz[1 + atomicAdd(&s_nz, 1)] = j;  // first entry of class j
+    // (the exchanges were made in the L2; read there)
+    if (__hip_atomic_load(&head[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != e) continue;
+    const int rest = next[e] >= 0;  // the first of class j
+    nz[2 + rest * W + atomicAdd(&s_nz[rest], 1)] = j;
   }
   __syncthreads();
-  if (threadIdx.x == 0) nz[0] = s_nz;
+  if (threadIdx.x < 2) nz[threadIdx.x] = s_nz[threadIdx.x];
 }
 
-__global__ void __launch_bounds__(kV3Block) k_v3_refine_solve(const V3Launch *__restrict__ groups,
-                                                              const int2 *__restrict__ blocks,
-                                                              int nsub)
+__global__ void __launch_bounds__(kRefBlock) k_v3_refine_single(
+    const V3Launch *__restrict__ groups, const int2 *__restrict__ blocks, int nsub)
 {
   const int2 bb = blocks[blockIdx.x / (unsigned)nsub];
-  const int gid = (int)(blockIdx.x % (unsigned)nsub) * blockDim.x + threadIdx.x;
-  const int jj = gid / kRefOff, lane = gid % kRefOff;  // a group of kRefOff lanes a class
+  const int lane = threadIdx.x % kRefOff;  // a group of kRefOff lanes a class
   const V3Launch &a = groups[bb.x];
   const int s = bb.y;
   if (!a.refine || (a.status[s] & 1)) return;  // no barriers here
-  // one group per non-empty class (listed by k_v3_refine); a group returns
-  // or continues as a whole, so its shuffles see all its lanes
-  const int *nz = reinterpret_cast<const int *>(a.cv + (int64_t)s * a.Fcap);
-  if (jj >= nz[0]) return;
-  const int j = nz[1 + jj];
-  const int g0 = a.params[(int64_t)s * 6 + 4];
-  if (refine_class(a, s, g0, j, a.cf + (int64_t)s * a.Fcap, a.remi + (int64_t)s * a.Rcap * 3,
-                   a.map_keys + (int64_t)s * a.Mcap, a.map_vals + (int64_t)s * a.Mcap, lane) &&
-      lane == 0)
-    atomicOr(&a.status[s], 8);
+  int *nz = refine_lists(a, s);
+  const int cnt = nz[0], g0 = a.params[(int64_t)s * 6 + 4];
+  // a group's lanes take every branch together, so its shuffles see them all
+  for (int jj = (int)(blockIdx.x % (unsigned)nsub * blockDim.x + threadIdx.x) / kRefOff; jj < cnt;
+       jj += nsub * (kRefBlock / kRefOff)) {
+    const int j = nz[2 + jj];
+    if (!refine_single(a, s, g0, j, a.cf[(int64_t)s * a.Fcap + j],
+                       a.map_keys + (int64_t)s * a.Mcap, a.map_vals + (int64_t)s * a.Mcap, lane) &&
+        lane == 0)
+      nz[2 + a.W + atomicAdd(&nz[1], 1)] = j;
+  }
+}
+
+__global__ void __launch_bounds__(kRefBlock) k_v3_refine_solve(
+    const V3Launch *__restrict__ groups, const int2 *__restrict__ blocks, int nsub)
+{
+  const int2 bb = blocks[blockIdx.x / (unsigned)nsub];
+  const int lane = threadIdx.x % kRefOff;
+  const V3Launch &a = groups[bb.x];
+  const int s = bb.y;
+  if (!a.refine || (a.status[s] & 1)) return;
+  const int *nz = refine_lists(a, s);
+  const int cnt = nz[1], g0 = a.params[(int64_t)s * 6 + 4];
+  for (int jj = (int)(blockIdx.x % (unsigned)nsub * blockDim.x + threadIdx.x) / kRefOff; jj < cnt;
+       jj += nsub * (kRefBlock / kRefOff))
+    if (refine_class(a, s, g0, nz[2 + a.W + jj], a.cf + (int64_t)s * a.Fcap,
+                     a.remi + (int64_t)s * a.Rcap * 3, a.map_keys + (int64_t)s * a.Mcap,
+                     a.map_vals + (int64_t)s * a.Mcap, lane) &&
+        lane == 0)
+      atomicOr(&a.status[s], 8);
 }
 
 __global__ void __launch_bounds__(kV3Block) k_v3_refine_write(const V3Launch *__restrict__ groups,
@@ -2103,12 +2162,13 @@ int v3_multi(const V3Launch *h_groups, int G, const V3Launch *d_groups, const in
     lds = std::max(lds, h_groups[g].lds_bytes);
   }
   bool refine = false;
-  int nsub = 1;
+  int nsub = 1;  // solve workgroups per signal
   for (int g = 0; g < G; g++)
     if (h_groups[g].refine) {
       refine = true;
-      nsub = std::max(nsub, (h_groups[g].W * kRefOff + kV3Block - 1) / kV3Block);
+      nsub = std::max(nsub, (h_groups[g].W * kRefOff + kRefBlock - 1) / kRefBlock);
     }
+  nsub = std::min(nsub, std::max(1, kRefGrid / nblocks));
   const int nref = refine ? kRefOff : 0;
   allow_v3_lds(reinterpret_cast<const void *>(k_v3_run), lds);
   hipLaunchKernelGGL(k_v3_run, dim3((5 + nref) * nblocks), dim3(kV3Block), lds, st, d_groups,
@@ -2122,7 +2182,9 @@ int v3_multi(const V3Launch *h_groups, int G, const V3Launch *d_groups, const in
     // groups without refine write their result in k_v3_run; their blocks
     // return at once here
     hipLaunchKernelGGL(k_v3_refine, dim3(nblocks), dim3(kV3Block), 0, st, d_groups, d_blocks);
-    hipLaunchKernelGGL(k_v3_refine_solve, dim3(nblocks * nsub), dim3(kV3Block), 0, st, d_groups,
+    hipLaunchKernelGGL(k_v3_refine_single, dim3(nblocks * nsub), dim3(kRefBlock), 0, st,
+                       d_groups, d_blocks, nsub);
+    hipLaunchKernelGGL(k_v3_refine_solve, dim3(nblocks * nsub), dim3(kRefBlock), 0, st, d_groups,
                        d_blocks, nsub);
     allow_v3_lds(reinterpret_cast<const void *>(k_v3_refine_write), lds);
     hipLaunchKernelGGL(k_v3_refine_write, dim3(nblocks), dim3(kV3Block), lds, st, d_groups,

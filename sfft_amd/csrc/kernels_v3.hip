@@ -44,6 +44,9 @@ static_assert(6 * kStageChunk <= 65536, "list entries are 16 bits");
 
 __device__ __forceinline__ int ilog2v(int v) { return 31 - __clz(v); }
 
+// v / p for a power of two p (exact, like the division, but one instruction)
+__device__ __forceinline__ double div2(double v, int p) { return ldexp(v, -ilog2v(p)); }
+
 // Sum over the 64 lanes of a wave (every lane gets it).
 __device__ __forceinline__ int wave_sum(int v)
 {
@@ -120,7 +123,7 @@ __device__ __forceinline__ void ms_put(const Ctx &c, int h, double2 old, double2
   c.MS[2 * h] = now;
   c.MS[2 * h + 1] = now1;
   if (c.dirty) {
-    const double invW = 1.0 / c.W;
+    const double invW = div2(1.0, c.W);
     atomicOr(&c.dirty[h >> 5], 1u << (h & 31));
     const int d = ms_counted(now, invW) - ms_counted(old, invW);
     if (d) atomicAdd(c.cm, d);
@@ -204,7 +207,7 @@ __device__ __forceinline__ GaussIdx gauss_index(const Ctx &c, int key, int B)
   const unsigned n1 = (unsigned)n - 1;
   const unsigned nb = (unsigned)n >> ilog2v(B);
   GaussIdx x;
-  x.h = (int)(key * 1. / nb + 0.5) & (B - 1);
+  x.h = (int)(div2(key * 1., (int)nb) + 0.5) & (B - 1);
   const unsigned dist1 = ((unsigned)x.h * nb - (unsigned)key + (unsigned)n) & n1;
   x.dd[0] = dist1;
   x.dd[1] = (dist1 + (unsigned)n + nb) & n1;
@@ -216,7 +219,7 @@ __device__ __forceinline__ void gauss_values(const Ctx &c, int key, double2 valu
                                              const double2 F[3], double2 *r)
 {
   const int n = c.n;
-  const double PI2_DIV_N = 2 * M_PI / n;
+  const double PI2_DIV_N = div2(2 * M_PI, n);
   const double a1 = value.x, b1 = value.y;
   const int ko = smod(wmul(key, g), n);
   double b2, a2;
@@ -318,7 +321,7 @@ __device__ __forceinline__ void gauss_apply_few(double2 *S0, double2 *S1, int B,
 // update_mansour_loops2 (cf3 300-351), the removal at offset g
 __device__ __forceinline__ double2 mansour_value(const Ctx &c, int key, double2 value, int g)
 {
-  const double PI2_OVER_N = 2 * M_PI / c.n;
+  const double PI2_OVER_N = div2(2 * M_PI, c.n);
   const int W = c.W;
   const double vr = value.x, vi = value.y;
   double s0, c0;
@@ -687,7 +690,8 @@ __device__ __forceinline__ void found_at(const Ctx &c, int pos, int key, double2
 // One step of kV3Block buckets (bucket = step start + threadIdx.x) whose
 // results are in registers: the accepted ones are written at base + their
 // rank among the step's accepted buckets.  Returns the step's count
-// (uniform).  Uses NW ints at sh; contains barriers.
+// (uniform).  Uses NW ints at sh, which the next step must not (callers
+// alternate two sets); contains one barrier.
 __device__ __forceinline__ int emit_step(const Ctx &c, int base, bool ok, int out, double2 val,
                                          int *sh)
 {
@@ -703,7 +707,6 @@ __device__ __forceinline__ int emit_step(const Ctx &c, int base, bool ok, int ou
     off += q < wid ? t : 0;
     tot += t;
   }
-  __syncthreads();
   if (ok) {
     const int pos = off + __popcll(bal & ((1ull << lane) - 1));
     found_at(c, pos, out, val);
@@ -718,10 +721,10 @@ __device__ __forceinline__ int est_gauss(const Ctx &c, const double2 *S0, const 
   const int n = c.n;
   const unsigned n1 = (unsigned)n - 1, B1m = (unsigned)B - 1;
   const double PI2 = 2 * M_PI;
-  const double N_OVER_PI2 = n / PI2;
-  const double PI2_A_OFFSET_OVER_N = PI2 * a_ * c.gG / n;
-  const double BUCKETS_OVER_N = (double)B / n;
-  const int N_OVER_BUCKETS = n / B;
+  const double N_OVER_PI2 = n * (1 / PI2);  // (n a power of two: as n / PI2)
+  const double PI2_A_OFFSET_OVER_N = div2(PI2 * a_ * c.gG, n);
+  const double BUCKETS_OVER_N = div2((double)B, n);
+  const int N_OVER_BUCKETS = n >> ilog2v(B);
   int found = 0;
   for (int s0 = 0; s0 < B; s0 += blockDim.x) {
     const int bk = s0 + threadIdx.x;
@@ -732,24 +735,24 @@ __device__ __forceinline__ int est_gauss(const Ctx &c, const double2 *S0, const 
       const double zb = (a0 * a0 + b0 * b0) + (a1 * a1 + b1 * b1);
       if (zb > 1e-8) {
         const double c0 = a0 * a0 + b0 * b0, c1 = a1 * a1 + b1 * b1;
-        const double d0 = atan2(b0, a0), d1 = atan2(b1, a1);
         const double eb = c1 / c0 - 1;
         double err = eb * eb;
-        err /= n;
+        err = div2(err, n);
         if (err < 1e-12 && c0 > 0.01) {
+          const double d0 = atan2(b0, a0), d1 = atan2(b1, a1);
           const double slope = (d1 - d0) * 1.0;
           int freq = (int)rint(N_OVER_PI2 * slope) + n;
           freq = (int)((unsigned)freq & n1);
           const unsigned hashed = (unsigned)(long long)rint(freq * BUCKETS_OVER_N) & B1m;
           if (hashed == (unsigned)bk) {
+            const unsigned dist =
+                (hashed * (unsigned)N_OVER_BUCKETS - (unsigned)freq + (unsigned)n) & n1;
+            const double2 F = win_at(win, half, dist, n);  // in flight during the sine
             const double ph = d0 - PI2_A_OFFSET_OVER_N * freq;
             const double mag = sqrt(c0);
             double sn, cs;
             sincos(ph, &sn, &cs);
             const double mr = mag * cs, mi = mag * sn;
-            const unsigned dist =
-                (hashed * (unsigned)N_OVER_BUCKETS - (unsigned)freq + (unsigned)n) & n1;
-            const double2 F = win_at(win, half, dist, n);
             const double den = F.x * F.x + F.y * F.y;
             val = make_double2((mr * F.x + mi * F.y) / den, (mi * F.x - mr * F.y) / den);
             out = (int)(((unsigned)(timesmod(freq, a_, n) - b_ + n)) & n1);
@@ -757,7 +760,7 @@ __device__ __forceinline__ int est_gauss(const Ctx &c, const double2 *S0, const 
         }
       }
     }
-    found += emit_step(c, found, out >= 0, out, val, sh);
+    found += emit_step(c, found, out >= 0, out, val, sh + (s0 & kV3Block ? 8 : 0));
   }
   __threadfence_block();
   __syncthreads();
@@ -821,10 +824,10 @@ __device__ __forceinline__ int est_mansour(const Ctx &c, int *rank, int *sh)
   const int n = c.n, W = c.W;
   const double PI2 = 2 * M_PI;
   MansourConst m;
-  m.N_OVER_PI2 = n / PI2;
-  m.PI2_OVER_N = PI2 / n;
+  m.N_OVER_PI2 = n * (1 / PI2);  // (n a power of two: as n / PI2)
+  m.PI2_OVER_N = div2(PI2, n);
   m.FREQ_MASK = ((unsigned)n - 1) & ~((unsigned)W - 1);
-  m.NORM = 1. / W;
+  m.NORM = div2(1., W);
   m.NORM2 = m.NORM * m.NORM;
   m.err_max = n * 1e-10;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -888,22 +891,26 @@ __device__ __forceinline__ int est_mansour(const Ctx &c, int *rank, int *sh)
 // only: a bucket left unwritten holds the values that estimate rejected (an
 // accepted bucket is always written next, by the subtraction of what it
 // found), so it is rejected again and the result is the full sweep's.
-// Thread t takes bit word w = t (+ kV3Block ...), buckets 32 w .. 32 w + 31,
-// and clears it; a block scan over the threads' bit counts lists the set
-// bits in bucket order (list: kV3Block ints of LDS), and one thread tests and
-// estimates each listed bucket, one load latency and one estimate for all.
-__device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *list, int *sh)
+// Thread t takes bit word w = t, buckets 32 w .. 32 w + 31, and clears it.
+// most bounds the set bits.  Up to 64 (and no more words than threads): each
+// wave lists its lanes' bits in bucket order and tests and estimates them a
+// lane a bucket, one load latency and one estimate for all; a wave's buckets
+// lie below the next wave's, so emit_step ranks what was accepted.  More:
+// the block lists them together, kV3Block at a time.  list: kV3Block ints of
+// LDS.
+__device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int most, int *list, int *sh)
 {
   const int n = c.n, W = c.W;
   const double PI2 = 2 * M_PI;
   MansourConst m;
-  m.N_OVER_PI2 = n / PI2;
-  m.PI2_OVER_N = PI2 / n;
+  m.N_OVER_PI2 = n * (1 / PI2);  // (n a power of two: as n / PI2)
+  m.PI2_OVER_N = div2(PI2, n);
   m.FREQ_MASK = ((unsigned)n - 1) & ~((unsigned)W - 1);
-  m.NORM = 1. / W;
+  m.NORM = div2(1., W);
   m.NORM2 = m.NORM * m.NORM;
   m.err_max = n * 1e-10;
   const int words = (W + 31) >> 5;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   int found = 0;
   for (int w0 = 0; w0 < words; w0 += kV3Block) {
     const int wd = w0 + threadIdx.x;
@@ -911,6 +918,29 @@ __device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *list, int *s
     if (wd < words) {
       bits = c.dirty[wd];
       c.dirty[wd] = 0u;
+    }
+    if (most <= 64 && words <= kV3Block) {
+      int pos = 0, mine = 0;  // of the wave's bits: those of lower lanes, all
+      for (uint64_t bal = __ballot(bits != 0); bal; bal &= bal - 1) {
+        const int l = __ffsll((unsigned long long)bal) - 1;
+        const int cl = __popc((unsigned)__builtin_amdgcn_readlane((int)bits, l));
+        pos += l < lane ? cl : 0;
+        mine += cl;
+      }
+      int *wl = list + wid * 64;
+      for (; bits; bits &= bits - 1) wl[pos++] = wd * 32 + __ffs(bits) - 1;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      bool ok = false;
+      int o = -1;
+      double2 v = make_double2(0, 0);
+      if (lane < mine) {
+        const int bk = wl[lane];
+        ok = mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
+      }
+      found = emit_step(c, 0, ok, o, v, sh);
+      break;
     }
     int total;
     int pos = block_exclusive_scan(__popc(bits), sh, total);
@@ -924,7 +954,8 @@ __device__ __forceinline__ int est_mansour_dirty(const Ctx &c, int *list, int *s
         const int bk = list[threadIdx.x];
         ok = mansour_bucket<true>(c, m, bk, c.MS[2 * bk], c.MS[2 * bk + 1], o, v);
       }
-      found += emit_step(c, found, ok, o, v, sh);  // (its barriers free list)
+      found += emit_step(c, found, ok, o, v, sh);
+      __syncthreads();  // sh and list are used again
     }
   }
   __threadfence_block();
@@ -1435,7 +1466,7 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   extern __shared__ double2 lds[];
   __shared__ int sh[16];
   __shared__ int s_rank[kV3Block];
-  __shared__ int s_size, s_flag, s_cnt[3], s_cm, s_claim, s_ok;
+  __shared__ int s_size, s_flag, s_cnt[2][3], s_cm, s_claim, s_ok;
   __shared__ int s_lf[kFewPairs];
   __shared__ double2 s_lv[kFewPairs];
   // the empty map, written while the pre tasks run (Hcap: a power of two,
@@ -1508,13 +1539,13 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
     if (threadIdx.x == 0) s_flag |= 2;
   }
   for (int i = threadIdx.x; i < F; i += blockDim.x) {
-    const int h = c.ef[i] % W;  // one found per bucket
+    const int h = c.ef[i] & (W - 1);  // one found per bucket
     const double2 old = c.MS[2 * h];
     c.MS[2 * h] = make_double2(0, 0);
     c.MS[2 * h + 1] = make_double2(0, 0);
     if (c.dirty) {
       atomicOr(&c.dirty[h >> 5], 1u << (h & 31));
-      if (ms_counted(old, 1.0 / W)) atomicAdd(c.cm, -1);
+      if (ms_counted(old, div2(1.0, W))) atomicAdd(c.cm, -1);
     }
   }
   __threadfence_block();
@@ -1558,13 +1589,18 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
 
   // ---- round robin until the three bucket counts repeat (cf3 997-1076)
   int prev[3] = {0, 0, 0};
-  int pass = 0;
+  int pass = 0, round = 0;
+  int most = W;  // at least the Mansour buckets written since their last estimate
+  if (threadIdx.x < 3) s_cnt[0][threadIdx.x] = 0;  // (barriers before its use)
   bool cm_valid = false;  // s_cm holds the Mansour count (uniform)
   for (; pass < a.max_passes; pass++) {
     const int sel = pass % 3;
-    if (sel == 0) F = c.dirty ? est_mansour_dirty(c, s_rank, sh) : est_mansour(c, s_rank, sh);
-    else if (sel == 1) F = est_gauss(c, c.GS0, c.GS1, a.B1, 1, 0, a.win1, a.win1_half, sh);
+    if (sel == 0) {
+      F = c.dirty ? est_mansour_dirty(c, most, s_rank, sh) : est_mansour(c, s_rank, sh);
+      most = 0;
+    } else if (sel == 1) F = est_gauss(c, c.GS0, c.GS1, a.B1, 1, 0, a.win1, a.win1_half, sh);
     else F = est_gauss(c, c.GP0, c.GP1, a.B2, c.aa, c.b, a.win2, a.win2_half, sh);
+    most += F;
     if (!add_subtract(c, F, 7, sh, &s_size, &s_ok)) {
       // (what was subtracted all the same is not read again)
       if (threadIdx.x == 0) s_flag |= 2;
@@ -1572,8 +1608,10 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
       break;
     }
     if (sel == 2) {
-      if (threadIdx.x < 3) s_cnt[threadIdx.x] = 0;
-      __syncthreads();
+      // three counters a round, cleared one round ahead
+      int *const cnt = s_cnt[round & 1];
+      round++;
+      if (threadIdx.x < 3) s_cnt[round & 1][threadIdx.x] = 0;
       int c1 = 0, c2 = 0, cm = 0;
       for (int j = threadIdx.x; j < a.B1; j += blockDim.x) {
         // the reference counts elements 0..B1-1 of its interleaved array
@@ -1587,7 +1625,7 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
       // the Mansour count is kept up to date by every bucket write once it
       // has been counted in full (the first test)
       if (!cm_valid) {
-        const double invW = 1.0 / W;
+        const double invW = div2(1.0, W);
         for (int j0 = threadIdx.x; j0 < W; j0 += kSweepAhead * kV3Block) {
           double2 z[kSweepAhead];  // loaded together, clamped past the end
 #pragma unroll
@@ -1598,13 +1636,12 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
       }
       if (!cm_valid) cm = wave_sum(cm);
       if ((threadIdx.x & 63) == 0) {
-        if (!cm_valid) atomicAdd(&s_cnt[0], cm);
-        atomicAdd(&s_cnt[1], c1);
-        atomicAdd(&s_cnt[2], c2);
+        if (!cm_valid) atomicAdd(&cnt[0], cm);
+        atomicAdd(&cnt[1], c1);
+        atomicAdd(&cnt[2], c2);
       }
       __syncthreads();
-      const int now[3] = {cm_valid ? s_cm : s_cnt[0], s_cnt[1], s_cnt[2]};
-      __syncthreads();
+      const int now[3] = {cm_valid ? s_cm : cnt[0], cnt[1], cnt[2]};
       if (!cm_valid && c.dirty) {
         if (threadIdx.x == 0) s_cm = now[0];
         cm_valid = true;

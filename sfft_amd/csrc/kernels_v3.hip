@@ -25,10 +25,9 @@ namespace {
 
 constexpr int kV3Block = 512;
 static_assert((kV3Block & (kV3Block - 1)) == 0, "owner tests take residues by masking");
-// Passes that found up to this many pairs (a lane each) keep them and their
-// subtraction values in LDS.
+// Passes that found up to this many pairs give each a lane.
 constexpr int kFewPairs = 64;
-static_assert(kV3Block / 64 == 8, "subtract_few gives each of eight waves a part");
+static_assert(kV3Block / 64 >= 7, "six waves subtract a pass of few pairs, one adds them");
 // Steps of a sweep over the Mansour buckets whose loads are issued together.
 constexpr int kSweepAhead = 4;
 // Loads the pre-kernel's gathers and folds issue together per thread.
@@ -39,6 +38,7 @@ constexpr int kStageChunk = 1024, kMinStageChunk = 16;
 // Entries of one Gauss filter a thread ranks per chunk, values read ahead of
 // a bucket's subtractions, and hash slots of a chunk's Mansour buckets.
 constexpr int kStageRanks = (3 * kStageChunk + kV3Block - 1) / kV3Block, kStageAhead = 4;
+constexpr int kRankAhead = 4;  // entries a rank reads together
 constexpr int kMansourSlots = 256;
 static_assert(6 * kStageChunk <= 65536, "list entries are 16 bits");
 
@@ -115,13 +115,11 @@ __device__ __forceinline__ int ms_counted(double2 z, double invW)
   return re * re + im * im > 1e-6;
 }
 
-// MS bucket h becomes (now, now1), loop 0's value having been old: its
-// dirty bit set and the count updated.
-__device__ __forceinline__ void ms_put(const Ctx &c, int h, double2 old, double2 now,
-                                       double2 now1)
+// Loop 0's value of MS bucket h, old until now, becomes now: the bucket's
+// dirty bit is set and the count updated.
+__device__ __forceinline__ void ms_put(const Ctx &c, int h, double2 old, double2 now)
 {
   c.MS[2 * h] = now;
-  c.MS[2 * h + 1] = now1;
   if (c.dirty) {
     const double invW = div2(1.0, c.W);
     atomicOr(&c.dirty[h >> 5], 1u << (h & 31));
@@ -134,7 +132,8 @@ __device__ __forceinline__ void ms_put(const Ctx &c, int h, double2 old, double2
 __device__ __forceinline__ void ms_sub(const Ctx &c, int h, double2 r0, double2 r1)
 {
   const double2 old = c.MS[2 * h];
-  ms_put(c, h, old, csub(old, r0), csub(c.MS[2 * h + 1], r1));
+  c.MS[2 * h + 1] = csub(c.MS[2 * h + 1], r1);
+  ms_put(c, h, old, csub(old, r0));
 }
 
 // ---------------------------------------------------------------- map
@@ -249,75 +248,6 @@ __device__ void gauss_apply_pair(double2 *S0, double2 *S1, int B, int h, const d
   for (int q = 0; q < 3; q++) S1[bk[q]] = csub(S1[bk[q]], r[3 + q]);
 }
 
-// A few pairs (removal values in LDS, nv per pair, bucket indices nf per
-// pair, both from this filter's first on; cnt <= 64) applied by bucket
-// owners: thread t takes its buckets t, t + blockDim, ... and walks the
-// pairs in order, applying the parts that land on the bucket (h, h+1, h-1
-// within a pair) -- the order in which gauss_apply_pair applies them pair
-// after pair.  The bucket indices come from lanes (no LDS latency a pair),
-// kStageAhead pairs' values are read together, and a wave skips those of
-// which none lands on its buckets.
-__device__ __forceinline__ void gauss_apply_few(double2 *S0, double2 *S1, int B, const int *si,
-                                                int nf, const double2 *sv, int nv, int cnt)
-{
-  const int bm = B - 1;  // B a power of two
-  const int lane = threadIdx.x & 63;
-  const int hl = si[(lane < cnt ? lane : 0) * nf];
-  // whole waves throughout (lanes past the last bucket idle, not inactive):
-  // a lane holds a pair's index whether or not it has a bucket
-  const int w0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);
-  for (int t0 = w0; t0 < B; t0 += kV3Block) {
-    const int tb = t0 + lane;
-    const bool own = tb < B;
-    double2 a0 = S0[own ? tb : 0], a1 = S1[own ? tb : 0];
-    bool any = false;
-    if (B < 4) {  // a bucket can be several of a pair's three
-      for (int i = 0; i < cnt; i++) {
-        const int h = __builtin_amdgcn_readlane(hl, i);
-        const double2 *r = sv + i * nv;
-        const int bk[3] = {h, (h + 1) & bm, (h + bm) & bm};
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-          if (own && bk[q] == tb) {
-            a0 = csub(a0, r[q]);
-            a1 = csub(a1, r[3 + q]);
-            any = true;
-          }
-      }
-    } else {
-      for (int i0 = 0; i0 < cnt; i0 += kStageAhead) {
-        int d[kStageAhead];  // 0, 1, 2: this bucket is h - 1, h, h + 1
-        bool hit = false;
-#pragma unroll
-        for (int u = 0; u < kStageAhead; u++) {
-          const int h = __builtin_amdgcn_readlane(hl, min(i0 + u, cnt - 1));
-          d[u] = own && i0 + u < cnt ? (tb - h + 1) & bm : 3;
-          hit |= d[u] < 3;
-        }
-        if (!hit) continue;
-        any = true;
-        double2 v0[kStageAhead], v1[kStageAhead];
-#pragma unroll
-        for (int u = 0; u < kStageAhead; u++) {  // (of no pair: pair cnt - 1, unused)
-          const double2 *r = sv + min(i0 + u, cnt - 1) * nv + (d[u] == 1 ? 0 : (d[u] == 2 ? 1 : 2));
-          v0[u] = r[0];
-          v1[u] = r[3];
-        }
-#pragma unroll
-        for (int u = 0; u < kStageAhead; u++)
-          if (d[u] < 3) {
-            a0 = csub(a0, v0[u]);
-            a1 = csub(a1, v1[u]);
-          }
-      }
-    }
-    if (any) {
-      S0[tb] = a0;
-      S1[tb] = a1;
-    }
-  }
-}
-
 // update_mansour_loops2 (cf3 300-351), the removal at offset g
 __device__ __forceinline__ double2 mansour_value(const Ctx &c, int key, double2 value, int g)
 {
@@ -392,8 +322,9 @@ __device__ __forceinline__ size_t staged_fixed_bytes(int NB)
 // once, a barrier serving each:
 // - Gauss: the entries e = 3 u + q (pair u; q = 0, 1, 2 for its buckets h,
 //   h+1, h-1; Gauss-2's after Gauss-1's) are sorted by bucket -- counts, an
-//   exclusive scan, atomic placement, then every entry moved to its rank
-//   among the e of its bucket's list, one thread an entry.  (Sorted by
+//   exclusive scan, atomic placement of kV3Block entries at a time, then
+//   every entry moved to its rank among those of its bucket placed with it,
+//   one thread an entry.  (Sorted by
 //   insertion, a thread a bucket, the 48 pairs of an 8-bucket filter took
 //   14 us more.)  A thread for each bucket of each offset's array applies
 //   its entries in e order, which is pair order and h, h+1, h-1 within a
@@ -465,19 +396,28 @@ __device__ __forceinline__ void apply_staged(const Ctx &c, int which, const doub
     }
   }
   __syncthreads();
-  for (int e = t; e < E; e += T) list[atomicAdd(&pos[entry(e, vi)], 1)] = (unsigned short)e;
-  __syncthreads();  // pos[b] is the end of bin b
+  // T entries at a time, so a rank looks only among its bucket's entries of
+  // the same T (all at once, 962 pairs of a 128-bucket filter read 23 entries
+  // for each, and placing and ranking took 12.4 us; 5.9 so)
   int slot[MR];
 #pragma unroll
   for (int x = 0; x < MR; x++) {
+    if (x * T >= E) break;
     const int e = t + x * T;
-    if (e >= E) break;
-    const int b = entry(e, vi);
-    const int lo = b ? pos[b - 1] : 0, hi = pos[b];
-    int before = lo;
-    for (int i = lo; i < hi; i++) before += (int)list[i] < e;
-    slot[x] = before;
-  }
+    const int b = e < E ? entry(e, vi) : 0;
+    const int lo = pos[b];  // the end of bin b's earlier entries
+    __syncthreads();
+    if (e < E) list[atomicAdd(&pos[b], 1)] = (unsigned short)e;
+    __syncthreads();
+    if (e >= E) continue;
+    int at = lo;
+    const int hi = pos[b];
+    for (int i0 = lo; i0 < hi; i0 += kRankAhead)
+#pragma unroll
+      for (int u = 0; u < kRankAhead; u++)  // past the end: the last entry again
+        at += i0 + u < hi && (int)list[min(i0 + u, hi - 1)] < e;
+    slot[x] = at;
+  }  // pos[b] is the end of bin b
   __syncthreads();
 #pragma unroll
   for (int x = 0; x < MR; x++) {
@@ -498,7 +438,8 @@ __device__ __forceinline__ void apply_staged(const Ctx &c, int which, const doub
       }
       if (!first) continue;
       const double2 *r = sv + j * nv + 6 * ng;
-      ms_put(c, h, z0[x], csub(z0[x], r[0]), csub(z1[x], r[1]));
+      c.MS[2 * h + 1] = csub(z1[x], r[1]);
+      ms_put(c, h, z0[x], csub(z0[x], r[0]));
       for (int cur = j; more;) {  // later pairs of this bucket, ascending
         int nxt = m;
         for (int q = head[h & (kMansourSlots - 1)]; q >= 0; q = next[q])
@@ -533,79 +474,93 @@ __device__ __forceinline__ void apply_staged(const Ctx &c, int which, const doub
   }
 }
 
-// Few pairs: kept, like their removal values, in LDS.
-__device__ __forceinline__ bool few_pairs(const Ctx &c, int cnt)
+// Whether cnt pairs are few: a lane for each, and no more than per_bucket
+// pairs for each bucket of the smallest Gauss filter in which, since pairs
+// that share buckets take turns (48 pairs of an 8-bucket filter took 10 us
+// in turns, 7 us staged; 40 of a 32-bucket one 6.4 and 4.9; a pass that also
+// adds its pairs to the map gains by the wave that does so meanwhile, 8
+// pairs of an 8-bucket filter 1.9 and 7.8).
+__device__ __forceinline__ bool few_pairs(const Ctx &c, int cnt, int which, int per_bucket)
 {
-  return cnt <= kFewPairs && !c.a->serial_all &&
-         c.room >= (size_t)cnt * (14 * sizeof(double2) + 3 * sizeof(int));
+  const int B = which & 2 ? min(c.B2, which & 1 ? c.B1 : INT_MAX) : c.B1;
+  return cnt <= min(kFewPairs, per_bucket * B) && !c.a->serial_all;
 }
 
 // The subtraction of the 0 < cnt <= kFewPairs pairs in lf, lv: a wave for
-// each filter and offset computes its removals, a lane a pair (both offsets
-// on one lane took their sines in turn); the owner of a Gauss bucket applies
-// them in pair order, and each Mansour bucket (in HBM) is updated by the
-// lane of its first pair, in pair order -- every bucket sees the same
-// subtractions in the same order.  The last wave (no removal is computed
-// there) loads the Mansour buckets meanwhile.  Contains barriers, none after
-// the last update.
+// each filter and offset, a lane a pair.  A lane computes its removal and
+// applies it to the wave's bucket array itself, once every earlier pair that
+// shares a bucket with it has been applied: all pairs that share none at
+// once, the rest in rounds, so every bucket sees its subtractions in pair
+// order.  (Owners of buckets walking the pairs read each from LDS: a pass of
+// 36 pairs took 8.6 us, 9 4.4 and 4 2.2; so 4.4, 2.0 and 1.8.)  No barriers.
 __device__ __forceinline__ void subtract_few(const Ctx &c, int cnt, int which)
 {
   const V3Launch &a = *c.a;
-  double2 *const sv = c.stage;
-  const int nv = removal_values(which), nf = removal_indices(which);
-  int *const si = reinterpret_cast<int *>(sv + cnt * nv);
-  const int g1 = which & 1, g2 = (which >> 1) & 1;
+  const int nf = removal_indices(which), g1 = which & 1;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const bool mansour = (which & 4) && wave == kV3Block / 64 - 1;
-  int mh = -1;
-  bool first = false, more = false;
-  double2 z0 = make_double2(0, 0), z1 = make_double2(0, 0);
-  if (mansour) {
-    if (lane < cnt) {
-      mh = c.lf[lane] & (c.W - 1);
-      z0 = c.MS[2 * mh];
-      z1 = c.MS[2 * mh + 1];
+  if (wave >= 2 * nf) return;
+  const int f = wave >> 1, off = wave & 1;  // f-th filter here
+  const bool act = lane < cnt;
+  const int key = act ? c.lf[lane] : 0;
+  const double2 v = act ? c.lv[lane] : make_double2(0, 0);
+  const uint64_t all = cnt < 64 ? (1ull << cnt) - 1 : ~0ull;
+  if ((which & 4) && f == nf - 1) {
+    const int h = key & (c.W - 1);
+    double2 *const ms = c.MS + 2 * h + off;
+    const double2 early = *ms;  // in flight during the sine
+    uint64_t before = 0;
+    for (int q = 0; q < cnt; q++)
+      before |= (uint64_t)(q < lane && __builtin_amdgcn_readlane(h, q) == h) << q;
+    const double2 r = mansour_value(c, key, v, c.g0 + off);
+    for (uint64_t done = 0; done != all;) {
+      const bool now = act && !((done >> lane) & 1) && !(before & ~done);
+      if (now) {
+        const double2 old = before ? *ms : early;
+        const double2 z = csub(old, r);
+        if (off) *ms = z;
+        else ms_put(c, h, old, z);
+      }
+      done |= __ballot(now);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    first = lane < cnt;
-    for (int q = 0; q < cnt; q++) {
-      const int hq = __builtin_amdgcn_readlane(mh, q);
-      first &= !(q < lane && hq == mh);
-      more |= q > lane && hq == mh;
-    }
+    return;
   }
-  if (wave < 2 * nf && lane < cnt) {
-    const int f = wave >> 1, off = wave & 1;  // f-th filter here
-    const int key = c.lf[lane];
-    const double2 v = c.lv[lane];
-    double2 *r = sv + lane * nv;
-    if ((which & 4) && f == nf - 1) {
-      if (off == 0) si[lane * nf + f] = key & (c.W - 1);
-      r[6 * f + off] = mansour_value(c, key, v, c.g0 + off);
-    } else {
-      const bool second = f == 1 || !g1;  // Gauss-2
-      const int kf = second ? smod(timesmod(key, c.ai, c.n) + c.shift, c.n) : key;
-      const int g = second ? wmul(c.aa, c.gG) : c.gG;
-      const double2 *win = second ? a.win2 : a.win1;
-      const int half = second ? a.win2_half : a.win1_half;
-      const GaussIdx x = gauss_index(c, kf, second ? c.B2 : c.B1);
-      double2 F[3];
+  const bool second = f == 1 || !g1;  // Gauss-2
+  const int B = second ? c.B2 : c.B1, bm = B - 1;
+  const int kf = second ? smod(timesmod(key, c.ai, c.n) + c.shift, c.n) : key;
+  const int g = second ? wmul(c.aa, c.gG) : c.gG;
+  const double2 *win = second ? a.win2 : a.win1;
+  const int half = second ? a.win2_half : a.win1_half;
+  // GS0, GS1, GP0, GP1 lie one after the other
+  double2 *const S = c.GS0 + (second ? 2 * c.B1 + off * c.B2 : off * c.B1);
+  const GaussIdx x = gauss_index(c, kf, B);
+  double2 F[3], r[3];
 #pragma unroll
-      for (int q = 0; q < 3; q++) F[q] = win_at(win, half, x.dd[q], c.n);
-      if (off == 0) si[lane * nf + f] = x.h;
-      gauss_values(c, kf, v, (int)((unsigned)g + (unsigned)off), F, r + 6 * f + 3 * off);
+  for (int q = 0; q < 3; q++) F[q] = win_at(win, half, x.dd[q], c.n);
+  uint64_t before = 0;  // earlier pairs within two buckets (mod B) share one
+  for (int q = 0; q < cnt; q++)
+    before |=
+        (uint64_t)(q < lane && ((x.h - __builtin_amdgcn_readlane(x.h, q) + 2) & bm) <= 4) << q;
+  gauss_values(c, kf, v, (int)((unsigned)g + (unsigned)off), F, r);
+  const int bk[3] = {x.h, (x.h + 1) & bm, (x.h + bm) & bm};
+  for (uint64_t done = 0; done != all;) {
+    const bool now = act && !((done >> lane) & 1) && !(before & ~done);
+    if (now) {
+      if (B >= 4) {
+        double2 z[3];
+#pragma unroll
+        for (int q = 0; q < 3; q++) z[q] = S[bk[q]];
+#pragma unroll
+        for (int q = 0; q < 3; q++) S[bk[q]] = csub(z[q], r[q]);
+      } else {  // some of the three are one bucket
+#pragma unroll
+        for (int q = 0; q < 3; q++) S[bk[q]] = csub(S[bk[q]], r[q]);
+      }
     }
+    done |= __ballot(now);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
-  __syncthreads();
-  if (mansour && first) {
-    const double2 *r = sv + 6 * (g1 + g2);
-    ms_put(c, mh, z0, csub(z0, r[lane * nv]), csub(z1, r[lane * nv + 1]));
-    if (more)
-      for (int i = lane + 1; i < cnt; i++)
-        if (si[i * nf + g1 + g2] == mh) ms_sub(c, mh, r[i * nv], r[i * nv + 1]);
-  }
-  if (g1) gauss_apply_few(c.GS0, c.GS1, c.B1, si, nf, sv, nv, cnt);
-  if (g2) gauss_apply_few(c.GP0, c.GP1, c.B2, si + g1, nf, sv + 6 * g1, nv, cnt);
 }
 
 // Subtraction of cnt (key, value) pairs from the buckets of the filters in
@@ -615,7 +570,7 @@ __device__ __forceinline__ void subtract(const Ctx &c, const int *keys, const do
                                          int cnt, int which)
 {
   if (cnt == 0) return;
-  if (few_pairs(c, cnt)) {
+  if (few_pairs(c, cnt, which, 1)) {
     if ((int)threadIdx.x < cnt) {
       c.lf[threadIdx.x] = keys[threadIdx.x];
       c.lv[threadIdx.x] = vals[threadIdx.x];
@@ -1040,13 +995,13 @@ __device__ __forceinline__ bool add_subtract(const Ctx &c, int F, int which, int
                                              int *s_size, int *s_ok)
 {
   if (F == 0) return true;
-  if (!few_pairs(c, F)) {
+  if (!few_pairs(c, F, which, 3)) {
     const bool ok = map_add_found(c, F, sh, s_size);
     __syncthreads();
     subtract(c, c.ef, c.ev, F, which);
     return ok;
   }
-  if ((threadIdx.x >> 6) == kV3Block / 64 - 2) map_add_wave(c, F, s_size, s_ok);
+  if ((threadIdx.x >> 6) == kV3Block / 64 - 1) map_add_wave(c, F, s_size, s_ok);
   subtract_few(c, F, which);
   __threadfence_block();
   __syncthreads();

@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(kBlock) k_comb_merge(V12Launch a)
 // One block per (signal, loop).  Each thread owns buckets m = tid + q*T and
 // sums, in ascending tap order like the reference, x[(i*ai) mod n]*tap[i]
 // over the taps i = m + r*B < w.  LDS: B double2.  FP64 only (the FP32
-// form folds in k_fold_chunks).
+// form folds in k_fold_sorted).
 constexpr int kQ = 8;  // buckets per thread in flight (independent gathers)
 
 __global__ void __launch_bounds__(kBlock) k_fold_fft64(V12Launch a, int l0, int nl)
@@ -278,8 +278,8 @@ __global__ void __launch_bounds__(kBlock) k_fold_fft64(V12Launch a, int l0, int 
 //         chunk order.
 //
 // Bound by HBM on batches: the 850,060 gathers of a signal (n = 2^22, k = 64)
-// touch 422,076 lines, 13.83 GB per 256 signals, read in 2.96 ms (4.7 TB/s,
-// the rate of a large copy).  Before, with the gathers of a 256-row chunk in
+// touch 422,076 lines, 13.83 GB per 256 signals, read in 2.76 ms (5.0 TB/s;
+// a large copy reaches 4.7).  Before, with the gathers of a 256-row chunk in
 // flight at a time in tap order, 3.72 ms; the FP64 form, one wave per 64
 // buckets in tap order, took 1.03 ms per 64 signals against 0.80 ms.  One
 // signal is bound by the phases' latency: 19 us against 36 us (FP32), 17 us
@@ -643,8 +643,8 @@ __global__ void __launch_bounds__(1024) k_bucket_fft_v1(V12Launch a)
 constexpr int kVoteChunk = 8 * kBlock;
 static_assert(kVoteChunk == 2048, "vote_chunks() assumes chunks of 2048 candidates");
 
-// (the kernels evaluate a thread's eight candidates together, so that their
-// dependent reads overlap).
+// Both kernels evaluate a thread's eight candidates together, so that their
+// dependent reads overlap.
 struct VoteCtx {
   const int *prm, *J;
   const unsigned *selbits;
@@ -1768,11 +1768,11 @@ static bool fold_part(const V12Launch &a, bool fp32, int l0, int nl, int B, int 
 static bool fold_parts(const V12Launch &a, int from, int n64, FoldParts &f, size_t &lds)
 {
   // 16 residues (256 contiguous bytes of a row) read HBM 5-10 % faster than
-  // 8 on batches (FP32 256 x n = 2^22, k = 64: 3.20 against 3.56 ms beside
-  // the estimation; FP64 64 signals: 0.81 against 0.86 ms); a launch of few
-  // workgroups is faster spread over twice as many (one signal: 19.0 against
-  // 20.8 us), and a workgroup's LDS does not hold 16 residues of many FP64
-  // loops
+  // 8 on batches (with the groups in their natural order: FP32 256 x n =
+  // 2^22, k = 64: 3.20 against 3.56 ms beside the estimation; FP64 64
+  // signals: 0.81 against 0.86 ms); a launch of few workgroups is faster
+  // spread over twice as many (one signal: 19.0 against 20.8 us), and a
+  // workgroup's LDS does not hold 16 residues of many FP64 loops
   f = FoldParts{};
   lds = 0;
   int np = 0;

@@ -74,7 +74,7 @@ def parse():
     return ap.parse_args()
 
 
-TRAFFIC_PROFILE = "profiles/traffic_fold_chunks_v2_n22_k64_b256.md"
+TRAFFIC_PROFILE = "profiles/traffic_fold_sorted_v2_n22_k64_b256.md"
 
 
 def measured_traffic(kernel, S, n, k):

@@ -1136,9 +1136,7 @@ __global__ void __launch_bounds__(kBlock) k_estimate_comb(V12Launch a, int tiles
           } else {
             U = xs64[s_off[l] + hashed];
             const double den = t_den[l * kTI + il];
-            vr[l] = (U.x * g.x + U.y * g.y) / den;
-            const double q = (U.x * g.y - U.y * g.x) / den;
-            vi[l] = conj ? q : -q;
+            divide_by_filter(U, g, den, conj, vr[l], vi[l]);
           }
         } else {
           vr[l] = __longlong_as_double(0x7ff0000000000000ll);  // +inf pads
@@ -1357,11 +1355,14 @@ constexpr int kRI = 16, kRIsmall = 4;
 // its residual is exact to 2^-53 of itself, and where the quotient lies next
 // to a rounding midpoint q0 is half an ulp away, so the corrected sum lies
 // on the quotient's side of the midpoint (Markstein).  Holds while nothing
-// over- or underflows: see plain_value.
+// over- or underflows: see plain_value.  The residual is formed negated and
+// multiplied by -inv: for a = -0 the product is then -0, which leaves q0 = -0
+// as it is, where a - den q0 = +0 would turn it into +0 (the same
+// instructions; the signs are operand modifiers).
 __device__ __forceinline__ double div_by(double a, double den, double inv)
 {
   const double q0 = a * inv;
-  return fma(fma(-den, q0, a), inv, q0);
+  return fma(fma(den, q0, -a), -inv, q0);
 }
 
 // v, negated where flip is the sign bit (exact; an integer operation)
@@ -1402,6 +1403,15 @@ __device__ __forceinline__ double2 rows_median(const char *xs, const RowEntry32 
   return lower_median<LMAX>(vr, vi, FULL ? LMAX : L);
 }
 
+// The imaginary numerator of divide_by_filter: u.x gy - u.y gx, or with flip
+// (the unconjugated estimate) u.y gx - u.x gy, the same difference of
+// products with their signs flipped (a flipped result would turn a zero
+// difference's +0 into -0).
+__device__ __forceinline__ double imag_part(double2 u, const RowEntry64 &e, unsigned flip)
+{
+  return flip_sign(u.x, flip) * e.gy - flip_sign(u.y, flip) * e.gx;
+}
+
 // FP64: the reference's operation order (cf12 383-398); odd: with divisions,
 // one part and one quotient at a time (rare, so with few registers).
 template <int LMAX, bool FULL>
@@ -1416,7 +1426,7 @@ __device__ __forceinline__ double2 rows_median(const char *xs, const RowEntry64 
         const RowEntry64 e = tab[l];
         const double2 u = row_bucket<double2>(xs, e, jm, row_mask);
         vr[l] = div_by(u.x * e.gx + u.y * e.gy, e.den, e.inv);
-        vi[l] = flip_sign(div_by(u.x * e.gy - u.y * e.gx, e.den, e.inv), flip);
+        vi[l] = div_by(imag_part(u, e, flip), e.den, e.inv);
       } else {
         vr[l] = __longlong_as_double(0x7ff0000000000000ll);
         vi[l] = vr[l];
@@ -1433,8 +1443,7 @@ __device__ __forceinline__ double2 rows_median(const char *xs, const RowEntry64 
       if (FULL || l < L) {
         const RowEntry64 e = tab[l];
         const double2 u = row_bucket<double2>(xs, e, jm, row_mask);
-        v[l] = c == 0 ? (u.x * e.gx + u.y * e.gy) / e.den
-                      : flip_sign((u.x * e.gy - u.y * e.gx) / e.den, flip);
+        v[l] = (c == 0 ? u.x * e.gx + u.y * e.gy : imag_part(u, e, flip)) / e.den;
       } else {
         v[l] = __longlong_as_double(0x7ff0000000000000ll);
       }

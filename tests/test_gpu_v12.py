@@ -588,6 +588,27 @@ def test_alias_row_quotients(torch_cuda, kind):
             assert np.array_equal(a[i][1].view(np.float64), b[i][1].view(np.float64), equal_nan=True)
 
 
+@pytest.mark.parametrize("zero", [0.0, -0.0])
+def test_alias_row_signs_of_zero(torch_cuda, zero):
+    """Quotients of zero buckets keep the division's sign: for a signal of
+    zeros the alias-row estimation (schedule 1) gives the bits of the
+    natural-order one (schedule 2), which divides, estimates of -0 among
+    them, with the reference's conjugation and without."""
+    n, k = 1 << 18, 64
+    print(f"case signs of zero {zero}", flush=True)
+    x = np.full(n, complex(zero, zero))
+    neg = np.uint64(1 << 63)
+    for conj in (True, False):
+        bits = []
+        for mode in (1, 2):
+            plan = _gpu_plan(2, n, k)
+            plan.set_schedule(mode, 0)
+            plan.set_reference_conjugate(conj)
+            bits.append(_run_gpu_dense(torch_cuda, plan, x).view(np.uint64))
+        assert np.array_equal(bits[0], bits[1]), conj
+        assert (bits[1] == neg).any(), conj
+
+
 @pytest.mark.parametrize("version,precision,mode", [
     (1, "fp64", 0), (1, "fp64", 1), (1, "fp32_refine", 0), (2, "fp64", 2), (2, "fp32_refine", 1)])
 def test_dense_outputs_are_cleared(torch_cuda, version, precision, mode):

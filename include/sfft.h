@@ -70,11 +70,15 @@ sfft_plan *sfft_make_plan(int n, int k, sfft_version version,
 void sfft_free_plan(sfft_plan *plan);
 
 /* src/sfft.h:165 / src/sfft.cc:119-137.  out (n values) is zero-filled and
- * the located coefficients are written, as the reference does. */
+ * the located coefficients are written, as the reference does.  A device
+ * output may share memory with a device input: it is cleared first, as in
+ * the reference, so the input's shared part is read as zero. */
 void sfft_exec(sfft_plan *plan, complex_t *in, complex_t *out);
 
 /* src/sfft.h:166 / src/sfft.cc:139-147.  All signals go to the GPU as one
- * batch; RNG draws are consumed in signal order 0..num-1. */
+ * batch (in several where the workspace would pass 4 GiB); RNG draws are
+ * consumed in signal order 0..num-1.  Device outputs that share memory with
+ * inputs or outputs of their batch are cleared before any input is read. */
 void sfft_exec_many(sfft_plan *plan, int num, complex_t **in,
                     complex_t **out);
 

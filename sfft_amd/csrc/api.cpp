@@ -40,6 +40,26 @@ int chunk_signals(const Plan *P, bool host_inputs)
   return (int)std::max<int64_t>(1, std::min<int64_t>(4096, budget / per));
 }
 
+// Whether one of the dense device outputs (entries may be null) shares memory
+// with an input or with another output, all of n values.  Sorted by address,
+// the nearest neighbour of a range that overlaps any other overlaps it too.
+bool dense_overlaps(const std::vector<double2 *> &out, const std::vector<const double2 *> &in,
+                    int64_t n)
+{
+  std::vector<std::pair<uintptr_t, bool>> at;  // start, is an output
+  at.reserve(out.size() + in.size());
+  for (const double2 *p : out)
+    if (p) at.push_back({reinterpret_cast<uintptr_t>(p), true});
+  if (at.empty()) return false;
+  for (const double2 *p : in) at.push_back({reinterpret_cast<uintptr_t>(p), false});
+  std::sort(at.begin(), at.end());
+  for (size_t i = 1; i < at.size(); i++)
+    if ((at[i].second || at[i - 1].second) &&
+        at[i].first - at[i - 1].first < (size_t)n * sizeof(double2))
+      return true;
+  return false;
+}
+
 // Runs num signals.  Exactly one of (dense, sparse) is non-null.
 int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
         sfft_output_c *sparse)
@@ -106,7 +126,7 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
         }
         if (kinds.is_device(o)) {
           de[s] = reinterpret_cast<double2 *>(o);
-          // v1/v2 batches clear their dense outputs themselves
+          // v1/v2 batches clear their dense outputs themselves (below)
           if (P->version == SFFT_VERSION_3 && k::zero_dense(de[s], n, st) != 0) return fail(c0);
         } else {
           via_ws[s] = 1;
@@ -143,7 +163,14 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
     io.freq = any_sparse ? fr.data() : nullptr;
     io.val = any_sparse ? va.data() : nullptr;
     io.dense = dense ? de.data() : nullptr;
-    io.zero_dense = P->version != SFFT_VERSION_3;
+    // v1/v2 dense outputs are cleared in the fold's launch, part by part in
+    // large batches; those that share memory with an input or each other
+    // before anything else instead, as the reference does
+    // (src/sfft.cc:121-123): the input is then read as cleared
+    const bool first = dense && P->version != SFFT_VERSION_3 && dense_overlaps(de, ins, n);
+    for (int s = 0; s < S && first; s++)
+      if (de[s] && k::zero_dense(de[s], n, st) != 0) return fail(c0);
+    io.zero_dense = P->version != SFFT_VERSION_3 && !first;
     io.cap = cap;
     io.counts = counts.data();
     const int rc = exec_batch(P, io);

@@ -634,3 +634,86 @@ def test_dense_outputs_are_cleared(torch_cuda, version, precision, mode):
     plan.seed(17, 4242)
     plan.execute_device(xd[0], outs[1])
     assert torch.equal(outs[1], want[0])
+
+
+@pytest.mark.parametrize("version,precision", [(1, "fp64"), (2, "fp64"), (2, "fp32_refine")])
+def test_dense_outputs_sharing_memory(torch_cuda, version, precision):
+    """A dense device output that shares memory with an input of the call is
+    cleared before the inputs are read: the results are those of inputs
+    whose shared samples are zero."""
+    torch = torch_cuda
+    n, k = 1 << 16, 64
+    print(f"case shared memory v{version} {precision}", flush=True)
+    xs = [torch.from_numpy(signal_np(n, k, seed=90 + i, snr_db=30.0)[0]).cuda() for i in range(3)]
+    plan = _gpu_plan(version, n, k, precision)
+
+    def run(ins, outs):
+        plan.seed(17, 4242)
+        plan.execute_many_device(ins, outs)
+        torch.cuda.synchronize()
+
+    def fresh(cnt):
+        return [torch.empty(n, dtype=torch.complex128, device="cuda") for _ in range(cnt)]
+
+    # half of the output over half of the input, and the other way round
+    for shift in (n // 2, -(n // 2)):
+        buf = torch.zeros(2 * n, dtype=torch.complex128, device="cuda")
+        a, b = (0, shift) if shift > 0 else (-shift, 0)
+        buf[a:a + n] = xs[0]
+        x = xs[0].clone()
+        x[max(0, b - a):min(n, b - a + n)] = 0
+        want = fresh(1)
+        run([x], want)
+        run([buf[a:a + n]], [buf[b:b + n]])
+        assert torch.equal(buf[b:b + n], want[0]), shift
+    # an output that is another signal's input, and one that is its own
+    want = fresh(3)
+    run([xs[0], torch.zeros_like(xs[1]), torch.zeros_like(xs[2])], want)
+    ins = [x.clone() for x in xs]
+    outs = [ins[1], ins[2], fresh(1)[0]]
+    run(ins, outs)
+    for i in range(3):
+        assert torch.equal(outs[i], want[i]), i
+
+
+def test_dense_outputs_of_a_parted_batch(torch_cuda):
+    """Dense device outputs of 70 FP32 signals, a batch that runs in parts
+    (each part's clear on one stream, its estimates on another): every
+    output, filled before, holds its signal's located values and zeros.  Two
+    signals of different parts that share an output leave both spectra."""
+    torch = torch_cuda
+    n, k, S = 1 << 16, 64, 70
+    print(f"case dense parted n={n} k={k} S={S}", flush=True)
+    xs = [torch.from_numpy(signal_np(n, k, seed=300 + i, snr_db=30.0)[0]).cuda() for i in range(S)]
+    plan = _gpu_plan(2, n, k, "fp32_refine")
+    fr, va = plan.make_sparse_outputs(S)
+    counts = plan.execute_many_sparse(xs, fr, va)
+    want = torch.zeros((S, n), dtype=torch.complex128, device="cuda")
+    for i in range(S):
+        want[i, fr[i, :int(counts[i])].long()] = va[i, :int(counts[i])]
+    outs = [torch.full((n,), 7 + 7j, dtype=torch.complex128, device="cuda") for _ in range(S)]
+    for graphs in (False, True, True):
+        plan.enable_graphs(graphs)
+        plan.seed(17, 4242)
+        for o in outs:
+            o.fill_(5 - 3j)
+        plan.execute_many_device(xs, outs)
+        for i in range(S):
+            assert torch.equal(outs[i], want[i]), (graphs, i)
+    plan.enable_graphs(False)
+    first, last = 1, S - 2
+    shared = list(outs)
+    shared[last] = shared[first]
+    plan.seed(17, 4242)
+    plan.execute_many_device(xs, shared)
+    only = (want[first] != 0) & (want[last] == 0)
+    other = (want[first] == 0) & (want[last] != 0)
+    none = (want[first] == 0) & (want[last] == 0)
+    got = shared[first]
+    assert only.any() and other.any()
+    assert torch.equal(got[only], want[first][only])
+    assert torch.equal(got[other], want[last][other])
+    assert not got[none].any()
+    for i in range(S):
+        if i not in (first, last):
+            assert torch.equal(outs[i], want[i]), i

@@ -115,6 +115,15 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
         ins[s] = dst;
       }
     }
+    // on an error from here on the chunk's device outputs read as zero too
+    // (best effort; the call's error stays)
+    auto fail_chunk = [&]() {
+      const std::string why = last_error();
+      for (int s = 0; s < S; s++)
+        if (de[s]) (void)k::zero_dense(de[s], n, st);
+      set_error(why);
+      return fail(c0);
+    };
     // outputs
     int nws = 0;
     for (int s = 0; s < S; s++) {
@@ -122,7 +131,7 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
         complex_t *o = dense[c0 + s];
         if (!o) {
           set_error("null output signal");
-          return fail(c0);
+          return fail_chunk();
         }
         if (kinds.is_device(o)) {
           de[s] = reinterpret_cast<double2 *>(o);
@@ -147,7 +156,7 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
     if (nws) {
       if (!P->ws->out_freq.ensure((size_t)nws * cap * 4) ||
           !P->ws->out_val.ensure((size_t)nws * cap * 16))
-        return fail(c0);
+        return fail_chunk();
       int q = 0;
       for (int s = 0; s < S; s++) {
         if (!via_ws[s]) continue;
@@ -174,14 +183,7 @@ int run(Plan *P, int num, const complex_t *const *in, complex_t *const *dense,
     io.cap = cap;
     io.counts = counts.data();
     const int rc = exec_batch(P, io);
-    if (rc < 0) {
-      // (what follows is best effort; the call's error stays)
-      const std::string why = last_error();
-      for (int s = 0; s < S; s++)
-        if (de[s]) (void)k::zero_dense(de[s], n, st);
-      set_error(why);
-      return fail(c0);
-    }
+    if (rc < 0) return fail_chunk();
     partial |= rc > 0;
     // results that went through the plan's buffers
     for (int s = 0; s < S; s++) {

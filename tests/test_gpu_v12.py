@@ -717,3 +717,24 @@ def test_dense_outputs_of_a_parted_batch(torch_cuda):
     for i in range(S):
         if i not in (first, last):
             assert torch.equal(outs[i], want[i]), i
+
+
+@pytest.mark.parametrize("version", [1, 2])
+def test_refused_dense_call_clears_device_outputs(torch_cuda, version):
+    """A batch refused for a null output leaves the device outputs before it
+    cleared, as the reference's zero fill comes before anything else."""
+    torch = torch_cuda
+    n, k = 1 << 14, 50
+    print(f"case refused dense call v{version}", flush=True)
+
+    class Null:
+        def data_ptr(self):
+            return 0
+
+    plan = _gpu_plan(version, n, k)
+    xs = [torch.from_numpy(signal_np(n, k, seed=5 + i)[0]).cuda() for i in range(2)]
+    out = torch.full((n,), 3 + 4j, dtype=torch.complex128, device="cuda")
+    with pytest.raises(sfft_amd.SfftError, match="null output"):
+        plan.execute_many_device(xs, [out, Null()])
+    torch.cuda.synchronize()
+    assert not out.any()

@@ -515,10 +515,12 @@ void free_plan(Plan *P)
   }
   for (const auto &g : P->graphs) (void)hipGraphExecDestroy(g.exec);
   P->own_ws.release();
-  if (P->ev_made) {
-    for (hipEvent_t e : P->ev) (void)hipEventDestroy(e);
-    for (hipEvent_t e : P->ev_comb) (void)hipEventDestroy(e);
-  }
+  // (v3 plans make no comb events; destroying a null one leaves an error
+  // that the next launch check would report)
+  for (hipEvent_t e : P->ev)
+    if (e) (void)hipEventDestroy(e);
+  for (hipEvent_t e : P->ev_comb)
+    if (e) (void)hipEventDestroy(e);
   if (P->ev_fork) (void)hipEventDestroy(P->ev_fork);
   if (P->ev_join) (void)hipEventDestroy(P->ev_join);
   for (hipEvent_t e : P->ev_part)

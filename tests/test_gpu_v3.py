@@ -401,3 +401,24 @@ def test_v3_few_pairs_equal_serial(torch_cuda, n, k):
         c = int(ca[i])
         assert torch.equal(fa[i, :c], fb[i, :c])
         assert torch.equal(va[i, :c], vb[i, :c])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32_refine"])
+def test_v3_stage_timing(torch_cuda, precision):
+    """A timed v3 plan reports its stage, gives the untimed results, and
+    leaves no error behind when it is freed: the next plan is made and
+    runs."""
+    n, k = 1 << 16, 50
+    print(f"case v3 timing {precision}", flush=True)
+    x, f, v = signal_np(n, k, seed=5050)
+
+    def run(timed):
+        plan = sfft_amd.sfft(n, k, 3, precision=precision, seed=(17, 4242))
+        plan.enable_timing(timed)
+        res = plan.execute_sparse_host(x)
+        return res, plan.stage_times()["v3"]
+
+    a, (ms, launches) = run(True)
+    b, untimed = run(False)
+    assert ms > 0 and launches > 0 and untimed == (0, 0)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])

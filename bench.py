@@ -203,7 +203,8 @@ def main():
         "dtype": "fp32+fp64", "data": "synthetic",
         "eager": {"value": tps32_eager, "unit": "transforms/s",
                   "ms_per_step": S / tps32_eager * 1e3,
-                  "form": "the same batch launched eagerly (stage events on)"},
+                  "form": "the same batch launched eagerly with stage events on, which runs "
+                          "it in one part with the comb in its own launch"},
         "config": {"workload": "sFFT v2 batched exec_many_sparse replayed from a HIP graph, "
                                "FP32 buckets + FP64 estimation, %d signals, n=2^%d, k=%d, "
                                "SNR %g dB" % (S, int(np.log2(n)), k, args.snr),

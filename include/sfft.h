@@ -246,7 +246,12 @@ int sfft_plan_enable_timing(sfft_plan *plan, int enabled);
 /* Totals since timing was enabled: for stage s (0 comb, 1 fold (gather and
  * bucket sums; includes the bucket FFTs when they are fused into it),
  * 2 bucket FFTs, 3 selection+votes, 4 estimation, 5 v3) ms[s] = summed
- * milliseconds and launches[s] = kernel launches timed.  Arrays of 6. */
+ * milliseconds and launches[s] = kernel launches timed.  Arrays of 6.
+ * Timed v1/v2 execs run each stage as whole-batch launches of its own, so
+ * their schedule is not that of untimed ones: the v2 comb (with the table
+ * the estimation reads behind it) has its own launches beside the fold
+ * instead of workgroups in the fold's launch, large v2 FP32 batches run
+ * unparted, and graphs are not replayed.  Results are the same. */
 int sfft_plan_stage_times(const sfft_plan *plan, double *ms6,
                           int64_t *launches6);
 

@@ -805,10 +805,11 @@ int exec_multi_v3(Plan *const *plans, BatchIO *ios, int G, hipStream_t st, Works
     timer->ev_made = true;
   }
   if (timing) (void)hipEventRecord(timer->ev[0], st);
-  if (k::v3_multi(groups.data(), G, reinterpret_cast<k::V3Launch *>(sg.d),
+  const int launches =
+      k::v3_multi(groups.data(), G, reinterpret_cast<k::V3Launch *>(sg.d),
                   reinterpret_cast<int2 *>(sg.d + desc_bytes), (int)blocks.size(),
-                  reinterpret_cast<int *>(sg.d + desc_bytes + blk_bytes), st) != 0)
-    return -1;
+                  reinterpret_cast<int *>(sg.d + desc_bytes + blk_bytes), st);
+  if (launches < 0) return -1;
   if (timing) (void)hipEventRecord(timer->ev[1], st);
   HIP_OK(hipMemcpyAsync(sg.h + up_total, sg.d + up_total, dn, hipMemcpyDeviceToHost, st));
   HIP_OK(hipStreamSynchronize(st));
@@ -816,7 +817,7 @@ int exec_multi_v3(Plan *const *plans, BatchIO *ios, int G, hipStream_t st, Works
     float ms = 0;
     if (hipEventElapsedTime(&ms, timer->ev[0], timer->ev[1]) == hipSuccess) {
       timer->stage_ms[5] += ms;
-      timer->stage_launches[5] += 1;
+      timer->stage_launches[5] += launches;
     }
   }
   int rc = 0;  // 1: some map overflowed (every result written)
@@ -1112,7 +1113,7 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
       if (two_streams) {
         HIP_OK(hipEventRecord(P->ev_fork, st));
         HIP_OK(hipStreamWaitEvent(st2, P->ev_fork, 0));
-        if (k::comb(a, st2) != 0 || k::rows_table(a, st2) != 0) return -1;
+        if (k::comb(a, st2) < 0 || k::rows_table(a, st2) < 0) return -1;
         HIP_OK(hipEventRecord(P->ev_join, st2));
         HIP_OK(hipStreamWaitEvent(st3, P->ev_join, 0));
       }
@@ -1133,30 +1134,34 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
     // the fold is enqueued before the comb: for a single signal the host's
     // launch calls are on the latency path, and the fold branch is longer
     if ((launches[1] = k::fold_fft(a, st, 0)) < 0) return -1;
+    // the comb, and the estimation's table of the alias-row layout behind it
+    auto run_comb = [&](hipStream_t on) -> int {
+      const int c = k::comb(a, on), t = c < 0 ? -1 : k::rows_table(a, on);
+      return t < 0 ? -1 : c + t;
+    };
     if (p.comb && !two_streams && !a.comb_fused) {
-      if (k::comb(a, st) != 0 || k::rows_table(a, st) != 0) return -1;
-      launches[0] = cl > 1 ? 2 : 1;
+      if ((launches[0] = run_comb(st)) < 0) return -1;
     } else if (two_streams) {
       hipStream_t st2 = P->stream2;
       HIP_OK(hipStreamWaitEvent(st2, P->ev_fork, 0));
       if (timed) (void)hipEventRecord(P->ev_comb[0], st2);
-      if (k::comb(a, st2) != 0) return -1;
+      if ((launches[0] = run_comb(st2)) < 0) return -1;
       if (timed) (void)hipEventRecord(P->ev_comb[1], st2);
-      if (k::rows_table(a, st2) != 0) return -1;
       HIP_OK(hipEventRecord(P->ev_join, st2));
-      launches[0] = cl > 1 ? 2 : 1;
     }
     mark(2);
     if ((launches[2] = k::fold_fft(a, st, 1)) < 0) return -1;
     mark(3);
-    if (!p.comb && k::select_vote_v1(a, st) != 0) return -1;
-    launches[3] = p.comb ? 0 : 3;
+    if (!p.comb && (launches[3] = k::select_vote_v1(a, st)) < 0) return -1;
     if (two_streams) HIP_OK(hipStreamWaitEvent(st, P->ev_join, 0));
     mark(4);
     if (k::estimate(a, st) != 0) return -1;
     launches[4] = 1;
-    if (dbg_votes && k::comb_vote_keys(a, P->ws->votes.as<int64_t>(), 2 * cap, st) != 0)
-      return -1;
+    if (dbg_votes) {
+      const int v = k::comb_vote_keys(a, P->ws->votes.as<int64_t>(), 2 * cap, st);
+      if (v < 0) return -1;
+      launches[4] += v;
+    }
     mark(5);
     return deliver_counts();
   };

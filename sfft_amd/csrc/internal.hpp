@@ -441,7 +441,7 @@ struct V3Launch {
 };
 // G groups in one launch; d_groups / d_blocks: the descriptors and the
 // nblocks (group, signal) pairs, d_claims 4 nblocks zeroed ints, already on
-// the device (enqueued on st).
+// the device (enqueued on st).  Returns launches or -1.
 int v3_multi(const V3Launch *h_groups, int G, const V3Launch *d_groups, const int2 *d_blocks,
              int nblocks, int *d_claims, hipStream_t st);
 
@@ -458,6 +458,7 @@ int batch_fft32(float2 *data, float2 *tmp, int N, int64_t nb_outer, int nb_inner
 // Forward radix-2 DIT FFTs of any power-of-two size with the plan's twiddle
 // table, bit-identical to the in-LDS form; tmp (same layout as data) is
 // needed when N exceeds kMaxLdsFft64 (FP64) / 2*kMaxLdsFft64 (FP32).
+// Returns launches or -1.
 int radix2_fft64(double2 *data, double2 *tmp, int N, int64_t nb_outer, int nb_inner, int64_t so,
                  int64_t si, const double2 *tw, int tw_nmax, hipStream_t st);
 int radix2_fft32(float2 *data, float2 *tmp, int N, int64_t nb_outer, int nb_inner, int64_t so,
@@ -475,6 +476,7 @@ constexpr size_t kNoAllocScratch = (size_t)32 << 20;
 int noalloc_setup();
 void *noalloc_scratch(int dev);
 
+// The functions below that enqueue return their launches, or -1.
 int comb(const V12Launch &a, hipStream_t st);
 // Whether the fold's launch can run the combs too (V12Launch::comb_fused).
 bool fuse_comb(const V12Launch &a);
@@ -482,7 +484,7 @@ bool fuse_comb(const V12Launch &a);
 // FFTs' launch writes them).
 int rows_table(const V12Launch &a, hipStream_t st);
 // part 0: the fold (fused with the bucket FFTs when fold_mode == 0);
-// part 1: the bucket FFTs (nothing when fused).  Returns launches or -1.
+// part 1: the bucket FFTs (nothing when fused).
 int fold_fft(const V12Launch &a, hipStream_t st, int part);
 int select_vote_v1(const V12Launch &a, hipStream_t st);
 // Diagnostic of v2 plans in FP64 with buckets in natural order: the
@@ -490,6 +492,7 @@ int select_vote_v1(const V12Launch &a, hipStream_t st);
 // pair (append key, frequency) of the reference's comb votes, key -1 for a
 // frequency never appended; keys holds S x stride int64.
 int comb_vote_keys(const V12Launch &a, int64_t *keys, int64_t stride, hipStream_t st);
+// The estimation, one launch.  Returns 0 or -1 (so do those below).
 int estimate(const V12Launch &a, hipStream_t st);
 int zero_dense(double2 *out, int64_t n, hipStream_t st);
 // total values of uniform noise in [-1, 1)^2 (synthetic tuning input)

@@ -266,7 +266,7 @@ int radix2(T2 *data, T2 *tmp, int N, int C, int64_t nb_outer, int nb_inner, int6
     if (nb >= (1LL << 31)) return -1;
     hipLaunchKernelGGL(k_lds_fft_batch<T2>, dim3((unsigned)nb), dim3(fft_threads(N)), lds, st, data,
                        logN, nb_inner, so, si, tw, tw_nmax / N);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    return hipGetLastError() == hipSuccess ? 1 : -1;
   }
   logC = run_log(logN, logC, nb);
   const size_t run_lds = sizeof(T2) << logC, col_lds = (sizeof(T2) * kCols) << (logN - logC);
@@ -277,7 +277,7 @@ int radix2(T2 *data, T2 *tmp, int N, int C, int64_t nb_outer, int nb_inner, int6
                      st, data, tmp, logN, logC, nb_inner, so, si, tw, tw_nmax);
   hipLaunchKernelGGL((k_r2_cols<T2, false>), dim3((unsigned)(nb << (logC - 4))), dim3(kBlock),
                      col_lds, st, tmp, data, nullptr, logN, logC, nb_inner, so, si, tw, tw_nmax);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  return hipGetLastError() == hipSuccess ? 2 : -1;
 }
 
 template <typename T2>

@@ -1650,7 +1650,7 @@ void *noalloc_scratch(int dev)
 
 // The a.num largest of each of `rows` rows of `len` entries (powers at mag,
 // null: the v1 loops' |xs64|^2) into out, a.num per row; lists: 2 len ints of
-// scratch per row.
+// scratch per row.  Returns launches or -1.
 static int top_levels(const V12Launch &a, hipStream_t st, const double *mag, int len, int rows,
                       int *lists, int *out, bool comb_last)
 {
@@ -1664,7 +1664,7 @@ static int top_levels(const V12Launch &a, hipStream_t st, const double *mag, int
     set_error("selection of more than 4096 entries above the LDS size");
     return -1;
   }
-  while (true) {
+  for (int launches = 1;; launches++) {
     v.list_len = len;
     const bool last = len <= kTopLast;
     // every level at least halves the list: num is at most half a chunk
@@ -1679,7 +1679,7 @@ static int top_levels(const V12Launch &a, hipStream_t st, const double *mag, int
     hipLaunchKernelGGL(k_top_level, dim3((unsigned)(rows * v.chunks)), dim3(kTopThreads), lds, st,
                        a, v);
     if (launched("top_level") != 0) return -1;
-    if (last) return 0;
+    if (last) return launches;
     v.list = next;
     std::swap(next, other);
     len = left;
@@ -1693,6 +1693,7 @@ static int comb_merge(const V12Launch &a, hipStream_t st);
 
 int comb(const V12Launch &a, hipStream_t st)
 {
+  int launches = 1;
   if (a.W <= kMaxLdsComb) {
     const size_t lds = (size_t)a.W * sizeof(double2);
     if (a.S * a.comb_loops < kFewCombs) {
@@ -1710,11 +1711,13 @@ int comb(const V12Launch &a, hipStream_t st)
       return -1;
     }
     int *lists = reinterpret_cast<int *>(a.comb_buf);  // the transforms are done
-    if (top_levels(a, st, a.mag_buf, a.W, a.S * a.comb_loops, lists, a.approved,
-                   a.comb_loops == 1) != 0)
-      return -1;
+    const int levels = top_levels(a, st, a.mag_buf, a.W, a.S * a.comb_loops, lists, a.approved,
+                                  a.comb_loops == 1);
+    if (levels < 0) return -1;
+    launches = 2 + levels;
   }
-  return a.comb_loops > 1 ? comb_merge(a, st) : 0;
+  if (a.comb_loops == 1) return launches;
+  return comb_merge(a, st) == 0 ? launches + 1 : -1;
 }
 
 size_t rows_entry_bytes(bool fp32) { return fp32 ? sizeof(RowEntry32) : sizeof(RowEntry64); }
@@ -1730,7 +1733,7 @@ int rows_table(const V12Launch &a, hipStream_t st)
   const dim3 grid((unsigned)((rows_entries(a) + kBlock - 1) / kBlock));
   if (a.fp32) hipLaunchKernelGGL(k_rows_table<true>, grid, dim3(kBlock), 0, st, a);
   else hipLaunchKernelGGL(k_rows_table<false>, grid, dim3(kBlock), 0, st, a);
-  return launched("rows_table");
+  return launched("rows_table") == 0 ? 1 : -1;
 }
 
 // The part of loops [l0, l0 + nl) with `res` residues per workgroup and its
@@ -1851,8 +1854,8 @@ static int fold_sorted(const V12Launch &a, hipStream_t st, int from, int n64)
   allow_lds(k_fold_sorted, lds);
   hipLaunchKernelGGL(k_fold_sorted, dim3((unsigned)blocks), dim3(kFoldThreads), lds, st, a, f);
   if (launched("fold_sorted") != 0) return -1;
-  if (f.combs && a.comb_loops > 1 && comb_merge(a, st) != 0) return -1;
-  return 1;
+  if (!f.combs || a.comb_loops == 1) return 1;
+  return comb_merge(a, st) == 0 ? 2 : -1;
 }
 
 // Whether the bucket FFTs of a v1 batch select the top buckets too.
@@ -1941,14 +1944,15 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
                                       a.S, l1 - l0, a.xs, B, a.tw64, a.tw_nmax, st)
                        : radix2_fft32(a.xs32 + off, a.tmp32 ? a.tmp32 + off : nullptr, B,
                                       a.S, l1 - l0, a.xs, B, a.tw32, a.tw_nmax, st);
-    if (rc != 0) return launch_failed("bucket FFT");
-    launches++;
+    if (rc < 0) return launch_failed("bucket FFT");
+    launches += rc;
   }
   return launches;
 }
 
 // The top buckets of every location loop: in LDS up to its size, above it
-// in levels; more picks than a level takes, over the HBM array.
+// in levels; more picks than a level takes, over the HBM array.  Returns
+// launches or -1.
 static int select_loops(const V12Launch &a, hipStream_t st)
 {
   if (a.B_loc <= kMaxLdsSelect) {
@@ -1960,30 +1964,32 @@ static int select_loops(const V12Launch &a, hipStream_t st)
   } else {
     hipLaunchKernelGGL(k_select<true>, dim3(a.S * a.Lloc), dim3(kBlock), 0, st, a);
   }
-  return launched("select");
+  return launched("select") == 0 ? 1 : -1;
 }
 
 int select_vote_v1(const V12Launch &a, hipStream_t st)
 {
-  if (!v1_fft_select(a) && select_loops(a, st) != 0) return -1;
+  const int selects = v1_fft_select(a) ? 0 : select_loops(a, st);
+  if (selects < 0) return -1;
   const size_t lb = (size_t)a.Lloc * ((a.B_loc + 31) / 32) * 4;
   const int chunks = vote_chunks(a.n, a.B_loc, a.num, a.Lloc, a.thr);
   const dim3 grid((unsigned)((int64_t)a.S * chunks));
   hipLaunchKernelGGL(k_vote_count, grid, dim3(kBlock), lb, st, a, chunks);
   if (launched("vote_count") != 0) return -1;
   hipLaunchKernelGGL(k_vote_write, grid, dim3(kBlock), lb, st, a, chunks);
-  return launched("vote_write");
+  return launched("vote_write") == 0 ? selects + 2 : -1;
 }
 
 int comb_vote_keys(const V12Launch &a, int64_t *keys, int64_t stride, hipStream_t st)
 {
-  if (select_loops(a, st) != 0) return -1;
+  const int selects = select_loops(a, st);
+  if (selects < 0) return -1;
   const int64_t chunks = (a.est_cap + kBlock - 1) / kBlock;
   const size_t lb = (size_t)a.Lloc * ((a.B_loc + 31) / 32) * 4;
   allow_lds(k_comb_vote_keys, lb);
   hipLaunchKernelGGL(k_comb_vote_keys, dim3((unsigned)((int64_t)a.S * chunks)), dim3(kBlock), lb,
                      st, a, chunks, keys, stride);
-  return launched("comb_vote_keys");
+  return launched("comb_vote_keys") == 0 ? selects + 1 : -1;
 }
 
 // Blocks that keep every CU busy with several wavefronts.

@@ -2128,20 +2128,23 @@ __global__ void k_v3_mansour_gather(V3Launch a)
   a.ms_pre[t] = a.x[s][(off + (unsigned)i * sigma) & ((unsigned)a.n - 1)];
 }
 
-// Mansour pre-pass of one plan group whose W exceeds the LDS size.
+// Mansour pre-pass of one plan group whose W exceeds the LDS size.  Returns
+// launches or -1.
 static int mansour_prepass(const V3Launch &a, hipStream_t st)
 {
   if (!a.ms_pre) return 0;
   const int64_t total = (int64_t)a.S * a.ms_loops * a.W;
   hipLaunchKernelGGL(k_v3_mansour_gather, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
                      st, a);
-  if (hipGetLastError() != hipSuccess ||
-      radix2_fft64(a.ms_pre, a.ms_tmp, a.W, (int64_t)a.S * a.ms_loops, 1, a.W, a.W, a.tw64,
-                   a.tw_nmax, st) != 0) {
+  const int rc = hipGetLastError() != hipSuccess
+                     ? -1
+                     : radix2_fft64(a.ms_pre, a.ms_tmp, a.W, (int64_t)a.S * a.ms_loops, 1, a.W,
+                                    a.W, a.tw64, a.tw_nmax, st);
+  if (rc < 0) {
     set_error("v3: Mansour pre-pass launch failed");
     return -1;
   }
-  return 0;
+  return 1 + rc;
 }
 
 static void allow_v3_lds(const void *kernel, size_t bytes)
@@ -2153,8 +2156,11 @@ int v3_multi(const V3Launch *h_groups, int G, const V3Launch *d_groups, const in
              int nblocks, int *d_claims, hipStream_t st)
 {
   size_t lds = 0;
+  int launches = 1;
   for (int g = 0; g < G; g++) {
-    if (mansour_prepass(h_groups[g], st) != 0) return -1;
+    const int pre = mansour_prepass(h_groups[g], st);
+    if (pre < 0) return -1;
+    launches += pre;
     lds = std::max(lds, h_groups[g].lds_bytes);
   }
   bool refine = false;
@@ -2185,13 +2191,14 @@ int v3_multi(const V3Launch *h_groups, int G, const V3Launch *d_groups, const in
     allow_v3_lds(reinterpret_cast<const void *>(k_v3_refine_write), lds);
     hipLaunchKernelGGL(k_v3_refine_write, dim3(nblocks), dim3(kV3Block), lds, st, d_groups,
                        d_blocks);
+    launches += 4;
     e = hipGetLastError();
     if (e != hipSuccess) {
       set_error(std::string("v3 refine: ") + hipGetErrorString(e));
       return -1;
     }
   }
-  return 0;
+  return launches;
 }
 
 }  // namespace k

@@ -738,3 +738,27 @@ def test_refused_dense_call_clears_device_outputs(torch_cuda, version):
         plan.execute_many_device(xs, [out, Null()])
     torch.cuda.synchronize()
     assert not out.any()
+
+
+@pytest.mark.parametrize("version,n,k,precision,mode,launches", [
+    # comb, fold, bucket FFTs, selection + votes, estimate, v3
+    (1, 1 << 18, 100, "fp64", 1, (0, 1, 1, 2, 1, 0)),         # the FFTs select too
+    (1, 1 << 18, 100, "fp64", 0, (0, 1, 0, 3, 1, 0)),         # FFTs in the fold, a selection
+    (2, 1 << 18, 64, "fp32_refine", 1, (2, 1, 1, 0, 1, 0)),   # comb and alias-row table
+    (2, 1 << 16, 50, "fp64", 1, (2, 1, 2, 0, 1, 0)),          # comb and merge; two bucket counts
+    (2, 1 << 20, 50, "fp32_refine", 1, (5, 1, 1, 0, 1, 0)),   # runs, columns, level, merge, table
+    (3, 1 << 16, 50, "fp64", 1, (0, 0, 0, 0, 0, 1)),
+    (3, 1 << 16, 50, "fp32_refine", 1, (0, 0, 0, 0, 0, 5)),   # and the four refine kernels
+])
+def test_stage_launch_counts(torch_cuda, version, n, k, precision, mode, launches):
+    """Stage timing counts the kernels each stage launches."""
+    print(f"case stage launches v{version} n={n} k={k} {precision} mode={mode}", flush=True)
+    x, f, v = signal_np(n, k, seed=4200 + k)
+    plan = _gpu_plan(version, n, k, precision)
+    plan.set_schedule(mode, 0)
+    plan.enable_timing(True)
+    for _ in range(2):
+        plan.execute_sparse_host(x)
+    st = plan.stage_times()
+    assert tuple(int(st[s][1]) for s in plan.STAGES) == tuple(2 * c for c in launches), st
+    assert all((st[s][0] > 0) == (c > 0) for s, c in zip(plan.STAGES, launches)), st

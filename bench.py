@@ -52,7 +52,7 @@ def parse():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-serve", action="store_true", help="skip the serving-loop run")
     ap.add_argument("--schedule", default=None,
-                    help="fold schedule MODE,BLOCKS instead of autotuning (profiling runs)")
+                    help="fold schedule MODE instead of autotuning (profiling runs)")
     ap.add_argument("--no-configs", action="store_true",
                     help="skip the v1 / v2 single-signal and batched v3 configurations")
     ap.add_argument("--serve-requests", type=int, default=160)
@@ -212,7 +212,7 @@ def main():
                    "params": dict(zip(["B_loc", "B_est", "B_thresh", "W_comb",
                                        "comb_loops", "loc_loops", "est_loops",
                                        "thr_loops", "w_loc", "w_est"], p32.params())),
-                   "fold_schedule": {"mode": schedule32[0], "resident_blocks": schedule32[1]}},
+                   "fold_schedule": {"mode": schedule32[0]}},
     }
 
     # ---------------------------------------------------------- roofline

@@ -165,9 +165,10 @@ int sfft_plan_set_precision(sfft_plan *plan, sfft_precision precision);
  * fold that walks the taps of all loops in address order, then the bucket
  * FFTs, which for v2 store the buckets by
  * alias row so that estimation reads them contiguously; 2: as 1 with the
- * buckets in natural order.  stream_blocks is accepted and reported back;
- * the folds size their own grids.  Schedules never change results.
- * Returns 0 or -1. */
+ * buckets in natural order.  Schedules never change results.  stream_blocks
+ * (0 .. 2^20) has no effect, the folds size their own grids; it stays for
+ * callers of the earlier streamed fold and is reported back, also after
+ * sfft_plan_autotune, which chooses fold_mode alone.  Returns 0 or -1. */
 int sfft_plan_set_schedule(sfft_plan *plan, int fold_mode, int stream_blocks);
 int sfft_plan_get_schedule(const sfft_plan *plan, int *fold_mode, int *stream_blocks);
 

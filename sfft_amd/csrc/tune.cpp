@@ -3,9 +3,9 @@
 // The schedules differ only in how the fold is mapped onto the GPU: the
 // fused kernel (one workgroup per (signal, loop) folding into LDS and
 // transforming there) or the sorted fold followed by the bucket-FFT batches.
-// Every bucket is summed in the same tap order in all of them, so the choice never changes a bit of
-// the result; B, the loop counts and the filters are the reference's and are
-// not tuned.  Candidates are timed on synthetic noise signals with a private
+// Every bucket is summed in the same tap order in all of them, so the choice
+// never changes a bit of the result; B, the loop counts and the filters are
+// the reference's and are not tuned.  Candidates are timed on synthetic noise signals with a private
 // RNG stream, so tuning does not advance the plan's own draws.
 #include <algorithm>
 #include <chrono>
@@ -29,7 +29,7 @@ struct TuneKey {
 };
 
 std::mutex g_tune_mu;
-std::map<TuneKey, std::pair<int, int>> g_tuned;  // key -> (fold_mode, stream_blocks)
+std::map<TuneKey, int> g_tuned;  // key -> fold_mode
 
 TuneKey key_of(const Plan *P)
 {
@@ -42,10 +42,7 @@ void apply_tuned_schedule(Plan *P)
 {
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tuned.find(key_of(P));
-  if (it != g_tuned.end()) {
-    P->fold_mode = it->second.first;
-    P->stream_blocks = it->second.second;
-  }
+  if (it != g_tuned.end()) P->fold_mode = it->second;
 }
 
 int autotune_plan(Plan *P, int batch)
@@ -73,17 +70,16 @@ int autotune_plan(Plan *P, int batch)
   io.in = in.data();
   io.counts = counts.data();
 
-  std::vector<std::pair<int, int>> cand;
-  if (std::max(p.B_loc, p.B_est) <= kMaxLdsFft64) cand.push_back({0, 0});
-  cand.push_back({1, 0});
-  if (P->precision == SFFT_PRECISION_FP32_REFINE && p.comb) cand.push_back({2, 0});
-  const int mode0 = P->fold_mode, blocks0 = P->stream_blocks;
+  std::vector<int> cand;  // fold modes
+  if (std::max(p.B_loc, p.B_est) <= kMaxLdsFft64) cand.push_back(0);
+  cand.push_back(1);
+  if (P->precision == SFFT_PRECISION_FP32_REFINE && p.comb) cand.push_back(2);
+  const int mode0 = P->fold_mode;
   double best = 1e30;
-  std::pair<int, int> pick{mode0, blocks0};
-  for (const auto &c : cand) {
+  int pick = mode0;
+  for (int c : cand) {
     if (rc != 0) break;
-    P->fold_mode = c.first;
-    P->stream_blocks = c.second;
+    P->fold_mode = c;
     double t = 1e30;
     for (int rep = 0; rep < 3 && rc == 0; rep++) {  // first run warms up
       const auto t0 = std::chrono::steady_clock::now();
@@ -100,11 +96,9 @@ int autotune_plan(Plan *P, int batch)
   (void)hipFree(x);
   if (rc != 0) {
     P->fold_mode = mode0;
-    P->stream_blocks = blocks0;
     return -1;
   }
-  P->fold_mode = pick.first;
-  P->stream_blocks = pick.second;
+  P->fold_mode = pick;
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tuned[key_of(P)] = pick;
   return 0;

@@ -140,7 +140,8 @@ class sfft:
 
     def set_schedule(self, fold_mode, stream_blocks=0):
         """Fold schedule (0 fused, 1 sorted, 2 sorted with the buckets in
-        natural order); never changes results."""
+        natural order); never changes results.  stream_blocks is kept and
+        reported by schedule(), without effect."""
         if self._L.sfft_plan_set_schedule(self.sfft_plan, fold_mode, stream_blocks) != 0:
             raise SfftError(_lib.last_error())
 

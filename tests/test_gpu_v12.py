@@ -762,3 +762,13 @@ def test_stage_launch_counts(torch_cuda, version, n, k, precision, mode, launche
     st = plan.stage_times()
     assert tuple(int(st[s][1]) for s in plan.STAGES) == tuple(2 * c for c in launches), st
     assert all((st[s][0] > 0) == (c > 0) for s, c in zip(plan.STAGES, launches)), st
+
+
+def test_autotune_keeps_stream_blocks(torch_cuda):
+    """The autotuner chooses the fold mode; the caller's stream_blocks is
+    reported back as it was set."""
+    print("case autotune stream_blocks", flush=True)
+    plan = _gpu_plan(2, 1 << 16, 64, "fp32_refine")
+    plan.set_schedule(0, 96)
+    mode, blocks = plan.autotune(batch=2)
+    assert mode in (0, 1, 2) and blocks == 96

@@ -1695,7 +1695,7 @@ __device__ void write_result(const V3Launch &a, int s, const int *keys, const do
                              int M, int flags, double2 *lds)
 {
   constexpr int T = kV3Block, C = kResultBins / T;
-  __shared__ int s_scan[T / 64], s_most;
+  __shared__ int s_scan[16], s_most;
   if (threadIdx.x == 0) {
     a.count[s] = M;
     a.status[s] = flags;

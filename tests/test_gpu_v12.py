@@ -772,3 +772,43 @@ def test_autotune_keeps_stream_blocks(torch_cuda):
     plan.set_schedule(0, 96)
     mode, blocks = plan.autotune(batch=2)
     assert mode in (0, 1, 2) and blocks == 96
+
+
+@pytest.mark.parametrize("kind", ["noise", "zeros"])
+def test_selection_of_three_levels(torch_cuda, kind):
+    """n = 2^26, k = 2000 (v1): 4000 of 65,536 buckets a loop, whose levels
+    leave 32,000 and 16,000 candidates.  The located set is that of the votes
+    counted over every frequency, with each loop's selection taken from the
+    plan's own buckets by sorting (ties to the lower index)."""
+    torch = torch_cuda
+    n, k = 1 << 26, 2000
+    print(f"case three levels {kind}", flush=True)
+    plan = _gpu_plan(1, n, k)
+    B, _, num, W, _, Lloc, Lest, thr = plan.params()[:8]
+    assert (B, num) == (65536, 4000)
+    x = torch.zeros(n, dtype=torch.complex128, device="cuda")
+    if kind == "noise":
+        g = torch.Generator(device="cuda")
+        g.manual_seed(26)
+        x.real.normal_(generator=g)
+        x.imag.normal_(generator=g)
+    fr, va = plan.make_sparse_outputs(1)
+    count = int(plan.execute_many_sparse([x], fr, va)[0])
+    print("transformed", flush=True)
+    buckets = plan.debug_buckets(0)[:Lloc * B].reshape(Lloc, B)
+    a, ai, off = (np.zeros(Lloc + Lest, np.int32) for _ in range(3))
+    oracle.seed_glibc(17, 4242)
+    oracle.lib().or_v12_draw(n, Lloc + Lest, 0, W, *(q.ctypes.data for q in (a, ai, off)))
+    f = torch.arange(n, dtype=torch.int64, device="cuda")
+    score = torch.zeros(n, dtype=torch.int32, device="cuda")
+    for l in range(Lloc):
+        power = buckets[l].real * buckets[l].real + buckets[l].imag * buckets[l].imag
+        sel = np.zeros(B, np.int32)
+        sel[np.lexsort((np.arange(B), -power))[:num]] = 1
+        bucket = (((f * int(ai[l]) & (n - 1)) + n // B // 2) & (n - 1)) // (n // B)
+        score += torch.from_numpy(sel).cuda()[bucket]
+    want = torch.nonzero(score >= thr).flatten()
+    assert count == want.numel() > 0
+    assert torch.equal(torch.sort(fr[0, :count].long()).values, want)
+    del x, fr, va, f, score
+    torch.cuda.empty_cache()

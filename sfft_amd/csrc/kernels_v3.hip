@@ -89,8 +89,6 @@ struct Ctx {
   int *keys;
   double2 *vals;
   int *hidx;
-  int *cf;
-  double2 *cv;
   int *ef;
   double2 *ev;
   double2 *rem;
@@ -1463,8 +1461,6 @@ __device__ __forceinline__ void v3_signal(const V3Launch &a, const int s, int *c
   c.keys = a.map_keys + (int64_t)s * a.Mcap;
   c.vals = a.map_vals + (int64_t)s * a.Mcap;
   c.hidx = a.map_hidx + (int64_t)s * a.Hcap;
-  c.cf = a.cf + (int64_t)s * a.Fcap;
-  c.cv = a.cv + (int64_t)s * a.Fcap;
   c.ef = a.ef + (int64_t)s * a.Fcap;
   c.ev = a.ev + (int64_t)s * a.Fcap;
   c.rem = a.rem + (int64_t)s * a.Rcap * 14;

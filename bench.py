@@ -167,9 +167,9 @@ def main():
         schedule32 = p32.autotune(batch=min(S, 64))
     cap = p32.capacity
     fr32, va32 = p32.make_sparse_outputs(S)
-    # headline: the batch replayed from a captured HIP graph (uploads, comb
-    # beside the fold on a second stream, fold, bucket FFTs, estimation,
-    # count read-back); the first exec of the shape captures it
+    # headline: the batch replayed from a captured HIP graph (upload, fold
+    # with the combs in its launch, bucket FFTs, estimation); the first exec
+    # of the shape captures it
     p32.enable_graphs(True)
     for _ in range(args.warmup):
         p32.execute_many_sparse(x, fr32, va32)

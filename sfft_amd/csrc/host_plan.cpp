@@ -1100,8 +1100,8 @@ static int exec_batch_v12(Plan *P, BatchIO &io, V12Pending *pd)
     for (hipEvent_t &e : P->ev_part) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     HIP_OK(hipEventCreateWithFlags(&P->ev_est, hipEventDisableTiming));
   }
-  // The stream work of one batch: uploads, kernels, counts back.  The v2
-  // comb (its own gathers and FFTs) runs on stream2 beside the fold.
+  // The stream work of one batch: upload, kernels, counts.  A v2 comb that
+  // is not in the fold's launch runs on stream2 beside it.
   auto enqueue = [&](bool timed) -> int {
     auto mark = [&](int i) {
       if (timed) (void)hipEventRecord(P->ev[i], st);

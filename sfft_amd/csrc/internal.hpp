@@ -247,7 +247,7 @@ struct Plan {
   hipEvent_t ev[kStages + 1] = {};
   hipEvent_t ev_comb[2] = {};  // comb start / end on stream2 (timing)
   bool ev_made = false;
-  // The v2 comb runs on a second stream beside the fold and bucket FFTs;
+  // A v2 comb not in the fold's launch runs on a second stream beside it;
   // fork after the uploads, join before estimation.
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -347,7 +347,7 @@ struct V12Launch {
   int *num_comb;   // S
   int *J;          // S x Lloc x num
   int *hits;       // S x hits_cap
-  int *vote_cnt;   // v1: S x vote_chunks hit counts, then offsets
+  int *vote_cnt;   // v1: S x vote_chunks hit counts
   int64_t hits_cap;
   int64_t *count;  // S located counts
   int64_t *count_host;      // the same in pinned host memory, or null

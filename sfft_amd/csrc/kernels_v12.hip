@@ -1913,8 +1913,8 @@ int fold_fft(const V12Launch &a, hipStream_t st, int part)
     return launched("bucket_fft_v1") == 0 ? 1 : -1;
   }
   // the location and estimation loops as batches of one bucket count and
-  // precision: in LDS up to the LDS size, else radix-2 runs plus global
-  // passes; FP64 loops fused into their fold (schedule 0) are done
+  // precision: in LDS up to the LDS size, else radix-2 runs plus columns;
+  // FP64 loops fused into their fold (schedule 0) are done
   const int f0 = a.fold_mode == 0 ? n64 : 0;  // first loop still to transform
   int groups[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
   int ng = 0;
